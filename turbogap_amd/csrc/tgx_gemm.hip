@@ -202,74 +202,198 @@ __device__ __forceinline__ void epilogue(const VecT (&acc)[TI][TJ], int m0, int 
   }
 }
 
-// FP64 NT GEMM. M, N multiples of 128; K multiple of 16.
-// LDS holds both operands k-major ([k][row], row stride 144 doubles: the four
-// k rows an MFMA fragment read touches fall on disjoint bank halves), in two
-// stages: the global loads for stage s+1 are in flight during the MFMAs of
-// stage s and land in the other buffer, one barrier per stage. Threads 0-127
-// stage one row of A each, 128-255 one row of B (16 doubles, 128 contiguous
-// bytes), so a wavefront's LDS writes cover 64 consecutive rows.
-template <int EPI, bool ZINT>
-__global__ __launch_bounds__(256, 2) void k_gemm_f64(int K, const double* __restrict__ A, int lda,
-                                                     const double* __restrict__ B, int ldb, EpiArgs e) {
-  constexpr int BK = 16, LS = BM + 16;
-  __shared__ __align__(16) double As[2][BK * LS];
-  __shared__ __align__(16) double Bs[2][BK * LS];
-  __shared__ double sE[2 * BM];
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N < 16, "vmcnt immediate");
+  __builtin_amdgcn_s_waitcnt(0x3F70 | N);  // vmcnt(N); expcnt and lgkmcnt not waited on
+}
+
+// FP64 NT GEMM fed by direct global-to-LDS loads: workgroup tile (32 TI) x
+// (32 TJ), four wavefronts of (16 TI) x (16 TJ), BK = 16 in a two-slot ring. A
+// stage is 32 (TI + TJ) rows of 128 bytes (the A rows, then the B rows); the
+// eight 16-byte chunks of row r sit at chunk c ^ (r & 7), so that a 16-byte
+// fragment read spreads over all banks. One load instruction fills eight rows.
+// A lane's chunk holds two consecutive k, which go to two MFMAs: the k of both
+// operands are permuted alike, so the product is the same. Each half stage's
+// fragments are read into registers while the other half's MFMAs run, and the
+// one barrier a stage sits between the halves: without it, the two workgroups
+// of a CU reach their fragment waits and barriers together and the matrix
+// cores idle. Bound by the FP64 MFMA rate.
+// M a multiple of 32 TI, N of 32 TJ, K of 16.
+__host__ __device__ constexpr int f64_stage_bytes(int ti, int tj) { return 32 * (ti + tj) * 128; }
+__host__ __device__ constexpr int f64_lds_bytes(int ti, int tj) { return 2 * f64_stage_bytes(ti, tj) + 2 * 32 * ti * 8; }
+
+template <int TI, int TJ>
+__device__ __forceinline__ void f64_read(const unsigned char* sb, int aoff, int boff, int cpos, double2 (&a)[TI],
+                                         double2 (&b)[TJ]) {
+#pragma unroll
+  for (int i = 0; i < TI; ++i) a[i] = *reinterpret_cast<const double2*>(sb + aoff + i * 16 * 128 + cpos);
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) b[j] = *reinterpret_cast<const double2*>(sb + boff + j * 16 * 128 + cpos);
+}
+
+template <int TI, int TJ>
+__device__ __forceinline__ void f64_mfma(f64x4 (&acc)[TI][TJ], const double2 (&a)[TI], const double2 (&b)[TJ]) {
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].x, acc[i][j], 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b[j].y, acc[i][j], 0, 0, 0);
+}
+
+template <int EPI, bool ZINT, int TI, int TJ, int OCC>
+__global__ __launch_bounds__(256, OCC) void k_gemm_f64(int K, const double* __restrict__ A, int lda,
+                                                       const double* __restrict__ B, int ldb, EpiArgs e) {
+  constexpr int BK = 16, SB = f64_stage_bytes(TI, TJ);
+  constexpr int NBA = 4 * TI, P = TI + TJ;  // load blocks of eight rows: A's, and per wavefront
+  extern __shared__ __align__(16) unsigned char dsm[];
+  double* sE = reinterpret_cast<double*>(dsm + 2 * SB);
   int tm, tn;
   tile_of<TILE_GM>(tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * 32 * TI, n0 = tn * 32 * TJ;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w >> 1, wn = w & 1;
-  const int srow = tid & 127;
-  const bool isB = tid >= 128;
-  const double* G = isB ? B + (size_t)(n0 + srow) * ldb : A + (size_t)(m0 + srow) * lda;
-  f64x4 acc[4][4];
+  const int lrow = lane >> 3, lchunk = (lane & 7) ^ lrow;
+  const double* src[P];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (f64x4){0, 0, 0, 0};
-  double2 r0, r1, r2, r3, r4, r5, r6, r7;
-  auto gload = [&](int k) {
-    const double2* g = reinterpret_cast<const double2*>(G + k);
-    r0 = g[0]; r1 = g[1]; r2 = g[2]; r3 = g[3]; r4 = g[4]; r5 = g[5]; r6 = g[6]; r7 = g[7];
-  };
-  auto lstore = [&](int buf) {
-    double* d = (isB ? Bs[buf] : As[buf]) + srow;
-    d[0 * LS] = r0.x; d[1 * LS] = r0.y; d[2 * LS] = r1.x; d[3 * LS] = r1.y;
-    d[4 * LS] = r2.x; d[5 * LS] = r2.y; d[6 * LS] = r3.x; d[7 * LS] = r3.y;
-    d[8 * LS] = r4.x; d[9 * LS] = r4.y; d[10 * LS] = r5.x; d[11 * LS] = r5.y;
-    d[12 * LS] = r6.x; d[13 * LS] = r6.y; d[14 * LS] = r7.x; d[15 * LS] = r7.y;
-  };
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  const int n_stages = K / BK;
-  for (int st = 0; st < n_stages; ++st) {
-    const int buf = st & 1;
-    gload(min(st + 1, n_stages - 1) * BK);  // the last stage reloads itself: always in bounds
-    __builtin_amdgcn_sched_barrier(0);
-    const double* as = As[buf] + wm * 64 + (lane & 15);
-    const double* bs = Bs[buf] + wn * 64 + (lane & 15);
-#pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      const int kr = (ks * 4 + (lane >> 4)) * LS;
-      double a[4], b[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        a[t] = as[kr + t * 16];
-        b[t] = bs[kr + t * 16];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    lstore(buf ^ 1);
-    __syncthreads();
+  for (int j = 0; j < P; ++j) {
+    const int b = w + 4 * j;
+    src[j] = b < NBA ? A + (size_t)(m0 + 8 * b + lrow) * lda + 2 * lchunk
+                     : B + (size_t)(n0 + 8 * (b - NBA) + lrow) * ldb + 2 * lchunk;
   }
-  epilogue<EPI, double, double, f64x4, true, ZINT>(acc, m0, n0, tn, wm, wn, e, sE);
+  auto issue = [&](int st, int slot) {
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+      __builtin_amdgcn_global_load_lds(const_cast<double*>(src[j] + st * BK), dsm + slot * SB + (w + 4 * j) * 1024, 16,
+                                       0, 0);
+  };
+  const int li = lane & 15, lg = lane >> 4;
+  const int aoff = (wm * 16 * TI + li) * 128, boff = (32 * TI + wn * 16 * TJ + li) * 128;
+  const int c0 = (lg ^ (li & 7)) << 4, c1 = ((lg + 4) ^ (li & 7)) << 4;
+  f64x4 acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = (f64x4){0, 0, 0, 0};
+  const int n_stages = K / BK;
+  issue(0, 0);
+  wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  issue(min(1, n_stages - 1), 1);
+  double2 a0[TI], b0[TJ], a1[TI], b1[TJ];
+  f64_read<TI, TJ>(dsm, aoff, boff, c0, a0, b0);
+  for (int st = 0; st < n_stages; ++st) {
+    const int slot = st & 1;
+    f64_read<TI, TJ>(dsm + slot * SB, aoff, boff, c1, a1, b1);
+    __builtin_amdgcn_sched_barrier(0);
+    f64_mfma<TI, TJ>(acc, a0, b0);
+    __builtin_amdgcn_sched_barrier(0);
+    // this wavefront's part of stage st + 1 has landed and its reads of stage st are done
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(min(st + 2, n_stages - 1), slot);  // an in-bounds repeat past the end
+    f64_read<TI, TJ>(dsm + (slot ^ 1) * SB, aoff, boff, c0, a0, b0);
+    __builtin_amdgcn_sched_barrier(0);
+    f64_mfma<TI, TJ>(acc, a1, b1);
+  }
+  wait_vmcnt<0>();  // the loads issued past the last stage land before the LDS is released
+  __builtin_amdgcn_sched_barrier(0);
+  epilogue<EPI, double, double, f64x4, true, ZINT, TI, TJ, 16 * TI, 16 * TJ, 32 * TI>(acc, m0, n0, tn, wm, wn, e, sE);
+}
+
+// FP64 NT GEMM for few rows: workgroup tile 32 x (32 NC), NC x KS wavefronts of
+// 32 x 32 that each take a K / KS range straight from global memory (nothing is
+// shared, so nothing is staged), and the KS partials are added through LDS in
+// order. A handful of 128 x 128 tiles would each walk the whole K alone: the
+// reduction is what fills the chip there. M a multiple of 32, N of 32 NC, K of
+// 16 KS.
+template <int EPI, bool ZINT, int NC, int KS>
+__global__ __launch_bounds__(64 * NC * KS) void k_gemm_f64_few(int K, const double* __restrict__ A, int lda,
+                                                               const double* __restrict__ B, int ldb, EpiArgs e) {
+  extern __shared__ __align__(16) unsigned char dsm[];
+  double* part = reinterpret_cast<double*>(dsm);  // [KS][32][32 NC]
+  constexpr int W = 32 * NC;
+  int tm, tn;
+  tile_of<TILE_GM>(tm, tn);
+  const int m0 = tm * 32, n0 = tn * W;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wc = w % NC, wk = w / NC, kr = K / KS;
+  const int li = lane & 15, lg = lane >> 4;
+  const double* Ap = A + (size_t)(m0 + li) * lda + wk * kr + 2 * lg;
+  const double* Bp = B + (size_t)(n0 + 32 * wc + li) * ldb + wk * kr + 2 * lg;
+  const size_t a16 = (size_t)16 * lda, b16 = (size_t)16 * ldb;
+  f64x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = (f64x4){0, 0, 0, 0};
+  // DEPTH rounds of 16 k in flight: two waves per SIMD do not cover a load's latency
+  constexpr int DEPTH = 4;
+  double2 a[DEPTH][2][2], b[DEPTH][2][2];
+  const int rounds = kr / 16;
+  auto load = [&](int it, double2(&ra)[2][2], double2(&rb)[2][2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k = 16 * it + 8 * h;
+      ra[h][0] = *reinterpret_cast<const double2*>(Ap + k);
+      ra[h][1] = *reinterpret_cast<const double2*>(Ap + a16 + k);
+      rb[h][0] = *reinterpret_cast<const double2*>(Bp + k);
+      rb[h][1] = *reinterpret_cast<const double2*>(Bp + b16 + k);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < DEPTH; ++u) load(min(u, rounds - 1), a[u], b[u]);
+  for (int it = 0; it < rounds; it += DEPTH) {
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u) {
+      if (it + u < rounds) {
+        f64_mfma<2, 2>(acc, a[u][0], b[u][0]);
+        f64_mfma<2, 2>(acc, a[u][1], b[u][1]);
+      }
+      load(min(it + u + DEPTH, rounds - 1), a[u], b[u]);  // in bounds past the end
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        part[(wk * 32 + i * 16 + tile_row<true>(lane, r)) * W + 32 * wc + j * 16 + li] = acc[i][j][r];
+  __syncthreads();
+  // thread: row tid / TR, columns tid % TR + TR c
+  constexpr int TR = 2 * NC * KS, CP = W / TR;
+  static_assert(W % TR == 0 && TR <= 64, "columns per thread");
+  const int row = tid / TR, c0 = tid % TR;
+  double er = 0.0;
+#pragma unroll
+  for (int c = 0; c < CP; ++c) {
+    const int col = c0 + c * TR;
+    double v = part[row * W + col];
+#pragma unroll
+    for (int k = 1; k < KS; ++k) v += part[(k * 32 + row) * W + col];
+    double* o = reinterpret_cast<double*>(e.out) + (size_t)(m0 + row) * e.ldo + n0 + col;
+    if (EPI == EPI_GAP) {
+      const double al = e.alpha[n0 + col];
+      double kz, kzm1;
+      kpow<double, ZINT>(v, e.zeta, e.zeta_int, kz, kzm1);
+      *o = e.pref * kzm1 * al;
+      er += al * kz;
+    } else {
+      *o = e.pref * v;
+    }
+  }
+  if (EPI == EPI_GAP) {
+#pragma unroll
+    for (int x = 1; x < TR; x <<= 1) er += __shfl_xor(er, x);
+    if (c0 == 0) e.epart[(size_t)(m0 + row) * e.n_tiles + tn] = er;
+  }
 }
 
 // BF16 NT GEMM with FP32 accumulation. M, N multiples of 128; K multiple of 64.
@@ -499,12 +623,6 @@ constexpr int DROW = DK * 2;                // bytes per staged row
 __host__ __device__ constexpr int dma_stage_bytes(int tm) { return (tm + BN) * DROW; }
 __host__ __device__ constexpr int dma_lds_bytes(int tm, int ns) { return ns * dma_stage_bytes(tm) + 2 * tm * 8; }
 
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 16, "vmcnt immediate");
-  __builtin_amdgcn_s_waitcnt(0x3F70 | N);  // vmcnt(N); expcnt and lgkmcnt not waited on
-}
-
 // One stage's loads of a wavefront: its P blocks of 16 rows, block b of the
 // stage into bytes [1024 b, 1024 b + 1024) of the stage buffer.
 template <int P>
@@ -679,17 +797,51 @@ static int launch_bf16(tgx_ctx* ctx, const char* name, int M, int N, int K, int 
   return TGX_OK;
 }
 
-static int launch_f64(tgx_ctx* ctx, int epi, int M, int N, int K, const double* A, int lda, const double* B, int ldb,
-                      EpiArgs e, const char* name) {
-  TGX_REQUIRE(M % BM == 0 && N % BN == 0 && K % 16 == 0, "gemm_f64: unpadded shape %d x %d x %d", M, N, K);
-  dim3 grid(N / BN, M / BM);
-  if (epi == EPI_GAP && e.zeta_int >= 1)
-    TGX_LAUNCH(ctx, name, (k_gemm_f64<EPI_GAP, true>), grid, dim3(256), 0, K, A, lda, B, ldb, e);
-  else if (epi == EPI_GAP)
-    TGX_LAUNCH(ctx, name, (k_gemm_f64<EPI_GAP, false>), grid, dim3(256), 0, K, A, lda, B, ldb, e);
-  else
-    TGX_LAUNCH(ctx, name, (k_gemm_f64<EPI_STORE, true>), grid, dim3(256), 0, K, A, lda, B, ldb, e);
+template <int EPI, bool ZINT, int TI, int TJ, int OCC>
+static int launch_f64_tile(tgx_ctx* ctx, const char* name, int M, int N, int K, const double* A, int lda,
+                           const double* B, int ldb, EpiArgs e) {
+  TGX_LAUNCH(ctx, name, (k_gemm_f64<EPI, ZINT, TI, TJ, OCC>), dim3(N / (32 * TJ), M / (32 * TI)), dim3(256),
+             f64_lds_bytes(TI, TJ), K, A, lda, B, ldb, e);
   return TGX_OK;
+}
+
+template <int EPI, bool ZINT, int NC, int KS>
+static int launch_f64_few(tgx_ctx* ctx, const char* name, int M, int N, int K, const double* A, int lda,
+                          const double* B, int ldb, EpiArgs e) {
+  TGX_LAUNCH(ctx, name, (k_gemm_f64_few<EPI, ZINT, NC, KS>), dim3(N / (32 * NC), M / 32), dim3(64 * NC * KS),
+             sizeof(double) * 32 * 32 * NC * KS, K, A, lda, B, ldb, e);
+  return TGX_OK;
+}
+
+// FP64 NT GEMM launch. 128 x 128 tiles while they fill the 256 CUs twice over
+// (32,768 x 1,280 x 4,096: 5.2 ms, 66 TFLOP/s; the half-tall tile 5.8), smaller
+// ones below (2,048 x 1,280 x 4,096: 0.60 ms on 160 tiles of 128 x 128, 0.41 on
+// 64 x 64; 1,024 x 2,048 x 384: 0.073 -> 0.047 on 64 x 128), and the kernel that
+// splits K between the wavefronts when even those leave most CUs empty (256 x
+// 384 x 2,048: 0.28 ms on 128 x 128, 0.12 on 64 x 64, 0.04 split). The lines lie
+// where the two sides measured alike. The energy partials of the GAP epilogue
+// are per 128 columns whatever the tile, so their layout does not depend on the
+// rule. shared: another block's kernels run beside this one and take the CUs a
+// last round leaves idle, so that the wide tile pays earlier (two blocks of
+// 8,000 centres, FP64 adjoint step: 11.33 ms with 64 x 64 tiles, 11.08 with 128 x
+// 128, although alone the latter's 630 tiles take 2.06 ms against 1.39). Every
+// tile adds an element's products in the same order, so the results do not
+// depend on it.
+template <int EPI, bool ZINT>
+static int launch_f64(tgx_ctx* ctx, bool shared, int M, int N, int K, const double* A, int lda, const double* B,
+                      int ldb, EpiArgs e, const char* name) {
+  TGX_REQUIRE(M % BM == 0 && N % BN == 0 && K % BN == 0, "gemm_f64: unpadded shape %d x %d x %d", M, N, K);
+  const int64_t tiles = (int64_t)(M / BM) * (N / BN);
+  if constexpr (EPI == EPI_GAP) {
+    if (tiles >= 512) return launch_f64_tile<EPI, ZINT, 4, 4, 2>(ctx, name, M, N, K, A, lda, B, ldb, e);
+    if (tiles >= 96) return launch_f64_tile<EPI, ZINT, 2, 4, 3>(ctx, name, M, N, K, A, lda, B, ldb, e);
+    return launch_f64_few<EPI, ZINT, 4, 2>(ctx, name, M, N, K, A, lda, B, ldb, e);
+  } else {
+    if (tiles >= (shared ? 512 : 1024))
+      return launch_f64_tile<EPI, ZINT, 4, 4, 2>(ctx, name, M, N, K, A, lda, B, ldb, e);
+    if (tiles >= 48) return launch_f64_tile<EPI, ZINT, 2, 2, 4>(ctx, name, M, N, K, A, lda, B, ldb, e);
+    return launch_f64_few<EPI, ZINT, 1, 8>(ctx, name, M, N, K, A, lda, B, ldb, e);
+  }
 }
 
 int tgx_gap_contract_f64(tgx_ctx* ctx, const tgx_model_t* m, int ns, const double* q, double* kd, double* epart,
@@ -698,13 +850,17 @@ int tgx_gap_contract_f64(tgx_ctx* ctx, const tgx_model_t* m, int ns, const doubl
   const int Mp = (int)tgx_round_up(ns, BM);
   const int Sp = m->Spad, Dp = m->Dpad;
   const int n_tiles = Sp / BN;
+  const bool shared = m->stream && ctx->stream == m->stream;  // blocks run concurrently
   EpiArgs e = gap_epi(m);
   e.epart = epart;
   e.n_tiles = n_tiles;
   e.alpha = m->alpha.as<double>();
   e.out = kd;
   e.ldo = Sp;
-  TGX_TRY(launch_f64(ctx, EPI_GAP, Mp, Sp, Dp, q, Dp, m->Qs.as<double>(), Dp, e, "gemm_kernel_f64"));
+  if (e.zeta_int >= 1)
+    TGX_TRY((launch_f64<EPI_GAP, true>(ctx, shared, Mp, Sp, Dp, q, Dp, m->Qs.as<double>(), Dp, e, "gemm_kernel_f64")));
+  else
+    TGX_TRY((launch_f64<EPI_GAP, false>(ctx, shared, Mp, Sp, Dp, q, Dp, m->Qs.as<double>(), Dp, e, "gemm_kernel_f64")));
   TGX_LAUNCH(ctx, "energy_finalize", k_energy_finalize, dim3((ns + 255) / 256), dim3(256), 0, ns, epart, n_tiles,
              m->delta * m->delta, m->e0, e_site);
   if (!qss) return TGX_OK;
@@ -712,7 +868,7 @@ int tgx_gap_contract_f64(tgx_ctx* ctx, const tgx_model_t* m, int ns, const doubl
   s.pref = 1.0;
   s.out = qss;
   s.ldo = Dp;
-  return launch_f64(ctx, EPI_STORE, Mp, Dp, Sp, kd, Sp, m->QsT.as<double>(), Sp, s, "gemm_qss_f64");
+  return launch_f64<EPI_STORE, true>(ctx, shared, Mp, Dp, Sp, kd, Sp, m->QsT.as<double>(), Sp, s, "gemm_qss_f64");
 }
 
 int tgx_gap_contract(tgx_ctx* ctx, tgx_model_t* m, int path, bool do_forces) {
