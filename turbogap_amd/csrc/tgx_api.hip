@@ -9,7 +9,8 @@
 #include "tgx_util.h"
 
 int tgx_energy_scatter(tgx_ctx* ctx, tgx_model_t* m);
-int tgx_block_seen(tgx_ctx* ctx, tgx_model_t* m, int* d_seen, bool clear);
+int tgx_block_seen(tgx_ctx* ctx, tgx_model_t* m, int* d_mark);
+int tgx_fold_out(tgx_ctx* ctx, const double* F, const int* d_mark);
 int tgx_radial_table_build(tgx_ctx* ctx, tgx_model_t* m);
 
 
@@ -168,6 +169,8 @@ extern "C" int tgx_finalize(tgx_ctx* ctx) {
   if (ctx->gate_host) (void)hipHostFree(ctx->gate_host);
   if (ctx->md_flag_host) (void)hipHostFree(ctx->md_flag_host);
   if (ctx->red_host) (void)hipHostFree(ctx->red_host);
+  if (ctx->pairs_host) (void)hipHostFree(ctx->pairs_host);
+  if (ctx->fold_host) (void)hipHostFree(ctx->fold_host);
   if (ctx->ev_blocks) (void)hipEventDestroy(ctx->ev_blocks);
   for (auto& r : ctx->prof) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
   for (auto e : ctx->ev_pool) (void)hipEventDestroy(e);
@@ -575,8 +578,7 @@ static int begin_step(tgx_ctx* ctx) {
   TGX_TRY(ctx->energies.ensure(sizeof(double) * (size_t)n));
   TGX_TRY(ctx->forces.ensure(sizeof(double) * 3 * (size_t)n));
   TGX_TRY(ctx->fglob.ensure(sizeof(double) * 3 * P));
-  TGX_TRY(tgx_zero(ctx, ctx->energies.p, sizeof(double) * (size_t)n));
-  TGX_TRY(tgx_zero(ctx, ctx->fglob.p, sizeof(double) * 3 * P));
+  TGX_TRY(tgx_zero2(ctx, ctx->energies.p, sizeof(double) * (size_t)n, ctx->fglob.p, sizeof(double) * 3 * P));
   ctx->results_n = n;
   return TGX_OK;
 }
@@ -596,9 +598,12 @@ static int memory_budget_bytes(tgx_ctx* ctx, double* bytes) {
     *bytes = ctx->mem_budget;
     return TGX_OK;
   }
-  size_t f = 0, t = 0;
-  TGX_CHECK_HIP(hipMemGetInfo(&f, &t));
-  *bytes = 0.8 * (double)t;
+  if (ctx->mem_total <= 0.0) {  // the device's size does not change: asked for once
+    size_t f = 0, t = 0;
+    TGX_CHECK_HIP(hipMemGetInfo(&f, &t));
+    ctx->mem_total = (double)t;
+  }
+  *bytes = 0.8 * ctx->mem_total;
   return TGX_OK;
 }
 
@@ -638,16 +643,9 @@ static int plain_batches(tgx_ctx* ctx, tgx_model_t* m, int lo, int hi, std::vect
 
 // A block's energies and pair forces over the centres of atoms [lo, hi),
 // batched by the memory budget on the FP64 plain path. Energies are added into
-// the context's per-atom energies and pair forces into fglob. When `sites` is
-// given, the centres' atoms and energies are appended to it and `seen` marks
-// (device) the atoms the pairs reach. Runs on ctx->stream.
-struct BlockOut {
-  std::vector<int>* atoms = nullptr;
-  std::vector<double>* e = nullptr;
-  int* d_seen = nullptr;
-};
-
-static int run_block_range(tgx_ctx* ctx, tgx_model_t* m, int path, bool do_forces, int lo, int hi, BlockOut* out,
+// the context's per-atom energies and pair forces into fglob. d_mark (device,
+// may be null) marks the atoms the block touches. Runs on ctx->stream.
+static int run_block_range(tgx_ctx* ctx, tgx_model_t* m, int path, bool do_forces, int lo, int hi, int* d_mark,
                            int* n_sites_tot, int64_t* n_pairs_tot) {
   const int save_lo = m->sel_lo, save_hi = m->sel_hi;
   struct Restore {
@@ -676,17 +674,7 @@ static int run_block_range(tgx_ctx* ctx, tgx_model_t* m, int path, bool do_force
     TGX_TRY(tgx_energy_scatter(ctx, m));
     ns_tot += m->n_sites_b;
     np_tot += m->n_pairs_b;
-    if (out && out->atoms && m->n_sites_b > 0) {
-      const size_t b0 = out->atoms->size();
-      out->atoms->resize(b0 + (size_t)m->n_sites_b);
-      out->e->resize(b0 + (size_t)m->n_sites_b);
-      TGX_CHECK_HIP(hipMemcpyAsync(out->atoms->data() + b0, m->site_atom.p, sizeof(int) * (size_t)m->n_sites_b,
-                                   hipMemcpyDeviceToHost, ctx->stream));
-      TGX_CHECK_HIP(hipMemcpyAsync(out->e->data() + b0, m->e_site.p, sizeof(double) * (size_t)m->n_sites_b,
-                                   hipMemcpyDeviceToHost, ctx->stream));
-      TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    }
-    if (out && out->d_seen) TGX_TRY(tgx_block_seen(ctx, m, out->d_seen, false));
+    if (d_mark) TGX_TRY(tgx_block_seen(ctx, m, d_mark));
   }
   if (n_sites_tot) *n_sites_tot = ns_tot;
   if (n_pairs_tot) *n_pairs_tot = np_tot;
@@ -710,44 +698,27 @@ static int get_gap_soap_impl(tgx_ctx* ctx, int path, int do_forces, int lo, int 
   TGX_TRY(begin_step(ctx));
   const int n = ctx->n_sites;
   TGX_REQUIRE(lo >= 0 && lo <= hi && hi <= n, "tgx_get_gap_soap: sites [%d, %d) outside [0, %d)", lo, hi, n);
-  std::vector<int> sa;
-  std::vector<double> es;
-  BlockOut out;
-  out.atoms = &sa;
-  out.e = &es;
-  if (do_forces) {
-    TGX_TRY(ctx->gate_mask.ensure(sizeof(int) * (size_t)n));
-    TGX_TRY(tgx_zero(ctx, ctx->gate_mask.p, sizeof(int) * (size_t)n));
-    out.d_seen = ctx->gate_mask.as<int>();
-  }
+  TGX_TRY(ctx->gate_mask.ensure(sizeof(int) * 2 * (size_t)n));
+  int* mark = ctx->gate_mask.as<int>();
+  TGX_TRY(tgx_zero(ctx, mark, sizeof(int) * 2 * (size_t)n));
   int ns_b = 0;
   int64_t np_b = 0;
-  TGX_TRY(run_block_range(ctx, m, path, do_forces != 0, lo, hi, &out, &ns_b, &np_b));
+  TGX_TRY(run_block_range(ctx, m, path, do_forces != 0, lo, hi, mark, &ns_b, &np_b));
   double vir[9] = {0};
-  std::vector<int> seen;
-  std::vector<double> F;
-  if (do_forces) {
-    TGX_TRY(tgx_gather_forces(ctx, nullptr, vir));
-    seen.resize((size_t)n);
-    F.resize(3 * (size_t)n);
-    TGX_CHECK_HIP(hipMemcpyAsync(seen.data(), ctx->gate_mask.p, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost,
-                                 ctx->stream));
-    TGX_CHECK_HIP(hipMemcpyAsync(F.data(), ctx->forces.p, sizeof(double) * F.size(), hipMemcpyDeviceToHost, ctx->stream));
-    TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-  }
+  if (do_forces) TGX_TRY(tgx_gather_forces_launch(ctx));
+  TGX_TRY(tgx_fold_out(ctx, do_forces ? ctx->forces.as<double>() : nullptr, mark));
+  TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  if (do_forces) TGX_TRY(tgx_gather_collect(ctx, vir, nullptr));
   // fold back like src/gap_interface.f90:422-431: assign, for touched atoms only
-  if (energies)
-    for (size_t s = 0; s < sa.size(); ++s) energies[sa[s]] = es[s];
-  if (do_forces) {
-    if (forces)
-      for (int i = 0; i < n; ++i)
-        if (seen[(size_t)i])
-          for (int k = 0; k < 3; ++k) forces[3 * (size_t)i + k] = F[3 * (size_t)i + k];
-    if (virial)
-      for (int k = 0; k < 9; ++k) virial[k] = vir[k];
-  } else if (virial) {
-    for (int k = 0; k < 9; ++k) virial[k] = 0.0;
+  const double *F = ctx->fold_host, *E = F + 3 * (size_t)n;
+  const int* touched = reinterpret_cast<const int*>(E + n);
+  for (int i = 0; i < n; ++i) {
+    if (energies && (touched[i] & 2)) energies[i] = E[i];
+    if (do_forces && forces && (touched[i] & 1))
+      for (int k = 0; k < 3; ++k) forces[3 * (size_t)i + k] = F[3 * (size_t)i + k];
   }
+  if (virial)
+    for (int k = 0; k < 9; ++k) virial[k] = vir[k];
   if (n_sites_block) *n_sites_block = ns_b;
   if (n_pairs_block) *n_pairs_block = np_b;
   return TGX_OK;

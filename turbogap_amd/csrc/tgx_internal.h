@@ -216,6 +216,7 @@ struct tgx_ctx {
   dbuf energies, forces, fglob, virial_part, scratch, red;
   dbuf fres;  // per-atom force residual of a force-loss training step
   int results_n = 0;  // atoms the energies / forces buffers hold results for (0: none)
+  double mem_total = 0.0;   // device memory in bytes
   double mem_budget = 0.0;  // device bytes the FP64 plain path may hold for one block (0: 80% of the device)
   // md
   int md_n = 0;       // atoms of the MD state (velocities, masses, previous step); 0: none
@@ -240,6 +241,10 @@ struct tgx_ctx {
   int64_t gate_sites = 0, gate_gated = 0;
   int* gate_host = nullptr;  // pinned: {count, max spread bits} of every block
   double* red_host = nullptr;  // pinned: virial and energy partials of the force gather
+  int gather_parts[2] = {0, 0};   // virial and energy partials of the last gather
+  double* fold_host = nullptr;    // pinned: a block's forces, energies and atom marks (get_gap_soap)
+  int fold_n = 0;
+  int64_t* pairs_host = nullptr;  // pinned: the list build's pair count
   int gate_host_n = 0;
   dbuf gate_mask;
   hipEvent_t ev_blocks = nullptr;  // recorded on the context stream before concurrent blocks start
@@ -308,6 +313,10 @@ int tgx_plain_pair_forces_q(tgx_ctx* ctx, tgx_model_t* m, const double* qss);
 int tgx_compress_descriptors(tgx_ctx* ctx, tgx_model_t* m, bool with_der);
 int tgx_compress_gradient(tgx_ctx* ctx, tgx_model_t* m);
 int tgx_gather_forces(tgx_ctx* ctx, double* energy_out, double* virial_out);
+// tgx_gather_forces without its wait: the launch, and, once the caller has
+// synchronised the stream, the check and the virial.
+int tgx_gather_forces_launch(tgx_ctx* ctx);
+int tgx_gather_collect(tgx_ctx* ctx, double* virial_out, double* energy_out);
 // F (device, n x 3) and the pair virial (host, 9, optional) from per-entry pair
 // forces fglob (device, n_pairs x 3) on the resident list.
 int tgx_gather_pair_forces(tgx_ctx* ctx, const double* fglob, double* F, double* virial_out,

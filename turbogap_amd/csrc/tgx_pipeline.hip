@@ -6,6 +6,8 @@
 // global pair index, and atom j sums the entries of the pairs that point at it
 // by walking its own list through the reverse-pair index, in list order. The
 // result is the same bits on every run.
+#include <algorithm>
+
 #include "tgx_internal.h"
 #include "tgx_util.h"
 
@@ -24,23 +26,34 @@ struct SpeciesMap {
 // A site is a centre of the block when its species is the block's central
 // species (or the block takes every atom); a pair is kept when it lies inside
 // the block's largest cutoff and the block sees the neighbour's species.
-// Only atoms in [lo, hi) can be centres (a batch of the block's sites).
-__global__ void k_select_count(int n, int lo, int hi, SpeciesMap sm, int central, double rcut,
-                               const int* __restrict__ n_neigh, const int64_t* __restrict__ off,
-                               const int* __restrict__ species, const double* __restrict__ rjs,
-                               const int* __restrict__ nspec, int* __restrict__ flag, int* __restrict__ npairs) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Only atoms in [lo, hi) can be centres (a batch of the block's sites). Two
+// atoms per wavefront, 32 lanes each, as the fill (one thread walking its
+// atom's list took 18 us, 37 at 53 neighbours; this takes 5).
+__global__ __launch_bounds__(256) void k_select_count(int n, int lo, int hi, SpeciesMap sm, int central, double rcut,
+                                                    const int* __restrict__ n_neigh, const int64_t* __restrict__ off,
+                                                    const int* __restrict__ species, const double* __restrict__ rjs,
+                                                    const int* __restrict__ nspec, int* __restrict__ flag,
+                                                    int* __restrict__ npairs) {
+  const int lane = threadIdx.x & 63, sub = lane & 31;
+  const uint64_t half = (lane < 32 ? 0xffffffffull : 0xffffffff00000000ull);
+  const int i = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 2 + (lane >> 5);
   if (i >= n) return;
   const int sc = sm.index(species[i]);
-  const bool sel = i >= lo && i < hi && n_neigh[i] > 0 && sc >= 0 && (central == 0 || sc == central - 1);
+  const int nn = n_neigh[i];
+  const bool sel = i >= lo && i < hi && nn > 0 && sc >= 0 && (central == 0 || sc == central - 1);
   int cnt = 0;
   if (sel) {
     const int64_t b = off[i];
-    for (int k = 0; k < n_neigh[i]; ++k)
-      if (rjs[b + k] < rcut && sm.index(nspec[b + k]) >= 0) ++cnt;
+    for (int base = 0; base < nn; base += 32) {
+      const int k = base + sub;
+      const bool keep = k < nn && rjs[b + k] < rcut && sm.index(nspec[b + k]) >= 0;
+      cnt += __popcll(__ballot(keep) & half);
+    }
   }
-  flag[i] = sel ? 1 : 0;
-  npairs[i] = cnt;
+  if (sub == 0) {
+    flag[i] = sel ? 1 : 0;
+    npairs[i] = cnt;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_select_fill(int n, SpeciesMap sm, double rcut, const int* __restrict__ flag,
@@ -52,7 +65,8 @@ __global__ __launch_bounds__(256) void k_select_fill(int n, SpeciesMap sm, doubl
                                                    int* __restrict__ site_atom, int64_t* __restrict__ site_beg,
                                                    int64_t* __restrict__ pr_gidx, int* __restrict__ pr_nbr,
                                                    int* __restrict__ pr_spec, double* __restrict__ pr_r,
-                                                   double* __restrict__ pr_xyz, int* __restrict__ seen) {
+                                                   double* __restrict__ pr_xyz) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) site_beg[site_idx[n]] = pair_off[n];
   // two atoms per wavefront, 32 lanes each (lists average about 22 entries);
   // each half's ballot bits are masked to its own lanes
   const int lane = threadIdx.x & 63, sub = lane & 31;
@@ -85,79 +99,108 @@ __global__ __launch_bounds__(256) void k_select_fill(int n, SpeciesMap sm, doubl
       pr_xyz[3 * p] = xyz[3 * g];
       pr_xyz[3 * p + 1] = xyz[3 * g + 1];
       pr_xyz[3 * p + 2] = xyz[3 * g + 2];
-      if (seen) seen[j] = 1;
     }
     kept += __popcll(mask);
   }
 }
 
-__global__ void k_set_last(int64_t* __restrict__ site_beg, int ns, const int64_t* __restrict__ pair_off, int n) {
-  site_beg[ns] = pair_off[n];
-}
-
+// The end of a force evaluation in one launch: workgroups [0, n_gather) gather
+// forces, the next n_vir sum the virial, the rest the energies. The partials and
+// the missing-reverse flag go straight to pinned host memory, so that the step
+// ends with one kernel and one wait (five launches and a copy before: 25 us of
+// gaps and small kernels).
+//
 // F_j = sum over j's list entries q of fglob[rev[q]], in list order.
 // GATHER_LANES lanes per atom: lane t sums entries t, t + GATHER_LANES, ... in
 // order, then the lanes' sums combine by a fixed xor butterfly, so every run
-// adds in the same order.
+// adds in the same order. Virial: 0.5 (f x^T + x f^T) summed over a fixed slice
+// of pairs per workgroup (column-major 3x3). Energies: a fixed slice per
+// workgroup in a fixed tree.
 constexpr int GATHER_LANES = 16;
+constexpr int VIRIAL_PARTS = 512;
 
-__global__ void k_gather(int n, const int* __restrict__ n_neigh, const int64_t* __restrict__ off,
-                         const int64_t* __restrict__ rev, const double* __restrict__ fglob, double* __restrict__ F,
-                         int* __restrict__ bad) {
-  const int t = threadIdx.x % GATHER_LANES;
-  const int j = (blockIdx.x * blockDim.x + threadIdx.x) / GATHER_LANES;
-  const bool live = j < n;
-  double f0 = 0, f1 = 0, f2 = 0;
-  if (live) {
-    const int64_t b = off[j];
-    const int nn = n_neigh[j];
-    for (int k = t; k < nn; k += GATHER_LANES) {
-      const int64_t r = rev[b + k];
-      if (r < 0) { atomicExch(bad, 1); continue; }
-      f0 += fglob[3 * r];
-      f1 += fglob[3 * r + 1];
-      f2 += fglob[3 * r + 2];
-    }
-  }
-#pragma unroll
-  for (int o = GATHER_LANES / 2; o > 0; o >>= 1) {  // every lane of the wavefront takes part
-    f0 += __shfl_xor(f0, o);
-    f1 += __shfl_xor(f1, o);
-    f2 += __shfl_xor(f2, o);
-  }
-  if (live && t == 0) {
-    F[3 * j] = f0;
-    F[3 * j + 1] = f1;
-    F[3 * j + 2] = f2;
-  }
-}
+struct FinishArgs {
+  int n;
+  int64_t P;
+  const int* n_neigh;
+  const int64_t* off;
+  const int64_t* rev;
+  const double* fglob;
+  const double* xyz;
+  const double* energies;
+  double* F;
+  double* vpart;  // pinned: [n_vir][9]
+  double* epart;  // pinned: [n_e]
+  int* bad;       // pinned, set when a pair has no reverse entry
+  int n_gather, n_vir, n_e;
+};
 
-// Virial partials: 0.5 (f x^T + x f^T) summed over a fixed slice of pairs per
-// block (column-major 3x3).
-__global__ __launch_bounds__(256) void k_virial(int64_t P, const double* __restrict__ fglob,
-                                                const double* __restrict__ xyz, double* __restrict__ part) {
+__global__ __launch_bounds__(256) void k_finish(FinishArgs a) {
   __shared__ double sh[9][256];
-  const int64_t per = (P + gridDim.x - 1) / gridDim.x;
-  const int64_t b = (int64_t)blockIdx.x * per, e = b + per < P ? b + per : P;
+  int blk = blockIdx.x;
+  if (blk < a.n_gather) {
+    const int t = threadIdx.x % GATHER_LANES;
+    const int j = (blk * 256 + (int)threadIdx.x) / GATHER_LANES;
+    const bool live = j < a.n;
+    double f0 = 0, f1 = 0, f2 = 0;
+    if (live) {
+      const int64_t b = a.off[j];
+      const int nn = a.n_neigh[j];
+      for (int k = t; k < nn; k += GATHER_LANES) {
+        const int64_t r = a.rev[b + k];
+        if (r < 0) { *a.bad = 1; continue; }
+        f0 += a.fglob[3 * r];
+        f1 += a.fglob[3 * r + 1];
+        f2 += a.fglob[3 * r + 2];
+      }
+    }
+#pragma unroll
+    for (int o = GATHER_LANES / 2; o > 0; o >>= 1) {  // every lane of the wavefront takes part
+      f0 += __shfl_xor(f0, o);
+      f1 += __shfl_xor(f1, o);
+      f2 += __shfl_xor(f2, o);
+    }
+    if (live && t == 0) {
+      a.F[3 * (size_t)j] = f0;
+      a.F[3 * (size_t)j + 1] = f1;
+      a.F[3 * (size_t)j + 2] = f2;
+    }
+    return;
+  }
+  blk -= a.n_gather;
+  const bool vir = blk < a.n_vir;
+  const int nv = vir ? 9 : 1;
   double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for (int64_t p = b + threadIdx.x; p < e; p += 256) {
-    const double f[3] = {fglob[3 * p], fglob[3 * p + 1], fglob[3 * p + 2]};
-    const double x[3] = {xyz[3 * p], xyz[3 * p + 1], xyz[3 * p + 2]};
+  if (vir) {
+    const int64_t per = (a.P + a.n_vir - 1) / a.n_vir;
+    const int64_t b = (int64_t)blk * per, e = b + per < a.P ? b + per : a.P;
+    for (int64_t p = b + threadIdx.x; p < e; p += 256) {
+      const double f[3] = {a.fglob[3 * p], a.fglob[3 * p + 1], a.fglob[3 * p + 2]};
+      const double x[3] = {a.xyz[3 * p], a.xyz[3 * p + 1], a.xyz[3 * p + 2]};
 #pragma unroll
-    for (int k1 = 0; k1 < 3; ++k1)
+      for (int k1 = 0; k1 < 3; ++k1)
 #pragma unroll
-      for (int k2 = 0; k2 < 3; ++k2) v[3 * k2 + k1] += 0.5 * (f[k1] * x[k2] + f[k2] * x[k1]);
+        for (int k2 = 0; k2 < 3; ++k2) v[3 * k2 + k1] += 0.5 * (f[k1] * x[k2] + f[k2] * x[k1]);
+    }
+  } else {
+    blk -= a.n_vir;
+    const int per = (a.n + a.n_e - 1) / a.n_e;
+    const int b = blk * per, e = b + per < a.n ? b + per : a.n;
+    for (int i = b + (int)threadIdx.x; i < e; i += 256) v[0] += a.energies[i];
   }
 #pragma unroll
-  for (int k = 0; k < 9; ++k) sh[k][threadIdx.x] = v[k];
+  for (int k = 0; k < 9; ++k)
+    if (k < nv) sh[k][threadIdx.x] = v[k];
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
     if (threadIdx.x < o)
-#pragma unroll
-      for (int k = 0; k < 9; ++k) sh[k][threadIdx.x] += sh[k][threadIdx.x + o];
+      for (int k = 0; k < nv; ++k) sh[k][threadIdx.x] += sh[k][threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x < 9) part[9 * blockIdx.x + threadIdx.x] = sh[threadIdx.x][0];
+  if (threadIdx.x < nv) {
+    if (vir) a.vpart[9 * blk + threadIdx.x] = sh[threadIdx.x][0];
+    else a.epart[blk] = sh[0][0];
+  }
 }
 
 __global__ void k_energy_scatter(int ns, const int* __restrict__ site_atom, const double* __restrict__ e_site,
@@ -175,8 +218,8 @@ static SpeciesMap species_map(const tgx_model_t* m) {
   return sm;
 }
 
-// Block selection in two halves: the count and scans with the two totals copied
-// to pinned host memory (no wait), then, once the caller has synchronised the
+// Block selection in two halves: the count and scans, which leave the two totals
+// in pinned host memory (no wait), then, once the caller has synchronised the
 // stream, the allocation and the fill. Several blocks can have their counts in
 // flight before one wait.
 struct SelectView {
@@ -203,14 +246,11 @@ int tgx_block_select_count(tgx_ctx* ctx, tgx_model_t* m) {
   const SelectView v = select_view(m, n);
   SpeciesMap sm = species_map(m);
   const int lo = m->sel_lo > 0 ? m->sel_lo : 0, hi = (m->sel_hi >= 0 && m->sel_hi < n) ? m->sel_hi : n;
-  TGX_LAUNCH(ctx, "select_count", k_select_count, dim3((n + 255) / 256), dim3(256), 0, n, lo, hi, sm,
+  TGX_LAUNCH(ctx, "select_count", k_select_count, dim3((n + 7) / 8), dim3(256), 0, n, lo, hi, sm,
              m->central_species, m->rcut_max, ctx->n_neigh.as<int>(), ctx->nl_off.as<int64_t>(),
              ctx->species_sc.as<int>(), ctx->rjs.as<double>(), ctx->nspec.as<int>(), v.flag, v.npairs);
-  TGX_TRY(tgx_scan2_i32(ctx, v.flag, v.site_idx, v.npairs, v.pair_off, n, m->scan_tmp));
   if (!m->sel_host) TGX_CHECK_HIP(hipHostMalloc((void**)&m->sel_host, 2 * sizeof(int64_t), hipHostMallocDefault));
-  TGX_CHECK_HIP(hipMemcpyAsync(m->sel_host, v.site_idx + n, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
-  TGX_CHECK_HIP(hipMemcpyAsync(m->sel_host + 1, v.pair_off + n, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
-  return TGX_OK;
+  return tgx_scan2_i32(ctx, v.flag, v.site_idx, v.npairs, v.pair_off, n, m->scan_tmp, m->sel_host);
 }
 
 int tgx_block_select_counts_host(tgx_ctx* ctx, tgx_model_t* m, std::vector<int>& flag, std::vector<int64_t>& pair_off) {
@@ -244,8 +284,7 @@ int tgx_block_select_fill(tgx_ctx* ctx, tgx_model_t* m) {
              v.site_idx, v.pair_off, ctx->n_neigh.as<int>(), ctx->nl_off.as<int64_t>(), ctx->nlist.as<int>(),
              ctx->rjs.as<double>(), ctx->xyz.as<double>(), ctx->nspec.as<int>(), m->site_atom.as<int>(),
              m->site_beg.as<int64_t>(), m->pr_gidx.as<int64_t>(), m->pr_nbr.as<int>(), m->pr_spec.as<int>(),
-             m->pr_r.as<double>(), m->pr_xyz.as<double>(), (int*)nullptr);
-  TGX_LAUNCH(ctx, "select_last", k_set_last, dim3(1), dim3(1), 0, m->site_beg.as<int64_t>(), (int)ns, v.pair_off, n);
+             m->pr_r.as<double>(), m->pr_xyz.as<double>());
   return TGX_OK;
 }
 
@@ -263,47 +302,66 @@ int tgx_gather_forces(tgx_ctx* ctx, double* energy_out, double* virial_out) {
                                 ctx->energies.as<double>(), energy_out);
 }
 
-// Layout of ctx->red (and its pinned host copy): 512 blocks x 9 virial
-// partials, TGX_SUM_PARTS energy partials, the missing-reverse flag; one
-// readback and one synchronisation for all of them.
-int tgx_gather_pair_forces(tgx_ctx* ctx, const double* fglob, double* F, double* virial_out,
-                           const double* d_energies, double* energy_out) {
-  const int n = ctx->n_sites;
-  const int64_t P = ctx->n_pairs;
-  const int nbk = 512;
-  const size_t nred = 9 * (size_t)nbk + TGX_SUM_PARTS + 1;
-  TGX_TRY(ctx->red.ensure(sizeof(double) * nred));
+// Layout of ctx->red_host (pinned): VIRIAL_PARTS x 9 virial partials,
+// TGX_SUM_PARTS energy partials, the missing-reverse flag.
+static int gather_launch(tgx_ctx* ctx, const double* fglob, double* F, bool with_virial, const double* d_energies) {
+  const size_t nred = 9 * (size_t)VIRIAL_PARTS + TGX_SUM_PARTS + 1;
   if (!ctx->red_host) TGX_CHECK_HIP(hipHostMalloc((void**)&ctx->red_host, sizeof(double) * nred, hipHostMallocDefault));
-  double* vpart = ctx->red.as<double>();
-  double* epart = vpart + 9 * nbk;
-  int* bad = reinterpret_cast<int*>(epart + TGX_SUM_PARTS);
-  TGX_TRY(tgx_zero(ctx, bad, sizeof(double)));
-  TGX_LAUNCH(ctx, "force_gather", k_gather, dim3((unsigned)(((int64_t)n * GATHER_LANES + 255) / 256)), dim3(256), 0,
-             n, ctx->n_neigh.as<int>(),
-             ctx->nl_off.as<int64_t>(), ctx->rev.as<int64_t>(), fglob, F, bad);
-  TGX_LAUNCH(ctx, "virial", k_virial, dim3(nbk), dim3(256), 0, P, fglob, ctx->xyz.as<double>(), vpart);
-  const bool with_e = energy_out && d_energies;
-  if (with_e) TGX_TRY(tgx_device_sum_launch(ctx, d_energies, n, epart));
-  TGX_CHECK_HIP(hipMemcpyAsync(ctx->red_host, vpart, sizeof(double) * nred, hipMemcpyDeviceToHost, ctx->stream));
-  TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-  const double* hv = ctx->red_host;
-  int badh = 0;
-  std::memcpy(&badh, hv + 9 * nbk + TGX_SUM_PARTS, sizeof(int));
-  if (badh) {
+  FinishArgs a;
+  a.n = ctx->n_sites;
+  a.P = ctx->n_pairs;
+  a.n_neigh = ctx->n_neigh.as<int>();
+  a.off = ctx->nl_off.as<int64_t>();
+  a.rev = ctx->rev.as<int64_t>();
+  a.fglob = fglob;
+  a.xyz = ctx->xyz.as<double>();
+  a.energies = d_energies;
+  a.F = F;
+  a.vpart = ctx->red_host;
+  a.epart = a.vpart + 9 * VIRIAL_PARTS;
+  a.bad = reinterpret_cast<int*>(a.epart + TGX_SUM_PARTS);
+  *a.bad = 0;  // every use of the buffer ends with a wait: no kernel holds it now
+  // about 2,048 pairs or atoms a partial, so that a small system writes few of them
+  auto parts = [](int64_t n, int most) { return (int)std::min<int64_t>(most, std::max<int64_t>(1, (n + 2047) / 2048)); };
+  a.n_gather = (int)(((int64_t)a.n * GATHER_LANES + 255) / 256);
+  a.n_vir = with_virial ? parts(a.P, VIRIAL_PARTS) : 0;
+  a.n_e = d_energies ? parts(a.n, TGX_SUM_PARTS) : 0;
+  ctx->gather_parts[0] = a.n_vir;
+  ctx->gather_parts[1] = a.n_e;
+  TGX_LAUNCH(ctx, "force_gather", k_finish, dim3((unsigned)(a.n_gather + a.n_vir + a.n_e)), dim3(256), 0, a);
+  return TGX_OK;
+}
+
+int tgx_gather_collect(tgx_ctx* ctx, double* virial_out, double* energy_out) {
+  const double* vp = ctx->red_host;
+  const double* ep = vp + 9 * VIRIAL_PARTS;
+  if (*reinterpret_cast<const int*>(ep + TGX_SUM_PARTS)) {
     tgx_set_error("force gather: a pair has no reverse entry (an atom without its own list); build with do_list = all");
     return TGX_ERR_UNSUPPORTED;
   }
   if (virial_out) {
     for (int k = 0; k < 9; ++k) virial_out[k] = 0.0;
-    for (int b = 0; b < nbk; ++b)
-      for (int k = 0; k < 9; ++k) virial_out[k] += hv[9 * b + k];
+    for (int b = 0; b < ctx->gather_parts[0]; ++b)
+      for (int k = 0; k < 9; ++k) virial_out[k] += vp[9 * b + k];
   }
-  if (with_e) {
+  if (energy_out && ctx->gather_parts[1] > 0) {
     double e = 0.0;
-    for (int i = 0; i < TGX_SUM_PARTS; ++i) e += hv[9 * nbk + i];
+    for (int i = 0; i < ctx->gather_parts[1]; ++i) e += ep[i];
     *energy_out = e;
   }
   return TGX_OK;
+}
+
+int tgx_gather_forces_launch(tgx_ctx* ctx) {
+  TGX_TRY(ctx->forces.ensure(sizeof(double) * 3 * (size_t)ctx->n_sites));
+  return gather_launch(ctx, ctx->fglob.as<double>(), ctx->forces.as<double>(), true, nullptr);
+}
+
+int tgx_gather_pair_forces(tgx_ctx* ctx, const double* fglob, double* F, double* virial_out,
+                           const double* d_energies, double* energy_out) {
+  TGX_TRY(gather_launch(ctx, fglob, F, virial_out != nullptr, energy_out ? d_energies : nullptr));
+  TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  return tgx_gather_collect(ctx, virial_out, energy_out);
 }
 
 int tgx_energy_scatter(tgx_ctx* ctx, tgx_model_t* m) {
@@ -314,17 +372,49 @@ int tgx_energy_scatter(tgx_ctx* ctx, tgx_model_t* m) {
   return TGX_OK;
 }
 
-// Atoms a block touches: its centres and every kept neighbour.
-__global__ void k_mark_seen(int64_t np, const int* __restrict__ pr_nbr, int* __restrict__ seen) {
+// Marks (two ints an atom) of the atoms a block touches: mark[0][j] for every
+// kept neighbour (a centre's self entry among them), mark[1][i] for the centres.
+__global__ void k_mark_seen(int64_t np, int ns, int n, const int* __restrict__ pr_nbr,
+                            const int* __restrict__ site_atom, int* __restrict__ mark) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < np) seen[pr_nbr[p]] = 1;
+  if (p < np) mark[pr_nbr[p]] = 1;
+  if (p < ns) mark[n + site_atom[p]] = 1;
 }
 
-int tgx_block_seen(tgx_ctx* ctx, tgx_model_t* m, int* d_seen, bool clear) {
-  if (clear) TGX_TRY(tgx_zero(ctx, d_seen, sizeof(int) * (size_t)ctx->n_sites));
-  const int64_t np = m->n_pairs_b;
+int tgx_block_seen(tgx_ctx* ctx, tgx_model_t* m, int* d_mark) {
+  const int64_t np = std::max<int64_t>(m->n_pairs_b, m->n_sites_b);
   if (np == 0) return TGX_OK;
-  TGX_LAUNCH(ctx, "mark_seen", k_mark_seen, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, np, m->pr_nbr.as<int>(),
-             d_seen);
+  TGX_LAUNCH(ctx, "mark_seen", k_mark_seen, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, m->n_pairs_b,
+             m->n_sites_b, ctx->n_sites, m->pr_nbr.as<int>(), m->site_atom.as<int>(), d_mark);
+  return TGX_OK;
+}
+
+// Forces, energies and marks of every atom into pinned host memory (4 doubles an
+// atom, then one int an atom: 1 force, 2 energy). F may be null.
+__global__ void k_fold_out(int n, const double* __restrict__ F, const double* __restrict__ energies,
+                           const int* __restrict__ mark, double* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  if (F) {
+    out[3 * (size_t)i] = F[3 * (size_t)i];
+    out[3 * (size_t)i + 1] = F[3 * (size_t)i + 1];
+    out[3 * (size_t)i + 2] = F[3 * (size_t)i + 2];
+  }
+  out[3 * (size_t)n + i] = energies[i];
+  reinterpret_cast<int*>(out + 4 * (size_t)n)[i] = (mark[i] ? 1 : 0) | (mark[n + i] ? 2 : 0);
+}
+
+int tgx_fold_out(tgx_ctx* ctx, const double* F, const int* d_mark) {
+  const int n = ctx->n_sites;
+  if (ctx->fold_n < n) {
+    if (ctx->fold_host) (void)hipHostFree(ctx->fold_host);
+    ctx->fold_host = nullptr;
+    ctx->fold_n = 0;
+    TGX_CHECK_HIP(hipHostMalloc((void**)&ctx->fold_host, (sizeof(double) * 4 + sizeof(int)) * (size_t)n,
+                                hipHostMallocDefault));
+    ctx->fold_n = n;
+  }
+  TGX_LAUNCH(ctx, "fold_out", k_fold_out, dim3((n + 255) / 256), dim3(256), 0, n, F, ctx->energies.as<double>(), d_mark,
+             ctx->fold_host);
   return TGX_OK;
 }

@@ -2,17 +2,22 @@
 #pragma once
 #include "tgx_internal.h"
 
+// Zero two device ranges (bytes, multiples of four) in one launch.
+int tgx_zero2(tgx_ctx* ctx, void* p, size_t np, void* q, size_t nq);
+
 // Exclusive prefix sum of n int32 values into int64 offsets; out has n + 1
-// entries (out[n] is the total). When total is not NULL the total is copied to
-// the host (this synchronises the stream). The block totals go to tmp, or to
-// the context's own scratch when tmp is NULL; scans that may run on different
-// streams at once must each bring their own.
+// entries (out[n] is the total). total, when not NULL, is pinned host memory
+// that the scan's kernel stores the total into (valid once the stream has been
+// synchronised; a copy of its own costs a launch and its gap). The block totals
+// go to tmp, or to the context's own scratch when tmp is NULL; scans that may
+// run on different streams at once must each bring their own.
 int tgx_scan_i32(tgx_ctx* ctx, const int* in, int64_t* out, int64_t n, int64_t* total, dbuf* tmp = nullptr);
-// The same for two arrays of n values (two launches for both when 16,384 < n <=
-// 65,536, four or six otherwise); block totals in tmp, which belongs to the
-// caller so that scans on different streams do not share it.
+// The same for two arrays of n values, their totals in totals[0] and totals[1]
+// (one launch for both up to 8,192 values, two up to 65,536, six above); block
+// totals in tmp, which belongs to the caller so that scans on different streams
+// do not share it.
 int tgx_scan2_i32(tgx_ctx* ctx, const int* in0, int64_t* out0, const int* in1, int64_t* out1, int64_t n,
-                  dbuf& tmp);
+                  dbuf& tmp, int64_t* totals);
 
 // Partial sums of n doubles into TGX_SUM_PARTS device values, each over a fixed
 // contiguous slice in a fixed tree (summed on the host in order).

@@ -1,15 +1,27 @@
 // Device utilities: zero fill, deterministic exclusive scan, deterministic sum.
+#include <algorithm>
+
 #include "tgx_util.h"
 
 namespace {
 
 constexpr int SCAN_BLOCK = 1024;
-constexpr int64_t SCAN_SINGLE_MAX = 16 * 1024;  // one workgroup scans up to this many values
+constexpr int64_t SCAN_SINGLE_MAX = 8 * 1024;  // one workgroup scans up to this many values (8,192: 6 us; 16,001: 18, in two launches 10)
 
 __global__ void k_fill_zero(uint32_t* __restrict__ p, size_t n_words) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (; i < n_words; i += stride) p[i] = 0u;
+}
+
+// Two ranges in one launch.
+__global__ void k_fill_zero2(uint32_t* __restrict__ p, size_t np, uint32_t* __restrict__ q, size_t nq) {
+  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (; i < np + nq; i += stride) {
+    if (i < np) p[i] = 0u;
+    else q[i - np] = 0u;
+  }
 }
 
 __global__ void k_fill_zero_bytes(uint8_t* __restrict__ p, size_t n) {
@@ -61,37 +73,14 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_sums(int64_t* __restrict__ 
   if (threadIdx.x == 0) sums[nb] = carry;
 }
 
-__global__ void k_scan_add(int64_t* __restrict__ out, int64_t n, const int64_t* __restrict__ sums) {
+__global__ void k_scan_add(int64_t* __restrict__ out, int64_t n, const int64_t* __restrict__ sums,
+                           int64_t* __restrict__ tot) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] += sums[i / SCAN_BLOCK];
-  if (i == 0) out[n] = sums[(n + SCAN_BLOCK - 1) / SCAN_BLOCK];
-}
-
-// Whole exclusive scan in one workgroup (n up to SCAN_SINGLE_MAX = 16 per
-// thread): thread t owns the contiguous chunk [t c, (t+1) c), loaded at once into
-// registers; the 1024 chunk sums are scanned in LDS and each thread writes its
-// chunk's prefixes; out[n] is the total.
-constexpr int SCAN_CMAX = 16;
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_single(const int* __restrict__ in, int64_t* __restrict__ out,
-                                                           int64_t n) {
-  __shared__ int64_t sh[SCAN_BLOCK];
-  const int c = (int)((n + SCAN_BLOCK - 1) / SCAN_BLOCK);
-  const int64_t b = (int64_t)threadIdx.x * c;
-  int v[SCAN_CMAX];
-  int64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < SCAN_CMAX; ++k) {
-    v[k] = (k < c && b + k < n) ? in[b + k] : 0;
-    s += v[k];
+  if (i == 0) {
+    out[n] = sums[(n + SCAN_BLOCK - 1) / SCAN_BLOCK];
+    if (tot) *tot = sums[(n + SCAN_BLOCK - 1) / SCAN_BLOCK];
   }
-  int64_t tot;
-  int64_t run = block_exclusive_scan(s, sh, &tot);
-#pragma unroll
-  for (int k = 0; k < SCAN_CMAX; ++k) {
-    if (k < c && b + k < n) out[b + k] = run;
-    run += v[k];
-  }
-  if (threadIdx.x == 0) out[n] = tot;
 }
 
 // Exclusive scan of one value per thread over a 1024-thread workgroup: wave
@@ -121,6 +110,40 @@ __device__ int64_t block_exclusive_scan_waves(int64_t v, int64_t* sh, int64_t* t
   return (w > 0 ? sh[NW + w - 1] : 0) + x - v;
 }
 
+// Whole exclusive scan in one workgroup (n up to SCAN_SINGLE_MAX = 8 per
+// thread), one or two arrays (blockIdx.y): thread t owns the contiguous chunk
+// [t c, (t+1) c), loaded at once into registers; the 1024 chunk sums are scanned
+// and each thread writes its chunk's prefixes; out[n] is the total, also stored
+// at tot (pinned host memory) when given.
+constexpr int SCAN_CMAX = 8;
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_single(const int* __restrict__ in0, int64_t* __restrict__ out0,
+                                                           const int* __restrict__ in1, int64_t* __restrict__ out1,
+                                                           int64_t n, int64_t* __restrict__ tot) {
+  __shared__ int64_t sh[2 * SCAN_BLOCK / 64];
+  const int* in = blockIdx.y ? in1 : in0;
+  int64_t* out = blockIdx.y ? out1 : out0;
+  const int c = (int)((n + SCAN_BLOCK - 1) / SCAN_BLOCK);
+  const int64_t b = (int64_t)threadIdx.x * c;
+  int v[SCAN_CMAX];
+  int64_t s = 0;
+#pragma unroll
+  for (int k = 0; k < SCAN_CMAX; ++k) {
+    v[k] = (k < c && b + k < n) ? in[b + k] : 0;
+    s += v[k];
+  }
+  int64_t total;
+  int64_t run = block_exclusive_scan_waves(s, sh, &total);
+#pragma unroll
+  for (int k = 0; k < SCAN_CMAX; ++k) {
+    if (k < c && b + k < n) out[b + k] = run;
+    run += v[k];
+  }
+  if (threadIdx.x == 0) {
+    out[n] = total;
+    if (tot) tot[blockIdx.y] = total;
+  }
+}
+
 // Two-launch exclusive scan of up to SCAN_2L_MAX values, one or two arrays
 // (blockIdx.y picks in0/out0 or in1/out1): k_scan_local2 scans each block of
 // 1024 values and stores the block totals; k_scan_add2 adds to every block the
@@ -142,7 +165,8 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_local2(const int* __restric
 }
 
 __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add2(int64_t* __restrict__ out0, int64_t* __restrict__ out1,
-                                                         int64_t n, const int64_t* __restrict__ sums) {
+                                                         int64_t n, const int64_t* __restrict__ sums,
+                                                         int64_t* __restrict__ tot) {
   __shared__ int64_t off;
   int64_t* out = blockIdx.y ? out1 : out0;
   const int64_t* bs = sums + (size_t)blockIdx.y * gridDim.x;
@@ -156,7 +180,10 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add2(int64_t* __restrict__ 
   __syncthreads();
   const int64_t i = (int64_t)blockIdx.x * SCAN_BLOCK + threadIdx.x;
   if (i < n) out[i] += off;
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = off + bs[blockIdx.x];
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    out[n] = off + bs[blockIdx.x];
+    if (tot) tot[blockIdx.y] = off + bs[blockIdx.x];
+  }
 }
 
 // Streaming copy, 16 bytes per thread and iteration (the HBM reference).
@@ -198,47 +225,59 @@ int tgx_zero(tgx_ctx* ctx, void* p, size_t bytes) {
   return TGX_OK;
 }
 
+int tgx_zero2(tgx_ctx* ctx, void* p, size_t np, void* q, size_t nq) {
+  TGX_REQUIRE(((np | nq) & 3) == 0, "tgx_zero2: sizes must be multiples of four bytes");
+  const size_t w = (np + nq) / 4;
+  if (w == 0) return TGX_OK;
+  TGX_LAUNCH(ctx, "fill_zero", k_fill_zero2, dim3((unsigned)std::min<size_t>((w + 255) / 256, 65536)), dim3(256), 0,
+             (uint32_t*)p, np / 4, (uint32_t*)q, nq / 4);
+  return TGX_OK;
+}
+
 int tgx_scan_i32(tgx_ctx* ctx, const int* in, int64_t* out, int64_t n, int64_t* total, dbuf* tmp) {
   const int64_t nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
   dbuf& sb = tmp ? *tmp : ctx->scan_tmp;
   TGX_TRY(sb.ensure(sizeof(int64_t) * (size_t)(nb + 2)));
   int64_t* sums = sb.as<int64_t>();
   if (n > 0 && n <= SCAN_SINGLE_MAX) {
-    TGX_LAUNCH(ctx, "scan_single", k_scan_single, dim3(1), dim3(SCAN_BLOCK), 0, in, out, n);
+    TGX_LAUNCH(ctx, "scan_single", k_scan_single, dim3(1), dim3(SCAN_BLOCK), 0, in, out, (const int*)nullptr,
+               (int64_t*)nullptr, n, total);
   } else if (n > 0 && n <= SCAN_2L_MAX) {
     TGX_LAUNCH(ctx, "scan_local", k_scan_local2, dim3((unsigned)nb, 1), dim3(SCAN_BLOCK), 0, in, out,
                (const int*)nullptr, (int64_t*)nullptr, n, sums);
     TGX_LAUNCH(ctx, "scan_add", k_scan_add2, dim3((unsigned)nb, 1), dim3(SCAN_BLOCK), 0, out, (int64_t*)nullptr, n,
-               (const int64_t*)sums);
+               (const int64_t*)sums, total);
   } else if (n > 0) {
     TGX_LAUNCH(ctx, "scan_local", k_scan_local, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, in, out, n, sums);
     TGX_LAUNCH(ctx, "scan_sums", k_scan_sums, dim3(1), dim3(SCAN_BLOCK), 0, sums, nb);
-    TGX_LAUNCH(ctx, "scan_add", k_scan_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, out, n, sums);
+    TGX_LAUNCH(ctx, "scan_add", k_scan_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, out, n,
+               (const int64_t*)sums, total);
   } else {
     TGX_TRY(tgx_zero(ctx, out, sizeof(int64_t)));
-  }
-  if (total) {
-    TGX_CHECK_HIP(hipMemcpyAsync(total, out + n, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
-    TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    if (total) *total = 0;
   }
   return TGX_OK;
 }
 
 int tgx_scan2_i32(tgx_ctx* ctx, const int* in0, int64_t* out0, const int* in1, int64_t* out1, int64_t n,
-                  dbuf& tmp) {
-  if (n > SCAN_SINGLE_MAX && n <= SCAN_2L_MAX) {
+                  dbuf& tmp, int64_t* totals) {
+  if (n > 0 && n <= SCAN_SINGLE_MAX) {
+    TGX_LAUNCH(ctx, "scan_single", k_scan_single, dim3(1, 2), dim3(SCAN_BLOCK), 0, in0, out0, in1, out1, n, totals);
+    return TGX_OK;
+  }
+  if (n > 0 && n <= SCAN_2L_MAX) {
     const int64_t nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
     TGX_TRY(tmp.ensure(sizeof(int64_t) * 2 * (size_t)nb));
     int64_t* sums = tmp.as<int64_t>();
     TGX_LAUNCH(ctx, "scan_local", k_scan_local2, dim3((unsigned)nb, 2), dim3(SCAN_BLOCK), 0, in0, out0, in1, out1, n,
                sums);
     TGX_LAUNCH(ctx, "scan_add", k_scan_add2, dim3((unsigned)nb, 2), dim3(SCAN_BLOCK), 0, out0, out1, n,
-               (const int64_t*)sums);
+               (const int64_t*)sums, totals);
     return TGX_OK;
   }
   // one after the other on the caller's stream, both through the caller's tmp
-  TGX_TRY(tgx_scan_i32(ctx, in0, out0, n, nullptr, &tmp));
-  return tgx_scan_i32(ctx, in1, out1, n, nullptr, &tmp);
+  TGX_TRY(tgx_scan_i32(ctx, in0, out0, n, totals, &tmp));
+  return tgx_scan_i32(ctx, in1, out1, n, totals ? totals + 1 : nullptr, &tmp);
 }
 
 int tgx_device_sum_launch(tgx_ctx* ctx, const double* d_x, int64_t n, double* d_part) {
