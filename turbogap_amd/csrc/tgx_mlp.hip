@@ -33,213 +33,395 @@ __device__ __forceinline__ float silu(float z) { return tgx_silu(z); }
 __device__ __forceinline__ float silu1(float z) { return tgx_silu1(z); }
 __device__ __forceinline__ float silu2(float z) { return tgx_silu2(z); }
 
-// layer 1: z1 += b1; h1 = silu(z1) (bf16 and fp32); s1 = silu'(z1); s1pp = silu''(z1)
-__global__ void k_l1(int64_t n, int H, float* __restrict__ z1, const float* __restrict__ b1, __bf16* __restrict__ h1b,
-                     float* __restrict__ h1, float* __restrict__ s1, float* __restrict__ s1pp) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float z = z1[i] + b1[i % H];
-  z1[i] = z;
-  const float h = silu(z);
-  h1b[i] = (__bf16)h;
-  if (h1) h1[i] = h;
-  s1[i] = silu1(z);
-  if (s1pp) s1pp[i] = silu2(z);
-}
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-// layer 2 and output, one wavefront per row: z2 += b2, E = w3 . silu(z2) + b3,
-// a2 = w3 * silu'(z2); optional training copies.
-__global__ __launch_bounds__(256) void k_l2(int rows, int H, float* __restrict__ z2, const float* __restrict__ b2,
-                                            const float* __restrict__ w3, const float* __restrict__ b3,
-                                            float* __restrict__ E, __bf16* __restrict__ a2b, float* __restrict__ a2,
-                                            float* __restrict__ h2, float* __restrict__ s2p,
-                                            float* __restrict__ s2pp) {
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  float acc = 0.f;
-  for (int j = lane; j < H; j += 64) {
-    const size_t k = (size_t)row * H + j;
-    const float z = z2[k] + b2[j];
-    z2[k] = z;
-    const float h = silu(z), d1 = silu1(z);
-    acc += w3[j] * h;
-    const float a = w3[j] * d1;
-    a2b[k] = (__bf16)a;
-    if (a2) a2[k] = a;
-    if (h2) h2[k] = h;
-    if (s2p) s2p[k] = d1;
-    if (s2pp) s2pp[k] = silu2(z);
+// Products of the training pass (NT, BF16 operands, FP32 accumulation) with the
+// elementwise work that follows each fused into its epilogue. Only z1, z2, v1 and
+// tau0 are kept in FP32; everything else is formed again from them, which costs
+// less than storing and reading it:
+//   TR_L1    z1 = acc + b1;  h1 = silu(z1) out in BF16, and transposed (wgrad operand)
+//   TR_L2    z2 = acc + b2;  a2 = w3 silu'(z2) out in BF16 and transposed; row sums of w3 silu(z2)
+//   TR_BACK2 v1 = acc;       a1 = v1 silu'(z1) out in BF16 and transposed
+//   TR_JVP1  tau0 = acc;     tau1 = silu'(z1) tau0 out in BF16; dE h1 + cG tau1 transposed
+//   TR_JVP2  tau2 = acc;     zeta2 = w3 tau2 silu''(z2) out in BF16, cG zeta2 transposed; column
+//                            sums of dE a2 + cG zeta2 and dE h2 + cG gamma2, gamma2 = silu'(z2) tau2
+//   TR_VJP2  acc = W2^T zeta2; zeta1 = v1 tau0 silu''(z1) + acc silu'(z1), cG zeta1 transposed;
+//                            column sums of dE a1 + cG zeta1
+//   TR_PART  acc out in FP32 (a K chunk of a weight gradient, blockIdx.z)
+enum { TR_L1, TR_L2, TR_BACK2, TR_JVP1, TR_JVP2, TR_VJP2, TR_PART };
+
+struct TrainArgs {
+  int B, H;
+  bool train;             // transposed operands wanted
+  const float* bias;      // b1 (TR_L1) or b2 (TR_L2)
+  const float* w3;
+  float *z1, *z2, *v1, *t0;
+  __bf16* row;            // [B][H] BF16 output
+  __bf16* tr;             // [H][2B] transposed operand
+  const float* dE;
+  float cG;
+  float* epart;           // [B][H / 32] partial energies (TR_L2)
+  double* cpart;          // [3][B / 32][H] column partials (b1, b2, w3)
+  float* out;             // TR_PART: [z][M][N]
+  int ldo;
+  int64_t sOut;
+};
+
+// Workgroup tile 64 x 64, four wavefronts of 32 x 32, BK = 64 in a four-slot ring
+// of direct global-to-LDS loads, three stages in flight. A stage is 128 rows of
+// 128 bytes (A, then B); the eight 16-byte chunks of row r sit at c ^ (r & 7), so
+// that a fragment read covers all banks. The layers are 4,096 x 256: 128 x 128
+// tiles left 64 workgroups on 256 CUs (15 us for K = 1,280 and 8 for K = 256, and
+// 5 to 8 for each elementwise pass; now 8 and 5 with nothing after them).
+// M and N multiples of 64, K of 64.
+constexpr int TR_SB = 128 * 128, TR_NS = 4;
+
+template <int OP>
+__global__ __launch_bounds__(256, 2) void k_train_gemm(int K, const __bf16* __restrict__ A, int lda,
+                                                       const __bf16* __restrict__ B, int ldb, TrainArgs e) {
+  __shared__ __align__(16) unsigned char dsm[TR_NS * TR_SB];
+  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wm = w >> 1, wn = w & 1;
+  if (OP == TR_PART) {  // this workgroup's K chunk
+    A += (size_t)blockIdx.z * K;
+    B += (size_t)blockIdx.z * K;
   }
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-  if (lane == 0) E[row] = acc + b3[0];
+  const int lrow = lane >> 3, lchunk = (lane & 7) ^ lrow;
+  const __bf16* src[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int b = w + 4 * j;  // eight rows each: A's 0..7, B's 8..15
+    src[j] = b < 8 ? A + (size_t)(m0 + 8 * b + lrow) * lda + 8 * lchunk
+                   : B + (size_t)(n0 + 8 * (b - 8) + lrow) * ldb + 8 * lchunk;
+  }
+  const int n_stages = K / 64;
+  auto issue = [&](int st) {
+    const int k0 = min(st, n_stages - 1) * 64;  // an in-bounds repeat past the end
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_global_load_lds(const_cast<__bf16*>(src[j] + k0),
+                                       dsm + (st & (TR_NS - 1)) * TR_SB + (w + 4 * j) * 1024, 16, 0, 0);
+  };
+  const int li = lane & 15, lg = lane >> 4;
+  const int aoff = (wm * 32 + li) * 128, boff = (64 + wn * 32 + li) * 128;
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < TR_NS - 1; ++s) issue(s);
+  for (int st = 0; st < n_stages; ++st) {
+    __builtin_amdgcn_sched_barrier(0);  // every read of the last round stays before the barrier
+    __builtin_amdgcn_s_waitcnt(0x3F70 | (4 * (TR_NS - 2)));  // this wavefront's part of stage st has landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(st + TR_NS - 1);  // into the slot that every wavefront read in the last round
+    const unsigned char* sb = dsm + (st & (TR_NS - 1)) * TR_SB;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int cp = ((4 * ks + lg) ^ (li & 7)) << 4;
+      bf16x8 a[2], b[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        a[t] = *reinterpret_cast<const bf16x8*>(sb + aoff + t * 16 * 128 + cp);
+        b[t] = *reinterpret_cast<const bf16x8*>(sb + boff + t * 16 * 128 + cp);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x3F70);  // the loads issued past the last stage land before the LDS is released
+  __builtin_amdgcn_sched_barrier(0);
+  const int H = e.H;
+  const size_t B2 = 2 * (size_t)e.B;
+  double cs0[2] = {0.0, 0.0}, cs1[2] = {0.0, 0.0};
+#pragma unroll
+  for (int ti = 0; ti < 2; ++ti) {
+    const int row = m0 + wm * 32 + ti * 16 + 4 * lg;  // rows row .. row + 3
+    float er[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int tj = 0; tj < 2; ++tj) {
+      const int col = n0 + wn * 32 + tj * 16 + li;
+      bf16x4 tr;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float v = acc[ti][tj][r];
+        const size_t k = (size_t)(row + r) * H + col;
+        if constexpr (OP == TR_L1) {
+          const float z = v + e.bias[col], h = silu(z);
+          e.z1[k] = z;
+          e.row[k] = (__bf16)h;
+          tr[r] = (__bf16)h;
+        } else if constexpr (OP == TR_L2) {
+          const float z = v + e.bias[col], a = e.w3[col] * silu1(z);
+          e.z2[k] = z;
+          e.row[k] = (__bf16)a;
+          tr[r] = (__bf16)a;
+          er[r] += e.w3[col] * silu(z);
+        } else if constexpr (OP == TR_BACK2) {
+          const float a = v * silu1(e.z1[k]);
+          if (e.train) e.v1[k] = v;
+          e.row[k] = (__bf16)a;
+          tr[r] = (__bf16)a;
+        } else if constexpr (OP == TR_JVP1) {
+          const float z = e.z1[k], t = silu1(z) * v;
+          e.t0[k] = v;
+          e.row[k] = (__bf16)t;
+          tr[r] = (__bf16)(e.dE[row + r] * silu(z) + e.cG * t);
+        } else if constexpr (OP == TR_JVP2) {
+          const float z = e.z2[k], w3 = e.w3[col], s = silu1(z), zet = w3 * v * silu2(z);
+          const double de = (double)e.dE[row + r], cg = (double)e.cG;
+          e.row[k] = (__bf16)zet;
+          tr[r] = (__bf16)(e.cG * zet);
+          cs0[tj] += de * (double)(w3 * s) + cg * (double)zet;
+          cs1[tj] += de * (double)silu(z) + cg * (double)(s * v);
+        } else if constexpr (OP == TR_VJP2) {
+          const float z = e.z1[k], s = silu1(z), v1 = e.v1[k], zet = v1 * e.t0[k] * silu2(z) + v * s;
+          tr[r] = (__bf16)(e.cG * zet);
+          cs0[tj] += (double)e.dE[row + r] * (double)(v1 * s) + (double)e.cG * (double)zet;
+        } else {
+          e.out[(size_t)blockIdx.z * e.sOut + (size_t)(row + r) * e.ldo + col] = v;
+        }
+      }
+      if constexpr (OP != TR_PART) {
+        // first half of the concatenated batch: a2, a1, dE h1 + cG tau1; second: h1, zeta2, zeta1
+        const size_t half = OP == TR_L1 || OP == TR_JVP2 || OP == TR_VJP2 ? (size_t)e.B : 0;
+        if (e.train) *reinterpret_cast<bf16x4*>(e.tr + (size_t)col * B2 + half + row) = tr;
+      }
+    }
+    if constexpr (OP == TR_L2) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = er[r];
+        v += __shfl_xor(v, 1);
+        v += __shfl_xor(v, 2);
+        v += __shfl_xor(v, 4);
+        v += __shfl_xor(v, 8);
+        if (li == 0) e.epart[(size_t)(row + r) * (H / 32) + (n0 >> 5) + wn] = v;
+      }
+    }
+  }
+  if constexpr (OP == TR_JVP2 || OP == TR_VJP2) {
+    // this wavefront's 32 rows of each column, in a fixed order
+    const int chunk = (m0 >> 5) + wm;
+    const size_t task = (size_t)(e.B / 32) * H;
+#pragma unroll
+    for (int tj = 0; tj < 2; ++tj) {
+      const int col = n0 + wn * 32 + tj * 16 + li;
+      double a = cs0[tj], b = cs1[tj];
+      a += __shfl_xor(a, 16);
+      a += __shfl_xor(a, 32);
+      if (OP == TR_JVP2) {
+        b += __shfl_xor(b, 16);
+        b += __shfl_xor(b, 32);
+      }
+      if (lg == 0) {
+        const size_t k = (size_t)chunk * H + col;
+        if (OP == TR_VJP2) {
+          e.cpart[k] = a;
+        } else {
+          e.cpart[task + k] = a;
+          e.cpart[2 * task + k] = b;
+        }
+      }
+    }
+  }
 }
 
-// a1 = v1 * silu'(z1)
-__global__ void k_a1(int64_t n, const float* __restrict__ v1, const float* __restrict__ s1, float* __restrict__ a1,
-                     __bf16* __restrict__ a1b) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float a = v1[i] * s1[i];
-  if (a1) a1[i] = a;
-  a1b[i] = (__bf16)a;
+// E = b3 + the partial energies of a row, in order.
+__device__ __forceinline__ float energy_of(const float* __restrict__ epart, int np, int row,
+                                           const float* __restrict__ b3) {
+  double s = 0.0;
+  for (int k = 0; k < np; ++k) s += (double)epart[(size_t)row * np + k];
+  return (float)s + b3[0];
+}
+
+__global__ void k_esum(int rows, int np, const float* __restrict__ epart, const float* __restrict__ b3,
+                       float* __restrict__ E) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < rows) E[r] = energy_of(epart, np, r, b3);
 }
 
 // Per row: residuals of the normalised targets, u = P(g - g_n), loss partials,
-// dE = 2 w_E (E - E_n)/B. One wavefront per row.
-__global__ __launch_bounds__(256) void k_loss(int rows, int Dp, const float* __restrict__ E, const double* __restrict__ e_ref,
-                                              const float* __restrict__ g, const float* __restrict__ g_ref,
-                                              const float* __restrict__ q, double shift, double inv_scale, float w_e,
+// dE = 2 w_E (E - E_n)/B. One wavefront per row, the row's g - g_n in LDS between
+// the two passes. Row r of q and g_ref is row idx[r] of their arrays (idx null: r).
+// The energies come from E, or, E null, from the second layer's partials.
+__global__ __launch_bounds__(256) void k_loss(int rows, int Dp, const float* __restrict__ E,
+                                              const float* __restrict__ epart, int np, const float* __restrict__ b3,
+                                              const double* __restrict__ e_ref, const float* __restrict__ g,
+                                              const float* __restrict__ g_ref, const float* __restrict__ q,
+                                              const int* __restrict__ idx, double shift, double inv_scale, float w_e,
                                               float* __restrict__ u, __bf16* __restrict__ ub, float* __restrict__ dE,
                                               double* __restrict__ le, double* __restrict__ lg) {
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  extern __shared__ float sdiff[];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int row = blockIdx.x * 4 + w;
   if (row >= rows) return;
-  const float* gr = g + (size_t)row * Dp;
-  const float* gf = g_ref + (size_t)row * Dp;
-  const float* qr = q + (size_t)row * Dp;
+  float* diff = sdiff + (size_t)w * Dp;
+  const int src = idx ? idx[row] : row;
+  const float2* gr = reinterpret_cast<const float2*>(g + (size_t)row * Dp);
+  const float2* gf = reinterpret_cast<const float2*>(g_ref + (size_t)src * Dp);
+  const float2* qr = reinterpret_cast<const float2*>(q + (size_t)src * Dp);
   float qd = 0.f;
-  for (int j = lane; j < Dp; j += 64) qd += qr[j] * (gr[j] - (float)(gf[j] * inv_scale));
+  for (int j = lane; j < Dp / 2; j += 64) {
+    const float2 a = gr[j], t = gf[j], x = qr[j];
+    const float d0 = a.x - (float)(t.x * inv_scale), d1 = a.y - (float)(t.y * inv_scale);
+    diff[2 * j] = d0;
+    diff[2 * j + 1] = d1;
+    qd += x.x * d0;
+    qd += x.y * d1;
+  }
   for (int o = 32; o > 0; o >>= 1) qd += __shfl_xor(qd, o);
   float uu = 0.f;
-  for (int j = lane; j < Dp; j += 64) {
-    const size_t k = (size_t)row * Dp + j;
-    const float v = (gr[j] - (float)(gf[j] * inv_scale)) - qr[j] * qd;
-    u[k] = v;
-    ub[k] = (__bf16)v;
-    uu += v * v;
+  for (int j = lane; j < Dp / 2; j += 64) {
+    const float2 x = qr[j];
+    float2 v;
+    v.x = diff[2 * j] - x.x * qd;
+    v.y = diff[2 * j + 1] - x.y * qd;
+    reinterpret_cast<float2*>(u + (size_t)row * Dp)[j] = v;
+    __bf16* o = ub + (size_t)row * Dp + 2 * j;
+    o[0] = (__bf16)v.x;
+    o[1] = (__bf16)v.y;
+    uu += v.x * v.x;
+    uu += v.y * v.y;
   }
   for (int o = 32; o > 0; o >>= 1) uu += __shfl_xor(uu, o);
   if (lane == 0) {
-    const double r = (double)E[row] - (e_ref[row] - shift) * inv_scale;
+    const float en = E ? E[row] : energy_of(epart, np, row, b3);
+    const double r = (double)en - (e_ref[row] - shift) * inv_scale;
     dE[row] = (float)(2.0 * w_e * r / rows);
     le[row] = r * r;
     lg[row] = uu;
   }
 }
 
-// tau1 = silu'(z1) * tau0
-__global__ void k_t1(int64_t n, const float* __restrict__ s1, const float* __restrict__ t0, float* __restrict__ t1,
-                     __bf16* __restrict__ t1b) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float t = s1[i] * t0[i];
-  t1[i] = t;
-  t1b[i] = (__bf16)t;
-}
-
-// gamma2 = silu'(z2) tau2, zeta2 = w3 tau2 silu''(z2)
-__global__ void k_z2(int64_t n, int H, const float* __restrict__ t2, const float* __restrict__ s2p,
-                     const float* __restrict__ s2pp, const float* __restrict__ w3, float* __restrict__ gam2,
-                     float* __restrict__ zet2, __bf16* __restrict__ zet2b) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  gam2[i] = s2p[i] * t2[i];
-  const float z = w3[i % H] * t2[i] * s2pp[i];
-  zet2[i] = z;
-  zet2b[i] = (__bf16)z;
-}
-
-// zeta1 = v1 tau0 silu''(z1) + (W2^T zeta2) silu'(z1)
-__global__ void k_z1(int64_t n, const float* __restrict__ v1, const float* __restrict__ t0,
-                     const float* __restrict__ s1pp, const float* __restrict__ wz, const float* __restrict__ s1,
-                     float* __restrict__ zet1) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  zet1[i] = v1[i] * t0[i] * s1pp[i] + wz[i] * s1[i];
-}
-
-// Transposed BF16 operands of the weight-gradient GEMMs, with the batch of the
-// gradient's two terms concatenated along K (2B columns):
-//   out[c][b]     = bf16(dE[b] P[b][c] + beta U[b][c])   (dE null: P[b][c]; U null: no second term)
-//   out[c][B + b] = bf16(gamma V[b][c])
-// for b < B, c < cols. 64 x 64 tiles go through LDS so that the reads run along
-// c and the writes along b.
-__global__ __launch_bounds__(256) void k_pack_t(int B, int cols, const float* __restrict__ dE,
-                                                const float* __restrict__ P, float beta, const float* __restrict__ U,
-                                                float gamma, const float* __restrict__ V, __bf16* __restrict__ out) {
-  __shared__ float tile[64][65];
-  const int c0 = blockIdx.x * 64, b0 = blockIdx.y * 64, half = blockIdx.z;
+// Transposed BF16 operand of the first layer's weight gradient, with the batch of
+// the gradient's two terms concatenated along K (2B columns): for b < B, c < Dp,
+//   out[c][b]     = bf16(dE[b] q[b][c] + cG u[b][c])
+//   out[c][B + b] = bf16(q[b][c])
+// 64 x 64 tiles go through LDS so that the reads run along c and the writes along
+// b. Row b of q is row idx[b] of its array (idx null: b). B and Dp multiples of 64.
+__global__ __launch_bounds__(256) void k_pack_q(int B, int Dp, const float* __restrict__ dE,
+                                                const float* __restrict__ q, const int* __restrict__ idx, float cG,
+                                                const float* __restrict__ u, __bf16* __restrict__ out) {
+  __shared__ float tq[64][65], tx[64][65];
+  const int c0 = blockIdx.x * 64, b0 = blockIdx.y * 64;
   const int tc = threadIdx.x & 63, tr = threadIdx.x >> 6;
-#pragma unroll 4
-  for (int i = 0; i < 16; ++i) {
-    const int rr = tr + 4 * i, b = b0 + rr, c = c0 + tc;
-    float v = 0.f;
-    if (b < B && c < cols) {
-      const size_t k = (size_t)b * cols + c;
-      if (half == 0) {
-        v = dE ? dE[b] * P[k] : P[k];
-        if (U) v += beta * U[k];
-      } else {
-        v = gamma * V[k];
-      }
+  const int lc = 4 * (threadIdx.x & 15), lr = threadIdx.x >> 4;  // 16-byte loads, 16 rows at a time
+  float4 xq[4], xu[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int b = b0 + lr + 16 * i;
+    xq[i] = *reinterpret_cast<const float4*>(q + (size_t)(idx ? idx[b] : b) * Dp + c0 + lc);
+    xu[i] = *reinterpret_cast<const float4*>(u + (size_t)b * Dp + c0 + lc);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int rr = lr + 16 * i;
+    const float de = dE[b0 + rr];
+    const float qv[4] = {xq[i].x, xq[i].y, xq[i].z, xq[i].w}, uv[4] = {xu[i].x, xu[i].y, xu[i].z, xu[i].w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      tq[rr][lc + k] = qv[k];
+      tx[rr][lc + k] = de * qv[k] + cG * uv[k];
     }
-    tile[rr][tc] = v;
   }
   __syncthreads();
+  // lanes 0..31: the first half's b pairs, 32..63: the second's
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const int half = tc >> 5, bb = 2 * (tc & 31);
 #pragma unroll 4
   for (int i = 0; i < 16; ++i) {
-    const int cc = tr + 4 * i, c = c0 + cc, b = b0 + tc;
-    if (c < cols && b < B) out[(size_t)c * (2 * (size_t)B) + (size_t)half * B + b] = (__bf16)tile[tc][cc];
+    const int cc = tr + 4 * i;
+    bf16x2 v;
+    v[0] = (__bf16)(half ? tq[bb][cc] : tx[bb][cc]);
+    v[1] = (__bf16)(half ? tq[bb + 1][cc] : tx[bb + 1][cc]);
+    *reinterpret_cast<bf16x2*>(out + (size_t)(c0 + cc) * (2 * (size_t)B) + (size_t)half * B + b0 + bb) = v;
   }
 }
 
-// out[i] = sum_z part[z][i] over the split-K partials, in z order.
-__global__ void k_splitk_sum(int64_t n, int nz, const float* __restrict__ part, float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.f;
-  for (int z = 0; z < nz; ++z) s += part[(size_t)z * n + i];
-  out[i] = s;
-}
-
-// Column sums out[j] = sum_b (dE[b] X[b][j] + c Y[b][j]) (X null: X = 1; Y null:
-// no second term) of up to four arrays at once (blockIdx.z), in two fixed-order
-// passes: every 64-row chunk of 64 columns summed by 4 row groups in FP64, then
-// the chunks added in order.
-struct ColTask {
-  const float* X;
-  const float* Y;
-  float c;
-  int cols;
-  float* out;
-};
-struct ColTasks {
-  ColTask t[4];
-  const float* dE;
-  int rows;
+// Weight gradients from their partials, every sum in a fixed order: workgroups
+// [0, n1) add the nz1 K chunks of W1's, the next n2 those of W2's, the next the
+// chunks of 32 rows of the b1, b2 and w3 columns (16 lanes a column, then a fixed
+// xor butterfly), the last one sums dE for b3.
+struct GradArgs {
+  int64_t n1, n2;  // elements of W1, W2
+  int nz1, nz2, H, B, g1, g2, g3;
+  const float *p1, *p2, *dE;
+  const double* cpart;
+  float *W1, *W2, *b1, *b2, *w3, *b3;
 };
 
-__global__ __launch_bounds__(256) void k_colsum_part(ColTasks ts, double* __restrict__ part) {
-  __shared__ double sh[4][64];
-  const ColTask& t = ts.t[blockIdx.z];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int j = blockIdx.x * 64 + tx;
-  const int r0 = blockIdx.y * 64, r1 = min(ts.rows, r0 + 64);
-  double acc = 0.0;
-  if (j < t.cols)
-    for (int b = r0 + ty; b < r1; b += 4) {
-      double v = (double)ts.dE[b] * (t.X ? (double)t.X[(size_t)b * t.cols + j] : 1.0);
-      if (t.Y) v += (double)t.c * (double)t.Y[(size_t)b * t.cols + j];
-      acc += v;
+__global__ __launch_bounds__(256) void k_grad_finish(GradArgs a) {
+  __shared__ double sh[256];
+  int blk = blockIdx.x;
+  if (blk < a.g1 + a.g2) {
+    const bool first = blk < a.g1;
+    const int64_t n = first ? a.n1 : a.n2;
+    const int nz = first ? a.nz1 : a.nz2;
+    const float4* p = reinterpret_cast<const float4*>(first ? a.p1 : a.p2);
+    const int64_t i = (int64_t)(first ? blk : blk - a.g1) * 256 + threadIdx.x;
+    if (i >= n / 4) return;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int z = 0; z < nz; ++z) {
+      const float4 v = p[(size_t)z * (n / 4) + i];
+      s.x += v.x;
+      s.y += v.y;
+      s.z += v.z;
+      s.w += v.w;
     }
-  sh[ty][tx] = acc;
-  __syncthreads();
-  if (ty == 0 && j < t.cols)
-    part[((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x * 64 + j] = (sh[0][tx] + sh[1][tx]) + (sh[2][tx] + sh[3][tx]);
-}
-
-__global__ void k_colsum_fin(ColTasks ts, int nch, int ldp, const double* __restrict__ part) {
-  const ColTask& t = ts.t[blockIdx.z];
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= t.cols) return;
+    reinterpret_cast<float4*>(first ? a.W1 : a.W2)[i] = s;
+    return;
+  }
+  blk -= a.g1 + a.g2;
+  if (blk < a.g3) {
+    const int t = threadIdx.x & 15, c = (blk * 256 + (int)threadIdx.x) >> 4;  // column of the three tasks
+    const int task = c / a.H, j = c - task * a.H, nch = a.B / 32;
+    double s = 0.0;
+    if (task < 3)
+      for (int k = t; k < nch; k += 16) s += a.cpart[((size_t)task * nch + k) * a.H + j];
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (task < 3 && t == 0) (task == 0 ? a.b1 : task == 1 ? a.b2 : a.w3)[j] = (float)s;
+    return;
+  }
   double s = 0.0;
-  for (int k = 0; k < nch; ++k) s += part[((size_t)blockIdx.z * nch + k) * ldp + j];
-  t.out[j] = (float)s;
+  for (int b = threadIdx.x; b < a.B; b += 256) s += (double)a.dE[b];
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) a.b3[0] = (float)sh[0];
 }
 
+__device__ __forceinline__ void pack_weight(int64_t i, int H, int Dp, int64_t oW2, float x, __bf16* __restrict__ W1b,
+                                            __bf16* __restrict__ W1Tb, __bf16* __restrict__ W2b,
+                                            __bf16* __restrict__ W2Tb) {
+  const int64_t n1 = (int64_t)H * Dp, k = i - oW2;
+  const __bf16 v = (__bf16)x;
+  if (i < n1) {
+    const int h = (int)(i / Dp), d = (int)(i % Dp);
+    W1b[i] = v;
+    W1Tb[(size_t)d * H + h] = v;
+  } else if (k >= 0 && k < (int64_t)H * H) {
+    W2b[k] = v;
+    W2Tb[(size_t)(k % H) * H + k / H] = v;
+  }
+}
+
+// Adam, and the BF16 copies of the new weights.
 __global__ void k_adam(int64_t n, float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, float lr, float b1, float b2, float c1, float c2, float eps) {
+                       float* __restrict__ v, float lr, float b1, float b2, float c1, float c2, float eps, int H, int Dp,
+                       int64_t oW2, __bf16* __restrict__ W1b, __bf16* __restrict__ W1Tb, __bf16* __restrict__ W2b,
+                       __bf16* __restrict__ W2Tb) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float gi = g[i];
@@ -247,40 +429,33 @@ __global__ void k_adam(int64_t n, float* __restrict__ w, const float* __restrict
   const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
   m[i] = mi;
   v[i] = vi;
-  w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  const float x = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  w[i] = x;
+  pack_weight(i, H, Dp, oW2, x, W1b, W1Tb, W2b, W2Tb);
 }
 
 // BF16 copies of W1 [H][Dp], W1^T [Dp][H], W2 [H][H], W2^T [H][H].
-__global__ void k_pack(int H, int Dp, const float* __restrict__ W1, const float* __restrict__ W2, __bf16* __restrict__ W1b,
+__global__ void k_pack(int64_t n, int H, int Dp, int64_t oW2, const float* __restrict__ w, __bf16* __restrict__ W1b,
                        __bf16* __restrict__ W1Tb, __bf16* __restrict__ W2b, __bf16* __restrict__ W2Tb) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n1 = (int64_t)H * Dp;
-  if (i < n1) {
-    const int h = (int)(i / Dp), d = (int)(i % Dp);
-    const __bf16 v = (__bf16)W1[i];
-    W1b[i] = v;
-    W1Tb[(size_t)d * H + h] = v;
-  } else if (i < n1 + (int64_t)H * H) {
-    const int64_t k = i - n1;
-    const int a = (int)(k / H), b = (int)(k % H);
-    const __bf16 v = (__bf16)W2[k];
-    W2b[k] = v;
-    W2Tb[(size_t)b * H + a] = v;
-  }
+  if (i < n) pack_weight(i, H, Dp, oW2, w[i], W1b, W1Tb, W2b, W2Tb);
 }
 
-// Gather dataset rows into the batch buffers.
+// The batch's BF16 descriptors and energies from the dataset rows idx; the FP32
+// rows are read in place (k_loss, k_pack_q).
 __global__ void k_gather_rows(int rows, int Dp, const int* __restrict__ idx, const float* __restrict__ q,
-                              const float* __restrict__ g, const double* __restrict__ e, float* __restrict__ bq,
-                              __bf16* __restrict__ bqb, float* __restrict__ bg, double* __restrict__ be) {
+                              const double* __restrict__ e, __bf16* __restrict__ bqb, double* __restrict__ be) {
   const int r = blockIdx.x;
   if (r >= rows) return;
   const int src = idx[r];
-  for (int j = threadIdx.x; j < Dp; j += blockDim.x) {
-    const float v = q[(size_t)src * Dp + j];
-    bq[(size_t)r * Dp + j] = v;
-    bqb[(size_t)r * Dp + j] = (__bf16)v;
-    bg[(size_t)r * Dp + j] = g[(size_t)src * Dp + j];
+  for (int j = threadIdx.x; j < Dp / 4; j += blockDim.x) {
+    const float4 v = reinterpret_cast<const float4*>(q + (size_t)src * Dp)[j];
+    bf16x4 o;
+    o[0] = (__bf16)v.x;
+    o[1] = (__bf16)v.y;
+    o[2] = (__bf16)v.z;
+    o[3] = (__bf16)v.w;
+    reinterpret_cast<bf16x4*>(bqb + (size_t)r * Dp)[j] = o;
   }
   if (threadIdx.x == 0) be[r] = e[src];
 }
@@ -427,16 +602,24 @@ struct tgx_mlp {
   int n = 0, cap = 0;
   dbuf dq, dg, de;
   // batch work space
-  dbuf idx, bq, bqb, bg, be, z1, h1, h1b, s1, s1pp, z2, h2, a2, a2b, s2p, s2pp, E, v1, a1, a1b, G, u, ub, t0, t1, t1b,
-      t2, gam2, zet2, zet2b, wz, zet1, dE, packA, packB, cpart, kpart, lossb;
+  dbuf idx, bq, bqb, bg, be, z1, z2, v1, t0, h1b, a2b, a1b, t1b, zet2b, E, epart, G, u, ub, dE, packA1, packA2, packB1,
+      packB2, cpart, kpart, lossb;
   dbuf fdg;  // force-loss step: -(g_hat - g) rows in FP64
   uint64_t seed = 0;
 };
 
+// K chunks of a weight gradient M x N (K = 2B): enough 64 x 64 tiles for two to
+// three workgroups per CU, at least 256 of K each.
+static int wgrad_chunks(int M, int N, int K) {
+  const int tiles = (M / 64) * (N / 64);
+  int nz = 1;
+  while (nz < 64 && tiles * nz * 2 <= 768 && (K / (nz * 2)) % 64 == 0 && K / (nz * 2) >= 256) nz *= 2;
+  return nz;
+}
+
 static int mlp_workspace(tgx_mlp* m, int B) {
   const size_t H = m->H, Dp = m->Dp, b = (size_t)B;
-  dbuf* f_bh[] = {&m->z1, &m->h1, &m->s1, &m->s1pp, &m->z2, &m->h2, &m->a2, &m->s2p, &m->s2pp, &m->v1, &m->a1,
-                  &m->t0, &m->t1, &m->t2, &m->gam2, &m->zet2, &m->wz, &m->zet1};
+  dbuf* f_bh[] = {&m->z1, &m->z2, &m->v1, &m->t0};
   for (dbuf* x : f_bh) TGX_TRY(x->ensure(sizeof(float) * b * H));
   dbuf* h_bh[] = {&m->h1b, &m->a2b, &m->a1b, &m->t1b, &m->zet2b};
   for (dbuf* x : h_bh) TGX_TRY(x->ensure(sizeof(__bf16) * b * H));
@@ -446,22 +629,23 @@ static int mlp_workspace(tgx_mlp* m, int B) {
   TGX_TRY(m->ub.ensure(sizeof(__bf16) * b * Dp));
   TGX_TRY(m->be.ensure(sizeof(double) * b));
   TGX_TRY(m->E.ensure(sizeof(float) * b));
+  TGX_TRY(m->epart.ensure(sizeof(float) * b * (H / 32)));
   TGX_TRY(m->dE.ensure(sizeof(float) * b));
   TGX_TRY(m->lossb.ensure(sizeof(double) * 2 * b));
   TGX_TRY(m->idx.ensure(sizeof(int) * b));
   // weight-gradient operands over the concatenated batch, column-sum partials
-  TGX_TRY(m->packA.ensure(sizeof(__bf16) * H * 2 * b));
-  TGX_TRY(m->packB.ensure(sizeof(__bf16) * (Dp > H ? Dp : H) * 2 * b));
-  TGX_TRY(m->cpart.ensure(sizeof(double) * 4 * ((b + 63) / 64) * (size_t)tgx_round_up((int64_t)H, 64)));
+  dbuf* packs[] = {&m->packA1, &m->packA2, &m->packB2};
+  for (dbuf* x : packs) TGX_TRY(x->ensure(sizeof(__bf16) * H * 2 * b));
+  TGX_TRY(m->packB1.ensure(sizeof(__bf16) * Dp * 2 * b));
+  TGX_TRY(m->cpart.ensure(sizeof(double) * 3 * (b / 32) * H));
   return TGX_OK;
 }
 
 static int mlp_pack(tgx_mlp* m) {
   tgx_ctx* ctx = m->ctx;
-  const float* th = m->theta.as<float>();
-  const int64_t n = (int64_t)m->H * m->Dp + (int64_t)m->H * m->H;
-  TGX_LAUNCH(ctx, "mlp_pack", k_pack, g1(n), dim3(256), 0, m->H, m->Dp, th + m->oW1, th + m->oW2, m->W1b.as<__bf16>(),
-             m->W1Tb.as<__bf16>(), m->W2b.as<__bf16>(), m->W2Tb.as<__bf16>());
+  TGX_LAUNCH(ctx, "mlp_pack", k_pack, g1(m->nparam), dim3(256), 0, m->nparam, m->H, m->Dp, m->oW2,
+             (const float*)m->theta.as<float>(), m->W1b.as<__bf16>(), m->W1Tb.as<__bf16>(), m->W2b.as<__bf16>(),
+             m->W2Tb.as<__bf16>());
   return TGX_OK;
 }
 
@@ -519,10 +703,9 @@ extern "C" int tgx_mlp_destroy(tgx_mlp* m) {
   (void)hipSetDevice(m->ctx->device);
   (void)hipStreamSynchronize(m->ctx->stream);
   dbuf* all[] = {&m->theta, &m->grad, &m->mom, &m->vel, &m->W1b, &m->W1Tb, &m->W2b, &m->W2Tb, &m->dq, &m->dg, &m->de,
-                 &m->idx, &m->bq, &m->bqb, &m->bg, &m->be, &m->z1, &m->h1, &m->h1b, &m->s1, &m->s1pp, &m->z2, &m->h2,
-                 &m->a2, &m->a2b, &m->s2p, &m->s2pp, &m->E, &m->v1, &m->a1, &m->a1b, &m->G, &m->u, &m->ub, &m->t0,
-                 &m->t1, &m->t1b, &m->t2, &m->gam2, &m->zet2, &m->zet2b, &m->wz, &m->zet1, &m->dE, &m->packA,
-                 &m->packB, &m->cpart, &m->kpart, &m->lossb, &m->fdg};
+                 &m->idx, &m->bq, &m->bqb, &m->bg, &m->be, &m->z1, &m->z2, &m->v1, &m->t0, &m->h1b, &m->a2b, &m->a1b,
+                 &m->t1b, &m->zet2b, &m->E, &m->epart, &m->G, &m->u, &m->ub, &m->dE, &m->packA1, &m->packA2,
+                 &m->packB1, &m->packB2, &m->cpart, &m->kpart, &m->lossb, &m->fdg};
   for (dbuf* b : all) b->release();
   delete m;
   return TGX_OK;
@@ -530,75 +713,72 @@ extern "C" int tgx_mlp_destroy(tgx_mlp* m) {
 
 // Forward (energy and input gradient) on B rows of bqb (BF16) held in the batch
 // buffers. With training copies when `train`.
+template <int OP>
+static int train_gemm(tgx_ctx* ctx, const char* name, int M, int N, int K, int nz, const __bf16* A, int lda,
+                      const __bf16* B, int ldb, const TrainArgs& e) {
+  TGX_REQUIRE(M % 64 == 0 && N % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldb % 8 == 0 && nz >= 1,
+              "train_gemm %s: unpadded shape %d x %d x %d", name, M, N, K);
+  TGX_LAUNCH(ctx, name, k_train_gemm<OP>, dim3(N / 64, M / 64, nz), dim3(256), 0, K, A, lda, B, ldb, e);
+  return TGX_OK;
+}
+
+// The arguments shared by a batch's products.
+static TrainArgs train_args(tgx_mlp* m, int B, bool train) {
+  TrainArgs e{};
+  e.B = B;
+  e.H = m->H;
+  e.train = train;
+  e.w3 = m->theta.as<float>() + m->ow3;
+  e.z1 = m->z1.as<float>();
+  e.z2 = m->z2.as<float>();
+  e.v1 = m->v1.as<float>();
+  e.t0 = m->t0.as<float>();
+  e.dE = m->dE.as<float>();
+  e.epart = m->epart.as<float>();
+  e.cpart = m->cpart.as<double>();
+  return e;
+}
+
+// E (E_out; null leaves the partial energies to k_loss) and G = dE/dq of B rows xb.
 static int mlp_forward(tgx_mlp* m, int B, const __bf16* xb, bool train, float* E_out, float* G_out, double gscale) {
   tgx_ctx* ctx = m->ctx;
   const int H = m->H, Dp = m->Dp;
   const float* th = m->theta.as<float>();
-  const int64_t nbh = (int64_t)B * H;
-  TGX_TRY(tgx_gemm_bf16_nt(ctx, "mlp_l1", B, H, Dp, xb, Dp, m->W1b.as<__bf16>(), Dp, m->z1.as<float>(), H, 1.0));
-  TGX_LAUNCH(ctx, "mlp_act1", k_l1, g1(nbh), dim3(256), 0, nbh, H, m->z1.as<float>(), th + m->ob1, m->h1b.as<__bf16>(),
-             train ? m->h1.as<float>() : nullptr, m->s1.as<float>(), train ? m->s1pp.as<float>() : nullptr);
-  TGX_TRY(tgx_gemm_bf16_nt(ctx, "mlp_l2", B, H, H, m->h1b.as<__bf16>(), H, m->W2b.as<__bf16>(), H, m->z2.as<float>(), H,
-                           1.0));
-  TGX_LAUNCH(ctx, "mlp_act2", k_l2, dim3((B + 3) / 4), dim3(256), 0, B, H, m->z2.as<float>(), th + m->ob2, th + m->ow3,
-             th + m->ob3, E_out, m->a2b.as<__bf16>(), train ? m->a2.as<float>() : nullptr,
-             train ? m->h2.as<float>() : nullptr, train ? m->s2p.as<float>() : nullptr,
-             train ? m->s2pp.as<float>() : nullptr);
-  TGX_TRY(tgx_gemm_bf16_nt(ctx, "mlp_back2", B, H, H, m->a2b.as<__bf16>(), H, m->W2Tb.as<__bf16>(), H, m->v1.as<float>(),
-                           H, 1.0));
-  TGX_LAUNCH(ctx, "mlp_a1", k_a1, g1(nbh), dim3(256), 0, nbh, m->v1.as<float>(), m->s1.as<float>(),
-             train ? m->a1.as<float>() : nullptr, m->a1b.as<__bf16>());
-  TGX_TRY(tgx_gemm_bf16_nt(ctx, "mlp_back1", B, Dp, H, m->a1b.as<__bf16>(), H, m->W1Tb.as<__bf16>(), H, G_out, Dp,
-                           gscale));
-  return TGX_OK;
+  TrainArgs e = train_args(m, B, train);
+  e.bias = th + m->ob1;
+  e.row = m->h1b.as<__bf16>();
+  e.tr = m->packB2.as<__bf16>();
+  TGX_TRY(train_gemm<TR_L1>(ctx, "mlp_l1", B, H, Dp, 1, xb, Dp, m->W1b.as<__bf16>(), Dp, e));
+  e.bias = th + m->ob2;
+  e.row = m->a2b.as<__bf16>();
+  e.tr = m->packA2.as<__bf16>();
+  TGX_TRY(train_gemm<TR_L2>(ctx, "mlp_l2", B, H, H, 1, m->h1b.as<__bf16>(), H, m->W2b.as<__bf16>(), H, e));
+  if (E_out)
+    TGX_LAUNCH(ctx, "mlp_esum", k_esum, dim3((B + 255) / 256), dim3(256), 0, B, H / 32,
+               (const float*)m->epart.as<float>(), th + m->ob3, E_out);
+  e.row = m->a1b.as<__bf16>();
+  e.tr = m->packA1.as<__bf16>();
+  TGX_TRY(train_gemm<TR_BACK2>(ctx, "mlp_back2", B, H, H, 1, m->a2b.as<__bf16>(), H, m->W2Tb.as<__bf16>(), H, e));
+  return tgx_gemm_bf16_nt(ctx, "mlp_back1", B, Dp, H, m->a1b.as<__bf16>(), H, m->W1Tb.as<__bf16>(), H, G_out, Dp,
+                          gscale);
 }
 
-// C[M][N] = A[M][K] B[N][K]^T (BF16 operands, FP32) for the weight gradients, whose
-// M x N grid has few tiles against a long K: K is split into nz chunks run as a
-// batch of GEMMs into FP32 partials, which are then added in chunk order.
-static int wgrad_gemm(tgx_mlp* m, const char* name, int M, int N, int K, const __bf16* A, const __bf16* B, float* C) {
-  tgx_ctx* ctx = m->ctx;
-  const int tiles = (M / 128) * (N / 128);
-  int nz = 1;
-  while (nz < 32 && tiles * nz * 2 <= 1024 && (K / (nz * 2)) % 64 == 0 && K / (nz * 2) >= 256) nz *= 2;
-  if (nz == 1) return tgx_gemm_bf16_nt(ctx, name, M, N, K, A, K, B, K, C, N, 1.0);
-  const int64_t mn = (int64_t)M * N;
-  TGX_TRY(m->kpart.ensure(sizeof(float) * (size_t)(nz * mn)));
-  tgx_gemm_desc d;
-  d.epi = TGX_EPI_STORE_F32;
-  d.M = M;
-  d.N = N;
-  d.K = K / nz;
-  d.batch = nz;
-  d.A = A;
-  d.lda = K;
-  d.sA = K / nz;
-  d.B = B;
-  d.ldb = K;
-  d.sB = K / nz;
-  d.C = m->kpart.p;
-  d.ldc = N;
-  d.sC = mn;
-  d.scale = 1.0;
-  TGX_TRY(tgx_gemm_bf16(ctx, name, d));
-  TGX_LAUNCH(ctx, "mlp_splitk_sum", k_splitk_sum, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, mn, nz,
-             (const float*)m->kpart.as<float>(), C);
-  return TGX_OK;
-}
+static int mlp_backward_dirs(tgx_mlp* m, int B, float cG, const float* q, const int* idx);
 
-static int mlp_backward_dirs(tgx_mlp* m, int B, float cG);
-
-// Loss and weight gradients of the batch in the batch buffers (bq, bqb, bg, be).
-static int mlp_backward(tgx_mlp* m, int B, float w_e, float w_g, double* loss_e, double* loss_g) {
+// Loss and weight gradients of the batch in bqb and be, with the FP32 descriptors
+// and target gradients in rows idx of q and g (idx null: the first B rows).
+static int mlp_backward(tgx_mlp* m, int B, const float* q, const float* g, const int* idx, float w_e, float w_g,
+                        double* loss_e, double* loss_g) {
   tgx_ctx* ctx = m->ctx;
   const int Dp = m->Dp;
-  TGX_TRY(mlp_forward(m, B, m->bqb.as<__bf16>(), true, m->E.as<float>(), m->G.as<float>(), 1.0));
+  TGX_TRY(mlp_forward(m, B, m->bqb.as<__bf16>(), true, nullptr, m->G.as<float>(), 1.0));
   double* le = m->lossb.as<double>();
   double* lg = le + B;
-  TGX_LAUNCH(ctx, "mlp_loss", k_loss, dim3((B + 3) / 4), dim3(256), 0, B, Dp, m->E.as<float>(), m->be.as<double>(),
-             m->G.as<float>(), m->bg.as<float>(), m->bq.as<float>(), m->shift, 1.0 / m->scale, w_e, m->u.as<float>(),
-             m->ub.as<__bf16>(), m->dE.as<float>(), le, lg);
-  TGX_TRY(mlp_backward_dirs(m, B, 2.0f * w_g / (float)B));
+  TGX_LAUNCH(ctx, "mlp_loss", k_loss, dim3((B + 3) / 4), dim3(256), sizeof(float) * 4 * Dp, B, Dp, (const float*)nullptr,
+             (const float*)m->epart.as<float>(), m->H / 32, m->theta.as<float>() + m->ob3, m->be.as<double>(),
+             m->G.as<float>(), g, q, idx, m->shift, 1.0 / m->scale, w_e, m->u.as<float>(), m->ub.as<__bf16>(),
+             m->dE.as<float>(), le, lg);
+  TGX_TRY(mlp_backward_dirs(m, B, 2.0f * w_g / (float)B, q, idx));
   if (loss_e || loss_g) {
     double se = 0.0, sg = 0.0;
     TGX_TRY(tgx_device_sum(ctx, le, B, &se));
@@ -613,53 +793,62 @@ static int mlp_backward(tgx_mlp* m, int B, float w_e, float w_g, double* loss_e,
 // the energy residual weights dE (per row) and the gradient-loss direction u
 // (FP32 and BF16 rows) with its weight cG: the reverse-mode derivative of
 // sum_b dE_b E_b + cG u_b . g_b with dE and u fixed.
-static int mlp_backward_dirs(tgx_mlp* m, int B, float cG) {
+//   dW1 = a1^T (dE q + cG u) + cG zeta1^T q = [a1 | cG zeta1]^T [dE q + cG u ; q]
+//   dW2 = a2^T (dE h1 + cG tau1) + cG zeta2^T h1 = [a2 | cG zeta2]^T [dE h1 + cG tau1 ; h1]
+// each one BF16 product over the concatenated batch (K = 2B); the products before
+// them write those operands transposed as they go.
+static int mlp_backward_dirs(tgx_mlp* m, int B, float cG, const float* q, const int* idx) {
   tgx_ctx* ctx = m->ctx;
   const int H = m->H, Dp = m->Dp;
-  const int64_t nbh = (int64_t)B * H;
-  float* th = m->theta.as<float>();
   float* gr = m->grad.as<float>();
+  TrainArgs e = train_args(m, B, true);
+  e.cG = cG;
+  TGX_LAUNCH(ctx, "mlp_pack_q", k_pack_q, dim3(Dp / 64, B / 64), dim3(256), 0, B, Dp, (const float*)m->dE.as<float>(), q,
+             idx, cG, (const float*)m->u.as<float>(), m->packB1.as<__bf16>());
   // forward mode along u, then reverse
-  TGX_TRY(tgx_gemm_bf16_nt(ctx, "mlp_jvp1", B, H, Dp, m->ub.as<__bf16>(), Dp, m->W1b.as<__bf16>(), Dp, m->t0.as<float>(),
-                           H, 1.0));
-  TGX_LAUNCH(ctx, "mlp_t1", k_t1, g1(nbh), dim3(256), 0, nbh, m->s1.as<float>(), m->t0.as<float>(), m->t1.as<float>(),
-             m->t1b.as<__bf16>());
-  TGX_TRY(tgx_gemm_bf16_nt(ctx, "mlp_jvp2", B, H, H, m->t1b.as<__bf16>(), H, m->W2b.as<__bf16>(), H, m->t2.as<float>(),
-                           H, 1.0));
-  TGX_LAUNCH(ctx, "mlp_z2", k_z2, g1(nbh), dim3(256), 0, nbh, H, m->t2.as<float>(), m->s2p.as<float>(),
-             m->s2pp.as<float>(), th + m->ow3, m->gam2.as<float>(), m->zet2.as<float>(), m->zet2b.as<__bf16>());
-  TGX_TRY(tgx_gemm_bf16_nt(ctx, "mlp_vjp2", B, H, H, m->zet2b.as<__bf16>(), H, m->W2Tb.as<__bf16>(), H,
-                           m->wz.as<float>(), H, 1.0));
-  TGX_LAUNCH(ctx, "mlp_z1", k_z1, g1(nbh), dim3(256), 0, nbh, m->v1.as<float>(), m->t0.as<float>(), m->s1pp.as<float>(),
-             m->wz.as<float>(), m->s1.as<float>(), m->zet1.as<float>());
-  // dW1 = a1^T (dE q + cG u) + cG zeta1^T q = [a1 | cG zeta1]^T [dE q + cG u ; q], one
-  // BF16 GEMM with FP32 accumulation over the concatenated batch (K = 2B)
-  const dim3 gH(H / 64, B / 64, 2), gD(Dp / 64, B / 64, 2);
-  __bf16* pA = m->packA.as<__bf16>();
-  __bf16* pB = m->packB.as<__bf16>();
-  TGX_LAUNCH(ctx, "mlp_packA1", k_pack_t, gH, dim3(256), 0, B, H, (const float*)nullptr, m->a1.as<float>(), 0.0f,
-             (const float*)nullptr, cG, m->zet1.as<float>(), pA);
-  TGX_LAUNCH(ctx, "mlp_packB1", k_pack_t, gD, dim3(256), 0, B, Dp, m->dE.as<float>(), m->bq.as<float>(), cG,
-             m->u.as<float>(), 1.0f, m->bq.as<float>(), pB);
-  TGX_TRY(wgrad_gemm(m, "mlp_dW1", H, Dp, 2 * B, pA, pB, gr + m->oW1));
-  // dW2 = a2^T (dE h1 + cG tau1) + cG zeta2^T h1 = [a2 | cG zeta2]^T [dE h1 + cG tau1 ; h1]
-  TGX_LAUNCH(ctx, "mlp_packA2", k_pack_t, gH, dim3(256), 0, B, H, (const float*)nullptr, m->a2.as<float>(), 0.0f,
-             (const float*)nullptr, cG, m->zet2.as<float>(), pA);
-  TGX_LAUNCH(ctx, "mlp_packB2", k_pack_t, gH, dim3(256), 0, B, H, m->dE.as<float>(), m->h1.as<float>(), cG,
-             m->t1.as<float>(), 1.0f, m->h1.as<float>(), pB);
-  TGX_TRY(wgrad_gemm(m, "mlp_dW2", H, H, 2 * B, pA, pB, gr + m->oW2));
-  // biases and output weights: fixed-order column sums over 64-row chunks
-  ColTasks ct{};
-  ct.dE = m->dE.as<float>();
-  ct.rows = B;
-  ct.t[0] = ColTask{m->a1.as<float>(), m->zet1.as<float>(), cG, H, gr + m->ob1};
-  ct.t[1] = ColTask{m->a2.as<float>(), m->zet2.as<float>(), cG, H, gr + m->ob2};
-  ct.t[2] = ColTask{m->h2.as<float>(), m->gam2.as<float>(), cG, H, gr + m->ow3};
-  ct.t[3] = ColTask{nullptr, nullptr, 0.0f, 1, gr + m->ob3};
-  const int nch = (B + 63) / 64, ldp = (int)tgx_round_up(H, 64);
-  TGX_LAUNCH(ctx, "mlp_colsum", k_colsum_part, dim3(ldp / 64, nch, 4), dim3(256), 0, ct, m->cpart.as<double>());
-  TGX_LAUNCH(ctx, "mlp_colsum_fin", k_colsum_fin, dim3((ldp + 63) / 64, 1, 4), dim3(64), 0, ct, nch, ldp,
-             (const double*)m->cpart.as<double>());
+  e.row = m->t1b.as<__bf16>();
+  e.tr = m->packB2.as<__bf16>();
+  TGX_TRY(train_gemm<TR_JVP1>(ctx, "mlp_jvp1", B, H, Dp, 1, m->ub.as<__bf16>(), Dp, m->W1b.as<__bf16>(), Dp, e));
+  e.row = m->zet2b.as<__bf16>();
+  e.tr = m->packA2.as<__bf16>();
+  TGX_TRY(train_gemm<TR_JVP2>(ctx, "mlp_jvp2", B, H, H, 1, m->t1b.as<__bf16>(), H, m->W2b.as<__bf16>(), H, e));
+  e.tr = m->packA1.as<__bf16>();
+  TGX_TRY(train_gemm<TR_VJP2>(ctx, "mlp_vjp2", B, H, H, 1, m->zet2b.as<__bf16>(), H, m->W2Tb.as<__bf16>(), H, e));
+  // the weight gradients' K chunks, then every sum in one launch
+  GradArgs a{};
+  a.n1 = (int64_t)H * Dp;
+  a.n2 = (int64_t)H * H;
+  a.nz1 = wgrad_chunks(H, Dp, 2 * B);
+  a.nz2 = wgrad_chunks(H, H, 2 * B);
+  TGX_TRY(m->kpart.ensure(sizeof(float) * (size_t)(a.nz1 * a.n1 + a.nz2 * a.n2)));
+  float* p1 = m->kpart.as<float>();
+  float* p2 = p1 + a.nz1 * a.n1;
+  e.out = p1;
+  e.ldo = Dp;
+  e.sOut = a.n1;
+  TGX_TRY(train_gemm<TR_PART>(ctx, "mlp_dW1", H, Dp, 2 * B / a.nz1, a.nz1, m->packA1.as<__bf16>(), 2 * B,
+                              m->packB1.as<__bf16>(), 2 * B, e));
+  e.out = p2;
+  e.ldo = H;
+  e.sOut = a.n2;
+  TGX_TRY(train_gemm<TR_PART>(ctx, "mlp_dW2", H, H, 2 * B / a.nz2, a.nz2, m->packA2.as<__bf16>(), 2 * B,
+                              m->packB2.as<__bf16>(), 2 * B, e));
+  a.p1 = p1;
+  a.p2 = p2;
+  a.H = H;
+  a.B = B;
+  a.dE = m->dE.as<float>();
+  a.cpart = m->cpart.as<double>();
+  a.W1 = gr + m->oW1;
+  a.W2 = gr + m->oW2;
+  a.b1 = gr + m->ob1;
+  a.b2 = gr + m->ob2;
+  a.w3 = gr + m->ow3;
+  a.b3 = gr + m->ob3;
+  a.g1 = (int)((a.n1 / 4 + 255) / 256);
+  a.g2 = (int)((a.n2 / 4 + 255) / 256);
+  a.g3 = (3 * H * 16 + 255) / 256;
+  TGX_LAUNCH(ctx, "mlp_grad_finish", k_grad_finish, dim3(a.g1 + a.g2 + a.g3 + 1), dim3(256), 0, a);
   return TGX_OK;
 }
 
@@ -735,10 +924,11 @@ static int adam_step(tgx_mlp* m, float lr) {
   m->step += 1;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.f - (float)std::pow(b1, (double)m->step), c2 = 1.f - (float)std::pow(b2, (double)m->step);
-  TGX_LAUNCH(m->ctx, "mlp_adam", k_adam, g1(m->nparam), dim3(256), 0, m->nparam, m->theta.as<float>(),
-             m->grad.as<float>(), m->mom.as<float>(), m->vel.as<float>(), lr, b1, b2, c1, c2, 1e-8f);
   // padded columns of W1 stay zero: their gradient is zero (q is zero there)
-  return mlp_pack(m);
+  TGX_LAUNCH(m->ctx, "mlp_adam", k_adam, g1(m->nparam), dim3(256), 0, m->nparam, m->theta.as<float>(),
+             m->grad.as<float>(), m->mom.as<float>(), m->vel.as<float>(), lr, b1, b2, c1, c2, 1e-8f, m->H, m->Dp, m->oW2,
+             m->W1b.as<__bf16>(), m->W1Tb.as<__bf16>(), m->W2b.as<__bf16>(), m->W2Tb.as<__bf16>());
+  return TGX_OK;
 }
 
 extern "C" int tgx_mlp_train(tgx_mlp* m, int n_train, int epochs, int batch, float lr, float w_e, float w_g,
@@ -761,16 +951,13 @@ extern "C" int tgx_mlp_train(tgx_mlp* m, int n_train, int epochs, int batch, flo
     for (int b0 = 0; b0 + batch <= n_train; b0 += batch) {
       TGX_CHECK_HIP(hipMemcpyAsync(m->idx.p, p.data() + b0, sizeof(int) * batch, hipMemcpyHostToDevice, ctx->stream));
       TGX_LAUNCH(ctx, "mlp_gather", k_gather_rows, dim3(batch), dim3(256), 0, batch, m->Dp, m->idx.as<int>(),
-                 m->dq.as<float>(), m->dg.as<float>(), m->de.as<double>(), m->bq.as<float>(), m->bqb.as<__bf16>(),
-                 m->bg.as<float>(), m->be.as<double>());
+                 m->dq.as<float>(), m->de.as<double>(), m->bqb.as<__bf16>(), m->be.as<double>());
       double le = 0.0, lg = 0.0;
-      const bool last = b0 + 2 * batch > n_train;
-      TGX_TRY(mlp_backward(m, batch, w_e, w_g, (ep == epochs - 1) ? &le : nullptr, (ep == epochs - 1) ? &lg : nullptr));
+      TGX_TRY(mlp_backward(m, batch, m->dq.as<float>(), m->dg.as<float>(), m->idx.as<int>(), w_e, w_g, (ep == epochs - 1) ? &le : nullptr, (ep == epochs - 1) ? &lg : nullptr));
       TGX_TRY(adam_step(m, lr));
       le_sum += le;
       lg_sum += lg;
       ++nb;
-      (void)last;
     }
   }
   TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
@@ -795,12 +982,12 @@ extern "C" int tgx_mlp_evaluate(tgx_mlp* m, int begin, int end, double* e_mae, d
     for (int r = 0; r < B; ++r) idx[r] = b0 + std::min(r, rows - 1);
     TGX_CHECK_HIP(hipMemcpyAsync(m->idx.p, idx.data(), sizeof(int) * B, hipMemcpyHostToDevice, ctx->stream));
     TGX_LAUNCH(ctx, "mlp_gather", k_gather_rows, dim3(B), dim3(256), 0, B, m->Dp, m->idx.as<int>(), m->dq.as<float>(),
-               m->dg.as<float>(), m->de.as<double>(), m->bq.as<float>(), m->bqb.as<__bf16>(), m->bg.as<float>(),
-               m->be.as<double>());
+               m->de.as<double>(), m->bqb.as<__bf16>(), m->be.as<double>());
     TGX_TRY(mlp_forward(m, B, m->bqb.as<__bf16>(), false, m->E.as<float>(), m->G.as<float>(), 1.0));
     double* le = m->lossb.as<double>();
-    TGX_LAUNCH(ctx, "mlp_loss", k_loss, dim3((B + 3) / 4), dim3(256), 0, B, m->Dp, m->E.as<float>(), m->be.as<double>(),
-               m->G.as<float>(), m->bg.as<float>(), m->bq.as<float>(), m->shift, 1.0 / m->scale, 1.0f,
+    TGX_LAUNCH(ctx, "mlp_loss", k_loss, dim3((B + 3) / 4), dim3(256), sizeof(float) * 4 * m->Dp, B, m->Dp,
+               (const float*)m->E.as<float>(), (const float*)nullptr, 0, (const float*)nullptr, m->be.as<double>(),
+               m->G.as<float>(), m->dg.as<float>(), m->dq.as<float>(), m->idx.as<int>(), m->shift, 1.0 / m->scale, 1.0f,
                m->u.as<float>(), m->ub.as<__bf16>(), m->dE.as<float>(), le, le + B);
     TGX_CHECK_HIP(hipMemcpyAsync(er.data(), le, sizeof(double) * B, hipMemcpyDeviceToHost, ctx->stream));
     TGX_CHECK_HIP(hipMemcpyAsync(lg.data(), le + B, sizeof(double) * B, hipMemcpyDeviceToHost, ctx->stream));
@@ -866,7 +1053,7 @@ extern "C" int tgx_mlp_gradients_host(tgx_mlp* m, int batch, const float* q, con
   TGX_CHECK_HIP(hipMemcpyAsync(m->bg.p, gp.data(), sizeof(float) * gp.size(), hipMemcpyHostToDevice, ctx->stream));
   TGX_CHECK_HIP(hipMemcpyAsync(m->be.p, ep.data(), sizeof(double) * ep.size(), hipMemcpyHostToDevice, ctx->stream));
   TGX_TRY(tgx_f32_to_bf16(ctx, m->bq.as<float>(), m->bqb.as<__bf16>(), (int64_t)B * Dp));
-  TGX_TRY(mlp_backward(m, B, w_e, w_g, loss_e, loss_g));
+  TGX_TRY(mlp_backward(m, B, m->bq.as<float>(), m->bg.as<float>(), nullptr, w_e, w_g, loss_e, loss_g));
   (void)H;
   (void)D;
   return tgx_mlp_get_gradients(m, dW1, db1, dW2, db2, dw3, db3);
@@ -978,7 +1165,7 @@ extern "C" int tgx_mlp_force_gradients(tgx_ctx* ctx, int n_blocks, tgx_mlp* cons
     TGX_LAUNCH(ctx, "mlp_force_jvp", k_force_jvp, dim3(B), dim3(256), 0, ns, m->D, m->Dp,
                md[b]->site_beg.as<int64_t>(), md[b]->pr_nbr.as<int>(), md[b]->soap_der.as<double>(),
                (const double*)ctx->fres.as<double>(), -m->scale, m->u.as<float>(), m->ub.as<__bf16>());
-    TGX_TRY(mlp_backward_dirs(m, B, cF));
+    TGX_TRY(mlp_backward_dirs(m, B, cF, m->bq.as<float>(), nullptr));
     if (loss_e && ns > 0) {
       double e = 0.0;
       TGX_TRY(tgx_device_sum(ctx, le, B, &e));
