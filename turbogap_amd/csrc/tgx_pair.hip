@@ -9,7 +9,7 @@
 // r < rcut. Energies are per centre; the pair force acts on the centre (the
 // reference's forces(:, i) +=), and the virial is the half-symmetrised
 // -f (x) xyz summed over pairs, times 1/2. One wavefront per centre, lanes over
-// its pairs; per-centre virial rows are summed on the host in atom order.
+// its pairs; per-centre virial rows are summed on the device in a fixed order.
 #include "tgx_internal.h"
 
 namespace {
@@ -21,8 +21,8 @@ struct PairModelArgs {
   double rcut, buffer, delta2, inv_sig2, e0;  // 2b (rcut, buffer, e0 also 3b)
   double yp1, ypn;                            // core_pot end slopes
   int sc, ktype;                              // 3b: centre species, kernel 0 "exp" / 1 "pol"
-  double w1, w2, w3;                          // 3b: 1 / sigma_c^2
-  const double* a;  // 2b: Qs   core_pot: x   3b: (Q1, Q2, Q3, 2 delta^2 alpha cutoff) per sparse point
+  double w1, w2, w3;                          // 3b: 1 / sigma_c
+  const double* a;  // 2b: Qs   core_pot: x   3b: (Q_c / sigma_c, 2 delta^2 alpha cutoff) per sparse point
   const double* b;  // 2b: alphas * cutoff   core_pot: V
   const double* c;  // core_pot: d2V/dx2
 };
@@ -132,6 +132,29 @@ __global__ void k_pair_model(int n_sites, const int* __restrict__ n_neigh, const
   }
 }
 
+// The per-centre virial rows (six entries) added over a fixed slice of centres
+// per workgroup in a fixed tree; the host adds the parts in order.
+constexpr int VIRIAL_SUM_PARTS = 64;
+
+__global__ __launch_bounds__(256) void k_virial_sum(int n, const double* __restrict__ w, double* __restrict__ part) {
+  __shared__ double sh[6][256];
+  const int per = (n + gridDim.x - 1) / gridDim.x;
+  const int b = (int)blockIdx.x * per, e = min(n, b + per);
+  double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int i = b + (int)threadIdx.x; i < e; i += 256)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) v[k] += w[6 * (size_t)i + k];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) sh[k][threadIdx.x] = v[k];
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o)
+#pragma unroll
+      for (int k = 0; k < 6; ++k) sh[k][threadIdx.x] += sh[k][threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = sh[threadIdx.x][0];
+}
 
 // angle_3b. A centre i of species sc sees every unordered pair (j, k) of its
 // neighbours with species (s1, s2) in either order and r_ij, r_ik < rcut; the
@@ -153,6 +176,27 @@ __global__ void k_pair_model(int n_sites, const int* __restrict__ n_neigh, const
 // selection, the force on the centre itself in its self entry), which the
 // deterministic reverse-pair gather turns into per-atom forces and the pair
 // virial 1/2 (f x^T + x f^T) summed over entries, the reference's virial.
+//
+// Bound by FP64 issue in the loop over the sparse points. With descriptor and
+// points scaled by 1/sigma once, no branch at r = 1 and a square root by two
+// Newton steps on the hardware's reciprocal root, a (triplet, point) takes 26
+// FP64 instructions and one quarter-rate one instead of about 45.
+
+// sqrt(x), x >= 0: coupled Newton (Goldschmidt) steps on v_rsq_f64, whose
+// relative error is below 2^-20, and a last residual correction; within one ulp.
+// x is kept away from zero, where the reciprocal root is infinite: a squared
+// distance below 1e-200 is zero to every use of its root.
+__device__ __forceinline__ double sqrt_pos(double x) {
+  x = fmax(x, 1e-200);
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  e = fma(-g, g, x);
+  return fma(e, h, g);
+}
+
 template <int MAXP, int KT>
 __global__ __launch_bounds__(64) void k_angle_3b(const int* __restrict__ centres, const int* __restrict__ n_neigh,
                                                  const int64_t* __restrict__ off, const int* __restrict__ species,
@@ -249,31 +293,32 @@ __global__ __launch_bounds__(64) void k_angle_3b(const int* __restrict__ centres
           fc13 = (cos(arg) + 1.0) / 2.0;
           gc13 = sin(arg) / 2.0 * pi / m.buffer;
         }
-        const double q1 = r12 + r13, q2 = (r12 - r13) * (r12 - r13), q3 = r23;
-        double K = 0.0, H1 = 0.0, H2 = 0.0, H3 = 0.0;  // H_c = sum_s kd_s (q_c - Q_sc)
+        // descriptor and sparse points in units of sigma: K = sum_s p_s k_s and
+        // H_c = sum_s kd_s d_c, d_c the scaled difference, kd = -(dk/dr)/r
+        const double q1 = (r12 + r13) * m.w1, q2 = (r12 - r13) * (r12 - r13) * m.w2, q3 = r23 * m.w3;
+        double K = 0.0, H1 = 0.0, H2 = 0.0, H3 = 0.0;
 #pragma unroll 4
         for (int s = 0; s < m.n; ++s) {
           const double4 Q = qp[s];
           const double d1 = q1 - Q.x, d2 = q2 - Q.y, d3 = q3 - Q.z;
-          const double r2 = d1 * d1 * m.w1 + d2 * d2 * m.w2 + d3 * d3 * m.w3;
-          double kv, kd;
+          const double r2 = d1 * d1 + d2 * d2 + d3 * d3;
+          double kd;
           if (KT == 0) {
-            kv = Q.w * exp(-0.5 * r2);
-            kd = kv;  // -dk/d(r^2/2)
-          } else if (r2 < 1.0) {
-            const double r = sqrt(r2), om = 1.0 - r, om3 = om * om * om;
-            kv = Q.w * om3 * om * (4.0 * r + 1.0);
-            kd = 20.0 * Q.w * om3;  // -(dk/dr)/r
+            kd = Q.w * exp(-0.5 * r2);
+            K += kd;
           } else {
-            kv = kd = 0.0;
+            // (1 - r)^4 (4 r + 1) and 20 (1 - r)^3, both zero from r = 1 on
+            const double r = sqrt_pos(r2), om = fmax(1.0 - r, 0.0);
+            kd = Q.w * (om * om) * om;
+            K += kd * om * (4.0 * r + 1.0);
           }
-          K += kv;
           H1 += kd * d1;
           H2 += kd * d2;
           H3 += kd * d3;
         }
         // S_c = -dK/dq_c
-        const double S1 = H1 * m.w1, S2 = H2 * m.w2, S3 = H3 * m.w3;
+        const double ks = KT == 0 ? 1.0 : 20.0;
+        const double S1 = ks * H1 * m.w1, S2 = ks * H2 * m.w2, S3 = ks * H3 * m.w3;
         const double fcut = fc12 * fc13;
         const double A2 = 2.0 * (r12 - r13);
         // d fc / d x_i of each cutoff (the reference's dfcut12, dfcut13)
@@ -512,12 +557,12 @@ extern "C" int tgx_angle_3b_create(tgx_ctx* ctx, int species_center, int species
   m.rcut = rcut;
   m.buffer = buffer;
   m.e0 = e0;
-  m.w1 = 1.0 / (sigma[0] * sigma[0]);
-  m.w2 = 1.0 / (sigma[1] * sigma[1]);
-  m.w3 = 1.0 / (sigma[2] * sigma[2]);
+  m.w1 = 1.0 / sigma[0];
+  m.w2 = 1.0 / sigma[1];
+  m.w3 = 1.0 / sigma[2];
   std::vector<double> qp(4 * (size_t)n_sparse), none;
   for (int s = 0; s < n_sparse; ++s) {
-    for (int c = 0; c < 3; ++c) qp[4 * s + c] = Qs[3 * s + c];
+    for (int c = 0; c < 3; ++c) qp[4 * s + c] = Qs[3 * s + c] * (1.0 / sigma[c]);
     qp[4 * s + 3] = 2.0 * delta * delta * alphas[s] * cutoff[s];
   }
   return add_model(ctx, pm, qp, none, none, model_id);
@@ -525,22 +570,18 @@ extern "C" int tgx_angle_3b_create(tgx_ctx* ctx, int species_center, int species
 
 template <int KT>
 static int angle_3b_launch(tgx_ctx* ctx, const tgx_pair_model* pm, double* e, double* fglob, int* big) {
-  const int n = ctx->n_sites;
-  const double4* qp = reinterpret_cast<const double4*>(pm->m.a);
-  TGX_LAUNCH(ctx, "angle_3b", (k_angle_3b<128, KT>), dim3(n), dim3(64), 0, nullptr, ctx->n_neigh.as<int>(),
+  TGX_LAUNCH(ctx, "angle_3b", (k_angle_3b<128, KT>), dim3(ctx->n_sites), dim3(64), 0, nullptr, ctx->n_neigh.as<int>(),
              ctx->nl_off.as<int64_t>(), ctx->species_sc.as<int>(), ctx->nspec.as<int>(), ctx->rjs.as<double>(),
-             ctx->xyz.as<double>(), pm->m, qp, e, fglob, big);
-  int h[2] = {0, 0};
-  TGX_CHECK_HIP(hipMemcpyAsync(h, big, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-  TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-  if (h[0] > 0) {  // centres with more than 128 selected pairs
-    TGX_LAUNCH(ctx, "angle_3b_large", (k_angle_3b<1024, KT>), dim3(h[0]), dim3(64), 0, big + 2,
-               ctx->n_neigh.as<int>(), ctx->nl_off.as<int64_t>(), ctx->species_sc.as<int>(), ctx->nspec.as<int>(),
-               ctx->rjs.as<double>(), ctx->xyz.as<double>(), pm->m, qp, e, fglob, big);
-    TGX_CHECK_HIP(hipMemcpyAsync(h, big, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-    TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    TGX_REQUIRE(!h[1], "angle_3b: a centre has more than 1024 neighbours of the selected species inside rcut");
-  }
+             ctx->xyz.as<double>(), pm->m, reinterpret_cast<const double4*>(pm->m.a), e, fglob, big);
+  return TGX_OK;
+}
+
+// The nbig centres with more than 128 selected pairs.
+template <int KT>
+static int angle_3b_launch_large(tgx_ctx* ctx, const tgx_pair_model* pm, int nbig, double* e, double* fglob, int* big) {
+  TGX_LAUNCH(ctx, "angle_3b_large", (k_angle_3b<1024, KT>), dim3(nbig), dim3(64), 0, big + 2, ctx->n_neigh.as<int>(),
+             ctx->nl_off.as<int64_t>(), ctx->species_sc.as<int>(), ctx->nspec.as<int>(), ctx->rjs.as<double>(),
+             ctx->xyz.as<double>(), pm->m, reinterpret_cast<const double4*>(pm->m.a), e, fglob, big);
   return TGX_OK;
 }
 
@@ -553,9 +594,22 @@ static int angle_3b_run(tgx_ctx* ctx, const tgx_pair_model* pm, double* energies
   double* F = e + n;
   double* fglob = F + 3 * (size_t)n;
   int* big = reinterpret_cast<int*>(e + nd);
+  // the list build's pinned word takes the two counters: the build that wrote it is over
+  int* h = reinterpret_cast<int*>(ctx->pairs_host);
   TGX_TRY(tgx_zero(ctx, big, 2 * sizeof(int)));
   TGX_TRY(pm->m.ktype == 0 ? angle_3b_launch<0>(ctx, pm, e, fglob, big) : angle_3b_launch<1>(ctx, pm, e, fglob, big));
+  TGX_CHECK_HIP(hipMemcpyAsync(h, big, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  // the gather's wait also brings the counters; it is repeated in the rare case
+  // that large centres were left over
   TGX_TRY(tgx_gather_pair_forces(ctx, fglob, F, virial));
+  if (h[0] > 0) {
+    TGX_TRY(pm->m.ktype == 0 ? angle_3b_launch_large<0>(ctx, pm, h[0], e, fglob, big)
+                             : angle_3b_launch_large<1>(ctx, pm, h[0], e, fglob, big));
+    TGX_CHECK_HIP(hipMemcpyAsync(h, big, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    TGX_REQUIRE(!h[1], "angle_3b: a centre has more than 1024 neighbours of the selected species inside rcut");
+    TGX_TRY(tgx_gather_pair_forces(ctx, fglob, F, virial));
+  }
   if (energies) TGX_CHECK_HIP(hipMemcpyAsync(energies, e, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
   if (forces) TGX_CHECK_HIP(hipMemcpyAsync(forces, F, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, ctx->stream));
   TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
@@ -570,22 +624,26 @@ extern "C" int tgx_pair_energy_and_forces(tgx_ctx* ctx, int model_id, double* en
   TGX_REQUIRE(ctx->have_list, "tgx_pair_energy_and_forces: no neighbour list");
   if (pm->m.kind == 2) return angle_3b_run(ctx, pm, energies, forces, virial);
   const int n = ctx->n_sites;
-  TGX_TRY(ctx->scratch.ensure(sizeof(double) * 10 * (size_t)n));
+  TGX_TRY(ctx->scratch.ensure(sizeof(double) * (10 * (size_t)n + 6 * VIRIAL_SUM_PARTS)));
   double* e = ctx->scratch.as<double>();
   double* f = e + n;
   double* w = f + 3 * (size_t)n;
   TGX_LAUNCH(ctx, "pair_model", k_pair_model, dim3((n + 3) / 4), dim3(256), 0, n, ctx->n_neigh.as<int>(),
              ctx->nl_off.as<int64_t>(), ctx->species_sc.as<int>(), ctx->nspec.as<int>(), ctx->rjs.as<double>(),
              ctx->xyz.as<double>(), pm->m, e, f, w);
-  std::vector<double> wh(6 * (size_t)n);
+  double wh[6 * VIRIAL_SUM_PARTS];
+  double* wp = w + 6 * (size_t)n;
+  if (virial) {
+    TGX_LAUNCH(ctx, "pair_virial", k_virial_sum, dim3(VIRIAL_SUM_PARTS), dim3(256), 0, n, (const double*)w, wp);
+    TGX_CHECK_HIP(hipMemcpyAsync(wh, wp, sizeof(wh), hipMemcpyDeviceToHost, ctx->stream));
+  }
   if (energies) TGX_CHECK_HIP(hipMemcpyAsync(energies, e, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
   if (forces) TGX_CHECK_HIP(hipMemcpyAsync(forces, f, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, ctx->stream));
-  TGX_CHECK_HIP(hipMemcpyAsync(wh.data(), w, sizeof(double) * 6 * n, hipMemcpyDeviceToHost, ctx->stream));
   TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   if (virial) {
     double s[6] = {0, 0, 0, 0, 0, 0};
-    for (int i = 0; i < n; ++i)
-      for (int k = 0; k < 6; ++k) s[k] += wh[6 * (size_t)i + k];
+    for (int b = 0; b < VIRIAL_SUM_PARTS; ++b)
+      for (int k = 0; k < 6; ++k) s[k] += wh[6 * b + k];
     const int map[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};
     for (int k = 0; k < 9; ++k) virial[k] = s[map[k]];
   }
