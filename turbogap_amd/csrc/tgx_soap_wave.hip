@@ -1,11 +1,12 @@
 // Wavefront-per-site SOAP kernels (descriptor and adjoint forces).
 //
 // One wavefront owns one central site and synchronises only with itself, so a
-// workgroup's four wavefronts run four sites independently. Within a site the
-// lanes take the neighbour pairs (up to CH per pass):
-//   * each lane computes its pair's radial projections R_n (n in the pair's
-//     species block) from the Gaussian at the fixed quadrature nodes, and
-//     streams all real spherical harmonics from one recurrence in m and l;
+// workgroup's four wavefronts run four sites independently. Within a site
+// quads of lanes take the neighbour pairs (16 per pass):
+//   * a quad of lanes computes its pair's radial projections R_n (n in the pair's
+//     species block) from the Gaussian at the fixed quadrature nodes, a quarter
+//     of the nodes each, and streams all real spherical harmonics from
+//     recurrences in m and l, a quarter of the orders m each;
 //   * the expansion c(n, lm) = sum_j R_n(j) A_l(j) Y_lm(j) is then a small
 //     product of the staged R and W = A Y, with lanes over (n, lm) outputs;
 //   * the adjoint contracts H(n, lm) = d(g . p)/dc with dc/dr_j on the fly:
@@ -69,26 +70,44 @@ template <class T> struct Tables {
   }
 };
 
-// Radial projections of one pair (lane): R[n] and, when GRAD, dR[n]/dr.
+// Sum over the four lanes of a quad, which share a pair, by DPP on the VALU; the
+// same on all four.
+template <int CTRL> __device__ __forceinline__ float dpp_of(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_of(double x) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true));
+}
+template <class T> __device__ __forceinline__ T quad_sum(T v) {
+  v += dpp_of<0xB1>(v);         // quad_perm [1, 0, 3, 2]
+  return v + dpp_of<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+}
+
+// Radial projections of one pair by the four lanes of a quad: R[n] and, when
+// GRAD, dR[n]/dr, complete on every lane. Lane sub takes the nodes sub, sub + 4,
+// ...: a lane per pair left three quarters of the wavefront idle (16 pairs a
+// pass) through the Gaussians, the largest part of both kernels.
 template <class T, bool GRAD>
-__device__ __forceinline__ void lane_radial(const SoapParams& P, const Tables<T>& tb, int s, T r, T (&R)[TGX_MAX_NB],
-                                            T (&dR)[TGX_MAX_NB]) {
+__device__ __forceinline__ void quad_radial(const SoapParams& P, const Tables<T>& tb, int s, int sub, T r,
+                                            T (&R)[TGX_MAX_NB], T (&dR)[TGX_MAX_NB]) {
   const SpeciesParams& sp = P.sp[s];
   const T inv_rc = (T)sp.inv_rc;
   const T x = r * inv_rc;
   const T sig = (T)sp.sig_r * ((T)1 + (T)sp.sig_r_sc * r) * inv_rc;
   const T dsig = (T)(sp.sig_r * sp.sig_r_sc) * inv_rc;
   const T inv_s2 = (T)1 / (sig * sig);
+  const T d1 = inv_s2 * inv_rc, d2 = inv_s2 / sig * dsig, ex = -(T)0.5 * inv_s2;
 #pragma unroll
   for (int n = 0; n < TGX_MAX_NB; ++n) { R[n] = 0; dR[n] = 0; }
   const T* xq = tb.xq + s * TGX_MAX_Q;
   const T* Bt = tb.Bt + s * TGX_MAX_Q * TGX_MAX_NB;
   const int nb = sp.nb;
-  for (int q = 0; q < sp.nq; ++q) {
+  for (int q = sub; q < sp.nq; q += 4) {
     const T dx = xq[q] - x;
-    const T g = w_exp<T>(-(T)0.5 * dx * dx * inv_s2);
+    const T g = w_exp<T>(dx * dx * ex);
     T dg = 0;
-    if (GRAD) dg = g * (dx * inv_s2 * inv_rc + dx * dx * inv_s2 / sig * dsig);
+    if (GRAD) dg = g * (dx * d1 + dx * dx * d2);
     const T* b = Bt + q * TGX_MAX_NB;
 #pragma unroll
     for (int n = 0; n < TGX_MAX_NB; ++n) {
@@ -109,89 +128,104 @@ __device__ __forceinline__ void lane_radial(const SoapParams& P, const Tables<T>
     amp = 0;
     damp = 0;
   } else {
-    const T Pa = w_pow<T>(Pp, a);
+    const T Pa = a == (T)1 ? Pp : w_pow<T>(Pp, a);  // x^1 = x and x^0 = 1 exactly
     amp = Pa / sig;
-    damp = a * w_pow<T>(Pp, a - (T)1) * dPp / sig - Pa * dsig / (sig * sig);
+    damp = a * (a == (T)1 ? (T)1 : w_pow<T>(Pp, a - (T)1)) * dPp / sig - Pa * dsig / (sig * sig);
   }
   amp *= (T)sp.gs;
   damp *= (T)sp.gs;
 #pragma unroll
   for (int n = 0; n < TGX_MAX_NB; ++n) {
-    const T I = R[n];
-    R[n] = amp * I;
-    if (GRAD) dR[n] = damp * I + amp * dR[n];
+    if (n < nb) {
+      const T I = quad_sum(R[n]);
+      R[n] = amp * I;
+      if (GRAD) dR[n] = damp * I + amp * quad_sum(dR[n]);
+    }
   }
 }
 
-// Angular damping recurrence state: A_l = exp(-l(l+1) k).
+// Angular damping A_l = exp(-l(l+1) kk): A_l = prod_{k <= l} e2^k with e2 =
+// exp(-2 kk); -A_l'/A_l = l(l+1) dk.
 template <class T> struct Damp {
-  T e2, kk, dk;
+  T e2, dk;
   __device__ void init(const SpeciesParams& sp, T r) {
     const T st = (T)sp.sig_t * ((T)1 + (T)sp.sig_t_sc * r);
     const T dst = (T)(sp.sig_t * sp.sig_t_sc);
-    kk = st * st / ((T)2 * r * r);
-    dk = st * st / (r * r * r) - st * dst / (r * r);  // -dk/dr
-    const T e1 = w_exp<T>(-kk);
+    dk = st * st / (r * r * r) - st * dst / (r * r);
+    const T e1 = w_exp<T>(-(st * st / ((T)2 * r * r)));
     e2 = e1 * e1;
   }
 };
 
-// Streams every (l, m) of the real harmonics at u (and the gradient of the
-// solid harmonic when GRAD) to f(l, lm, Y, gx, gy, gz), m-major.
+// The real harmonics at u (and the gradient of the solid harmonic when GRAD) of
+// one pair by the four lanes of a quad, to f(l, lm, A_l, Y, gx, gy, gz). Lane sub
+// takes the orders m = sub, 7 - sub, 8 + sub, 15 - sub: for l_max = 8 at most 15
+// degrees against 45 for a lane on its own, the four lanes stepping through
+// their degrees together. The order's cos and sin factors c + i s = (ux + i
+// uy)^m, their gradient (m (c', s') of order m - 1) and A_m come from the powers
+// up to m.
 template <class T, bool GRAD, class F>
-__device__ __forceinline__ void ylm_stream(int L, const T* ynorm, T ux, T uy, T uz, F&& f) {
-  T c = 1, cx = 0, cy = 0, s = 0, sx = 0, sy = 0;
-  for (int m = 0; m <= L; ++m) {
-    if (m > 0) {
-      const T nc = c * ux - s * uy, ns = c * uy + s * ux;
-      if (GRAD) {
-        const T ncx = cx * ux + c - sx * uy, ncy = cy * ux - sy * uy - s;
-        const T nsx = cx * uy + sx * ux + s, nsy = cy * uy + c + sy * ux;
-        cx = ncx; cy = ncy; sx = nsx; sy = nsy;
-      }
-      c = nc;
-      s = ns;
+__device__ __forceinline__ void ylm_quad(int L, const T* ynorm, int sub, T ux, T uy, T uz, T e2, F&& f) {
+  T c = (T)1, s = (T)0, cp = (T)0, sp = (T)0, pw0 = (T)1, A0 = (T)1;
+  int k = 0;
+  for (int t = 0; 4 * t <= L; ++t) {
+    const int m = 8 * (t >> 1) + ((t & 1) ? 7 - sub : sub);
+    for (; k < m && k < L; ++k) {
+      cp = c;
+      sp = s;
+      c = cp * ux - sp * uy;
+      s = cp * uy + sp * ux;
+      pw0 *= e2;
+      A0 *= pw0;
     }
-    T q = 1, qx = 0, qy = 0, qz = 0, p = 0, px = 0, py = 0, pz = 0;
-    for (int l = m; l <= L; ++l) {
-      if (l == m + 1) {
+    const T dm = (T)m;
+    const T cx = dm * cp, cy = -dm * sp, sx = dm * sp, sy = dm * cp;
+    T q = (T)1, qx = (T)0, qy = (T)0, qz = (T)0, p = (T)0, px = (T)0, py = (T)0, pz = (T)0;
+    T Al = A0, pw = pw0;
+    for (int i = 0; i <= L; ++i) {
+      const int l = m + i;
+      if (l > L) break;
+      if (i == 1) {
         p = q; px = qx; py = qy; pz = qz;
-        q = (T)(2 * m + 1) * uz;
-        qx = 0; qy = 0; qz = (T)(2 * m + 1);
-      } else if (l > m + 1) {
-        const T a = (T)(2 * l - 1), b = (T)(l + m - 1), inv = (T)1 / (T)(l - m);
-        const T nq = (a * uz * q - b * p) * inv;
+        qz = (T)2 * dm + (T)1;
+        q = qz * uz;
+        qx = (T)0; qy = (T)0;
+      } else if (i > 1) {
+        const T inv = (T)1 / (T)i, a = ((T)2 * dm + (T)(2 * i - 1)) * inv,
+                     b = ((T)2 * dm + (T)(i - 1)) * inv;
+        const T nq = a * uz * q - b * p;
         if (GRAD) {
-          const T nqx = (a * uz * qx - b * ((T)2 * ux * p + px)) * inv;
-          const T nqy = (a * uz * qy - b * ((T)2 * uy * p + py)) * inv;
-          const T nqz = (a * (q + uz * qz) - b * ((T)2 * uz * p + pz)) * inv;
+          const T nqx = a * uz * qx - b * ((T)2 * ux * p + px);
+          const T nqy = a * uz * qy - b * ((T)2 * uy * p + py);
+          const T nqz = a * (q + uz * qz) - b * ((T)2 * uz * p + pz);
           px = qx; py = qy; pz = qz;
           qx = nqx; qy = nqy; qz = nqz;
         }
         p = q;
         q = nq;
       }
+      if (i > 0) {
+        pw *= e2;
+        Al *= pw;
+      }
       const int base = l * l + l;
       const T N = ynorm[base + m];
-      if (m == 0) {
-        f(l, base, N * q, N * qx, N * qy, N * qz);
-      } else {
-        f(l, base + m, N * q * c, N * (qx * c + q * cx), N * (qy * c + q * cy), N * qz * c);
-        f(l, base - m, N * q * s, N * (qx * s + q * sx), N * (qy * s + q * sy), N * qz * s);
-      }
+      f(l, base + m, Al, N * q * c, N * (qx * c + q * cx), N * (qy * c + q * cy), N * qz * c);
+      if (m > 0) f(l, base - m, Al, N * q * s, N * (qx * s + q * sx), N * (qy * s + q * sy), N * qz * s);
     }
   }
 }
 
 // Expansion coefficients of one site into C (LDS, [N][NLM]) by one wavefront.
-// Pass over chunks of CH pairs: pair lanes stage Rf[j][n] (stacked radial index,
+// Pass over chunks of CH pairs: quads of lanes stage Rf[j][n] (stacked radial index,
 // zero outside the pair's species block) and W[j][lm] = A_l Y_lm in LDS; then
 // lanes over lm accumulate C[n][lm] += sum_j Rf[j][n] W[j][lm] with the n
 // column in registers and Rf rows read as LDS broadcasts.
 template <class T, int CH, int NMAX>
 __device__ void wave_coefficients(const SoapParams& P, const Tables<T>& tb, const WaveArgs& a, int64_t b0, int nn, T* C,
                                   T* W, T* Rf) {
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, pj = lane >> 2, sub = lane & 3;  // a quad of lanes per pair
+  static_assert(CH <= 16, "a pass holds a pair per quad");
   const int NLM = P.NLM, N = P.N, L = P.L;
   T acc[2][NMAX];
 #pragma unroll
@@ -212,37 +246,31 @@ __device__ void wave_coefficients(const SoapParams& P, const Tables<T>& tb, cons
   for (int k0 = 1; k0 < nn; k0 += CH) {
     const int cnt = min(CH, nn - k0);
     wave_sync();
-    if (lane < cnt) {
-      const int64_t p = b0 + k0 + lane;
+    if (pj < cnt) {
+      const int64_t p = b0 + k0 + pj;
       int s = a.pr_spec[p];
       const double rr = a.pr_r[p];
       if (s >= 0 && !(rr < P.sp[s].rc)) s = -1;
-      T* rf = Rf + lane * NMAX;
-#pragma unroll
-      for (int n = 0; n < NMAX; ++n) rf[n] = 0;
+      T* rf = Rf + pj * NMAX;
+      for (int n = sub; n < NMAX; n += 4) rf[n] = 0;
+      T* w = W + pj * NLM;
       if (s >= 0) {
         const T r = (T)rr, inv = (T)1 / r;
         const T ux = (T)a.pr_xyz[3 * p] * inv, uy = (T)a.pr_xyz[3 * p + 1] * inv, uz = (T)a.pr_xyz[3 * p + 2] * inv;
         T R[TGX_MAX_NB], dR[TGX_MAX_NB];
-        lane_radial<T, false>(P, tb, s, r, R, dR);
+        quad_radial<T, false>(P, tb, s, sub, r, R, dR);
         const int off = P.sp[s].off, nb = P.sp[s].nb;
+        wave_sync();  // the quad's zeros before its values
+        if (sub == 0)
 #pragma unroll
-        for (int n = 0; n < TGX_MAX_NB; ++n)
-          if (n < nb) rf[off + n] = R[n];
+          for (int n = 0; n < TGX_MAX_NB; ++n)
+            if (n < nb) rf[off + n] = R[n];
         Damp<T> dmp;
         dmp.init(P.sp[s], r);
-        T Atab[TGX_MAX_L + 1];
-        T Al = 1, pw = 1;
-#pragma unroll
-        for (int l = 0; l <= TGX_MAX_L; ++l) {
-          if (l > 0) { pw *= dmp.e2; Al *= pw; }
-          Atab[l] = Al;
-        }
-        T* w = W + lane * NLM;
-        ylm_stream<T, false>(L, tb.ynorm, ux, uy, uz, [&](int l, int lm, T Y, T, T, T) { w[lm] = Atab[l] * Y; });
+        ylm_quad<T, false>(L, tb.ynorm, sub, ux, uy, uz, dmp.e2,
+                           [&](int l, int lm, T Al, T Y, T, T, T) { w[lm] = Al * Y; });
       } else {
-        T* w = W + lane * NLM;
-        for (int lm = 0; lm < NLM; ++lm) w[lm] = 0;
+        for (int lm = sub; lm < NLM; lm += 4) w[lm] = 0;
       }
     }
     wave_sync();
@@ -352,7 +380,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_adjoint_wave(SoapParams P, WaveA
   Tables<T> tb;
   tb.load(P, sm);
   __syncthreads();
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, pj = lane >> 2, sub = lane & 3;
   const int site = blockIdx.x * WAVES + w;
   if (site >= n_sites) return;
   const int NLM = P.NLM, N = P.N, L = P.L, D = P.D, CN = N * NLM;
@@ -416,30 +444,31 @@ __global__ __launch_bounds__(64 * WAVES) void k_adjoint_wave(SoapParams P, WaveA
   T s0 = 0, s1 = 0, s2 = 0;
   for (int k0 = 1; k0 < nn; k0 += CH) {
     const int cnt = min(CH, nn - k0);
-    // 1) pair lanes: radial values and derivatives
+    // 1) pair quads: radial values and derivatives
     int s = -1;
     T r = 0, ux = 0, uy = 0, uz = 0;
     int64_t p = 0;
     wave_sync();
-    if (lane < cnt) {
-      p = b0 + k0 + lane;
+    if (pj < cnt) {
+      p = b0 + k0 + pj;
       s = a.pr_spec[p];
       const double rr = a.pr_r[p];
       if (s >= 0 && !(rr < P.sp[s].rc)) s = -1;
-      T* rr_ = Rr + lane * NMAX;
-      T* dr_ = dRr + lane * NMAX;
-#pragma unroll
-      for (int n = 0; n < NMAX; ++n) { rr_[n] = 0; dr_[n] = 0; }
+      T* rr_ = Rr + pj * NMAX;
+      T* dr_ = dRr + pj * NMAX;
+      for (int n = sub; n < NMAX; n += 4) { rr_[n] = 0; dr_[n] = 0; }
       if (s >= 0) {
         r = (T)rr;
         const T inv = (T)1 / r;
         ux = (T)a.pr_xyz[3 * p] * inv; uy = (T)a.pr_xyz[3 * p + 1] * inv; uz = (T)a.pr_xyz[3 * p + 2] * inv;
         T R[TGX_MAX_NB], dR[TGX_MAX_NB];
-        lane_radial<T, true>(P, tb, s, r, R, dR);
+        quad_radial<T, true>(P, tb, s, sub, r, R, dR);
         const int off = P.sp[s].off, nb = P.sp[s].nb;
+        wave_sync();  // the quad's zeros before its values
+        if (sub == 0)
 #pragma unroll
-        for (int n = 0; n < TGX_MAX_NB; ++n)
-          if (n < nb) { rr_[off + n] = R[n]; dr_[off + n] = dR[n]; }
+          for (int n = 0; n < TGX_MAX_NB; ++n)
+            if (n < nb) { rr_[off + n] = R[n]; dr_[off + n] = dR[n]; }
       }
     }
     wave_sync();
@@ -462,38 +491,35 @@ __global__ __launch_bounds__(64 * WAVES) void k_adjoint_wave(SoapParams P, WaveA
         }
     }
     wave_sync();
-    // 3) pair lanes: contract with the harmonics and their gradients
+    // 3) pair quads: contract with the harmonics and their gradients
     T f0 = 0, f1 = 0, f2 = 0;
-    if (lane < cnt && s >= 0) {
+    if (pj < cnt && s >= 0) {
       const T inv_r = (T)1 / r;
       Damp<T> dmp;
       dmp.init(P.sp[s], r);
-      T Atab[TGX_MAX_L + 1], dAtab[TGX_MAX_L + 1];
-      T Al = 1, pw = 1;
-#pragma unroll
-      for (int l = 0; l <= TGX_MAX_L; ++l) {
-        if (l > 0) { pw *= dmp.e2; Al *= pw; }
-        Atab[l] = Al;
-        dAtab[l] = Al * (T)(l * (l + 1)) * dmp.dk;
-      }
-      const T* xa = Xa + lane * NLM;
-      const T* xb = Xb + lane * NLM;
-      ylm_stream<T, true>(L, tb.ynorm, ux, uy, uz, [&](int l, int lm, T Y, T gx, T gy, T gz) {
+      const T* xa = Xa + pj * NLM;
+      const T* xb = Xb + pj * NLM;
+      ylm_quad<T, true>(L, tb.ynorm, sub, ux, uy, uz, dmp.e2, [&](int l, int lm, T A, T Y, T gx, T gy, T gz) {
         const T x = xa[lm], y = xb[lm];
-        const T A = Atab[l], dA = dAtab[l];
-        const T rad = dA * x + A * y;
-        const T ang = A * x * inv_r;
-        const T lf = (T)l;
-        f0 += rad * Y * ux + ang * (gx - lf * Y * ux);
-        f1 += rad * Y * uy + ang * (gy - lf * Y * uy);
-        f2 += rad * Y * uz + ang * (gz - lf * Y * uz);
+        const T Ax = A * x, lf = (T)l;
+        const T ang = Ax * inv_r;
+        // rad Y u + ang (grad - l Y u), rad = A' x + A y
+        const T t = (Ax * (lf * (lf + (T)1) * dmp.dk) + A * y - ang * lf) * Y;
+        f0 += t * ux + ang * gx;
+        f1 += t * uy + ang * gy;
+        f2 += t * uz + ang * gz;
       });
+      f0 = quad_sum(f0);
+      f1 = quad_sum(f1);
+      f2 = quad_sum(f2);
     }
-    if (lane < cnt) {
+    if (pj < cnt && sub == 0) {
       const int64_t gi = a.pr_gidx[p];
       fglob[3 * gi] += (double)f0;
       fglob[3 * gi + 1] += (double)f1;
       fglob[3 * gi + 2] += (double)f2;
+    } else {
+      f0 = f1 = f2 = 0;  // one lane of a quad carries the pair into the self entry's sum
     }
     s0 += f0;
     s1 += f1;
