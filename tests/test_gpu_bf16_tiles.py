@@ -1,0 +1,39 @@
+"""Mixed-precision step against the FP64 one at the sizes where the BF16 products change tile: 32-row,
+64-row, 128-row and 256-row workgroups, with row counts that are no multiple of any of them."""
+import numpy as np
+import pytest
+
+from turbogap_amd import structures as S
+
+pytestmark = pytest.mark.gpu
+
+
+# atoms (half of them a block's centres), sparse points: 128 x 128 tiles per block of the kernel and
+# Qss products are (4, 20), (63, 70), (128, 160), (384 with 24 columns, 170), (1,184, 360), (2,304, 720)
+@pytest.mark.parametrize("n,n_sparse", [(300, 200), (1700, 1100), (4000, 1000), (4300, 3000), (9100, 4000),
+                                        (18300, 4000)])
+def test_mixed_matches_fp64(n, n_sparse):
+    from turbogap_amd import Context
+    rng = np.random.default_rng(n)
+    sysm = S.binary_system(n, seed=31)
+    with Context(0) as ctx:
+        ctx.set_system(sysm.positions, sysm.species, sysm.box)
+        ctx.build_neighbors_list(3.7, fetch=False)
+        scale = 0.0
+        for h in S.soap_binary():
+            probe = ctx.soap_model(h, np.zeros((1, h.dim)), np.zeros(1))
+            ctx.soap_backend_begin(probe)
+            q, _ = ctx.get_soap(derivatives=False)
+            ctx.soap_backend_end()
+            Qs = q[rng.integers(0, q.shape[0], n_sparse)]
+            al = rng.normal(scale=1e-3, size=n_sparse)
+            scale = max(scale, np.linalg.norm(al))
+            ctx.soap_model(h, Qs, al)
+        # the probe blocks have zero alphas: they add nothing
+        ctx.compute("fp64_adjoint")
+        e0, f0 = ctx.results()
+        ctx.compute("mixed")
+        e1, f1 = ctx.results()
+    # operands rounded to BF16 (2^-9 each): K^4 is off by 4 * 2 * 2^-9 at most, independently per sparse point
+    assert np.abs(e1 - e0).max() <= 5.0 * 4 * 2 * 2.0 ** -9 * scale
+    assert np.linalg.norm(f1 - f0) <= 2.0 ** -6 * np.linalg.norm(f0)

@@ -19,6 +19,7 @@ namespace {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 128, BN = 128;
 constexpr int TILE_GM = 8;  // tile rows per group of the GEMM tile order (tile_of)
@@ -82,81 +83,20 @@ __device__ __forceinline__ void kpow(T k, double zeta, int zi, T& kz, T& kzm1) {
   }
 }
 
-// Shared epilogue. acc holds, for tile (ti, tj) and register r, the element
-// (row0 + ti*16 + rr, col0 + tj*16 + lane%16) where the row within the tile is
-//   rr = 4*r + lane/16   for v_mfma_f64_16x16x4f64   (register-major)
-//   rr = 4*(lane/16) + r for the FP32-output MFMAs   (lane-group-major)
-// (checked against a host GEMM on the device).
-template <bool F64> __device__ __forceinline__ int tile_row(int lane, int r) {
-  return F64 ? 4 * r + (lane >> 4) : 4 * (lane >> 4) + r;
-}
+// FP64 epilogue. acc holds, for tile (ti, tj) and register r, the element
+// (row0 + ti*16 + 4*r + lane/16, col0 + tj*16 + lane%16) (the register-major
+// layout of v_mfma_f64_16x16x4f64, checked against a host GEMM on the device).
+__device__ __forceinline__ int tile_row(int lane, int r) { return 4 * r + (lane >> 4); }
 
 // TI x TJ MFMA tiles of 16 x 16 per wavefront (a WM x WN wave tile), the
 // workgroup tile BMT rows tall with two wavefronts along N.
-template <int EPI, class OutT, class AccT, class VecT, bool F64, bool ZINT, int TI = 4, int TJ = 4, int WM = 64,
-          int WN = 64, int BMT = BM>
-__device__ __forceinline__ void epilogue(const VecT (&acc)[TI][TJ], int m0, int n0, int tn, int wm, int wn, const EpiArgs& e,
-                         double* sE) {
+template <int EPI, bool ZINT, int TI, int TJ, int WM, int WN, int BMT>
+__device__ __forceinline__ void epilogue_f64(const f64x4 (&acc)[TI][TJ], int m0, int n0, int tn, int wm, int wn,
+                                             const EpiArgs& e, double* sE) {
   const int lane = threadIdx.x & 63;
   const int rbase = m0 + wm * WM;
   const int cbase = n0 + wn * WN + (lane & 15);
-  OutT* out = reinterpret_cast<OutT*>(e.out);
-  if (EPI == EPI_SILU || EPI == EPI_SCALE_AUX) {
-#pragma unroll
-    for (int tj = 0; tj < TJ; ++tj) {
-      const int col = cbase + tj * 16;
-      const float bc = EPI == EPI_SILU ? e.bias[col] : 0.0f;
-#pragma unroll
-      for (int ti = 0; ti < TI; ++ti)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const size_t row = (size_t)(rbase + ti * 16 + tile_row<F64>(lane, r));
-          if (EPI == EPI_SILU) {
-            const float v = (float)acc[ti][tj][r] + bc;
-            out[row * e.ldo + col] = (OutT)tgx_silu(v);
-            e.aux[row * e.ldaux + col] = tgx_silu1(v);
-          } else {
-            out[row * e.ldo + col] = (OutT)((float)acc[ti][tj][r] * e.aux[row * e.ldaux + col] * (float)e.pref);
-          }
-        }
-    }
-    return;
-  }
-  if (EPI == EPI_ACT2) {
-    // per 16-row slab: a2 = w3 silu'(v) out, and the row sums of w3 silu(v)
-    // over the tile's columns as partial energies (as the GAP epilogue's)
-#pragma unroll
-    for (int ti = 0; ti < TI; ++ti) {
-      double er[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int tj = 0; tj < TJ; ++tj) {
-        const int col = cbase + tj * 16;
-        const float bc = e.bias[col], wc = e.w3[col];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const size_t row = (size_t)(rbase + ti * 16 + tile_row<F64>(lane, r));
-          const float v = (float)acc[ti][tj][r] + bc;
-          out[row * e.ldo + col] = (OutT)(wc * tgx_silu1(v));
-          er[r] += (double)(wc * tgx_silu(v));
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        double v = er[r];
-        v += __shfl_xor(v, 1);
-        v += __shfl_xor(v, 2);
-        v += __shfl_xor(v, 4);
-        v += __shfl_xor(v, 8);
-        if ((lane & 15) == 0) sE[wn * BMT + wm * WM + ti * 16 + tile_row<F64>(lane, r)] = v;
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x < BMT) {
-      const int row = m0 + threadIdx.x;
-      e.epart[(size_t)row * e.n_tiles + tn] = sE[threadIdx.x] + sE[BMT + threadIdx.x];
-    }
-    return;
-  }
+  double* out = reinterpret_cast<double*>(e.out);
   if (EPI == EPI_STORE) {
 #pragma unroll
     for (int ti = 0; ti < TI; ++ti)
@@ -164,8 +104,7 @@ __device__ __forceinline__ void epilogue(const VecT (&acc)[TI][TJ], int m0, int 
       for (int tj = 0; tj < TJ; ++tj)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          out[(size_t)(rbase + ti * 16 + tile_row<F64>(lane, r)) * e.ldo + cbase + tj * 16] =
-              (OutT)((AccT)e.pref * acc[ti][tj][r]);
+          out[(size_t)(rbase + ti * 16 + tile_row(lane, r)) * e.ldo + cbase + tj * 16] = e.pref * acc[ti][tj][r];
     return;
   }
   // one 16-row slab at a time keeps only four row partials live
@@ -175,13 +114,13 @@ __device__ __forceinline__ void epilogue(const VecT (&acc)[TI][TJ], int m0, int 
 #pragma unroll
     for (int tj = 0; tj < TJ; ++tj) {
       const int col = cbase + tj * 16;
-      const AccT al = e.alpha_f ? (AccT)e.alpha_f[col] : (AccT)e.alpha[col];
+      const double al = e.alpha[col];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        AccT kz, kzm1;
-        kpow<AccT, ZINT>(acc[ti][tj][r], e.zeta, e.zeta_int, kz, kzm1);
-        out[(size_t)(rbase + ti * 16 + tile_row<F64>(lane, r)) * e.ldo + col] = (OutT)((AccT)e.pref * kzm1 * al);
-        er[r] += (double)(al * kz);
+        double kz, kzm1;
+        kpow<double, ZINT>(acc[ti][tj][r], e.zeta, e.zeta_int, kz, kzm1);
+        out[(size_t)(rbase + ti * 16 + tile_row(lane, r)) * e.ldo + col] = e.pref * kzm1 * al;
+        er[r] += al * kz;
       }
     }
     // reduce over the 16 lanes that share rows
@@ -192,13 +131,110 @@ __device__ __forceinline__ void epilogue(const VecT (&acc)[TI][TJ], int m0, int 
       v += __shfl_xor(v, 2);
       v += __shfl_xor(v, 4);
       v += __shfl_xor(v, 8);
-      if ((lane & 15) == 0) sE[wn * BMT + wm * WM + ti * 16 + tile_row<F64>(lane, r)] = v;
+      if ((lane & 15) == 0) sE[wn * BMT + wm * WM + ti * 16 + tile_row(lane, r)] = v;
     }
   }
   __syncthreads();
   if (threadIdx.x < BMT) {
     const int row = m0 + threadIdx.x;
     e.epart[(size_t)row * e.n_tiles + tn] = sE[threadIdx.x] + sE[BMT + threadIdx.x];
+  }
+}
+
+// BF16 epilogues (FP32 accumulators), in two layouts.
+// Straight, v_mfma(A, B): register r of tile (ti, tj) is the element (row0 + ti*16
+// + 4*(lane/16) + r, col0 + tj*16 + lane%16), so that a store instruction writes
+// 64-byte runs of FP32; for the epilogues with an FP32 output or factor.
+// Exchanged, v_mfma(B, A): a lane's four registers are four consecutive columns
+// of one row, row0 + ti*16 + lane%16, columns col0 + tj*16 + 4*(lane/16) + r; for
+// the epilogues that write BF16 only and sum rows: 8-byte stores instead of four
+// 2-byte ones and two shuffles a row sum instead of four a register (GAP product
+// 32,768 x 4,096 x 1,280: 0.431 -> 0.402 ms; exchanged, the FP32 stores of the
+// 32,768 x 1,280 x 768 product cost 0.095 ms against 0.082).
+template <int EPI> constexpr bool exchanged() { return EPI == EPI_GAP || EPI == EPI_ACT2; }
+
+template <int EPI>
+__device__ __forceinline__ f32x4 mfma_bf16(const bf16x8& a, const bf16x8& b, const f32x4& c) {
+  return exchanged<EPI>() ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, c, 0, 0, 0)
+                          : __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x4 load4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+// TI x 4 MFMA tiles per wavefront (a WM x 64 wave tile), the workgroup tile BMT
+// rows tall with two wavefronts along N.
+template <int EPI, class OutT, bool ZINT, int TI, int WM, int BMT>
+__device__ __forceinline__ void epilogue_bf16(const f32x4 (&acc)[TI][4], int m0, int n0, int tn, int wm, int wn,
+                                              const EpiArgs& e, double* sE) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  OutT* out = reinterpret_cast<OutT*>(e.out);
+  const float pref = (float)e.pref;
+  if constexpr (!exchanged<EPI>()) {
+    const int rbase = m0 + wm * WM + 4 * lg, cbase = n0 + wn * 64 + li;
+#pragma unroll
+    for (int ti = 0; ti < TI; ++ti)
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj) {
+        const int col = cbase + tj * 16;
+        const float b = EPI == EPI_SILU ? e.bias[col] : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const size_t row = (size_t)(rbase + ti * 16 + r);
+          const float x = acc[ti][tj][r];
+          if constexpr (EPI == EPI_SILU) {
+            out[row * e.ldo + col] = (OutT)tgx_silu(x + b);
+            e.aux[row * e.ldaux + col] = tgx_silu1(x + b);
+          } else if constexpr (EPI == EPI_SCALE_AUX) {
+            out[row * e.ldo + col] = (OutT)(x * e.aux[row * e.ldaux + col] * pref);
+          } else {
+            out[row * e.ldo + col] = (OutT)(pref * x);
+          }
+        }
+      }
+    return;
+  } else {
+    const int cbase = n0 + wn * 64 + 4 * lg;
+#pragma unroll
+    for (int ti = 0; ti < TI; ++ti) {
+      const int trow = wm * WM + ti * 16 + li;
+      const size_t row = (size_t)(m0 + trow);
+      double er = 0.0;
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj) {
+        const int col = cbase + tj * 16;
+        const f32x4 x = acc[ti][tj];
+        bf16x4 o;
+        if constexpr (EPI == EPI_ACT2) {
+          // a2 = w3 silu'(v) out, and the row sums of w3 silu(v) over the tile's
+          // columns as partial energies (as the GAP epilogue's)
+          const f32x4 b = load4(e.bias + col), w3 = load4(e.w3 + col);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float v = x[r] + b[r];
+            o[r] = (__bf16)(w3[r] * tgx_silu1(v));
+            er += (double)(w3[r] * tgx_silu(v));
+          }
+        } else {
+          const f32x4 al = load4(e.alpha_f + col);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float kz, kzm1;
+            kpow<float, ZINT>(x[r], e.zeta, e.zeta_int, kz, kzm1);
+            o[r] = (__bf16)(pref * kzm1 * al[r]);
+            er += (double)(al[r] * kz);
+          }
+        }
+        *reinterpret_cast<bf16x4*>(out + row * e.ldo + col) = o;
+      }
+      er += __shfl_xor(er, 16);
+      er += __shfl_xor(er, 32);
+      if (lane < 16) sE[wn * BMT + trow] = er;
+    }
+    __syncthreads();
+    if (threadIdx.x < BMT) {
+      const int row = m0 + threadIdx.x;
+      e.epart[(size_t)row * e.n_tiles + tn] = sE[threadIdx.x] + sE[BMT + threadIdx.x];
+    }
   }
 }
 
@@ -303,7 +339,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_f64(int K, const double* __re
   }
   wait_vmcnt<0>();  // the loads issued past the last stage land before the LDS is released
   __builtin_amdgcn_sched_barrier(0);
-  epilogue<EPI, double, double, f64x4, true, ZINT, TI, TJ, 16 * TI, 16 * TJ, 32 * TI>(acc, m0, n0, tn, wm, wn, e, sE);
+  epilogue_f64<EPI, ZINT, TI, TJ, 16 * TI, 16 * TJ, 32 * TI>(acc, m0, n0, tn, wm, wn, e, sE);
 }
 
 // FP64 NT GEMM for few rows: workgroup tile 32 x (32 NC), NC x KS wavefronts of
@@ -365,7 +401,7 @@ __global__ __launch_bounds__(64 * NC * KS) void k_gemm_f64_few(int K, const doub
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        part[(wk * 32 + i * 16 + tile_row<true>(lane, r)) * W + 32 * wc + j * 16 + li] = acc[i][j][r];
+        part[(wk * 32 + i * 16 + tile_row(lane, r)) * W + 32 * wc + j * 16 + li] = acc[i][j][r];
   __syncthreads();
   // thread: row tid / TR, columns tid % TR + TR c
   constexpr int TR = 2 * NC * KS, CP = W / TR;
@@ -436,14 +472,13 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int K, const __bf16* __restri
   // 64 registers fit in the two waves per SIMD that the LDS allows)
   float auxv[4][4][4];
   if constexpr (EPI == EPI_SCALE_AUX) {
-    const int rb = m0 + wm * 64, cb = n0 + wn * 64 + (lane & 15);
+    const int rb = m0 + wm * 64 + 4 * (lane >> 4), cb = n0 + wn * 64 + (lane & 15);
 #pragma unroll
     for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
       for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          auxv[ti][tj][r] = e.aux[(size_t)(rb + ti * 16 + tile_row<false>(lane, r)) * e.ldaux + cb + tj * 16];
+        for (int r = 0; r < 4; ++r) auxv[ti][tj][r] = e.aux[(size_t)(rb + ti * 16 + r) * e.ldaux + cb + tj * 16];
   }
   f32x4 acc[4][4];
 #pragma unroll
@@ -495,7 +530,7 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int K, const __bf16* __restri
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < 4; ++j) acc[i][j] = mfma_bf16<EPI>(a[i], b[j], acc[i][j]);
     }
     __builtin_amdgcn_sched_barrier(0);
     lstore(buf ^ 1);
@@ -503,103 +538,18 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int K, const __bf16* __restri
   }
   if constexpr (EPI == EPI_SCALE_AUX) {
     OutT* out = reinterpret_cast<OutT*>(e.out);
-    const int rb = m0 + wm * 64, cb = n0 + wn * 64 + (lane & 15);
+    const int rb = m0 + wm * 64 + 4 * (lane >> 4), cb = n0 + wn * 64 + (lane & 15);
 #pragma unroll
     for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
       for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          out[(size_t)(rb + ti * 16 + tile_row<false>(lane, r)) * e.ldo + cb + tj * 16] =
-              (OutT)((float)acc[ti][tj][r] * auxv[ti][tj][r] * (float)e.pref);
+          out[(size_t)(rb + ti * 16 + r) * e.ldo + cb + tj * 16] =
+              (OutT)(acc[ti][tj][r] * auxv[ti][tj][r] * (float)e.pref);
   } else {
-    epilogue<EPI, OutT, float, f32x4, false, ZINT>(acc, m0, n0, tn, wm, wn, e, sE);
+    epilogue_bf16<EPI, OutT, ZINT, 4, 64, BM>(acc, m0, n0, tn, wm, wn, e, sE);
   }
-}
-
-// BF16 NT GEMM, workgroup tile 256 x 128: four wavefronts of 128 x 64 (8 x 4
-// MFMA tiles), BK = 32 in two LDS stages of (256 + 128) rows x 80 bytes
-// (61 KB: two workgroups per CU). A wavefront reads 12 fragments per 32 MFMAs
-// against 8 per 16 in the 128 x 128 kernel, a quarter less LDS traffic per
-// flop. M a multiple of 256, N of 128, K of 32.
-template <int EPI, class OutT, bool ZINT>
-__global__ __launch_bounds__(256, 2) void k_gemm_bf16_w(int K, const __bf16* __restrict__ A, int lda,
-                                                        const __bf16* __restrict__ B, int ldb, EpiArgs e) {
-  constexpr int TM = 256, BK = 32, LS = BK + 8;  // 80-byte rows: 16-byte fragment reads hit distinct banks
-  __shared__ __align__(16) __bf16 As[2][TM * LS];
-  __shared__ __align__(16) __bf16 Bs[2][BN * LS];
-  __shared__ double sE[2 * TM];
-  int tm, tn;
-  tile_of<TILE_GM>(tm, tn);
-  const int m0 = tm * TM, n0 = tn * BN;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w >> 1, wn = w & 1;
-  // rows lr + 64 j, 16-byte chunk lc; the eight lanes of a store group take rows r and r + 4 of an
-  // 8-row run (at the 80-byte pitch rows r and r + 1 would share a bank at byte 128)
-  const int jr = tid >> 2;
-  const int lr = (jr & ~7) | ((jr & 1) << 2) | ((jr >> 1) & 3), lc = (tid & 3) * 8;
-  {
-    const int z = blockIdx.z;
-    A += z * e.sA;
-    B += z * e.sB;
-    e.out = reinterpret_cast<OutT*>(e.out) + z * e.sOut;
-    if (e.aux) e.aux += z * e.sAux;
-    if (e.bias) e.bias += z * e.sBias;
-    if (e.w3) e.w3 += z * e.sW3;
-    if (e.epart) e.epart += z * e.sEpart;
-    if (e.zscale) e.pref = e.zscale[z];
-  }
-  const __bf16* Ag = A + (size_t)(m0 + lr) * lda + lc;
-  const __bf16* Bg = B + (size_t)(n0 + lr) * ldb + lc;
-  const size_t a64 = (size_t)64 * lda, b64 = (size_t)64 * ldb;
-  f32x4 acc[8][4];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4){0, 0, 0, 0};
-  uint4 ra0, ra1, ra2, ra3, rb0, rb1;  // named: arrays of staging registers are demoted to private memory
-  auto gload = [&](int k) {
-    ra0 = *reinterpret_cast<const uint4*>(Ag + k);
-    ra1 = *reinterpret_cast<const uint4*>(Ag + a64 + k);
-    ra2 = *reinterpret_cast<const uint4*>(Ag + 2 * a64 + k);
-    ra3 = *reinterpret_cast<const uint4*>(Ag + 3 * a64 + k);
-    rb0 = *reinterpret_cast<const uint4*>(Bg + k);
-    rb1 = *reinterpret_cast<const uint4*>(Bg + b64 + k);
-  };
-  auto lstore = [&](int buf) {
-    __bf16* as = &As[buf][lr * LS + lc];
-    __bf16* bs = &Bs[buf][lr * LS + lc];
-    *reinterpret_cast<uint4*>(as) = ra0;
-    *reinterpret_cast<uint4*>(as + 64 * LS) = ra1;
-    *reinterpret_cast<uint4*>(as + 128 * LS) = ra2;
-    *reinterpret_cast<uint4*>(as + 192 * LS) = ra3;
-    *reinterpret_cast<uint4*>(bs) = rb0;
-    *reinterpret_cast<uint4*>(bs + 64 * LS) = rb1;
-  };
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  const int n_stages = K / BK;
-  for (int st = 0; st < n_stages; ++st) {
-    const int buf = st & 1;
-    gload(min(st + 1, n_stages - 1) * BK);
-    __builtin_amdgcn_sched_barrier(0);
-    const __bf16* as = &As[buf][(wm * 128 + (lane & 15)) * LS + 8 * (lane >> 4)];
-    const __bf16* bs = &Bs[buf][(wn * 64 + (lane & 15)) * LS + 8 * (lane >> 4)];
-    bf16x8 b[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) b[t] = *reinterpret_cast<const bf16x8*>(bs + t * 16 * LS);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(as + i * 16 * LS);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[i][j], 0, 0, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    lstore(buf ^ 1);
-    __syncthreads();
-  }
-  epilogue<EPI, OutT, float, f32x4, false, ZINT, 8, 4, 128, 64, TM>(acc, m0, n0, tn, wm, wn, e, sE);
 }
 
 // BF16 NT GEMM fed by direct global-to-LDS loads (global_load_lds_dwordx4):
@@ -640,20 +590,20 @@ __device__ __forceinline__ void pf_read(const unsigned char* sb, int aoff, int b
   for (int i = 0; i < TI; ++i) a[i] = *reinterpret_cast<const bf16x8*>(sb + aoff + i * 16 * DROW);
 }
 
-template <int TI, int I0, int I1>
+template <int EPI, int TI, int I0, int I1>
 __device__ __forceinline__ void pf_mfma(f32x4 (&acc)[TI][4], const bf16x8 (&a)[TI], const bf16x8 (&b)[4]) {
 #pragma unroll
   for (int i = I0; i < I1; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    for (int j = 0; j < 4; ++j) acc[i][j] = mfma_bf16<EPI>(a[i], b[j], acc[i][j]);
 }
 
-template <int TI, int P, int NS, int SB>
+template <int EPI, int TI, int P, int NS, int SB>
 __device__ __forceinline__ void pf_stage(f32x4 (&acc)[TI][4], const bf16x8 (&a)[TI], const bf16x8 (&b)[4],
                                          bf16x8 (&an)[TI], bf16x8 (&bn)[4], const __bf16* const (&src)[P],
                                          unsigned char* dsm, int st, int n_stages, int& slot, int aoff, int boff,
                                          int w) {
-  pf_mfma<TI, 0, TI / 2>(acc, a, b);
+  pf_mfma<EPI, TI, 0, TI / 2>(acc, a, b);
   __builtin_amdgcn_sched_barrier(0);
   wait_vmcnt<(NS - 2) * P>();
   __builtin_amdgcn_s_barrier();
@@ -663,7 +613,7 @@ __device__ __forceinline__ void pf_stage(f32x4 (&acc)[TI][4], const bf16x8 (&a)[
   slot = slot + 1 == NS ? 0 : slot + 1;
   pf_read<TI>(dsm + slot * SB, aoff, boff, an, bn);
   __builtin_amdgcn_sched_barrier(0);
-  pf_mfma<TI, TI / 2, TI>(acc, a, b);
+  pf_mfma<EPI, TI, TI / 2, TI>(acc, a, b);
 }
 
 template <int EPI, class OutT, bool ZINT, int TM, int NS, int OCC>
@@ -719,14 +669,98 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_bf16_pf(int K, const __bf16* 
   pf_read<TI>(dsm, aoff, boff, a0, b0);
   int slot = 0, st = 0;
   for (; st + 1 < n_stages; st += 2) {
-    pf_stage<TI, P, NS, SB>(acc, a0, b0, a1, b1, src, dsm, st, n_stages, slot, aoff, boff, w);
-    pf_stage<TI, P, NS, SB>(acc, a1, b1, a0, b0, src, dsm, st + 1, n_stages, slot, aoff, boff, w);
+    pf_stage<EPI, TI, P, NS, SB>(acc, a0, b0, a1, b1, src, dsm, st, n_stages, slot, aoff, boff, w);
+    pf_stage<EPI, TI, P, NS, SB>(acc, a1, b1, a0, b0, src, dsm, st + 1, n_stages, slot, aoff, boff, w);
   }
-  if (st < n_stages) pf_stage<TI, P, NS, SB>(acc, a0, b0, a1, b1, src, dsm, st, n_stages, slot, aoff, boff, w);
+  if (st < n_stages) pf_stage<EPI, TI, P, NS, SB>(acc, a0, b0, a1, b1, src, dsm, st, n_stages, slot, aoff, boff, w);
   // the loads issued past the last stage land before the workgroup's LDS is released
   wait_vmcnt<0>();
   __builtin_amdgcn_sched_barrier(0);
-  epilogue<EPI, OutT, float, f32x4, false, ZINT, TI, 4, TM / 2, 64, TM>(acc, m0, n0, tn, wm, wn, e, sE);
+  epilogue_bf16<EPI, OutT, ZINT, TI, TM / 2, TM>(acc, m0, n0, tn, wm, wn, e, sE);
+}
+
+// BF16 NT GEMM for few tiles: workgroup tile (32 TI) x 128, four wavefronts of
+// (16 TI) x 64, BK = 64 in a three-slot ring of direct global-to-LDS loads (two
+// stages in flight), stages laid out as in k_gemm_f64: rows of 128 bytes with
+// chunk c of row r at c ^ (r & 7). Small systems leave 128 x 128 tiles on a
+// fraction of the 256 CUs, each walking the whole K alone. M a multiple of 32 TI,
+// N of 128, K of 64.
+__host__ __device__ constexpr int few_stage_bytes(int ti) { return (32 * ti + BN) * 128; }
+__host__ __device__ constexpr int few_lds_bytes(int ti) { return 3 * few_stage_bytes(ti) + 2 * 32 * ti * 8; }
+
+template <int EPI, class OutT, bool ZINT, int TI>
+__global__ __launch_bounds__(256, 2) void k_gemm_bf16_few(int K, const __bf16* __restrict__ A, int lda,
+                                                          const __bf16* __restrict__ B, int ldb, EpiArgs e) {
+  constexpr int SB = few_stage_bytes(TI), NS = 3, P = TI + 4, NBA = 4 * TI;
+  extern __shared__ __align__(16) unsigned char dsm[];
+  double* sE = reinterpret_cast<double*>(dsm + NS * SB);
+  int tm, tn;
+  tile_of<TILE_GM>(tm, tn);
+  const int m0 = tm * 32 * TI, n0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wm = w >> 1, wn = w & 1;
+  {
+    const int z = blockIdx.z;
+    A += z * e.sA;
+    B += z * e.sB;
+    e.out = reinterpret_cast<OutT*>(e.out) + z * e.sOut;
+    if (e.aux) e.aux += z * e.sAux;
+    if (e.bias) e.bias += z * e.sBias;
+    if (e.w3) e.w3 += z * e.sW3;
+    if (e.epart) e.epart += z * e.sEpart;
+    if (e.zscale) e.pref = e.zscale[z];
+  }
+  const int lrow = lane >> 3, lchunk = (lane & 7) ^ lrow;
+  const __bf16* src[P];
+#pragma unroll
+  for (int j = 0; j < P; ++j) {
+    const int b = w + 4 * j;
+    src[j] = b < NBA ? A + (size_t)(m0 + 8 * b + lrow) * lda + 8 * lchunk
+                     : B + (size_t)(n0 + 8 * (b - NBA) + lrow) * ldb + 8 * lchunk;
+  }
+  const int n_stages = K / 64;
+  auto issue = [&](int st, int slot) {
+    const int k0 = min(st, n_stages - 1) * 64;  // an in-bounds repeat past the end
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+      __builtin_amdgcn_global_load_lds(const_cast<__bf16*>(src[j] + k0), dsm + slot * SB + (w + 4 * j) * 1024, 16, 0, 0);
+  };
+  const int li = lane & 15, lg = lane >> 4;
+  const int aoff = (wm * 16 * TI + li) * 128, boff = (32 * TI + wn * 64 + li) * 128;
+  f32x4 acc[TI][4];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4){0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) issue(s, s);
+  int slot = 0, fill = NS - 1;
+  for (int st = 0; st < n_stages; ++st) {
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<(NS - 2) * P>();  // this wavefront's part of stage st has landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(st + NS - 1, fill);  // into the slot that every wavefront read in the last round
+    fill = fill + 1 == NS ? 0 : fill + 1;
+    const unsigned char* sb = dsm + slot * SB;
+    slot = slot + 1 == NS ? 0 : slot + 1;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int cp = ((4 * ks + lg) ^ (li & 7)) << 4;
+      bf16x8 a[TI], b[4];
+#pragma unroll
+      for (int t = 0; t < TI; ++t) a[t] = *reinterpret_cast<const bf16x8*>(sb + aoff + t * 16 * 128 + cp);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) b[t] = *reinterpret_cast<const bf16x8*>(sb + boff + t * 16 * 128 + cp);
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = mfma_bf16<EPI>(a[i], b[j], acc[i][j]);
+    }
+  }
+  wait_vmcnt<0>();  // the loads issued past the last stage land before the LDS is released
+  __builtin_amdgcn_sched_barrier(0);
+  epilogue_bf16<EPI, OutT, ZINT, TI, 16 * TI, 32 * TI>(acc, m0, n0, tn, wm, wn, e, sE);
 }
 
 // E_i = delta^2 sum_t epart[i][t] + e0. 16 lanes a row, lane t adding partials
@@ -762,44 +796,58 @@ static EpiArgs gap_epi(const tgx_model_t* m) {
   return e;
 }
 
-// BF16 NT GEMM launch. Plain FP32 stores with at least 512 tiles of 256 x 128
-// (one round of two workgroups per CU) go to the kernel fed by direct LDS
-// loads (0.389 -> 0.345 ms on the 32,768 x 1,280 x 4,096 Qss product, with the
-// grouped tile order); the GAP and second-layer epilogues to its 128 x 128
-// form with three workgroups per CU (GAP kernel 0.495 -> 0.476 ms, second
-// layer 0.052 -> 0.047 ms). The SiLU and scaled epilogues measured faster on
-// the register-staged kernels.
-// Otherwise 256 x 128 tiles when M is a multiple of 256 and there are at least
-// 1,024 of them (two rounds of two workgroups per CU; with fewer, the last
-// round's imbalance costs more than the wider tile saves, measured on the
-// 32,768-row MLP shapes), else 128 x 128. The GAP epilogue writes one energy
-// partial per row and 128-column tile either way.
+template <int EPI, class OutT, bool ZINT, int TM, int NS, int OCC>
+static int launch_pf(tgx_ctx* ctx, const char* name, int M, int N, int K, int batch, const __bf16* A, int lda,
+                     const __bf16* B, int ldb, EpiArgs e) {
+  TGX_LAUNCH(ctx, name, (k_gemm_bf16_pf<EPI, OutT, ZINT, TM, NS, OCC>), dim3(N / BN, M / TM, batch), dim3(256),
+             dma_lds_bytes(TM, NS), K, A, lda, B, ldb, e);
+  return TGX_OK;
+}
+
+template <int EPI, class OutT, bool ZINT, int TI>
+static int launch_few(tgx_ctx* ctx, const char* name, int M, int N, int K, int batch, const __bf16* A, int lda,
+                      const __bf16* B, int ldb, EpiArgs e) {
+  TGX_LAUNCH(ctx, name, (k_gemm_bf16_few<EPI, OutT, ZINT, TI>), dim3(N / BN, M / (32 * TI), batch), dim3(256),
+             few_lds_bytes(TI), K, A, lda, B, ldb, e);
+  return TGX_OK;
+}
+
+// BF16 NT GEMM launch, by the number of 128 x 128 tiles t (256 CUs, two or three
+// workgroups each), all times alone on the card:
+//   t <= 96    32-row tiles (512 x 768 x 1,280, 24 tiles: 0.012 ms, 128-row tiles 0.017-0.023)
+//   t < 384    64-row tiles (1,024 x 4,096 x 1,280, 256 tiles: 0.020 against 0.026); plain products with a long
+//              K up to 1,023 (8,192 x 1,280 x 4,096, 640 tiles: 0.104 against 0.106-0.117)
+//   M a multiple of 256, t >= 1,024: the 256-row direct-load kernel for plain and GAP epilogues (32,768 x 1,280 x
+//              4,096: 0.356 ms, 128-row tiles 0.412; GAP 32,768 x 4,096 x 1,280: 0.392 against 0.501)
+//   else       the 128-row direct-load kernel for plain, GAP and second-layer epilogues, and the register-staged
+//              one for the two that read or write an FP32 factor (32,768 x 256 x 256 x 3 alike at 0.041 ms; beside
+//              the other block the 256-row SiLU kernel, faster alone, is not: 0.239 against 0.232)
+// The GAP and second-layer epilogues write one energy partial per row and
+// 128-column tile whatever the rule.
 template <int EPI, class OutT, bool ZINT>
 static int launch_bf16(tgx_ctx* ctx, const char* name, int M, int N, int K, int batch, const __bf16* A, int lda,
                        const __bf16* B, int ldb, EpiArgs e) {
   TGX_REQUIRE(M % BM == 0 && N % BN == 0 && K % 64 == 0 && lda % 8 == 0 && ldb % 8 == 0,
               "gemm_bf16 %s: unpadded shape %d x %d x %d", name, M, N, K);
-  if constexpr (EPI == EPI_STORE) {
-    if (M % 256 == 0 && (long)(M / 256) * (N / BN) * batch >= 512) {
-      TGX_LAUNCH(ctx, name, (k_gemm_bf16_pf<EPI, OutT, ZINT, 256, 3, 2>), dim3(N / BN, M / 256, batch), dim3(256),
-                 dma_lds_bytes(256, 3), K, A, lda, B, ldb, e);
-      return TGX_OK;
-    }
+  if constexpr (exchanged<EPI>())  // four columns at a time
+    TGX_REQUIRE(e.ldo % 4 == 0 && e.sOut % 4 == 0 && e.sBias % 4 == 0 && e.sW3 % 4 == 0 && (uintptr_t)e.out % 8 == 0 &&
+                    ((uintptr_t)e.bias | (uintptr_t)e.w3 | (uintptr_t)e.alpha_f) % 16 == 0,
+                "gemm_bf16 %s: misaligned epilogue operands", name);
+  const int64_t t = (int64_t)(M / BM) * (N / BN) * batch;
+  if (t <= 96) return launch_few<EPI, OutT, ZINT, 1>(ctx, name, M, N, K, batch, A, lda, B, ldb, e);
+  if (t < 384 || (EPI == EPI_STORE && K >= 2048 && t < 1024))
+    return launch_few<EPI, OutT, ZINT, 2>(ctx, name, M, N, K, batch, A, lda, B, ldb, e);
+  if constexpr (EPI == EPI_STORE || EPI == EPI_GAP) {
+    if (M % 256 == 0 && t >= 1024)
+      return launch_pf<EPI, OutT, ZINT, 256, 3, 2>(ctx, name, M, N, K, batch, A, lda, B, ldb, e);
   }
-  if constexpr (EPI == EPI_GAP || EPI == EPI_ACT2) {
-    if (K % DK == 0) {
-      TGX_LAUNCH(ctx, name, (k_gemm_bf16_pf<EPI, OutT, ZINT, 128, 3, 3>), dim3(N / BN, M / BM, batch), dim3(256),
-                 dma_lds_bytes(128, 3), K, A, lda, B, ldb, e);
-      return TGX_OK;
-    }
-  }
-  if (M % 256 == 0 && (long)(M / 256) * (N / BN) * batch >= 1024)
-    TGX_LAUNCH(ctx, name, (k_gemm_bf16_w<EPI, OutT, ZINT>), dim3(N / BN, M / 256, batch), dim3(256), 0, K, A, lda, B,
-               ldb, e);
-  else
+  if constexpr (EPI == EPI_STORE || EPI == EPI_GAP || EPI == EPI_ACT2) {
+    return launch_pf<EPI, OutT, ZINT, 128, 3, 3>(ctx, name, M, N, K, batch, A, lda, B, ldb, e);
+  } else {
     TGX_LAUNCH(ctx, name, (k_gemm_bf16<EPI, OutT, ZINT>), dim3(N / BN, M / BM, batch), dim3(256), 0, K, A, lda, B, ldb,
                e);
-  return TGX_OK;
+    return TGX_OK;
+  }
 }
 
 template <int EPI, bool ZINT, int TI, int TJ, int OCC>
@@ -879,18 +927,21 @@ int tgx_gap_contract_f64(tgx_ctx* ctx, const tgx_model_t* m, int ns, const doubl
 int tgx_gap_contract(tgx_ctx* ctx, tgx_model_t* m, int path, bool do_forces) {
   const int ns = m->n_sites_b;
   if (ns == 0) return TGX_OK;
-  const int Mp = (int)tgx_round_up(ns, BM);
   const int Sp = m->Spad, Dp = m->Dpad;
   const int n_tiles = Sp / BN;
-  TGX_TRY(m->epart.ensure(sizeof(double) * (size_t)Mp * n_tiles));
-  TGX_TRY(m->e_site.ensure(sizeof(double) * (size_t)Mp));
   if (path == TGX_PATH_FP64_PLAIN || path == TGX_PATH_FP64_ADJOINT) {
+    const int Mp = (int)tgx_round_up(ns, BM);
+    TGX_TRY(m->epart.ensure(sizeof(double) * (size_t)Mp * n_tiles));
+    TGX_TRY(m->e_site.ensure(sizeof(double) * (size_t)Mp));
     TGX_TRY(m->kd64.ensure(sizeof(double) * (size_t)Mp * Sp));
     if (do_forces) TGX_TRY(m->qss64.ensure(sizeof(double) * (size_t)Mp * Dp));
     return tgx_gap_contract_f64(ctx, m, ns, m->q64.as<double>(), m->kd64.as<double>(), m->epart.as<double>(),
                                 m->e_site.as<double>(), do_forces ? m->qss64.as<double>() : nullptr);
   }
   // mixed path: qbf (BF16 descriptors) comes from the FP32 descriptor pass
+  const int Mp = tgx_rows_bf16(ns);
+  TGX_TRY(m->epart.ensure(sizeof(double) * (size_t)Mp * n_tiles));
+  TGX_TRY(m->e_site.ensure(sizeof(double) * (size_t)Mp));
   EpiArgs e = gap_epi(m);
   e.epart = m->epart.as<double>();
   e.n_tiles = n_tiles;

@@ -45,6 +45,11 @@ void tgx_set_error(const char* fmt, ...);
 
 static inline int64_t tgx_round_up(int64_t x, int64_t g) { return (x + g - 1) / g * g; }
 
+// Rows of a block's arrays that the BF16 products read or write, for ns centres:
+// whole 128-row tiles, and from 4,096 on whole 256-row ones (the wider tile is
+// the faster one there; at most 127 rows more work).
+static inline int tgx_rows_bf16(int64_t ns) { return (int)tgx_round_up(ns, ns >= 4096 ? 256 : 128); }
+
 // Growable device buffer.
 struct dbuf {
   void* p = nullptr;

@@ -1400,7 +1400,7 @@ int tgx_surrogate_eval(tgx_ctx* ctx, tgx_model_t* m, bool selected) {
   const int ns = m->n_sites_b;
   if (ns == 0) return TGX_OK;
   TGX_TRY(tgx_soap_descriptors(ctx, m, TGX_PATH_MIXED, false));
-  const int Mp = (int)tgx_round_up(ns, 128), Dp = m->Dpad;
+  const int Mp = tgx_rows_bf16(ns), Dp = m->Dpad;
   TGX_TRY(ensemble_pack(ctx, sl, K, Dp));
   const EnsemblePack& pk = sl.pack;
   const int KH = K * H;
@@ -1477,7 +1477,7 @@ int tgx_surrogate_eval(tgx_ctx* ctx, tgx_model_t* m, bool selected) {
 int tgx_surrogate_finish(tgx_ctx* ctx, tgx_model_t* m, int ng) {
   const int ns = m->n_sites_b;
   if (ns == 0) return TGX_OK;
-  const int Mp = (int)tgx_round_up(ns, 128), Dp = m->Dpad;
+  const int Mp = tgx_rows_bf16(ns), Dp = m->Dpad;
   if (ng > 0) {
     const int ngp = (int)tgx_round_up(ng, 128);
     TGX_TRY(m->q64.ensure(sizeof(double) * (size_t)ngp * Dp));

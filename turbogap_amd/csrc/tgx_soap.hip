@@ -1419,7 +1419,7 @@ int tgx_soap_descriptors(tgx_ctx* ctx, tgx_model_t* m, int path, bool with_der) 
       TGX_TRY(tgx_desc_f32(ctx, m));  // writes the BF16 copy as well
     } else {
       TGX_TRY(tgx_desc_wave(ctx, m, false, nullptr, ns, m->q32.p, m->pnorm.p));
-      TGX_TRY(m->qbf.ensure(sizeof(__bf16) * nsp * m->Dpad));
+      TGX_TRY(m->qbf.ensure(sizeof(__bf16) * (size_t)tgx_rows_bf16(ns) * m->Dpad));
       TGX_TRY(tgx_f32_to_bf16(ctx, m->q32.as<float>(), m->qbf.as<__bf16>(), (int64_t)nsp * m->Dpad));
     }
   }

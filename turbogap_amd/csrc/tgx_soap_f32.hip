@@ -1496,7 +1496,7 @@ int tgx_desc_f32(tgx_ctx* ctx, tgx_model_t* m) {
   }
   const size_t lds = sizeof(float) * (size_t)WAVES * desc_wave_floats(m->P);
   TGX_REQUIRE(lds <= 160 * 1024, "FP32 descriptor kernel needs %zu bytes of LDS", lds);
-  TGX_TRY(m->qbf.ensure(sizeof(__bf16) * (size_t)tgx_round_up(ns, 128) * m->Dpad));
+  TGX_TRY(m->qbf.ensure(sizeof(__bf16) * (size_t)tgx_rows_bf16(ns) * m->Dpad));
   // the matrix-core adjoint forms the power spectrum from the coefficients
   // again: the FP32 descriptors and norms are written only for the other one
   const bool fp32_copy = !adjoint_on_mfma(m, a);
