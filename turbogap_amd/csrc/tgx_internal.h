@@ -252,7 +252,6 @@ struct tgx_ctx {
   int64_t* pairs_host = nullptr;  // pinned: the list build's pair count
   int gate_host_n = 0;
   dbuf gate_mask;
-  hipEvent_t ev_blocks = nullptr;  // recorded on the context stream before concurrent blocks start
   int block_streams = 1;           // blocks of distinct central species on streams of their own: 0 off, 1 default, 2 every path
   // profiling
   bool profiling = false;
@@ -292,6 +291,8 @@ int tgx_block_select(tgx_ctx* ctx, tgx_model_t* m);
 // pinned memory (no wait), then, after the caller has synchronised the stream,
 // allocation and fill.
 int tgx_block_select_count(tgx_ctx* ctx, tgx_model_t* m);
+// The same for several blocks at once on the context's stream.
+int tgx_blocks_select_count(tgx_ctx* ctx, tgx_model_t* const* models, int count);
 // Host copies of the count half's per-atom centre flags and pair offsets
 // (n and n + 1 values), after the stream has been synchronised.
 int tgx_block_select_counts_host(tgx_ctx* ctx, tgx_model_t* m, std::vector<int>& flag, std::vector<int64_t>& pair_off);

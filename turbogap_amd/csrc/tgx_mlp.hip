@@ -484,7 +484,7 @@ __global__ void k_append(int n_take, int stride, int offset, int Dp, const doubl
 __global__ void k_surrogate_out(int n, int K, const double* __restrict__ epart, int ldm, int nt,
                                 const float* __restrict__ b3, const double* __restrict__ shift,
                                 const double* __restrict__ scale, double* __restrict__ e_site, float threshold,
-                                int* __restrict__ stat, int* __restrict__ gated) {
+                                int* __restrict__ stat, int* __restrict__ gated, int* __restrict__ host) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const bool in = i < n;
   double s = 0.0, lo = 1e300, hi = -1e300;
@@ -510,6 +510,15 @@ __global__ void k_surrogate_out(int n, int K, const double* __restrict__ epart, 
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
     if ((threadIdx.x & 63) == 0) atomicMax(&stat[1], m);
     if (in && sp > threshold) gated[atomicAdd(&stat[0], 1)] = i;
+    // the last workgroup hands the two counters to pinned memory and clears them
+    // (and the count of workgroups, stat[2]) for the next step
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(&stat[2], 1) == (int)gridDim.x - 1) {
+      host[0] = atomicExch(&stat[0], 0);
+      host[1] = atomicExch(&stat[1], 0);
+      atomicExch(&stat[2], 0);
+    }
   }
 }
 
@@ -1385,7 +1394,7 @@ extern "C" int tgx_surrogate_stats(tgx_ctx* ctx, double* gated_fraction, double*
 //           w3_k silu(z2_k + b2_k), from which the output kernel forms E_k
 //   back2 : a1_k = -(scale_k/K) (a2_k W2_k) o s1_k           batched over k
 //   back1 : Qss = a1 W1Tcat^T = -(1/K) sum_k scale_k dE_k/dq  one GEMM, depth K H
-int tgx_surrogate_eval(tgx_ctx* ctx, tgx_model_t* m, bool selected) {
+int tgx_surrogate_eval(tgx_ctx* ctx, tgx_model_t* m, bool selected, int* gate_host) {
   int model_id = -1;
   for (int k = 0; k < (int)ctx->models.size(); ++k)
     if (ctx->models[k] == m) model_id = k;
@@ -1461,13 +1470,14 @@ int tgx_surrogate_eval(tgx_ctx* ctx, tgx_model_t* m, bool selected) {
   b1.C = m->qss32.p; b1.ldc = Dp;
   TGX_TRY(tgx_gemm_bf16(ctx, "mlp_back1", b1));
 
-  TGX_TRY(m->gate_stat.ensure(sizeof(int) * 2));
+  const bool fresh = !m->gate_stat.p;
+  TGX_TRY(m->gate_stat.ensure(sizeof(int) * 3));
+  if (fresh) TGX_TRY(tgx_zero(ctx, m->gate_stat.p, sizeof(int) * 3));  // later steps find it cleared
   TGX_TRY(m->gate_list.ensure(sizeof(int) * (size_t)Mp));
-  TGX_TRY(tgx_zero(ctx, m->gate_stat.p, sizeof(int) * 2));
   TGX_LAUNCH(ctx, "mlp_out", k_surrogate_out, g1(ns), dim3(256), 0, ns, K, (const double*)e2part, Mp, nt2,
              pk.b3.as<float>(), pk.shift.as<double>(),
              pk.scale.as<double>(), m->e_site.as<double>(), (float)ctx->gate_threshold, m->gate_stat.as<int>(),
-             m->gate_list.as<int>());
+             m->gate_list.as<int>(), gate_host);
   return TGX_OK;
 }
 

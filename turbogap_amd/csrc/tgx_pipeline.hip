@@ -29,30 +29,42 @@ struct SpeciesMap {
 // Only atoms in [lo, hi) can be centres (a batch of the block's sites). Two
 // atoms per wavefront, 32 lanes each, as the fill (one thread walking its
 // atom's list took 18 us, 37 at 53 neighbours; this takes 5).
-__global__ __launch_bounds__(256) void k_select_count(int n, int lo, int hi, SpeciesMap sm, int central, double rcut,
-                                                    const int* __restrict__ n_neigh, const int64_t* __restrict__ off,
-                                                    const int* __restrict__ species, const double* __restrict__ rjs,
-                                                    const int* __restrict__ nspec, int* __restrict__ flag,
-                                                    int* __restrict__ npairs) {
+// One block per blockIdx.y.
+struct SelectTask {
+  SpeciesMap sm;
+  int lo, hi, central;
+  double rcut;
+  int* flag;
+  int* npairs;
+};
+constexpr int SELECT_TASKS = TGX_SCAN_TASKS / 2;
+struct SelectTasks {
+  SelectTask t[SELECT_TASKS];
+};
+
+__global__ __launch_bounds__(256) void k_select_count(int n, SelectTasks ts, const int* __restrict__ n_neigh,
+                                                    const int64_t* __restrict__ off, const int* __restrict__ species,
+                                                    const double* __restrict__ rjs, const int* __restrict__ nspec) {
+  const SelectTask& t = ts.t[blockIdx.y];
   const int lane = threadIdx.x & 63, sub = lane & 31;
   const uint64_t half = (lane < 32 ? 0xffffffffull : 0xffffffff00000000ull);
   const int i = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 2 + (lane >> 5);
   if (i >= n) return;
-  const int sc = sm.index(species[i]);
+  const int sc = t.sm.index(species[i]);
   const int nn = n_neigh[i];
-  const bool sel = i >= lo && i < hi && nn > 0 && sc >= 0 && (central == 0 || sc == central - 1);
+  const bool sel = i >= t.lo && i < t.hi && nn > 0 && sc >= 0 && (t.central == 0 || sc == t.central - 1);
   int cnt = 0;
   if (sel) {
     const int64_t b = off[i];
     for (int base = 0; base < nn; base += 32) {
       const int k = base + sub;
-      const bool keep = k < nn && rjs[b + k] < rcut && sm.index(nspec[b + k]) >= 0;
+      const bool keep = k < nn && rjs[b + k] < t.rcut && t.sm.index(nspec[b + k]) >= 0;
       cnt += __popcll(__ballot(keep) & half);
     }
   }
   if (sub == 0) {
-    flag[i] = sel ? 1 : 0;
-    npairs[i] = cnt;
+    t.flag[i] = sel ? 1 : 0;
+    t.npairs[i] = cnt;
   }
 }
 
@@ -203,10 +215,17 @@ __global__ __launch_bounds__(256) void k_finish(FinishArgs a) {
   }
 }
 
-__global__ void k_energy_scatter(int ns, const int* __restrict__ site_atom, const double* __restrict__ e_site,
-                                 double* __restrict__ energies) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s < ns) energies[site_atom[s]] += e_site[s];
+// Centre energies into their atoms, one block per blockIdx.y (blocks of one launch
+// have no centre in common).
+struct ScatterTasks {
+  int ns[SELECT_TASKS];
+  const int* atom[SELECT_TASKS];
+  const double* e[SELECT_TASKS];
+};
+
+__global__ void k_energy_scatter(ScatterTasks t, double* __restrict__ energies) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
+  if (s < t.ns[k]) energies[t.atom[k][s]] += t.e[k][s];
 }
 
 }  // namespace
@@ -238,20 +257,32 @@ static SelectView select_view(tgx_model_t* m, int n) {
   return v;
 }
 
-int tgx_block_select_count(tgx_ctx* ctx, tgx_model_t* m) {
+int tgx_blocks_select_count(tgx_ctx* ctx, tgx_model_t* const* models, int count) {
   TGX_REQUIRE(ctx->have_list, "no neighbour list: call tgx_build_neighbors_list first");
   const int n = ctx->n_sites;
-  // the block's own scratch: blocks may be selected while another block's kernels still run
-  TGX_TRY(m->sel_scratch.ensure(sizeof(int) * 2 * (size_t)n + sizeof(int64_t) * 2 * (size_t)(n + 1) + 256));
-  const SelectView v = select_view(m, n);
-  SpeciesMap sm = species_map(m);
-  const int lo = m->sel_lo > 0 ? m->sel_lo : 0, hi = (m->sel_hi >= 0 && m->sel_hi < n) ? m->sel_hi : n;
-  TGX_LAUNCH(ctx, "select_count", k_select_count, dim3((n + 7) / 8), dim3(256), 0, n, lo, hi, sm,
-             m->central_species, m->rcut_max, ctx->n_neigh.as<int>(), ctx->nl_off.as<int64_t>(),
-             ctx->species_sc.as<int>(), ctx->rjs.as<double>(), ctx->nspec.as<int>(), v.flag, v.npairs);
-  if (!m->sel_host) TGX_CHECK_HIP(hipHostMalloc((void**)&m->sel_host, 2 * sizeof(int64_t), hipHostMallocDefault));
-  return tgx_scan2_i32(ctx, v.flag, v.site_idx, v.npairs, v.pair_off, n, m->scan_tmp, m->sel_host);
+  for (int k0 = 0; k0 < count; k0 += SELECT_TASKS) {
+    const int cnt = std::min(SELECT_TASKS, count - k0);
+    SelectTasks st{};
+    tgx_scan_tasks sc{};
+    for (int k = 0; k < cnt; ++k) {
+      tgx_model_t* m = models[k0 + k];
+      // the block's own scratch: blocks may be selected while another block's kernels still run
+      TGX_TRY(m->sel_scratch.ensure(sizeof(int) * 2 * (size_t)n + sizeof(int64_t) * 2 * (size_t)(n + 1) + 256));
+      if (!m->sel_host) TGX_CHECK_HIP(hipHostMalloc((void**)&m->sel_host, 2 * sizeof(int64_t), hipHostMallocDefault));
+      const SelectView v = select_view(m, n);
+      const int lo = m->sel_lo > 0 ? m->sel_lo : 0, hi = (m->sel_hi >= 0 && m->sel_hi < n) ? m->sel_hi : n;
+      st.t[k] = SelectTask{species_map(m), lo, hi, m->central_species, m->rcut_max, v.flag, v.npairs};
+      sc.t[2 * k] = tgx_scan_task{v.flag, v.site_idx, m->sel_host};
+      sc.t[2 * k + 1] = tgx_scan_task{v.npairs, v.pair_off, m->sel_host + 1};
+    }
+    TGX_LAUNCH(ctx, "select_count", k_select_count, dim3((n + 7) / 8, cnt), dim3(256), 0, n, st, ctx->n_neigh.as<int>(),
+               ctx->nl_off.as<int64_t>(), ctx->species_sc.as<int>(), ctx->rjs.as<double>(), ctx->nspec.as<int>());
+    TGX_TRY(tgx_scan_many(ctx, sc, 2 * cnt, n, &models[k0]->scan_tmp));
+  }
+  return TGX_OK;
 }
+
+int tgx_block_select_count(tgx_ctx* ctx, tgx_model_t* m) { return tgx_blocks_select_count(ctx, &m, 1); }
 
 int tgx_block_select_counts_host(tgx_ctx* ctx, tgx_model_t* m, std::vector<int>& flag, std::vector<int64_t>& pair_off) {
   const int n = ctx->n_sites;
@@ -364,13 +395,26 @@ int tgx_gather_pair_forces(tgx_ctx* ctx, const double* fglob, double* F, double*
   return tgx_gather_collect(ctx, virial_out, energy_out);
 }
 
-int tgx_energy_scatter(tgx_ctx* ctx, tgx_model_t* m) {
-  const int ns = m->n_sites_b;
-  if (ns == 0) return TGX_OK;
-  TGX_LAUNCH(ctx, "energy_scatter", k_energy_scatter, dim3((ns + 255) / 256), dim3(256), 0, ns, m->site_atom.as<int>(),
-             m->e_site.as<double>(), ctx->energies.as<double>());
+int tgx_energy_scatter_blocks(tgx_ctx* ctx, tgx_model_t* const* models, int count) {
+  for (int k0 = 0; k0 < count; k0 += SELECT_TASKS) {
+    const int cnt = std::min(SELECT_TASKS, count - k0);
+    ScatterTasks t{};
+    int most = 0;
+    for (int k = 0; k < cnt; ++k) {
+      tgx_model_t* m = models[k0 + k];
+      t.ns[k] = m->n_sites_b;
+      t.atom[k] = m->site_atom.as<int>();
+      t.e[k] = m->e_site.as<double>();
+      most = std::max(most, m->n_sites_b);
+    }
+    if (most == 0) continue;
+    TGX_LAUNCH(ctx, "energy_scatter", k_energy_scatter, dim3((most + 255) / 256, cnt), dim3(256), 0, t,
+               ctx->energies.as<double>());
+  }
   return TGX_OK;
 }
+
+int tgx_energy_scatter(tgx_ctx* ctx, tgx_model_t* m) { return tgx_energy_scatter_blocks(ctx, &m, 1); }
 
 // Marks (two ints an atom) of the atoms a block touches: mark[0][j] for every
 // kept neighbour (a centre's self entry among them), mark[1][i] for the centres.
@@ -401,7 +445,7 @@ __global__ void k_fold_out(int n, const double* __restrict__ F, const double* __
     out[3 * (size_t)i + 2] = F[3 * (size_t)i + 2];
   }
   out[3 * (size_t)n + i] = energies[i];
-  reinterpret_cast<int*>(out + 4 * (size_t)n)[i] = (mark[i] ? 1 : 0) | (mark[n + i] ? 2 : 0);
+  if (mark) reinterpret_cast<int*>(out + 4 * (size_t)n)[i] = (mark[i] ? 1 : 0) | (mark[n + i] ? 2 : 0);
 }
 
 int tgx_fold_out(tgx_ctx* ctx, const double* F, const int* d_mark) {

@@ -12,12 +12,18 @@ int tgx_zero2(tgx_ctx* ctx, void* p, size_t np, void* q, size_t nq);
 // go to tmp, or to the context's own scratch when tmp is NULL; scans that may
 // run on different streams at once must each bring their own.
 int tgx_scan_i32(tgx_ctx* ctx, const int* in, int64_t* out, int64_t n, int64_t* total, dbuf* tmp = nullptr);
-// The same for two arrays of n values, their totals in totals[0] and totals[1]
-// (one launch for both up to 8,192 values, two up to 65,536, six above); block
-// totals in tmp, which belongs to the caller so that scans on different streams
-// do not share it.
-int tgx_scan2_i32(tgx_ctx* ctx, const int* in0, int64_t* out0, const int* in1, int64_t* out1, int64_t n,
-                  dbuf& tmp, int64_t* totals);
+// The same for several arrays of n values at once (one launch for all of them up
+// to 8,192 values, two up to 65,536, three each above).
+constexpr int TGX_SCAN_TASKS = 16;
+struct tgx_scan_task {
+  const int* in;
+  int64_t* out;
+  int64_t* tot;
+};
+struct tgx_scan_tasks {
+  tgx_scan_task t[TGX_SCAN_TASKS];
+};
+int tgx_scan_many(tgx_ctx* ctx, const tgx_scan_tasks& ts, int count, int64_t n, dbuf* tmp);
 
 // Partial sums of n doubles into TGX_SUM_PARTS device values, each over a fixed
 // contiguous slice in a fixed tree (summed on the host in order).

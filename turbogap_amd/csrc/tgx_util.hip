@@ -111,17 +111,16 @@ __device__ int64_t block_exclusive_scan_waves(int64_t v, int64_t* sh, int64_t* t
 }
 
 // Whole exclusive scan in one workgroup (n up to SCAN_SINGLE_MAX = 8 per
-// thread), one or two arrays (blockIdx.y): thread t owns the contiguous chunk
-// [t c, (t+1) c), loaded at once into registers; the 1024 chunk sums are scanned
-// and each thread writes its chunk's prefixes; out[n] is the total, also stored
-// at tot (pinned host memory) when given.
+// thread) of the arrays of a task list (blockIdx.y): thread t owns the contiguous
+// chunk [t c, (t+1) c), loaded at once into registers; the 1024 chunk sums are
+// scanned and each thread writes its chunk's prefixes; out[n] is the total, also
+// stored at tot (pinned host memory) when given.
 constexpr int SCAN_CMAX = 8;
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_single(const int* __restrict__ in0, int64_t* __restrict__ out0,
-                                                           const int* __restrict__ in1, int64_t* __restrict__ out1,
-                                                           int64_t n, int64_t* __restrict__ tot) {
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_single(tgx_scan_tasks ts, int64_t n) {
   __shared__ int64_t sh[2 * SCAN_BLOCK / 64];
-  const int* in = blockIdx.y ? in1 : in0;
-  int64_t* out = blockIdx.y ? out1 : out0;
+  const tgx_scan_task& task = ts.t[blockIdx.y];
+  const int* __restrict__ in = task.in;
+  int64_t* __restrict__ out = task.out;
   const int c = (int)((n + SCAN_BLOCK - 1) / SCAN_BLOCK);
   const int64_t b = (int64_t)threadIdx.x * c;
   int v[SCAN_CMAX];
@@ -140,22 +139,20 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_single(const int* __restric
   }
   if (threadIdx.x == 0) {
     out[n] = total;
-    if (tot) tot[blockIdx.y] = total;
+    if (task.tot) *task.tot = total;
   }
 }
 
-// Two-launch exclusive scan of up to SCAN_2L_MAX values, one or two arrays
-// (blockIdx.y picks in0/out0 or in1/out1): k_scan_local2 scans each block of
-// 1024 values and stores the block totals; k_scan_add2 adds to every block the
-// sum of the totals before it (at most 63 of them, summed by its first
-// wavefront), and the last block writes out[n].
+// Two-launch exclusive scan of up to SCAN_2L_MAX values, each array of a task
+// list (blockIdx.y): k_scan_local2 scans each block of 1024 values and stores the
+// block totals; k_scan_add2 adds to every block the sum of the totals before it
+// (at most 63 of them, summed by its first wavefront), and the last block writes
+// out[n].
 constexpr int64_t SCAN_2L_MAX = 64 * (int64_t)SCAN_BLOCK;
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_local2(const int* __restrict__ in0, int64_t* __restrict__ out0,
-                                                           const int* __restrict__ in1, int64_t* __restrict__ out1,
-                                                           int64_t n, int64_t* __restrict__ sums) {
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_local2(tgx_scan_tasks ts, int64_t n, int64_t* __restrict__ sums) {
   __shared__ int64_t sh[2 * SCAN_BLOCK / 64];
-  const int* in = blockIdx.y ? in1 : in0;
-  int64_t* out = blockIdx.y ? out1 : out0;
+  const int* __restrict__ in = ts.t[blockIdx.y].in;
+  int64_t* __restrict__ out = ts.t[blockIdx.y].out;
   const int64_t i = (int64_t)blockIdx.x * SCAN_BLOCK + threadIdx.x;
   const int64_t v = i < n ? in[i] : 0;
   int64_t tot;
@@ -164,11 +161,10 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_local2(const int* __restric
   if (threadIdx.x == 0) sums[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = tot;
 }
 
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add2(int64_t* __restrict__ out0, int64_t* __restrict__ out1,
-                                                         int64_t n, const int64_t* __restrict__ sums,
-                                                         int64_t* __restrict__ tot) {
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add2(tgx_scan_tasks ts, int64_t n,
+                                                         const int64_t* __restrict__ sums) {
   __shared__ int64_t off;
-  int64_t* out = blockIdx.y ? out1 : out0;
+  int64_t* __restrict__ out = ts.t[blockIdx.y].out;
   const int64_t* bs = sums + (size_t)blockIdx.y * gridDim.x;
   if (threadIdx.x < 64) {
     int64_t v = 0;
@@ -182,7 +178,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add2(int64_t* __restrict__ 
   if (i < n) out[i] += off;
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
     out[n] = off + bs[blockIdx.x];
-    if (tot) tot[blockIdx.y] = off + bs[blockIdx.x];
+    if (ts.t[blockIdx.y].tot) *ts.t[blockIdx.y].tot = off + bs[blockIdx.x];
   }
 }
 
@@ -234,50 +230,42 @@ int tgx_zero2(tgx_ctx* ctx, void* p, size_t np, void* q, size_t nq) {
   return TGX_OK;
 }
 
-int tgx_scan_i32(tgx_ctx* ctx, const int* in, int64_t* out, int64_t n, int64_t* total, dbuf* tmp) {
+int tgx_scan_many(tgx_ctx* ctx, const tgx_scan_tasks& ts, int count, int64_t n, dbuf* tmp) {
+  TGX_REQUIRE(count >= 1 && count <= TGX_SCAN_TASKS, "tgx_scan_many: %d arrays", count);
   const int64_t nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
   dbuf& sb = tmp ? *tmp : ctx->scan_tmp;
-  TGX_TRY(sb.ensure(sizeof(int64_t) * (size_t)(nb + 2)));
-  int64_t* sums = sb.as<int64_t>();
   if (n > 0 && n <= SCAN_SINGLE_MAX) {
-    TGX_LAUNCH(ctx, "scan_single", k_scan_single, dim3(1), dim3(SCAN_BLOCK), 0, in, out, (const int*)nullptr,
-               (int64_t*)nullptr, n, total);
+    TGX_LAUNCH(ctx, "scan_single", k_scan_single, dim3(1, count), dim3(SCAN_BLOCK), 0, ts, n);
   } else if (n > 0 && n <= SCAN_2L_MAX) {
-    TGX_LAUNCH(ctx, "scan_local", k_scan_local2, dim3((unsigned)nb, 1), dim3(SCAN_BLOCK), 0, in, out,
-               (const int*)nullptr, (int64_t*)nullptr, n, sums);
-    TGX_LAUNCH(ctx, "scan_add", k_scan_add2, dim3((unsigned)nb, 1), dim3(SCAN_BLOCK), 0, out, (int64_t*)nullptr, n,
-               (const int64_t*)sums, total);
-  } else if (n > 0) {
-    TGX_LAUNCH(ctx, "scan_local", k_scan_local, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, in, out, n, sums);
-    TGX_LAUNCH(ctx, "scan_sums", k_scan_sums, dim3(1), dim3(SCAN_BLOCK), 0, sums, nb);
-    TGX_LAUNCH(ctx, "scan_add", k_scan_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, out, n,
-               (const int64_t*)sums, total);
+    TGX_TRY(sb.ensure(sizeof(int64_t) * (size_t)count * (size_t)nb));
+    TGX_LAUNCH(ctx, "scan_local", k_scan_local2, dim3((unsigned)nb, count), dim3(SCAN_BLOCK), 0, ts, n,
+               sb.as<int64_t>());
+    TGX_LAUNCH(ctx, "scan_add", k_scan_add2, dim3((unsigned)nb, count), dim3(SCAN_BLOCK), 0, ts, n,
+               (const int64_t*)sb.as<int64_t>());
   } else {
-    TGX_TRY(tgx_zero(ctx, out, sizeof(int64_t)));
-    if (total) *total = 0;
+    // one after the other, all through the same block totals
+    if (n > 0) TGX_TRY(sb.ensure(sizeof(int64_t) * (size_t)(nb + 2)));
+    for (int k = 0; k < count; ++k) {
+      const tgx_scan_task& t = ts.t[k];
+      if (n > 0) {
+        int64_t* sums = sb.as<int64_t>();
+        TGX_LAUNCH(ctx, "scan_local", k_scan_local, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, t.in, t.out, n, sums);
+        TGX_LAUNCH(ctx, "scan_sums", k_scan_sums, dim3(1), dim3(SCAN_BLOCK), 0, sums, nb);
+        TGX_LAUNCH(ctx, "scan_add", k_scan_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, t.out, n,
+                   (const int64_t*)sums, t.tot);
+      } else {
+        TGX_TRY(tgx_zero(ctx, t.out, sizeof(int64_t)));
+        if (t.tot) *t.tot = 0;
+      }
+    }
   }
   return TGX_OK;
 }
 
-int tgx_scan2_i32(tgx_ctx* ctx, const int* in0, int64_t* out0, const int* in1, int64_t* out1, int64_t n,
-                  dbuf& tmp, int64_t* totals) {
-  if (n > 0 && n <= SCAN_SINGLE_MAX) {
-    TGX_LAUNCH(ctx, "scan_single", k_scan_single, dim3(1, 2), dim3(SCAN_BLOCK), 0, in0, out0, in1, out1, n, totals);
-    return TGX_OK;
-  }
-  if (n > 0 && n <= SCAN_2L_MAX) {
-    const int64_t nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
-    TGX_TRY(tmp.ensure(sizeof(int64_t) * 2 * (size_t)nb));
-    int64_t* sums = tmp.as<int64_t>();
-    TGX_LAUNCH(ctx, "scan_local", k_scan_local2, dim3((unsigned)nb, 2), dim3(SCAN_BLOCK), 0, in0, out0, in1, out1, n,
-               sums);
-    TGX_LAUNCH(ctx, "scan_add", k_scan_add2, dim3((unsigned)nb, 2), dim3(SCAN_BLOCK), 0, out0, out1, n,
-               (const int64_t*)sums, totals);
-    return TGX_OK;
-  }
-  // one after the other on the caller's stream, both through the caller's tmp
-  TGX_TRY(tgx_scan_i32(ctx, in0, out0, n, totals, &tmp));
-  return tgx_scan_i32(ctx, in1, out1, n, totals ? totals + 1 : nullptr, &tmp);
+int tgx_scan_i32(tgx_ctx* ctx, const int* in, int64_t* out, int64_t n, int64_t* total, dbuf* tmp) {
+  tgx_scan_tasks ts{};
+  ts.t[0] = tgx_scan_task{in, out, total};
+  return tgx_scan_many(ctx, ts, 1, n, tmp);
 }
 
 int tgx_device_sum_launch(tgx_ctx* ctx, const double* d_x, int64_t n, double* d_part) {
