@@ -14,6 +14,7 @@
 // quadrature nodes, the (l, m) harmonics and the (n, l) channel sums of a pair;
 // the power spectrum and its derivative are split over threads by component.
 #include "tgx_internal.h"
+#include "tgx_soap_lanes.h"
 
 int tgx_desc_wave(tgx_ctx* ctx, tgx_model_t* m, bool fp64, const int* d_sites, int n_rows, void* q_out, void* pn_out);
 int tgx_adjoint_wave(tgx_ctx* ctx, tgx_model_t* m, bool fp64);
@@ -144,74 +145,6 @@ __device__ void pair_step1(const SoapParams& P, int s, T r, T ux, T uy, T uz, in
     ylm_one<T>(l, m, (T)P.ynorm[lm], ux, uy, uz, Y, gx, gy, gz);
     ps.Y[lm] = Y;
     if (need_grad) { ps.gY[3 * lm] = gx; ps.gY[3 * lm + 1] = gy; ps.gY[3 * lm + 2] = gz; }
-  }
-}
-
-// Real harmonics of one pair by lanes over m, for a compile-time l_max LL:
-// lane t = m + LL (t <= 2 LL) runs the l recurrence of its |m| and writes
-// Y_lm, and with GRAD the gradient of the solid harmonic r^l Y_lm at the unit
-// vector (xyz interleaved), for l = |m|..LL. Same recurrences and constants
-// as ylm_one; rinv[k] = 1/k replaces the division. With PACK (and GRAD) the
-// four values of lm go to Y[4 lm .. 4 lm + 3] = (Y, gx, gy, gz) instead.
-template <int LL, bool GRAD, bool PACK = false>
-__device__ __forceinline__ void harmonics_m(int t, const double* ynorm, const double* rinv, double ux, double uy,
-                                            double uz, double* Y, double* gY) {
-  static_assert(!PACK || GRAD, "the packed layout carries gradients");
-  if (t > 2 * LL) return;
-  // opaque to the optimiser: the per-lane recurrence constants are rebuilt per call, not hoisted
-  // out of the caller's pair loop where they would stay live across the whole site
-  asm volatile("" : "+v"(t));
-  const int m = t - LL, am = m < 0 ? -m : m;
-  double c = 1, cx = 0, cy = 0, s = 0, sx = 0, sy = 0;
-#pragma unroll
-  for (int k = 0; k < LL; ++k) {
-    if (k < am) {
-      const double nc = c * ux - s * uy, ns = c * uy + s * ux;
-      if (GRAD) {
-        const double ncx = cx * ux + c - sx * uy, ncy = cy * ux - sy * uy - s;
-        const double nsx = cx * uy + sx * ux + s, nsy = cy * uy + c + sy * ux;
-        cx = ncx; cy = ncy; sx = nsx; sy = nsy;
-      }
-      c = nc;
-      s = ns;
-    }
-  }
-  const double f = m < 0 ? s : c, fx = m < 0 ? sx : cx, fy = m < 0 ? sy : cy;
-  double q = 1, qx = 0, qy = 0, qz = 0, p = 0, px = 0, py = 0, pz = 0;
-#pragma unroll
-  for (int l = 0; l <= LL; ++l) {
-    if (l < am) continue;
-    if (l == am + 1) {
-      p = q; px = qx; py = qy; pz = qz;
-      q = (double)(2 * am + 1) * uz;
-      qx = 0; qy = 0; qz = (double)(2 * am + 1);
-    } else if (l > am + 1) {
-      const double a = (double)(2 * l - 1), b = (double)(l + am - 1), inv = rinv[l - am];
-      const double nq = (a * uz * q - b * p) * inv;
-      if (GRAD) {
-        const double nqx = (a * uz * qx - b * (2.0 * ux * p + px)) * inv;
-        const double nqy = (a * uz * qy - b * (2.0 * uy * p + py)) * inv;
-        const double nqz = (a * (q + uz * qz) - b * (2.0 * uz * p + pz)) * inv;
-        px = qx; py = qy; pz = qz;
-        qx = nqx; qy = nqy; qz = nqz;
-      }
-      p = q;
-      q = nq;
-    }
-    const int lm = l * l + l + m;
-    const double Nn = ynorm[lm];
-    if (PACK) {
-      double2* y4 = reinterpret_cast<double2*>(Y + 4 * lm);
-      y4[0] = make_double2(Nn * q * f, Nn * (qx * f + q * fx));
-      y4[1] = make_double2(Nn * (qy * f + q * fy), Nn * qz * f);
-    } else {
-      Y[lm] = Nn * q * f;
-      if (GRAD) {
-        gY[3 * lm] = Nn * (qx * f + q * fx);
-        gY[3 * lm + 1] = Nn * (qy * f + q * fy);
-        gY[3 * lm + 2] = Nn * qz * f;
-      }
-    }
   }
 }
 
@@ -748,478 +681,479 @@ __global__ __launch_bounds__(WG, 2) void k_soap_der(SoapParams P, SiteArgs a, in
 }
 
 // ---- The same dq/dr for a compile-time l_max and at most two species of at
-// most eight radial functions each. Every wavefront works on its own pairs in
-// both pair phases; the site's pair data, the radial basis and the nodes sit in
-// registers, so a pair's set-up does not wait on memory.
+// most eight radial functions each (16 stacked rows).
 
 template <int LL> struct DerL {
-  static constexpr int L1 = LL + 1, NLM = L1 * L1, NL = 16 * L1;
-  static constexpr int PS = 2 * TGX_MAX_Q + 2 * TGX_MAX_NB + 2 * L1 + 4 * NLM;  // PairScratch
-  static constexpr int SL = 6 * NL + 8 + PS;                                    // one pair slot
+  static constexpr int L1 = LL + 1, NLM = L1 * L1, NL = 16 * L1, D = 16 * 17 / 2 * L1;
+  static constexpr int CHK = 32;             // pairs prepared together, eight lanes each
+  static constexpr int TABS = 2 * TGX_MAX_Q * 9;  // the species' nodes and basis [q][8]
+  static constexpr int ST = 33;              // one pair's record, see der_prepare
+  static constexpr int CP = 17;              // row of c or H at one (l, m), padded
+  static constexpr int SL = 6 * NL;          // one pair's channel tables
+  static constexpr int SPW = sizeof(SpeciesParams) / 8;     // doubles of a species' parameters
+  static_assert(sizeof(SpeciesParams) % 8 == 0, "copied to LDS in doubles");
+  static constexpr int HEAD = NLM + CHK * ST + 8 + 2 * SPW;
+  static constexpr int HEADP = HEAD + (HEAD & 1);
+  static constexpr int U1 = TABS + CHK * NLM;               // expansion: tables and W
+  static constexpr int U2 = NLM * CP + 1 + D;               // c, then H, and the spectrum
+  static constexpr int HG = 16;                             // pairs whose harmonics are kept
+  static constexpr int U3 = 4 * SL + HG * 4 * NLM + 48;     // four pairs' tables, harmonics, q . dp
+  static constexpr int U = U1 > U2 ? (U1 > U3 ? U1 : U3) : (U2 > U3 ? U2 : U3);
+  static constexpr size_t LDS = sizeof(double) * (HEADP + U);
 };
 
-__device__ __forceinline__ double lane_read(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)b, l);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
-// The pair-only factors of a pair's radial values and angular damping (what
-// der_radial and der_gauss would otherwise form in every lane for every pair):
-// the amplitude A(r) = global_scaling / s (1 + 2x^3 - 3x^2)^amplitude_scaling
-// and dA/dr, and e = exp(-k) and -dk/dr of the damping exponent
-// k = st^2 / (2 r^2). Zero for a pair outside the cutoff or unseen.
-struct PairAmp {
-  double amp, damp, ea, dk;
-};
-
-__device__ __forceinline__ PairAmp pair_amp(const SpeciesParams& sp, double r) {
-  PairAmp o;
-  const double inv_rc = sp.inv_rc;
-  const double x = r * inv_rc;
-  const double sig = sp.sig_r * (1.0 + sp.sig_r_sc * r) * inv_rc;
-  const double dsig = (sp.sig_r * sp.sig_r_sc) * inv_rc;
-  const double aa = sp.amp_a;
-  const double Pp = 1.0 + 2.0 * x * x * x - 3.0 * x * x;
-  const double dPp = (6.0 * x * x - 6.0 * x) * inv_rc;
-  double amp, damp;
-  if (aa == 0.0) {
-    amp = 1.0 / sig;
-    damp = -dsig / (sig * sig);
-  } else if (Pp <= 1.0e-10) {
-    amp = 0; damp = 0;
-  } else {
-    const double Pa = pow(Pp, aa);
-    amp = Pa / sig;
-    damp = aa * pow(Pp, aa - 1.0) * dPp / sig - Pa * dsig / (sig * sig);
-  }
-  o.amp = amp * sp.gs;
-  o.damp = damp * sp.gs;
-  const double st = sp.sig_t * (1.0 + sp.sig_t_sc * r);
-  const double dst = sp.sig_t * sp.sig_t_sc;
-  const double kk = st * st / (2.0 * r * r);
-  o.dk = st * st / (r * r * r) - st * dst / (r * r);  // -dk/dr
-  o.ea = exp(-kk);
-  return o;
-}
-
-// Register copies, per lane: pair 1 + lane of the site with its PairAmp;
-// B[s][n][q] at n = lane / 8, q = lane % 8 + 8 i; the node x_q of each species
-// at q = lane. At most two species (the blocks this kernel serves).
-struct DerRegs {
-  int spec;
-  double r, x, y, z;
-  PairAmp pa;
-  double B[2][8];
-  double xq[2];
-  __device__ void load(const SoapParams& P, const SiteArgs& a, int64_t b0, int nn, int lane) {
-    const int k = 1 + lane;
-    spec = -1;
-    r = 1.0; x = y = z = 0.0;
-    if (k < nn) {
-      spec = a.pr_spec[b0 + k];
-      r = a.pr_r[b0 + k];
-      x = a.pr_xyz[3 * (b0 + k)];
-      y = a.pr_xyz[3 * (b0 + k) + 1];
-      z = a.pr_xyz[3 * (b0 + k) + 2];
+// The species' nodes and basis (at most two species, eight functions) on their way
+// from memory to LDS, xq[s][q] and Bt[s][q][8]: loaded in registers at the kernel's
+// start, before anything that waits on the site's own offsets.
+struct DerTabs {
+  double x, b[4];
+  __device__ __forceinline__ void load(const double* xq, const double* B, int S) {
+    const int t = threadIdx.x;
+    x = t < S * TGX_MAX_Q ? xq[t] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = t + WG * u, sn = i / TGX_MAX_Q, q = i % TGX_MAX_Q;
+      b[u] = sn < 8 * S ? B[((size_t)(sn >> 3) * TGX_MAX_NB + (sn & 7)) * TGX_MAX_Q + q] : 0.0;
     }
-    pa = PairAmp{0.0, 0.0, 0.0, 0.0};
-    if (spec >= 0 && r < (spec == 0 ? P.sp[0].rc : P.sp[1].rc)) pa = pair_amp(spec == 0 ? P.sp[0] : P.sp[1], r);
-    const int n = lane >> 3, part = lane & 7;
+  }
+  __device__ __forceinline__ void store(double* tabs) const {
+    const int t = threadIdx.x;
+    if (t < 2 * TGX_MAX_Q) tabs[t] = x;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const bool have = s < P.n_species;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) B[s][i] = have ? P.B[((size_t)s * TGX_MAX_NB + n) * TGX_MAX_Q + part + 8 * i] : 0.0;
-      xq[s] = have ? P.xq[s * TGX_MAX_Q + lane] : 0.0;
+    for (int u = 0; u < 4; ++u) {
+      const int i = t + WG * u, sn = i / TGX_MAX_Q, q = i % TGX_MAX_Q;
+      tabs[2 * TGX_MAX_Q + ((sn >> 3) * TGX_MAX_Q + q) * 8 + (sn & 7)] = b[u];
     }
   }
 };
 
-struct DerPair {
-  int s;
-  bool ok;
-  double r, ux, uy, uz;
-  PairAmp pa;
-};
-
-// Pair k >= 1 of the site (wavefront-uniform): from the lanes for k <= 64, else from memory.
-__device__ __forceinline__ DerPair der_pair(const SoapParams& P, const SiteArgs& a, const DerRegs& R, int64_t b0,
-                                            int k) {
-  DerPair q;
-  double x, y, z;
-  const bool reg = k <= 64;
-  if (reg) {
-    q.s = __builtin_amdgcn_readlane(R.spec, k - 1);
-    q.r = lane_read(R.r, k - 1);
-    x = lane_read(R.x, k - 1);
-    y = lane_read(R.y, k - 1);
-    z = lane_read(R.z, k - 1);
-    q.pa.amp = lane_read(R.pa.amp, k - 1);
-    q.pa.damp = lane_read(R.pa.damp, k - 1);
-    q.pa.ea = lane_read(R.pa.ea, k - 1);
-    q.pa.dk = lane_read(R.pa.dk, k - 1);
-  } else {
-    const int64_t p = b0 + k;
-    q.s = a.pr_spec[p];
-    q.r = a.pr_r[p];
-    x = a.pr_xyz[3 * p];
-    y = a.pr_xyz[3 * p + 1];
-    z = a.pr_xyz[3 * p + 2];
-  }
-  // wavefront-uniform: the species parameters then come from scalar loads
-  q.s = __builtin_amdgcn_readfirstlane(q.s);
-  q.r = lane_read(q.r, 0);
-  x = lane_read(x, 0);
-  y = lane_read(y, 0);
-  z = lane_read(z, 0);
-  q.ok = q.s >= 0 && q.r < P.sp[q.s].rc;
-  if (!reg && q.ok) q.pa = pair_amp(P.sp[q.s], q.r);
-  const double inv = 1.0 / q.r;
-  q.ux = x * inv;
-  q.uy = y * inv;
-  q.uz = z * inv;
-  return q;
-}
-
-// pair_gauss with the nodes from registers (lane q < nq) and the damping on
-// lane 63 from the pair's e = exp(-k).
-__device__ __forceinline__ void der_gauss(const SoapParams& P, const DerRegs& R, const DerPair& pr, int lane,
-                                          PairScratch<double>& ps, bool need_grad) {
-  const int s = pr.s;
-  const double r = pr.r;
-  const SpeciesParams& sp = P.sp[s];
-  const double inv_rc = sp.inv_rc;
-  const double x = r * inv_rc;
-  const double sig = sp.sig_r * (1.0 + sp.sig_r_sc * r) * inv_rc;
-  const double dsig = (sp.sig_r * sp.sig_r_sc) * inv_rc;
-  const double inv_s2 = 1.0 / (sig * sig);
-  if (lane < sp.nq) {
-    const double dx = (s == 0 ? R.xq[0] : R.xq[1]) - x;
-    const double g = exp(-0.5 * dx * dx * inv_s2);
-    ps.G[lane] = g;
-    if (need_grad) ps.dG[lane] = g * (dx * inv_s2 * inv_rc + dx * dx * inv_s2 / sig * dsig);
-  }
-  if (lane == 63) {
-    const double dk = pr.pa.dk;
-    const double e1 = pr.pa.ea, e2 = e1 * e1;
-    double Al = 1, pw = 1;
-    for (int l = 0; l <= P.L; ++l) {
-      if (l > 0) { pw *= e2; Al *= pw; }
-      ps.A[l] = Al;
-      ps.dA[l] = Al * (double)(l * (l + 1)) * dk;
-    }
-  }
-}
-
-// pair_step2 for nb <= 8 (eight node slices per radial function) with B from
-// registers and the pair's amplitude; the node values are read before they
-// are summed, in the same order.
-__device__ __forceinline__ void der_radial(const SoapParams& P, const DerRegs& R, const DerPair& pr, int lane,
-                                           PairScratch<double>& ps, bool need_grad) {
-  const SpeciesParams& sp = P.sp[pr.s];
-  const double amp = pr.pa.amp, damp = pr.pa.damp;
-  const int n = lane >> 3, part = lane & 7, nq = sp.nq;
-  double g[8], dg[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int q = min(part + 8 * i, nq - 1);
-    g[i] = ps.G[q];
-    dg[i] = need_grad ? ps.dG[q] : 0.0;
-  }
-  double I = 0, dI = 0;
-  if (n < sp.nb) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (part + 8 * i < nq) {
-        const double b = pr.s == 0 ? R.B[0][i] : R.B[1][i];
-        I += b * g[i];
-        dI += b * dg[i];
-      }
-  }
-  for (int o = 1; o < 8; o <<= 1) {
-    I += __shfl_xor(I, o);
-    if (need_grad) dI += __shfl_xor(dI, o);
-  }
-  if (n < sp.nb && part == 0) {
-    ps.R[n] = amp * I;
-    if (need_grad) ps.dR[n] = damp * I + amp * dI;
-  }
-}
-
-// Channel tables of four pairs at once (slots 0..3 of U, pair data and
-// scratch filled by their wavefronts): lanes (n, p) = (lane & 15, lane >> 4)
-// take radial row n of pair p, and wavefront w the degrees of its set, so
-// every (n, l) entry of every pair is formed once and each c / H read serves
-// eight products. The pair's harmonics are packed (Y, gx, gy, gz) per lm.
-// Entry (n, l) of a slot is six doubles (s, E, v_x, v_y, v_z, Dd) at
-// 6 (n L1 + l), read back as three 16-byte loads:
-//   s(n,l) = sum_m Y c(n,lm),  v_k(n,l) = (sum_m dY_k c(n,lm) - l s u_k) / r,
-//   E(n,l) = R_n A_l,  Dd(n,l) = dR_n A_l + R_n dA_l  (rows of the pair's block),
-// and the pair's q . dp_k partial over the set, sum_(n,l) Dd h u_k +
-// E (h_k - l h u_k) / r with h = sum_m Y H(n,lm), h_k = sum_m dY_k H(n,lm),
-// reduced over the 16 row lanes into qpart[(w * 4 + p) * 3 + k].
-template <int LL>
-__device__ __forceinline__ void der_tables_w(const SoapParams& P, int w, int lane, int N, double* U, int SL,
-                                             const double* c, const double* H, double* qpart) {
-  static_assert(LL == 8, "degree sets are laid out for l_max = 8");
+// Records of the site's pairs k0 + 1 .. k0 + cnt, eight lanes each (cnt <= CHK), from
+// the species' parameters spl and tables tabs in LDS:
+//   R[8] | dR[8] | A[9] | -A'/(A l (l + 1)) | 1/r | u | seen (1 or 0) | first row, row count
+// (R, dR rows of the pair's own species block) and, with W, A_l Y_lm of every pair.
+template <int LL, bool W>
+__device__ __forceinline__ void der_prepare(const SpeciesParams* spl, const int* pr_spec, const double* pr_r,
+                                            const double* pr_xyz, int64_t b0, int k0, int cnt, const double* ynorm,
+                                            double* rec, const double* tabs, double* w) {
   using G = DerL<LL>;
-  constexpr int L1 = G::L1, NLM = G::NLM, NL = G::NL;
-  const int n = lane & 15, p = lane >> 4;
-  double* slot = U + p * SL;
-  const double* misc = slot + 6 * NL;
-  PairScratch<double> ps;
-  ps.bind(const_cast<double*>(misc) + 8, LL, NLM);
-  const bool ok = misc[0] != 0.0;
-  const int off = (int)misc[1], nb = (int)misc[2];
-  const double inv_r = 1.0 / misc[3], ux = misc[4], uy = misc[5], uz = misc[6];
-  const int nl = n - off;
-  const bool inb = ok && nl >= 0 && nl < nb;
-  const bool row = n < N;
-  const double* cr = c + n * NLM;
-  const double* hr = H + n * NLM;
-  double qx = 0.0, qy = 0.0, qz = 0.0;
-  const int nsets = w == 0 ? 3 : 2;
-  for (int li = 0; li < nsets; ++li) {
-    const int l = li == 0 ? LL - w : (li == 1 ? (w == 0 ? 0 : w + 1) : 1);
-    double s0 = 0.0, gx = 0.0, gy = 0.0, gz = 0.0, h0 = 0.0, hx = 0.0, hy = 0.0, hz = 0.0;
-    if (ok && row) {
-#pragma unroll 3
-      for (int lm = l * l; lm < (l + 1) * (l + 1); ++lm) {
-        const double2* y4 = reinterpret_cast<const double2*>(ps.Y + 4 * lm);  // (Y, gx), (gy, gz)
-        const double2 ya = y4[0], yb = y4[1];
-        const double y = ya.x, dx = ya.y, dy = yb.x, dz = yb.y;
-        const double cv = cr[lm], hv = hr[lm];
-        s0 += y * cv;
-        gx += dx * cv;
-        gy += dy * cv;
-        gz += dz * cv;
-        h0 += y * hv;
-        hx += dx * hv;
-        hy += dy * hv;
-        hz += dz * hv;
-      }
-    }
-    const double lf = (double)l;
-    const double E = inb ? ps.R[nl] * ps.A[l] : 0.0;
-    const double Dd = inb ? ps.dR[nl] * ps.A[l] + ps.R[nl] * ps.dA[l] : 0.0;
-    if (row) {
-      double2* t = reinterpret_cast<double2*>(slot + 6 * (n * L1 + l));
-      t[0] = make_double2(s0, E);
-      t[1] = make_double2((gx - lf * s0 * ux) * inv_r, (gy - lf * s0 * uy) * inv_r);
-      t[2] = make_double2((gz - lf * s0 * uz) * inv_r, Dd);
-    }
-    qx += Dd * h0 * ux + E * (hx - lf * h0 * ux) * inv_r;
-    qy += Dd * h0 * uy + E * (hy - lf * h0 * uy) * inv_r;
-    qz += Dd * h0 * uz + E * (hz - lf * h0 * uz) * inv_r;
+  const double* xq = tabs;
+  const double* Bt = tabs + 2 * TGX_MAX_Q;
+  const int j = threadIdx.x >> 3, sub = threadIdx.x & 7;
+  int s = -1;
+  double r = 1.0, ux = 0.0, uy = 0.0, uz = 0.0;
+  if (j < cnt) {
+    const int64_t p = b0 + k0 + 1 + j;
+    s = pr_spec[p];
+    r = pr_r[p];
+    const double inv = 1.0 / r;
+    ux = pr_xyz[3 * p] * inv;
+    uy = pr_xyz[3 * p + 1] * inv;
+    uz = pr_xyz[3 * p + 2] * inv;
   }
+  lds_barrier();
+  if (j >= cnt) return;
+  const SpeciesParams sp = spl[max(s, 0)];
+  if (s >= 0 && !(r < sp.rc)) s = -1;
+  double* st = rec + j * G::ST;
+  if (s >= 0) {
+    double R[8], dR[8];
+    radial_lanes<double, true, 8, 8>(sp, xq + s * TGX_MAX_Q, Bt + s * TGX_MAX_Q * 8, sub, r, R, dR);
+    Damp<double> dmp;
+    dmp.init(sp, r);
+    if (sub == 0) {
 #pragma unroll
-  for (int o = 1; o < 16; o <<= 1) {
-    qx += __shfl_xor(qx, o);
-    qy += __shfl_xor(qy, o);
-    qz += __shfl_xor(qz, o);
+      for (int n = 0; n < 8; ++n) st[n] = R[n];
+#pragma unroll
+      for (int n = 0; n < 8; ++n) st[8 + n] = dR[n];
+      double Al = 1.0, pw = 1.0;
+      st[16] = 1.0;
+#pragma unroll
+      for (int l = 1; l <= LL; ++l) {
+        pw *= dmp.e2;
+        Al *= pw;
+        st[16 + l] = Al;
+      }
+      st[25] = dmp.dk;
+      st[26] = 1.0 / r;
+      st[27] = ux;
+      st[28] = uy;
+      st[29] = uz;
+      st[30] = 1.0;
+      st[31] = (double)sp.off;
+      st[32] = (double)sp.nb;
+    }
+    if (W)
+      ylm_lanes<double, false, 8>(LL, ynorm, sub, ux, uy, uz, dmp.e2,
+                                  [&](int, int lm, double Al, double Y, double, double, double) {
+                                    w[j * G::NLM + lm] = Al * Y;
+                                  });
+  } else {
+    for (int i = sub; i < G::ST; i += 8) st[i] = 0.0;
+    if (W)
+      for (int lm = sub; lm < G::NLM; lm += 8) w[j * G::NLM + lm] = 0.0;
   }
-  if (n == 0) {
-    double* q = qpart + (w * 4 + p) * 3;
-    q[0] = qx;
-    q[1] = qy;
-    q[2] = qz;
+}
+
+// The records of a later chunk of a site with more than CHK pairs, tables included.
+// Not inlined: its registers would push the pair loop's, live across it, into
+// scratch for every site (9.41 -> 9.64 ms at 65,536 atoms, 50 -> 54 us at 216).
+template <int LL>
+__device__ __attribute__((noinline)) void der_prepare_again(const SpeciesParams* spl, const double* xq, const double* B,
+                                                            int S, const int* pr_spec, const double* pr_r,
+                                                            const double* pr_xyz, int64_t b0, int k0, int cnt,
+                                                            double* rec, double* tabs) {
+  lds_barrier();
+  DerTabs t;
+  t.load(xq, B, S);
+  t.store(tabs);
+  der_prepare<LL, false>(spl, pr_spec, pr_r, pr_xyz, b0, k0, cnt, nullptr, rec, tabs, nullptr);
+}
+
+// The wavefront's degrees of the channel tables, 20 or 21 (l, m) in all: {8, 0, 1},
+// {7, 2}, {6, 3} or {5, 4}; the i-th (l, m) of wavefront w.
+template <int LL> __device__ __forceinline__ int der_lm(int w, int i) {
+  static_assert(LL == 8, "degree sets are laid out for l_max = 8");
+  const int l = LL - w, k = 2 * l + 1;
+  return i < k ? l * l + i : (w == 0 ? i - k : (w + 1) * (w + 1) + min(i - k, 2 * w + 2));
+}
+
+struct DerLane {
+  double R, dR, dk, inv_r, ux, uy, uz;
+  bool ok;
+};
+
+// Entries (n, l) of one pair's channel tables, six doubles (s, E, v_x, v_y, v_z, Dd)
+// at 6 (n L1 + l), read back as three 16-byte loads:
+//   s(n,l) = sum_m Y c(n,lm),  v_k(n,l) = (sum_m dY_k c(n,lm) - l s u_k) / r,
+//   E(n,l) = R_n A_l,  Dd(n,l) = dR_n A_l + R_n A_l'  (rows of the pair's block),
+// and the row's part of q . dp_k, Dd h u_k + E (h_k - l h u_k) / r with
+// h = sum_m Y H(n,lm), h_k = sum_m dY_k H(n,lm). c and H of the row's (l, m) come in
+// registers I0, I0 + 1, ...; y holds the pair's (Y, gx, gy, gz).
+template <int LL, int l, int I0>
+__device__ __forceinline__ void der_channel(const DerLane& p, const double* y, const double* A, const double (&c)[21],
+                                            const double (&H)[21], double* slot, double& qx, double& qy, double& qz) {
+  double s0 = 0.0, gx = 0.0, gy = 0.0, gz = 0.0, h0 = 0.0, hx = 0.0, hy = 0.0, hz = 0.0;
+  if (p.ok) {
+#pragma unroll
+    for (int i = 0; i < 2 * l + 1; ++i) {
+      const double2* y4 = reinterpret_cast<const double2*>(y + 4 * (l * l + i));
+      const double2 ya = y4[0], yb = y4[1];
+      const double cv = c[I0 + i], hv = H[I0 + i];
+      s0 += ya.x * cv;
+      gx += ya.y * cv;
+      gy += yb.x * cv;
+      gz += yb.y * cv;
+      h0 += ya.x * hv;
+      hx += ya.y * hv;
+      hy += yb.x * hv;
+      hz += yb.y * hv;
+    }
   }
+  const double lf = (double)l, Al = A[l];
+  const double E = p.R * Al;
+  const double Dd = p.dR * Al + p.R * (Al * (lf * (lf + 1.0)) * p.dk);
+  double2* t = reinterpret_cast<double2*>(slot + 6 * l);
+  t[0] = make_double2(s0, E);
+  t[1] = make_double2((gx - lf * s0 * p.ux) * p.inv_r, (gy - lf * s0 * p.uy) * p.inv_r);
+  t[2] = make_double2((gz - lf * s0 * p.uz) * p.inv_r, Dd);
+  qx += Dd * h0 * p.ux + E * (hx - lf * h0 * p.ux) * p.inv_r;
+  qy += Dd * h0 * p.uy + E * (hy - lf * h0 * p.uy) * p.inv_r;
+  qz += Dd * h0 * p.uz + E * (hz - lf * h0 * p.uz) * p.inv_r;
 }
 
 // Plain-path dq/dr for l_max = LL (the output and element layout of
-// k_soap_der). Coefficients: wavefront w expands pairs 1 + w, 5 + w, ... with
-// lanes over (l, m) and the 16 rows in registers, and the four partial
-// expansions are added in wavefront order. Pairs go in groups of four: each
-// wavefront prepares one pair's Gaussians, harmonics and radial values, the
-// four wavefronts then form the four pairs' channel tables together
-// (der_tables_w), and each thread writes whole components d = tid + WG j (its
-// three Cartesian entries, from 13 LDS reads) of every pair of the group,
-// keeping the self-pair sums of its components in registers. J >= D / WG.
+// k_soap_der), one workgroup per site.
+//   * Pairs are prepared 32 at a time, eight lanes each (der_prepare), and their
+//     harmonics 16 at a time, a row of lanes each: with a wavefront per pair, five or
+//     six pairs in turn, a preparation took 13,000 cycles, nearly all of them the
+//     chain of exponentials, divisions and recurrences with 15 to 40 of 64 lanes idle.
+//   * The expansion c = sum_j R_j W_j, the power spectrum p_l = c_l c_l^T and
+//     H_l = S_l c_l are products on the FP64 matrix cores (16 rows n, the (l, m)
+//     or pairs of one degree as the other sides).
+//   * Each lane (n, p) keeps c and H of its row n at its wavefront's (l, m) in
+//     registers for the channel tables of four pairs at a time (der_channel); with
+//     neither in LDS the harmonics of 16 pairs fit beside two workgroups a CU
+//     (79 KB each; three of 48 KB with four pairs' harmonics spill at 168
+//     registers, 15.4 ms).
+//   * Each thread writes whole components d = tid + WG j (its three Cartesian
+//     entries) of every pair of the group and keeps the self-pair sums of its
+//     components in registers. J >= D / WG.
+// Bound by the 35 GB it writes at 65,536 atoms of two species (1.2 million pairs of
+// 1,224 components): 15.0 -> 9.45 ms, 3.7 TB/s; at 4,096 atoms 1.15 -> 0.61 ms,
+// at 216 atoms of one species, a workgroup a CU, 110 -> 50 us. Stores staged through
+// LDS to be contiguous (10.5 -> 11.6 ms) and non-temporal stores (10.6) lost.
 template <int LL, int J>
 __global__ __launch_bounds__(WG, 2) void k_soap_der_l(SoapParams P, SiteArgs a, int n_sites,
                                                       double* __restrict__ q_out, double* __restrict__ pnorm_out,
                                                       double* __restrict__ der_out) {
   using G = DerL<LL>;
-  constexpr int L1 = G::L1, NLM = G::NLM, NL = G::NL, SL = G::SL;
-  static_assert(SL % 2 == 0 && (NLM + L1) % 2 == 0, "pair slots and tables need 16-byte alignment");
+  constexpr int L1 = G::L1, NLM = G::NLM, SL = G::SL, CHK = G::CHK, ST = G::ST, CP = G::CP;
+  constexpr int NT = (NLM + 15) / 16;  // (l, m) tiles of the expansion
+  static_assert(NT <= 8 && LL <= 8, "two tiles a wavefront, a degree's (l, m) in at most two tiles");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   double* sm = reinterpret_cast<double*>(smem_raw);
   const int site = blockIdx.x;
   if (site >= n_sites) return;
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int N = P.N, D = P.D, D3 = 3 * D, CN = N * NLM;
-  double* ynorm = sm;                          // NLM
-  double* rinv = ynorm + NLM;                  // L1
-  double* c = rinv + L1;                       // N NLM
-  double* H = c + CN;                          // N NLM
-  double* X = H + CN;                          // D: p, then q
-  double* U = X + D + (D & 1);                 // max(4 SL + 48, 4 N NLM, WG), 16-byte aligned
+  const int li = lane & 15, lg = lane >> 4;
+  const int N = P.N, D = P.D, D3 = 3 * D;
+  double* ynorm = sm;               // NLM
+  double* rec = ynorm + NLM;        // CHK pair records
+  double* red = rec + CHK * ST;     // 8
+  SpeciesParams* spl = reinterpret_cast<SpeciesParams*>(red + 8);  // two species
+  double* U = sm + G::HEADP;
   const int64_t b0 = a.site_beg[site];
-  const int nn = (int)(a.site_beg[site + 1] - b0);
-  DerRegs RG;
-  RG.load(P, a, b0, nn, lane);
-  for (int i = tid; i < NLM; i += WG) ynorm[i] = P.ynorm[i];
-  if (tid < L1) rinv[tid] = tid > 0 ? 1.0 / (double)tid : 0.0;
-  lds_barrier();
-  // ---- expansion coefficients ----
+  const int nn = (int)(a.site_beg[site + 1] - b0), np1 = nn - 1;
+  DerTabs tabs;
+  tabs.load(P.xq, P.B, P.n_species);
+  const double yn = tid < NLM ? P.ynorm[tid] : 0.0;
+  const int sself = a.pr_spec[b0];
+  // components d = tid + WG j of this thread: row offsets of (n, l) and (n', l)
+  // in the tables, n == n'
+  int code[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int cd = P.dtab[min(tid + WG * j, D - 1)];
+    const int n = cd & 0xff, np = (cd >> 8) & 0xff, l = cd >> 16;
+    code[j] = (n * L1 + l) | ((np * L1 + l) << 8) | ((n == np ? 1 : 0) << 16);
+  }
+  if (tid < NLM) ynorm[tid] = yn;
+  if (tid < 2 * G::SPW) (red + 8)[tid] = reinterpret_cast<const double*>(P.sp)[tid];
+  tabs.store(U);
+  // ---- c(n, lm): (l, m) tiles w and w + 4
+  double* CH = U;                    // [NLM][CP]: c, then H
+  double* X = U + NLM * CP + 1;      // [D]: p, then q
   {
-    double acc[2][16];
+    double* W = U + G::TABS;         // [CHK][NLM]
+    f64x4_t acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+    for (int k0 = 0; k0 < np1; k0 += CHK) {
+      const int cnt = min(CHK, np1 - k0);
+      der_prepare<LL, true>(spl, a.pr_spec, a.pr_r, a.pr_xyz, b0, k0, cnt, ynorm, rec, U, W);
+      lds_barrier();
+      for (int j0 = 0; j0 < cnt; j0 += 4) {
+        const int j = j0 + lg;
+        const bool ok = j < cnt;
+        const double* st = rec + j * ST;
+        const int nl = ok ? li - (int)st[31] : -1;
+        const double av = ok && nl >= 0 && nl < (int)st[32] ? st[nl] : 0.0;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int n = 0; n < 16; ++n) acc[h][n] = 0.0;
-    PairScratch<double> ps;
-    ps.bind(U + w * G::PS, LL, NLM);
-    int lh[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) lh[h] = lm_l(lane + 64 * h);
-    for (int k = 1 + w; k < nn; k += 4) {
-      const DerPair pr = der_pair(P, a, RG, b0, k);
-      if (!pr.ok) continue;
-      der_gauss(P, RG, pr, lane, ps, false);
-      harmonics_m<LL, false>(lane, ynorm, rinv, pr.ux, pr.uy, pr.uz, ps.Y, nullptr);
-      der_wave_sync();
-      der_radial(P, RG, pr, lane, ps, false);
-      der_wave_sync();
-      const int nb = P.sp[pr.s].nb, off = P.sp[pr.s].off;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int lm = lane + 64 * h;
-        if (lm < NLM) {
-          const double al = ps.A[lh[h]], yv = ps.Y[lm];
-#pragma unroll
-          for (int n = 0; n < 16; ++n) {
-            const int nl = n - off;
-            if (nl >= 0 && nl < nb) acc[h][n] += ps.R[nl] * al * yv;
+        for (int t = 0; t < 2; ++t) {
+          const int lm = 16 * (w + 4 * t) + li;
+          if (w + 4 * t < NT) {
+            const double bv = ok && lm < NLM ? W[j * NLM + lm] : 0.0;
+            acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[t], 0, 0, 0);
           }
         }
       }
-      der_wave_sync();
+      lds_barrier();
     }
-    lds_barrier();  // the pair scratch is dead: the partial sums overlay it
+    if (w == 0 && li == 0 && sself >= 0) {  // central atom (self pair): its own species block, l = 0
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int lm = lane + 64 * h;
-      if (lm < NLM)
+      for (int r = 0; r < 4; ++r) {
+        const int nl = 4 * r + lg - P.sp[sself].off;
+        if (nl >= 0 && nl < P.sp[sself].nb) acc[0][r] += P.cen[sself * TGX_MAX_NB + nl];
+      }
+    }
 #pragma unroll
-        for (int n = 0; n < 16; ++n)
-          if (n < N) U[w * CN + n * NLM + lm] = acc[h][n];
+    for (int t = 0; t < 2; ++t) {
+      const int lm = 16 * (w + 4 * t) + li;
+      if (w + 4 * t < NT && lm < NLM)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) CH[lm * CP + 4 * r + lg] = acc[t][r];
     }
   }
   lds_barrier();
-  for (int e = tid; e < CN; e += WG) c[e] = ((U[e] + U[CN + e]) + U[2 * CN + e]) + U[3 * CN + e];
+  double cc[21], hh[21];
+#pragma unroll
+  for (int i = 0; i < 21; ++i) cc[i] = CH[der_lm<LL>(w, i) * CP + li];
+  // ---- power spectrum, degrees w, w + 4, w + 8
+  for (int l = w; l < L1; l += 4) {
+    const int K = 2 * l + 1;
+    f64x4_t g = {0.0, 0.0, 0.0, 0.0};
+    double v[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+      const int k = 4 * q + lg;
+      v[q] = k < K ? CH[(l * l + k) * CP + li] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < 5; ++q)
+      if (4 * q < K) g = __builtin_amdgcn_mfma_f64_16x16x4f64(v[q], v[q], g, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = 4 * r + lg, np = li;
+      if (n <= np && np < N) X[(n * N - n * (n - 1) / 2 + (np - n)) * L1 + l] = n == np ? g[r] : M_SQRT2 * g[r];
+    }
+  }
   lds_barrier();
+  double qd[J], nrm;
   {
-    // central atom (self pair): its own species block, l = 0
-    const int s = a.pr_spec[b0];
-    if (s >= 0)
-      for (int n = tid; n < P.sp[s].nb; n += WG) c[(P.sp[s].off + n) * NLM] += P.cen[s * TGX_MAX_NB + n];
-  }
-  lds_barrier();
-  const double nrm = power_spectrum<double>(P, c, X, U);
-  double* qrow = q_out + (size_t)site * P.Dpad;
-  for (int d = tid; d < P.Dpad; d += WG) qrow[d] = d < D ? X[d] : 0.0;
-  if (tid == 0) pnorm_out[site] = nrm;
-  contract_channel<double>(P, X, c, H);
-  // components d = tid + WG j of this thread: row offsets of (n, l) and (n', l)
-  // in the tables, n == n', d
-  int code[J];
-  double self[J][3];
+    double s2 = 0.0;
 #pragma unroll
-  for (int j = 0; j < J; ++j) code[j] = P.dtab[min(tid + WG * j, D - 1)];  // all loads in flight at once
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int d = tid + WG * j;
-    const int cd = code[j];
-    const int n = cd & 0xff, np = (cd >> 8) & 0xff, l = cd >> 16;
-    code[j] = d < D ? (n * L1 + l) | ((np * L1 + l) << 8) | ((n == np ? 1 : 0) << 16) | (d << 17) : -1;
-    self[j][0] = self[j][1] = self[j][2] = 0.0;
+    for (int j = 0; j < J; ++j) {
+      const int d = tid + WG * j;
+      qd[j] = d < D ? X[d] : 0.0;
+      s2 += qd[j] * qd[j];
+    }
+    for (int o = 32; o > 0; o >>= 1) s2 += __shfl_xor(s2, o);
+    if (lane == 0) red[w] = s2;
+    lds_barrier();
+    nrm = sqrt((red[0] + red[1]) + (red[2] + red[3]));
   }
   const double inv_n = nrm > 0.0 ? 1.0 / nrm : 0.0;
   const bool site_ok = nrm > 0.0;
-  double* qpart = U + 4 * SL;  // [wave][pair][k] partial q . dp
-  lds_barrier();
-  for (int g = 1; g < nn; g += 4) {
-    // (a) wavefront w: pair g + w's Gaussians, harmonics with gradients and radial values
-    {
-      double* slot = U + w * SL;
-      double* misc = slot + 6 * NL;
-      PairScratch<double> ps;
-      ps.bind(misc + 8, LL, NLM);
-      bool ok = false;
-      DerPair pr{};
-      if (g + w < nn) {
-        pr = der_pair(P, a, RG, b0, g + w);
-        ok = pr.ok && site_ok;
-      }
-      if (ok) {
-        der_gauss(P, RG, pr, lane, ps, true);
-        harmonics_m<LL, true, true>(lane, ynorm, rinv, pr.ux, pr.uy, pr.uz, ps.Y, nullptr);
-        der_wave_sync();
-        der_radial(P, RG, pr, lane, ps, true);
-      }
-      if (lane == 0) {
-        misc[0] = ok ? 1.0 : 0.0;
-        misc[1] = ok ? (double)P.sp[pr.s].off : 0.0;
-        misc[2] = ok ? (double)P.sp[pr.s].nb : 0.0;
-        misc[3] = ok ? pr.r : 1.0;
-        misc[4] = ok ? pr.ux : 0.0;
-        misc[5] = ok ? pr.uy : 0.0;
-        misc[6] = ok ? pr.uz : 0.0;
-      }
-    }
-    lds_barrier();
-    // (b) channel tables of the four pairs: lanes (n, pair), wavefront w takes
-    // the degrees {8, 0, 1}, {7, 2}, {6, 3} or {5, 4} (20 or 21 (l, m) each)
-    der_tables_w<LL>(P, w, lane, N, U, SL, c, H, qpart);
-    lds_barrier();
-    // (c) the slabs of the (up to) four pairs: thread owns components d, all three k
-    const int cnt = min(4, nn - g);
-    for (int pp = 0; pp < cnt; ++pp) {
-      const double* slot = U + pp * SL;
-      const double* misc = slot + 6 * NL;
-      const double* qp = qpart + 3 * pp;
-      const double q0 = ((qp[0] + qp[12]) + qp[24]) + qp[36];
-      const double q1 = ((qp[1] + qp[13]) + qp[25]) + qp[37];
-      const double q2 = ((qp[2] + qp[14]) + qp[26]) + qp[38];
-      const double ux = misc[4], uy = misc[5], uz = misc[6];
-      double* out = der_out + (size_t)(b0 + g + pp) * D3;
+  double* qrow = q_out + (size_t)site * P.Dpad;
 #pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const int cj = code[j];
-        if (cj < 0) continue;
-        const int i1 = cj & 0xff, i2 = (cj >> 8) & 0xff, d = cj >> 17;
-        const double wgt = ((cj >> 16) & 1) ? 1.0 : M_SQRT2;
-        const double qd = X[d];
-        const double2* t1 = reinterpret_cast<const double2*>(slot + 6 * i1);
-        const double2* t2 = reinterpret_cast<const double2*>(slot + 6 * i2);
-        const double2 a1 = t1[0], b1 = t1[1], c1 = t1[2];  // (s, E), (v_x, v_y), (v_z, Dd)
-        const double2 a2 = t2[0], b2 = t2[1], c2 = t2[2];
-        const double rad = c1.y * a2.x + c2.y * a1.x;
-        const double ox = (wgt * (rad * ux + a1.y * b2.x + a2.y * b1.x) - qd * q0) * inv_n;
-        const double oy = (wgt * (rad * uy + a1.y * b2.y + a2.y * b1.y) - qd * q1) * inv_n;
-        const double oz = (wgt * (rad * uz + a1.y * c2.x + a2.y * c1.x) - qd * q2) * inv_n;
-        out[3 * d] = ox;
-        out[3 * d + 1] = oy;
-        out[3 * d + 2] = oz;
-        self[j][0] -= ox;
-        self[j][1] -= oy;
-        self[j][2] -= oz;
+  for (int j = 0; j < J; ++j) {
+    const int d = tid + WG * j;
+    qd[j] *= inv_n;
+    if (d < D) X[d] = qd[j];
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int d = tid + WG * j;
+    if (d < P.Dpad) qrow[d] = qd[j];
+  }
+  for (int d = tid + WG * J; d < P.Dpad; d += WG) qrow[d] = 0.0;
+  if (tid == 0) pnorm_out[site] = nrm;
+  lds_barrier();
+  // ---- H_l = S_l c_l in place: l = 0..7, then (l, m) 64..79 and 80 of l = 8
+  for (int ht = w; ht < LL + 2; ht += 4) {
+    const int l = min(ht, LL);
+    const int base = ht <= LL ? l * l : l * l + 16;
+    const int width = ht < LL ? 2 * l + 1 : (ht == LL ? 16 : 2 * LL - 15);
+    f64x4_t h = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int n = li, np = 4 * s + lg;
+      const int u = min(n, np), v = max(n, np);
+      const double av =
+          v < N ? (n == np ? 2.0 : M_SQRT2) * X[(u * N - u * (u - 1) / 2 + (v - u)) * L1 + l] : 0.0;
+      const double bv = li < width ? CH[(base + li) * CP + np] : 0.0;
+      h = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, h, 0, 0, 0);
+    }
+    if (li < width)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) CH[(base + li) * CP + 4 * r + lg] = h[r];
+  }
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < 21; ++i) hh[i] = CH[der_lm<LL>(w, i) * CP + li];
+  lds_barrier();
+  // ---- pairs, four at a time
+  double* Yb = U + 4 * SL;              // [HG][NLM][4]
+  double* qpart = Yb + G::HG * 4 * NLM;     // [wave][pair][k] partial q . dp
+  double self[J][3];
+#pragma unroll
+  for (int j = 0; j < J; ++j) self[j][0] = self[j][1] = self[j][2] = 0.0;
+  for (int k0 = 0; k0 < np1; k0 += CHK) {
+    const int cntc = min(CHK, np1 - k0);
+    if (np1 > CHK)  // the records hold the expansion's last pairs: this chunk's again
+      der_prepare_again<LL>(spl, P.xq, P.B, P.n_species, a.pr_spec, a.pr_r, a.pr_xyz, b0, k0, cntc, rec, U);
+    for (int g = 0; g < cntc; g += 4) {
+      lds_barrier();
+      if (g % G::HG == 0) {  // harmonics with gradients of the next sixteen pairs, a row of lanes each
+        const int hj = tid >> 4;
+        const double* st = rec + min(g + hj, cntc - 1) * ST;
+        if (g + hj < cntc && st[30] != 0.0) {
+          double2* y = reinterpret_cast<double2*>(Yb + hj * 4 * NLM);
+          ylm_lanes<double, true, 16>(LL, ynorm, li, st[27], st[28], st[29], 1.0,
+                                      [&](int, int lm, double, double Y, double gx, double gy, double gz) {
+                                        y[2 * lm] = make_double2(Y, gx);
+                                        y[2 * lm + 1] = make_double2(gy, gz);
+                                      });
+        }
+        lds_barrier();
+      }
+      {
+        DerLane p;
+        const bool have = g + lg < cntc;
+        const double* st = rec + min(g + lg, cntc - 1) * ST;
+        p.ok = have && st[30] != 0.0 && site_ok;
+        const int nl = li - (int)st[31];
+        const bool inb = p.ok && nl >= 0 && nl < (int)st[32];
+        p.R = inb ? st[nl] : 0.0;
+        p.dR = inb ? st[8 + nl] : 0.0;
+        p.dk = st[25];
+        p.inv_r = st[26];
+        p.ux = st[27];
+        p.uy = st[28];
+        p.uz = st[29];
+        const double* y = Yb + (g % G::HG + lg) * 4 * NLM;
+        double* slot = U + lg * SL + 6 * li * L1;
+        double qx = 0.0, qy = 0.0, qz = 0.0;
+        if (w == 0) {
+          der_channel<LL, 8, 0>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+          der_channel<LL, 0, 17>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+          der_channel<LL, 1, 18>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+        } else if (w == 1) {
+          der_channel<LL, 7, 0>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+          der_channel<LL, 2, 15>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+        } else if (w == 2) {
+          der_channel<LL, 6, 0>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+          der_channel<LL, 3, 13>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+        } else {
+          der_channel<LL, 5, 0>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+          der_channel<LL, 4, 11>(p, y, st + 16, cc, hh, slot, qx, qy, qz);
+        }
+        qx = lanes_sum<16>(qx);
+        qy = lanes_sum<16>(qy);
+        qz = lanes_sum<16>(qz);
+        if (li == 0) {
+          double* q = qpart + (w * 4 + lg) * 3;
+          q[0] = qx;
+          q[1] = qy;
+          q[2] = qz;
+        }
+      }
+      lds_barrier();
+      const int cnt = min(4, cntc - g);
+      for (int pp = 0; pp < cnt; ++pp) {
+        const double* slot = U + pp * SL;
+        const double* st = rec + (g + pp) * ST;
+        const double* qp = qpart + 3 * pp;
+        const double q0 = ((qp[0] + qp[12]) + qp[24]) + qp[36];
+        const double q1 = ((qp[1] + qp[13]) + qp[25]) + qp[37];
+        const double q2 = ((qp[2] + qp[14]) + qp[26]) + qp[38];
+        const double ux = st[27], uy = st[28], uz = st[29];
+        double* out = der_out + (size_t)(b0 + 1 + k0 + g + pp) * D3;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const int d = tid + WG * j;
+          if (d >= D) continue;
+          const int cj = code[j];
+          const int i1 = cj & 0xff, i2 = (cj >> 8) & 0xff;
+          const double wgt = (cj >> 16) ? 1.0 : M_SQRT2;
+          const double2* t1 = reinterpret_cast<const double2*>(slot + 6 * i1);
+          const double2* t2 = reinterpret_cast<const double2*>(slot + 6 * i2);
+          const double2 a1 = t1[0], b1 = t1[1], c1 = t1[2];  // (s, E), (v_x, v_y), (v_z, Dd)
+          const double2 a2 = t2[0], b2 = t2[1], c2 = t2[2];
+          const double rad = c1.y * a2.x + c2.y * a1.x;
+          const double ox = (wgt * (rad * ux + a1.y * b2.x + a2.y * b1.x) - qd[j] * q0) * inv_n;
+          const double oy = (wgt * (rad * uy + a1.y * b2.y + a2.y * b1.y) - qd[j] * q1) * inv_n;
+          const double oz = (wgt * (rad * uz + a1.y * c2.x + a2.y * c1.x) - qd[j] * q2) * inv_n;
+          out[3 * d] = ox;
+          out[3 * d + 1] = oy;
+          out[3 * d + 2] = oz;
+          self[j][0] -= ox;
+          self[j][1] -= oy;
+          self[j][2] -= oz;
+        }
       }
     }
-    lds_barrier();
   }
   double* out = der_out + (size_t)b0 * D3;
 #pragma unroll
-  for (int j = 0; j < J; ++j)
-    if (code[j] >= 0) {
-      const int d = code[j] >> 17;
+  for (int j = 0; j < J; ++j) {
+    const int d = tid + WG * j;
+    if (d < D) {
       out[3 * d] = self[j][0];
       out[3 * d + 1] = self[j][1];
       out[3 * d + 2] = self[j][2];
     }
+  }
 }
 
 // Plain-path pair force: f_p = Qss_i . soap_cart_der(:, :, p), one wavefront per
@@ -1364,22 +1298,14 @@ int tgx_soap_descriptors(tgx_ctx* ctx, tgx_model_t* m, int path, bool with_der) 
       bool small_blocks = P.n_species <= 2;
       for (int sp = 0; sp < P.n_species; ++sp) small_blocks = small_blocks && P.sp[sp].nb <= 8 && P.sp[sp].nq <= 64;
       const int jd = (P.D + WG - 1) / WG;  // components per thread of k_soap_der_l
-      if (P.L == 8 && P.N <= 16 && small_blocks && P.D < 4096) {
-        using G = DerL<8>;
-        const size_t cn = (size_t)P.N * P.NLM;
-        size_t u = 4 * (size_t)G::SL + 48;  // four pair slots and the q . dp partials
-        if (4 * cn > u) u = 4 * cn;
-        if ((size_t)WG > u) u = WG;
-        const size_t lds = sizeof(double) * ((size_t)G::NLM + G::L1 + 2 * cn + P.D + (P.D & 1) + u);
+      if (P.L == 8 && P.N <= 16 && small_blocks) {
+        constexpr size_t lds = DerL<8>::LDS;
         TGX_TRY(check_lds(lds));
 #define TGX_SOAP_DER(J)                                                                                     \
   TGX_LAUNCH(ctx, "soap_site_der_f64", (k_soap_der_l<8, J>), dim3(ns), dim3(WG), lds, m->P, a, ns, \
              qout.as<double>(), m->pnorm.as<double>(), dout.as<double>())
         if (jd <= 2) TGX_SOAP_DER(2);
-        else if (jd <= 4) TGX_SOAP_DER(4);
-        else if (jd <= 5) TGX_SOAP_DER(5);
-        else if (jd <= 8) TGX_SOAP_DER(8);
-        else TGX_SOAP_DER(16);
+        else TGX_SOAP_DER(5);
 #undef TGX_SOAP_DER
       } else if (j_need <= 16 && NL <= 255 && P.D < 4096) {
         // coefficient, H and four pair slots; the slots overlay the spectrum and pair scratch

@@ -16,20 +16,11 @@
 // Same conventions and results as the workgroup-per-site kernels (the plain
 // dq/dr kernel keeps that form).
 #include "tgx_internal.h"
+#include "tgx_soap_lanes.h"
 
 namespace {
 
 constexpr int WAVES = 4;
-
-template <class T> __device__ __forceinline__ T w_exp(T x);
-template <> __device__ __forceinline__ double w_exp<double>(double x) { return exp(x); }
-template <> __device__ __forceinline__ float w_exp<float>(float x) { return __expf(x); }
-template <class T> __device__ __forceinline__ T w_pow(T x, T y);
-template <> __device__ __forceinline__ double w_pow<double>(double x, double y) { return pow(x, y); }
-template <> __device__ __forceinline__ float w_pow<float>(float x, float y) { return powf(x, y); }
-template <class T> __device__ __forceinline__ T w_sqrt(T x);
-template <> __device__ __forceinline__ double w_sqrt<double>(double x) { return sqrt(x); }
-template <> __device__ __forceinline__ float w_sqrt<float>(float x) { return sqrtf(x); }
 
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -69,152 +60,6 @@ template <class T> struct Tables {
     }
   }
 };
-
-// Sum over the four lanes of a quad, which share a pair, by DPP on the VALU; the
-// same on all four.
-template <int CTRL> __device__ __forceinline__ float dpp_of(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
-}
-template <int CTRL> __device__ __forceinline__ double dpp_of(double x) {
-  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true),
-                          __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true));
-}
-template <class T> __device__ __forceinline__ T quad_sum(T v) {
-  v += dpp_of<0xB1>(v);         // quad_perm [1, 0, 3, 2]
-  return v + dpp_of<0x4E>(v);   // quad_perm [2, 3, 0, 1]
-}
-
-// Radial projections of one pair by the four lanes of a quad: R[n] and, when
-// GRAD, dR[n]/dr, complete on every lane. Lane sub takes the nodes sub, sub + 4,
-// ...: a lane per pair left three quarters of the wavefront idle (16 pairs a
-// pass) through the Gaussians, the largest part of both kernels.
-template <class T, bool GRAD>
-__device__ __forceinline__ void quad_radial(const SoapParams& P, const Tables<T>& tb, int s, int sub, T r,
-                                            T (&R)[TGX_MAX_NB], T (&dR)[TGX_MAX_NB]) {
-  const SpeciesParams& sp = P.sp[s];
-  const T inv_rc = (T)sp.inv_rc;
-  const T x = r * inv_rc;
-  const T sig = (T)sp.sig_r * ((T)1 + (T)sp.sig_r_sc * r) * inv_rc;
-  const T dsig = (T)(sp.sig_r * sp.sig_r_sc) * inv_rc;
-  const T inv_s2 = (T)1 / (sig * sig);
-  const T d1 = inv_s2 * inv_rc, d2 = inv_s2 / sig * dsig, ex = -(T)0.5 * inv_s2;
-#pragma unroll
-  for (int n = 0; n < TGX_MAX_NB; ++n) { R[n] = 0; dR[n] = 0; }
-  const T* xq = tb.xq + s * TGX_MAX_Q;
-  const T* Bt = tb.Bt + s * TGX_MAX_Q * TGX_MAX_NB;
-  const int nb = sp.nb;
-  for (int q = sub; q < sp.nq; q += 4) {
-    const T dx = xq[q] - x;
-    const T g = w_exp<T>(dx * dx * ex);
-    T dg = 0;
-    if (GRAD) dg = g * (dx * d1 + dx * dx * d2);
-    const T* b = Bt + q * TGX_MAX_NB;
-#pragma unroll
-    for (int n = 0; n < TGX_MAX_NB; ++n) {
-      if (n < nb) {
-        R[n] += b[n] * g;
-        if (GRAD) dR[n] += b[n] * dg;
-      }
-    }
-  }
-  const T a = (T)sp.amp_a;
-  const T Pp = (T)1 + (T)2 * x * x * x - (T)3 * x * x;
-  const T dPp = ((T)6 * x * x - (T)6 * x) * inv_rc;
-  T amp, damp;
-  if (a == (T)0) {
-    amp = (T)1 / sig;
-    damp = -dsig / (sig * sig);
-  } else if (Pp <= (T)1.0e-10) {
-    amp = 0;
-    damp = 0;
-  } else {
-    const T Pa = a == (T)1 ? Pp : w_pow<T>(Pp, a);  // x^1 = x and x^0 = 1 exactly
-    amp = Pa / sig;
-    damp = a * (a == (T)1 ? (T)1 : w_pow<T>(Pp, a - (T)1)) * dPp / sig - Pa * dsig / (sig * sig);
-  }
-  amp *= (T)sp.gs;
-  damp *= (T)sp.gs;
-#pragma unroll
-  for (int n = 0; n < TGX_MAX_NB; ++n) {
-    if (n < nb) {
-      const T I = quad_sum(R[n]);
-      R[n] = amp * I;
-      if (GRAD) dR[n] = damp * I + amp * quad_sum(dR[n]);
-    }
-  }
-}
-
-// Angular damping A_l = exp(-l(l+1) kk): A_l = prod_{k <= l} e2^k with e2 =
-// exp(-2 kk); -A_l'/A_l = l(l+1) dk.
-template <class T> struct Damp {
-  T e2, dk;
-  __device__ void init(const SpeciesParams& sp, T r) {
-    const T st = (T)sp.sig_t * ((T)1 + (T)sp.sig_t_sc * r);
-    const T dst = (T)(sp.sig_t * sp.sig_t_sc);
-    dk = st * st / (r * r * r) - st * dst / (r * r);
-    const T e1 = w_exp<T>(-(st * st / ((T)2 * r * r)));
-    e2 = e1 * e1;
-  }
-};
-
-// The real harmonics at u (and the gradient of the solid harmonic when GRAD) of
-// one pair by the four lanes of a quad, to f(l, lm, A_l, Y, gx, gy, gz). Lane sub
-// takes the orders m = sub, 7 - sub, 8 + sub, 15 - sub: for l_max = 8 at most 15
-// degrees against 45 for a lane on its own, the four lanes stepping through
-// their degrees together. The order's cos and sin factors c + i s = (ux + i
-// uy)^m, their gradient (m (c', s') of order m - 1) and A_m come from the powers
-// up to m.
-template <class T, bool GRAD, class F>
-__device__ __forceinline__ void ylm_quad(int L, const T* ynorm, int sub, T ux, T uy, T uz, T e2, F&& f) {
-  T c = (T)1, s = (T)0, cp = (T)0, sp = (T)0, pw0 = (T)1, A0 = (T)1;
-  int k = 0;
-  for (int t = 0; 4 * t <= L; ++t) {
-    const int m = 8 * (t >> 1) + ((t & 1) ? 7 - sub : sub);
-    for (; k < m && k < L; ++k) {
-      cp = c;
-      sp = s;
-      c = cp * ux - sp * uy;
-      s = cp * uy + sp * ux;
-      pw0 *= e2;
-      A0 *= pw0;
-    }
-    const T dm = (T)m;
-    const T cx = dm * cp, cy = -dm * sp, sx = dm * sp, sy = dm * cp;
-    T q = (T)1, qx = (T)0, qy = (T)0, qz = (T)0, p = (T)0, px = (T)0, py = (T)0, pz = (T)0;
-    T Al = A0, pw = pw0;
-    for (int i = 0; i <= L; ++i) {
-      const int l = m + i;
-      if (l > L) break;
-      if (i == 1) {
-        p = q; px = qx; py = qy; pz = qz;
-        qz = (T)2 * dm + (T)1;
-        q = qz * uz;
-        qx = (T)0; qy = (T)0;
-      } else if (i > 1) {
-        const T inv = (T)1 / (T)i, a = ((T)2 * dm + (T)(2 * i - 1)) * inv,
-                     b = ((T)2 * dm + (T)(i - 1)) * inv;
-        const T nq = a * uz * q - b * p;
-        if (GRAD) {
-          const T nqx = a * uz * qx - b * ((T)2 * ux * p + px);
-          const T nqy = a * uz * qy - b * ((T)2 * uy * p + py);
-          const T nqz = a * (q + uz * qz) - b * ((T)2 * uz * p + pz);
-          px = qx; py = qy; pz = qz;
-          qx = nqx; qy = nqy; qz = nqz;
-        }
-        p = q;
-        q = nq;
-      }
-      if (i > 0) {
-        pw *= e2;
-        Al *= pw;
-      }
-      const int base = l * l + l;
-      const T N = ynorm[base + m];
-      f(l, base + m, Al, N * q * c, N * (qx * c + q * cx), N * (qy * c + q * cy), N * qz * c);
-      if (m > 0) f(l, base - m, Al, N * q * s, N * (qx * s + q * sx), N * (qy * s + q * sy), N * qz * s);
-    }
-  }
-}
 
 // Expansion coefficients of one site into C (LDS, [N][NLM]) by one wavefront.
 // Pass over chunks of CH pairs: quads of lanes stage Rf[j][n] (stacked radial index,
@@ -258,7 +103,8 @@ __device__ void wave_coefficients(const SoapParams& P, const Tables<T>& tb, cons
         const T r = (T)rr, inv = (T)1 / r;
         const T ux = (T)a.pr_xyz[3 * p] * inv, uy = (T)a.pr_xyz[3 * p + 1] * inv, uz = (T)a.pr_xyz[3 * p + 2] * inv;
         T R[TGX_MAX_NB], dR[TGX_MAX_NB];
-        quad_radial<T, false>(P, tb, s, sub, r, R, dR);
+        radial_lanes<T, false, 4, TGX_MAX_NB>(P.sp[s], tb.xq + s * TGX_MAX_Q, tb.Bt + s * TGX_MAX_Q * TGX_MAX_NB, sub, r,
+                                                R, dR);
         const int off = P.sp[s].off, nb = P.sp[s].nb;
         wave_sync();  // the quad's zeros before its values
         if (sub == 0)
@@ -267,7 +113,7 @@ __device__ void wave_coefficients(const SoapParams& P, const Tables<T>& tb, cons
             if (n < nb) rf[off + n] = R[n];
         Damp<T> dmp;
         dmp.init(P.sp[s], r);
-        ylm_quad<T, false>(L, tb.ynorm, sub, ux, uy, uz, dmp.e2,
+        ylm_lanes<T, false, 4>(L, tb.ynorm, sub, ux, uy, uz, dmp.e2,
                            [&](int l, int lm, T Al, T Y, T, T, T) { w[lm] = Al * Y; });
       } else {
         for (int lm = sub; lm < NLM; lm += 4) w[lm] = 0;
@@ -462,7 +308,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_adjoint_wave(SoapParams P, WaveA
         const T inv = (T)1 / r;
         ux = (T)a.pr_xyz[3 * p] * inv; uy = (T)a.pr_xyz[3 * p + 1] * inv; uz = (T)a.pr_xyz[3 * p + 2] * inv;
         T R[TGX_MAX_NB], dR[TGX_MAX_NB];
-        quad_radial<T, true>(P, tb, s, sub, r, R, dR);
+        radial_lanes<T, true, 4, TGX_MAX_NB>(P.sp[s], tb.xq + s * TGX_MAX_Q, tb.Bt + s * TGX_MAX_Q * TGX_MAX_NB, sub, r,
+                                             R, dR);
         const int off = P.sp[s].off, nb = P.sp[s].nb;
         wave_sync();  // the quad's zeros before its values
         if (sub == 0)
@@ -499,7 +346,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_adjoint_wave(SoapParams P, WaveA
       dmp.init(P.sp[s], r);
       const T* xa = Xa + pj * NLM;
       const T* xb = Xb + pj * NLM;
-      ylm_quad<T, true>(L, tb.ynorm, sub, ux, uy, uz, dmp.e2, [&](int l, int lm, T A, T Y, T gx, T gy, T gz) {
+      ylm_lanes<T, true, 4>(L, tb.ynorm, sub, ux, uy, uz, dmp.e2, [&](int l, int lm, T A, T Y, T gx, T gy, T gz) {
         const T x = xa[lm], y = xb[lm];
         const T Ax = A * x, lf = (T)l;
         const T ang = Ax * inv_r;
@@ -509,9 +356,9 @@ __global__ __launch_bounds__(64 * WAVES) void k_adjoint_wave(SoapParams P, WaveA
         f1 += t * uy + ang * gy;
         f2 += t * uz + ang * gz;
       });
-      f0 = quad_sum(f0);
-      f1 = quad_sum(f1);
-      f2 = quad_sum(f2);
+      f0 = lanes_sum<4>(f0);
+      f1 = lanes_sum<4>(f1);
+      f2 = lanes_sum<4>(f2);
     }
     if (pj < cnt && sub == 0) {
       const int64_t gi = a.pr_gidx[p];
