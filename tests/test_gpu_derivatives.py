@@ -30,3 +30,24 @@ def test_derivatives_match_oracle(ctx, orc, n, species, n_max):
     # up to 80 others
     np.testing.assert_allclose(q, qo, rtol=0, atol=1e-12)
     np.testing.assert_allclose(der, dero, rtol=0, atol=1e-11 * max(1.0, np.abs(dero).max()))
+
+
+@pytest.mark.parametrize("n,species,n_max", [(8, 1, 8), (75, 2, 8), (76, 2, 3), (120, 1, 7), (180, 2, 8)])
+def test_adjoint_matches_plain(ctx, n, species, n_max):
+    rng = np.random.default_rng(n)
+    codes = [S.SPECIES_A, S.SPECIES_B][:species]
+    sp = np.array(codes, np.int32)[rng.integers(0, species, n)]
+    ctx.set_system(S.rsa(n, 8.0, 0.9, 3 * n), sp, S.cubic_box(8.0))
+    ctx.build_neighbors_list(3.7, fetch=False)
+    h = S.soap_hypers(codes, central_species=0, n_max=n_max)
+    Qs = rng.random((40, h.dim))
+    ctx.soap_model(h, Qs / np.linalg.norm(Qs, axis=1, keepdims=True), rng.normal(scale=1e-2, size=40))
+    Ep, Wp = ctx.compute("fp64_plain")
+    ep, fp = ctx.results()
+    Ea, Wa = ctx.compute("fp64_adjoint")
+    ea, fa = ctx.results()
+    # the same sums in another order: up to 1,224 components by 80 pairs of one sign at most, 2^-53 each
+    tol = 1e-12 * max(1.0, np.abs(fp).max())
+    assert np.abs(ea - ep).max() <= 1e-13 and abs(Ea - Ep) <= 1e-13 * n
+    assert np.abs(fa - fp).max() <= tol
+    assert np.abs(Wa - Wp).max() <= tol * n * 3.7

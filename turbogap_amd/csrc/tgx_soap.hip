@@ -700,6 +700,9 @@ template <int LL> struct DerL {
   static constexpr int U3 = 4 * SL + HG * 4 * NLM + 48;     // four pairs' tables, harmonics, q . dp
   static constexpr int U = U1 > U2 ? (U1 > U3 ? U1 : U3) : (U2 > U3 ? U2 : U3);
   static constexpr size_t LDS = sizeof(double) * (HEADP + U);
+  static constexpr size_t LDS_DESC = sizeof(double) * (HEADP + (U1 > U2 ? U1 : U2));
+  static constexpr int U4 = HG * 4 * NLM + 4 * HG * 3;  // adjoint: harmonics, partials
+  static constexpr size_t LDS_ADJ = sizeof(double) * (HEADP + (U1 > U2 ? (U1 > U4 ? U1 : U4) : (U2 > U4 ? U2 : U4)));
 };
 
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
@@ -863,6 +866,190 @@ __device__ __forceinline__ void der_channel(const DerLane& p, const double* y, c
   qz += Dd * h0 * p.uz + E * (hz - lf * h0 * p.uz) * p.inv_r;
 }
 
+// What the three kernels of a site share. LDS: ynorm [NLM], CHK pair records, red [8],
+// the species' parameters, then U (its use differs).
+template <int LL> struct LSite {
+  using G = DerL<LL>;
+  double *ynorm, *rec, *red, *U;
+  SpeciesParams* spl;
+  int tid, w, lane, li, lg;
+  int64_t b0;
+  int np1;
+  __device__ __forceinline__ LSite(const SiteArgs& a, double* sm, int site) {
+    tid = threadIdx.x;
+    w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    lane = tid & 63;
+    li = lane & 15;
+    lg = lane >> 4;
+    ynorm = sm;
+    rec = ynorm + G::NLM;
+    red = rec + G::CHK * G::ST;
+    spl = reinterpret_cast<SpeciesParams*>(red + 8);
+    U = sm + G::HEADP;
+    b0 = a.site_beg[site];
+    np1 = (int)(a.site_beg[site + 1] - b0) - 1;
+  }
+};
+
+// c(n, lm) of the site into CH = U ([NLM][CP]), (l, m) tiles w and w + 4.
+template <int LL>
+__device__ __forceinline__ void l_expand(const SoapParams& P, const SiteArgs& a, const LSite<LL>& S) {
+  using G = DerL<LL>;
+  constexpr int NLM = G::NLM, CHK = G::CHK, ST = G::ST, CP = G::CP;
+  constexpr int NT = (NLM + 15) / 16;
+  static_assert(NT <= 8 && LL <= 8, "two tiles a wavefront, a degree's (l, m) in at most two tiles");
+  const int w = S.w, li = S.li, lg = S.lg, tid = S.tid;
+  double* CH = S.U;
+  DerTabs tabs;
+  tabs.load(P.xq, P.B, P.n_species);
+  const double yn = tid < NLM ? P.ynorm[tid] : 0.0;
+  const int sself = a.pr_spec[S.b0];
+  if (tid < NLM) S.ynorm[tid] = yn;
+  if (tid < 2 * G::SPW) (S.red + 8)[tid] = reinterpret_cast<const double*>(P.sp)[tid];
+  tabs.store(S.U);
+  double* W = S.U + G::TABS;         // [CHK][NLM]
+  f64x4_t acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+  for (int k0 = 0; k0 < S.np1; k0 += CHK) {
+    const int cnt = min(CHK, S.np1 - k0);
+    der_prepare<LL, true>(S.spl, a.pr_spec, a.pr_r, a.pr_xyz, S.b0, k0, cnt, S.ynorm, S.rec, S.U, W);
+    lds_barrier();
+    for (int j0 = 0; j0 < cnt; j0 += 4) {
+      const int j = j0 + lg;
+      const bool ok = j < cnt;
+      const double* st = S.rec + j * ST;
+      const int nl = ok ? li - (int)st[31] : -1;
+      const double av = ok && nl >= 0 && nl < (int)st[32] ? st[nl] : 0.0;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int lm = 16 * (w + 4 * t) + li;
+        if (w + 4 * t < NT) {
+          const double bv = ok && lm < NLM ? W[j * NLM + lm] : 0.0;
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[t], 0, 0, 0);
+        }
+      }
+    }
+    lds_barrier();
+  }
+  if (S.np1 <= 0) lds_barrier();  // the parameters, which the preparation's barrier covers otherwise
+  if (w == 0 && li == 0 && sself >= 0) {  // central atom (self pair): its own species block, l = 0
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int nl = 4 * r + lg - S.spl[sself].off;
+      if (nl >= 0 && nl < S.spl[sself].nb) acc[0][r] += P.cen[sself * TGX_MAX_NB + nl];
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int lm = 16 * (w + 4 * t) + li;
+    if (w + 4 * t < NT && lm < NLM)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) CH[lm * CP + 4 * r + lg] = acc[t][r];
+  }
+  lds_barrier();
+}
+
+// Power spectrum of CH into X [D], its norm, and this thread's components d = tid + WG j
+// of q = p / |p| (zero past D), also written to q_out's row; X holds p.
+template <int LL, int J>
+__device__ __forceinline__ double l_spectrum(const SoapParams& P, const LSite<LL>& S, double* X, double (&qd)[J],
+                                             double* qrow, double* pnorm) {
+  using G = DerL<LL>;
+  constexpr int L1 = G::L1, CP = G::CP;
+  const int w = S.w, lane = S.lane, li = S.li, lg = S.lg, tid = S.tid, N = P.N, D = P.D;
+  const double* CH = S.U;
+  double* red = S.red;
+  // degrees w, w + 4, w + 8
+  for (int l = w; l < L1; l += 4) {
+    const int K = 2 * l + 1;
+    f64x4_t g = {0.0, 0.0, 0.0, 0.0};
+    double v[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+      const int k = 4 * q + lg;
+      v[q] = k < K ? CH[(l * l + k) * CP + li] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < 5; ++q)
+      if (4 * q < K) g = __builtin_amdgcn_mfma_f64_16x16x4f64(v[q], v[q], g, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = 4 * r + lg, np = li;
+      if (n <= np && np < N) X[(n * N - n * (n - 1) / 2 + (np - n)) * L1 + l] = n == np ? g[r] : M_SQRT2 * g[r];
+    }
+  }
+  lds_barrier();
+  double nrm;
+  {
+    double s2 = 0.0;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int d = tid + WG * j;
+      qd[j] = d < D ? X[d] : 0.0;
+      s2 += qd[j] * qd[j];
+    }
+    for (int o = 32; o > 0; o >>= 1) s2 += __shfl_xor(s2, o);
+    if (lane == 0) red[w] = s2;
+    lds_barrier();
+    nrm = sqrt((red[0] + red[1]) + (red[2] + red[3]));
+  }
+  const double inv_n = nrm > 0.0 ? 1.0 / nrm : 0.0;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int d = tid + WG * j;
+    qd[j] *= inv_n;
+    if (d < P.Dpad) qrow[d] = qd[j];
+  }
+  for (int d = tid + WG * J; d < P.Dpad; d += WG) qrow[d] = 0.0;
+  if (tid == 0) *pnorm = nrm;
+  return nrm;
+}
+
+// H_l = S_l c_l in place of c, S(n, n') = 2 X or sqrt 2 X off the diagonal: l = 0..7, then
+// (l, m) 64..79 and 80 of l = 8.
+template <int LL>
+__device__ __forceinline__ void l_channel(const SoapParams& P, const LSite<LL>& S, const double* X) {
+  using G = DerL<LL>;
+  constexpr int L1 = G::L1, CP = G::CP;
+  const int w = S.w, li = S.li, lg = S.lg, N = P.N;
+  double* CH = S.U;
+  for (int ht = w; ht < LL + 2; ht += 4) {
+    const int l = min(ht, LL);
+    const int base = ht <= LL ? l * l : l * l + 16;
+    const int width = ht < LL ? 2 * l + 1 : (ht == LL ? 16 : 2 * LL - 15);
+    f64x4_t h = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int n = li, np = 4 * s + lg;
+      const int u = min(n, np), v = max(n, np);
+      const double av =
+          v < N ? (n == np ? 2.0 : M_SQRT2) * X[(u * N - u * (u - 1) / 2 + (v - u)) * L1 + l] : 0.0;
+      const double bv = li < width ? CH[(base + li) * CP + np] : 0.0;
+      h = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, h, 0, 0, 0);
+    }
+    if (li < width)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) CH[(base + li) * CP + 4 * r + lg] = h[r];
+  }
+  lds_barrier();
+}
+
+// Harmonics with gradients, (Y, gx, gy, gz) per lm, of the records g .. g + 15 (< cnt), a
+// row of lanes each.
+template <int LL>
+__device__ __forceinline__ void l_harmonics(const LSite<LL>& S, int g, int cnt, double* Yb) {
+  using G = DerL<LL>;
+  const int hj = S.tid >> 4;
+  const double* st = S.rec + min(g + hj, cnt - 1) * G::ST;
+  if (g + hj < cnt && st[30] != 0.0) {
+    double2* y = reinterpret_cast<double2*>(Yb + hj * 4 * G::NLM);
+    ylm_lanes<double, true, 16>(LL, S.ynorm, S.li, st[27], st[28], st[29], 1.0,
+                                [&](int, int lm, double, double Y, double gx, double gy, double gz) {
+                                  y[2 * lm] = make_double2(Y, gx);
+                                  y[2 * lm + 1] = make_double2(gy, gz);
+                                });
+  }
+}
+
 // Plain-path dq/dr for l_max = LL (the output and element layout of
 // k_soap_der), one workgroup per site.
 //   * Pairs are prepared 32 at a time, eight lanes each (der_prepare), and their
@@ -890,26 +1077,32 @@ __global__ __launch_bounds__(WG, 2) void k_soap_der_l(SoapParams P, SiteArgs a, 
                                                       double* __restrict__ der_out) {
   using G = DerL<LL>;
   constexpr int L1 = G::L1, NLM = G::NLM, SL = G::SL, CHK = G::CHK, ST = G::ST, CP = G::CP;
-  constexpr int NT = (NLM + 15) / 16;  // (l, m) tiles of the expansion
-  static_assert(NT <= 8 && LL <= 8, "two tiles a wavefront, a degree's (l, m) in at most two tiles");
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  double* sm = reinterpret_cast<double*>(smem_raw);
   const int site = blockIdx.x;
   if (site >= n_sites) return;
-  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int li = lane & 15, lg = lane >> 4;
-  const int N = P.N, D = P.D, D3 = 3 * D;
-  double* ynorm = sm;               // NLM
-  double* rec = ynorm + NLM;        // CHK pair records
-  double* red = rec + CHK * ST;     // 8
-  SpeciesParams* spl = reinterpret_cast<SpeciesParams*>(red + 8);  // two species
-  double* U = sm + G::HEADP;
-  const int64_t b0 = a.site_beg[site];
-  const int nn = (int)(a.site_beg[site + 1] - b0), np1 = nn - 1;
-  DerTabs tabs;
-  tabs.load(P.xq, P.B, P.n_species);
-  const double yn = tid < NLM ? P.ynorm[tid] : 0.0;
-  const int sself = a.pr_spec[b0];
+  const LSite<LL> S(a, reinterpret_cast<double*>(smem_raw), site);
+  const int tid = S.tid, w = S.w, li = S.li, lg = S.lg, np1 = S.np1;
+  const int D = P.D, D3 = 3 * D;
+  const int64_t b0 = S.b0;
+  double *U = S.U, *rec = S.rec;
+  l_expand<LL>(P, a, S);
+  const double* CH = U;
+  double* X = U + NLM * CP + 1;      // [D]: p, then q
+  double cc[21], hh[21], qd[J];
+#pragma unroll
+  for (int i = 0; i < 21; ++i) cc[i] = CH[der_lm<LL>(w, i) * CP + li];
+  const double nrm =
+      l_spectrum<LL, J>(P, S, X, qd, q_out + (size_t)site * P.Dpad, pnorm_out + site);
+  const double inv_n = nrm > 0.0 ? 1.0 / nrm : 0.0;
+  const bool site_ok = nrm > 0.0;
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    if (tid + WG * j < D) X[tid + WG * j] = qd[j];
+  lds_barrier();
+  l_channel<LL>(P, S, X);
+#pragma unroll
+  for (int i = 0; i < 21; ++i) hh[i] = CH[der_lm<LL>(w, i) * CP + li];
+  lds_barrier();
   // components d = tid + WG j of this thread: row offsets of (n, l) and (n', l)
   // in the tables, n == n'
   int code[J];
@@ -919,129 +1112,6 @@ __global__ __launch_bounds__(WG, 2) void k_soap_der_l(SoapParams P, SiteArgs a, 
     const int n = cd & 0xff, np = (cd >> 8) & 0xff, l = cd >> 16;
     code[j] = (n * L1 + l) | ((np * L1 + l) << 8) | ((n == np ? 1 : 0) << 16);
   }
-  if (tid < NLM) ynorm[tid] = yn;
-  if (tid < 2 * G::SPW) (red + 8)[tid] = reinterpret_cast<const double*>(P.sp)[tid];
-  tabs.store(U);
-  // ---- c(n, lm): (l, m) tiles w and w + 4
-  double* CH = U;                    // [NLM][CP]: c, then H
-  double* X = U + NLM * CP + 1;      // [D]: p, then q
-  {
-    double* W = U + G::TABS;         // [CHK][NLM]
-    f64x4_t acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-    for (int k0 = 0; k0 < np1; k0 += CHK) {
-      const int cnt = min(CHK, np1 - k0);
-      der_prepare<LL, true>(spl, a.pr_spec, a.pr_r, a.pr_xyz, b0, k0, cnt, ynorm, rec, U, W);
-      lds_barrier();
-      for (int j0 = 0; j0 < cnt; j0 += 4) {
-        const int j = j0 + lg;
-        const bool ok = j < cnt;
-        const double* st = rec + j * ST;
-        const int nl = ok ? li - (int)st[31] : -1;
-        const double av = ok && nl >= 0 && nl < (int)st[32] ? st[nl] : 0.0;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int lm = 16 * (w + 4 * t) + li;
-          if (w + 4 * t < NT) {
-            const double bv = ok && lm < NLM ? W[j * NLM + lm] : 0.0;
-            acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[t], 0, 0, 0);
-          }
-        }
-      }
-      lds_barrier();
-    }
-    if (w == 0 && li == 0 && sself >= 0) {  // central atom (self pair): its own species block, l = 0
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int nl = 4 * r + lg - P.sp[sself].off;
-        if (nl >= 0 && nl < P.sp[sself].nb) acc[0][r] += P.cen[sself * TGX_MAX_NB + nl];
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int lm = 16 * (w + 4 * t) + li;
-      if (w + 4 * t < NT && lm < NLM)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) CH[lm * CP + 4 * r + lg] = acc[t][r];
-    }
-  }
-  lds_barrier();
-  double cc[21], hh[21];
-#pragma unroll
-  for (int i = 0; i < 21; ++i) cc[i] = CH[der_lm<LL>(w, i) * CP + li];
-  // ---- power spectrum, degrees w, w + 4, w + 8
-  for (int l = w; l < L1; l += 4) {
-    const int K = 2 * l + 1;
-    f64x4_t g = {0.0, 0.0, 0.0, 0.0};
-    double v[5];
-#pragma unroll
-    for (int q = 0; q < 5; ++q) {
-      const int k = 4 * q + lg;
-      v[q] = k < K ? CH[(l * l + k) * CP + li] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < 5; ++q)
-      if (4 * q < K) g = __builtin_amdgcn_mfma_f64_16x16x4f64(v[q], v[q], g, 0, 0, 0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int n = 4 * r + lg, np = li;
-      if (n <= np && np < N) X[(n * N - n * (n - 1) / 2 + (np - n)) * L1 + l] = n == np ? g[r] : M_SQRT2 * g[r];
-    }
-  }
-  lds_barrier();
-  double qd[J], nrm;
-  {
-    double s2 = 0.0;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int d = tid + WG * j;
-      qd[j] = d < D ? X[d] : 0.0;
-      s2 += qd[j] * qd[j];
-    }
-    for (int o = 32; o > 0; o >>= 1) s2 += __shfl_xor(s2, o);
-    if (lane == 0) red[w] = s2;
-    lds_barrier();
-    nrm = sqrt((red[0] + red[1]) + (red[2] + red[3]));
-  }
-  const double inv_n = nrm > 0.0 ? 1.0 / nrm : 0.0;
-  const bool site_ok = nrm > 0.0;
-  double* qrow = q_out + (size_t)site * P.Dpad;
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int d = tid + WG * j;
-    qd[j] *= inv_n;
-    if (d < D) X[d] = qd[j];
-  }
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int d = tid + WG * j;
-    if (d < P.Dpad) qrow[d] = qd[j];
-  }
-  for (int d = tid + WG * J; d < P.Dpad; d += WG) qrow[d] = 0.0;
-  if (tid == 0) pnorm_out[site] = nrm;
-  lds_barrier();
-  // ---- H_l = S_l c_l in place: l = 0..7, then (l, m) 64..79 and 80 of l = 8
-  for (int ht = w; ht < LL + 2; ht += 4) {
-    const int l = min(ht, LL);
-    const int base = ht <= LL ? l * l : l * l + 16;
-    const int width = ht < LL ? 2 * l + 1 : (ht == LL ? 16 : 2 * LL - 15);
-    f64x4_t h = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int n = li, np = 4 * s + lg;
-      const int u = min(n, np), v = max(n, np);
-      const double av =
-          v < N ? (n == np ? 2.0 : M_SQRT2) * X[(u * N - u * (u - 1) / 2 + (v - u)) * L1 + l] : 0.0;
-      const double bv = li < width ? CH[(base + li) * CP + np] : 0.0;
-      h = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, h, 0, 0, 0);
-    }
-    if (li < width)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) CH[(base + li) * CP + 4 * r + lg] = h[r];
-  }
-  lds_barrier();
-#pragma unroll
-  for (int i = 0; i < 21; ++i) hh[i] = CH[der_lm<LL>(w, i) * CP + li];
-  lds_barrier();
   // ---- pairs, four at a time
   double* Yb = U + 4 * SL;              // [HG][NLM][4]
   double* qpart = Yb + G::HG * 4 * NLM;     // [wave][pair][k] partial q . dp
@@ -1051,20 +1121,11 @@ __global__ __launch_bounds__(WG, 2) void k_soap_der_l(SoapParams P, SiteArgs a, 
   for (int k0 = 0; k0 < np1; k0 += CHK) {
     const int cntc = min(CHK, np1 - k0);
     if (np1 > CHK)  // the records hold the expansion's last pairs: this chunk's again
-      der_prepare_again<LL>(spl, P.xq, P.B, P.n_species, a.pr_spec, a.pr_r, a.pr_xyz, b0, k0, cntc, rec, U);
+      der_prepare_again<LL>(S.spl, P.xq, P.B, P.n_species, a.pr_spec, a.pr_r, a.pr_xyz, b0, k0, cntc, rec, U);
     for (int g = 0; g < cntc; g += 4) {
       lds_barrier();
-      if (g % G::HG == 0) {  // harmonics with gradients of the next sixteen pairs, a row of lanes each
-        const int hj = tid >> 4;
-        const double* st = rec + min(g + hj, cntc - 1) * ST;
-        if (g + hj < cntc && st[30] != 0.0) {
-          double2* y = reinterpret_cast<double2*>(Yb + hj * 4 * NLM);
-          ylm_lanes<double, true, 16>(LL, ynorm, li, st[27], st[28], st[29], 1.0,
-                                      [&](int, int lm, double, double Y, double gx, double gy, double gz) {
-                                        y[2 * lm] = make_double2(Y, gx);
-                                        y[2 * lm + 1] = make_double2(gy, gz);
-                                      });
-        }
+      if (g % G::HG == 0) {
+        l_harmonics<LL>(S, g, cntc, Yb);
         lds_barrier();
       }
       {
@@ -1153,6 +1214,173 @@ __global__ __launch_bounds__(WG, 2) void k_soap_der_l(SoapParams P, SiteArgs a, 
       out[3 * d + 1] = self[j][1];
       out[3 * d + 2] = self[j][2];
     }
+  }
+}
+
+// FP64 descriptors for l_max = LL by the first half of k_soap_der_l, one workgroup
+// per site (listed or in order): a wavefront per site prepared its pairs 16 at a
+// time with four lanes each and formed the rest in loops over LDS. Bound by the
+// preparation's chains at three workgroups a CU (its floor, the pairs read and the
+// descriptors written, is 0.05 ms): 892 -> 342 us at 16,001 atoms of two species.
+template <int LL, int J>
+__global__ __launch_bounds__(WG, 3) void k_desc_l(SoapParams P, SiteArgs a, int n_sites, double* __restrict__ q_out,
+                                                  double* __restrict__ pnorm_out, const int* __restrict__ site_list) {
+  using G = DerL<LL>;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int row = blockIdx.x;
+  if (row >= n_sites) return;
+  const LSite<LL> S(a, reinterpret_cast<double*>(smem_raw), site_list ? site_list[row] : row);
+  l_expand<LL>(P, a, S);
+  double qd[J];
+  l_spectrum<LL, J>(P, S, S.U + G::NLM * G::CP + 1, qd, q_out + (size_t)row * P.Dpad, pnorm_out + row);
+}
+
+// FP64 adjoint pair forces for l_max = LL, one workgroup per site: c as above, H from
+// g = (Qss - (Qss . q) q) / |p|, then sixteen pairs at a time: x = sum_n R_n H(n, lm) and
+// y = sum_n R_n' H(n, lm) of all of them on the FP64 matrix cores, one (l, m) tile after
+// the other, and
+//   f_j = sum_lm [ (A' x + A y) Y u + A x (grad Y - l Y u) / r ]
+// summed by the lane that holds x and y of (j, lm), over the row's lanes, and over the
+// wavefronts (tiles w, w + 4) in order. A wavefront per site held H in registers and
+// walked x and y through LDS: 1,915 -> 752 us at 16,001 atoms of two species, bound as
+// the descriptors (c is formed again: reading it back would cost 10 KB a site).
+template <int LL, int J>
+__global__ __launch_bounds__(WG, 3) void k_adjoint_l(SoapParams P, SiteArgs a, int n_sites,
+                                                     const double* __restrict__ q_in,
+                                                     const double* __restrict__ pnorm_in,
+                                                     const double* __restrict__ qss, double* __restrict__ fglob) {
+  using G = DerL<LL>;
+  constexpr int NLM = G::NLM, CHK = G::CHK, ST = G::ST, CP = G::CP, HG = G::HG;
+  constexpr int NT = (NLM + 15) / 16;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int site = blockIdx.x;
+  if (site >= n_sites) return;
+  const LSite<LL> S(a, reinterpret_cast<double*>(smem_raw), site);
+  const int tid = S.tid, w = S.w, lane = S.lane, li = S.li, lg = S.lg, np1 = S.np1, D = P.D;
+  const int64_t b0 = S.b0;
+  double qd[J], sd[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int d = tid + WG * j;
+    qd[j] = d < D ? q_in[(size_t)site * P.Dpad + d] : 0.0;
+    sd[j] = d < D ? qss[(size_t)site * P.Dpad + d] : 0.0;
+  }
+  const double nrm = pnorm_in[site];
+  l_expand<LL>(P, a, S);
+  double* X = S.U + NLM * CP + 1;  // g
+  {
+    double sq = 0.0;
+#pragma unroll
+    for (int j = 0; j < J; ++j) sq += sd[j] * qd[j];
+    for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
+    if (lane == 0) S.red[w] = sq;
+    lds_barrier();
+    sq = (S.red[0] + S.red[1]) + (S.red[2] + S.red[3]);
+    const double inv_n = nrm > 0.0 ? 1.0 / nrm : 0.0;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int d = tid + WG * j;
+      if (d < D) X[d] = (sd[j] - sq * qd[j]) * inv_n;
+    }
+  }
+  lds_barrier();
+  l_channel<LL>(P, S, X);
+  double hreg[2][4];  // H(4 s + lg, lm) of this wavefront's tiles
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int lm = 16 * (w + 4 * t) + li;
+      hreg[t][s] = lm < NLM ? S.U[lm * CP + 4 * s + lg] : 0.0;
+    }
+  lds_barrier();
+  double* Yb = S.U;                    // [HG][NLM][4]
+  double* part = Yb + HG * 4 * NLM;    // [wave][pair][k]
+  const int oj = tid / 3, ok = tid - 3 * oj;  // pair and component of the thread's output (oj < HG)
+  double self = 0.0;
+  for (int k0 = 0; k0 < np1; k0 += CHK) {
+    const int cntc = min(CHK, np1 - k0);
+    if (np1 > CHK)  // the records hold the expansion's last pairs: this chunk's again
+      der_prepare_again<LL>(S.spl, P.xq, P.B, P.n_species, a.pr_spec, a.pr_r, a.pr_xyz, b0, k0, cntc, S.rec, S.U);
+    for (int g = 0; g < cntc; g += HG) {
+      lds_barrier();
+      l_harmonics<LL>(S, g, cntc, Yb);
+      const bool mine = oj < HG && g + oj < cntc;
+      const int64_t gi = mine ? a.pr_gidx[b0 + 1 + k0 + g + oj] : 0;
+      double ra[4], da[4];
+      {
+        const double* st = S.rec + min(g + li, cntc - 1) * ST;
+        const int off = (int)st[31], nb = (int)st[32];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int nl = 4 * s + lg - off;
+          const bool in = g + li < cntc && nl >= 0 && nl < nb;
+          ra[s] = in ? st[nl] : 0.0;
+          da[s] = in ? st[8 + nl] : 0.0;
+        }
+      }
+      lds_barrier();
+      double tu[4], fx[4], fy[4], fz[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tu[r] = fx[r] = fy[r] = fz[r] = 0.0;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        if (w + 4 * t >= NT) break;
+        f64x4_t x = {0.0, 0.0, 0.0, 0.0}, y = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          x = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[s], hreg[t][s], x, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f64_16x16x4f64(da[s], hreg[t][s], y, 0, 0, 0);
+        }
+        const int lm = 16 * (w + 4 * t) + li;
+        if (lm < NLM) {
+          const int l = lm_l(lm);
+          const double lf = (double)l, ll = lf * (lf + 1.0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int j = 4 * r + lg;  // pairs past the end or unseen: dropped below
+            const double* st = S.rec + min(g + j, cntc - 1) * ST;
+            const double2* yv = reinterpret_cast<const double2*>(Yb + j * 4 * NLM + 4 * lm);
+            const double2 ya = yv[0], yb = yv[1];
+            const double A = st[16 + l], Ax = A * x[r], ang = Ax * st[26];
+            tu[r] += (Ax * (ll * st[25]) + A * y[r] - ang * lf) * ya.x;
+            fx[r] += ang * ya.y;
+            fy[r] += ang * yb.x;
+            fz[r] += ang * yb.y;
+          }
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = 4 * r + lg;
+        const double* st = S.rec + min(g + j, cntc - 1) * ST;
+        const double tt = lanes_sum<16>(tu[r]);
+        const double vx = lanes_sum<16>(fx[r]) + tt * st[27], vy = lanes_sum<16>(fy[r]) + tt * st[28],
+                     vz = lanes_sum<16>(fz[r]) + tt * st[29];
+        if (li == 0) {
+          double* o = part + (w * HG + j) * 3;
+          o[0] = vx;
+          o[1] = vy;
+          o[2] = vz;
+        }
+      }
+      lds_barrier();
+      if (mine && S.rec[(g + oj) * ST + 30] != 0.0) {
+        const double* o = part + 3 * oj + ok;
+        const double f = ((o[0] + o[3 * HG]) + o[6 * HG]) + o[9 * HG];
+        fglob[3 * gi + ok] += f;
+        self += f;
+      }
+    }
+  }
+  // the self entry: minus the sum of the others, over the sixteen pairs' threads in order
+  lds_barrier();
+  if (oj < HG) part[tid] = self;
+  lds_barrier();
+  if (tid < 3) {
+    double v = 0.0;
+    for (int j = 0; j < HG; ++j) v += part[3 * j + tid];
+    fglob[3 * a.pr_gidx[b0] + tid] -= v;
   }
 }
 
@@ -1275,6 +1503,32 @@ static int check_lds(size_t bytes) {
   return TGX_OK;
 }
 
+// Blocks that the kernels for l_max = 8 take: at most two species of at most eight
+// radial functions, the sizes their degree sets, pair records and 16-row tiles are
+// laid out for. At 16,001 atoms 1.09 ms for descriptors and adjoint together, 2.81
+// for the wavefront-per-site kernels, which take every other block.
+static bool l_kernels(const SoapParams& P) {
+  bool ok = P.L == 8 && P.N <= 16 && P.n_species <= 2;
+  for (int s = 0; s < P.n_species; ++s) ok = ok && P.sp[s].nb <= 8;
+  return ok;
+}
+
+// FP64 descriptors of the block's (or the listed) sites.
+static int desc_f64(tgx_ctx* ctx, tgx_model_t* m, const int* d_sites, int n_rows, double* q_out, double* pn_out) {
+  const SoapParams& P = m->P;
+  if (!l_kernels(P)) return tgx_desc_wave(ctx, m, true, d_sites, n_rows, q_out, pn_out);
+  if (n_rows == 0) return TGX_OK;
+  SiteArgs a = site_args(m);
+  const char* name = d_sites ? "soap_desc_list_f64" : "soap_desc_f64";
+  if (P.D <= 2 * WG)
+    TGX_LAUNCH(ctx, name, (k_desc_l<8, 2>), dim3(n_rows), dim3(WG), DerL<8>::LDS_DESC, P, a, n_rows, q_out, pn_out,
+               d_sites);
+  else
+    TGX_LAUNCH(ctx, name, (k_desc_l<8, 5>), dim3(n_rows), dim3(WG), DerL<8>::LDS_DESC, P, a, n_rows, q_out, pn_out,
+               d_sites);
+  return TGX_OK;
+}
+
 int tgx_soap_descriptors(tgx_ctx* ctx, tgx_model_t* m, int path, bool with_der) {
   m->der_whole = false;  // set again by a whole-block FP64 plain evaluation
   const int ns = m->n_sites_b;
@@ -1295,16 +1549,12 @@ int tgx_soap_descriptors(tgx_ctx* ctx, tgx_model_t* m, int path, bool with_der) 
       const SoapParams& P = m->P;
       const int NL = P.N * (P.L + 1);
       const int j_need = (3 * P.D + WG - 1) / WG;
-      bool small_blocks = P.n_species <= 2;
-      for (int sp = 0; sp < P.n_species; ++sp) small_blocks = small_blocks && P.sp[sp].nb <= 8 && P.sp[sp].nq <= 64;
-      const int jd = (P.D + WG - 1) / WG;  // components per thread of k_soap_der_l
-      if (P.L == 8 && P.N <= 16 && small_blocks) {
+      if (l_kernels(P)) {
         constexpr size_t lds = DerL<8>::LDS;
-        TGX_TRY(check_lds(lds));
 #define TGX_SOAP_DER(J)                                                                                     \
   TGX_LAUNCH(ctx, "soap_site_der_f64", (k_soap_der_l<8, J>), dim3(ns), dim3(WG), lds, m->P, a, ns, \
              qout.as<double>(), m->pnorm.as<double>(), dout.as<double>())
-        if (jd <= 2) TGX_SOAP_DER(2);
+        if (P.D <= 2 * WG) TGX_SOAP_DER(2);
         else TGX_SOAP_DER(5);
 #undef TGX_SOAP_DER
       } else if (j_need <= 16 && NL <= 255 && P.D < 4096) {
@@ -1336,7 +1586,7 @@ int tgx_soap_descriptors(tgx_ctx* ctx, tgx_model_t* m, int path, bool with_der) 
 #undef TGX_SOAP_DER
       }
     } else {
-      TGX_TRY(tgx_desc_wave(ctx, m, true, nullptr, ns, qout.p, m->pnorm.p));
+      TGX_TRY(desc_f64(ctx, m, nullptr, ns, qout.as<double>(), m->pnorm.as<double>()));
     }
     if (m->compress) TGX_TRY(tgx_compress_descriptors(ctx, m, with_der));
   } else {
@@ -1357,6 +1607,22 @@ int tgx_adjoint_pair_forces(tgx_ctx* ctx, tgx_model_t* m, int path) {
   TGX_REQUIRE(!m->compress || fp64, "compressed SOAP blocks run on the FP64 paths only");
   if (m->compress) TGX_TRY(tgx_compress_gradient(ctx, m));
   if (!fp64 && m->P.N <= 16) return tgx_adjoint_f32(ctx, m);
+  const SoapParams& P = m->P;
+  if (fp64 && l_kernels(P)) {
+    const int ns = m->n_sites_b;
+    if (ns == 0) return TGX_OK;
+    SiteArgs a = site_args(m);
+    // a compressed block contracts the full-size gradient with the full descriptors
+    const double* q = (m->compress ? m->qf64 : m->q64).as<double>();
+    const double* g = (m->compress ? m->qssf64 : m->qss64).as<double>();
+    if (P.D <= 2 * WG)
+      TGX_LAUNCH(ctx, "soap_adjoint_f64", (k_adjoint_l<8, 2>), dim3(ns), dim3(WG), DerL<8>::LDS_ADJ, P, a, ns, q,
+                 m->pnorm.as<double>(), g, ctx->fglob.as<double>());
+    else
+      TGX_LAUNCH(ctx, "soap_adjoint_f64", (k_adjoint_l<8, 5>), dim3(ns), dim3(WG), DerL<8>::LDS_ADJ, P, a, ns, q,
+                 m->pnorm.as<double>(), g, ctx->fglob.as<double>());
+    return TGX_OK;
+  }
   return tgx_adjoint_wave(ctx, m, fp64);
 }
 
@@ -1413,5 +1679,5 @@ int tgx_local_property_finish(tgx_ctx* ctx, tgx_model_t* m, bool with_der, doubl
 // holding site d_sites[r] (used to re-evaluate gated sites with the GAP).
 int tgx_soap_descriptors_sites(tgx_ctx* ctx, tgx_model_t* m, const int* d_sites, int n_list, double* q_out,
                                double* pnorm_out) {
-  return tgx_desc_wave(ctx, m, true, d_sites, n_list, q_out, pnorm_out);
+  return desc_f64(ctx, m, d_sites, n_list, q_out, pnorm_out);
 }
