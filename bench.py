@@ -129,11 +129,11 @@ def roofline_entries(stats, n_atoms, blocks, n_pairs, members=1, hidden=256):
 # bench kernel label -> device kernel name in the rocprofv3 counter summary
 # (the Qss product and the network's first backward layer share one kernel
 # symbol, so the summary's average over both is not either one's traffic)
-KERNEL_SYMBOL = {"soap_adjoint_f32": "k_site_adjoint_mfma", "soap_desc_f32": "k_site_desc",
+KERNEL_SYMBOL = {"soap_adjoint_f32": "k_site_adjoint_mfma", "soap_desc_f32": "k_site_desc<8>",
                  "soap_pair_basis": "k_pair_basis8", "nbr_fill": "k_cell_neigh<1>",
                  "soap_site_der_f64": "k_soap_der_l<8, 5>", "plain_force": "k_plain_force",
-                 "gemm_kernel_f64": "k_gemm_f64<1, true>", "gemm_qss_f64": "k_gemm_f64<0, true>",
-                 "gemm_kernel_bf16": "k_gemm_bf16_pf<1, bool _Accum, bool, E, 128, 3, 3>",
+                 "gemm_kernel_f64": "k_gemm_f64<1, true, 4, 4, 2>", "gemm_qss_f64": "k_gemm_f64<0, true, 4, 4, 2>",
+                 "gemm_kernel_bf16": "k_gemm_bf16_pf<1, bool _Accum, bool, E, 256, 3, 2>",
                  "mlp_l1": "k_gemm_bf16<2, bool _Accum, bool, E>",
                  "mlp_l2": "k_gemm_bf16_pf<4, bool _Accum, bool, E, 128, 3, 3>",
                  "mlp_back2": "k_gemm_bf16<3, bool _Accum, bool, E>"}
@@ -400,7 +400,7 @@ def silicon_crystal(cells, perturb=0.05, seed=4):
 
 
 FAMILY_KERNELS = {"distance_2b": ["pair_model"], "core_pot": ["pair_model"],
-                  "angle_3b": ["angle_3b", "angle_3b_large", "force_gather", "virial"]}
+                  "angle_3b": ["angle_3b", "angle_3b_large", "force_gather", "pair_virial"]}
 
 
 def family_bench(args):

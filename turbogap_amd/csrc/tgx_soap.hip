@@ -1067,10 +1067,12 @@ __device__ __forceinline__ void l_harmonics(const LSite<LL>& S, int g, int cnt, 
 //   * Each thread writes whole components d = tid + WG j (its three Cartesian
 //     entries) of every pair of the group and keeps the self-pair sums of its
 //     components in registers. J >= D / WG.
-// Bound by the 35 GB it writes at 65,536 atoms of two species (1.2 million pairs of
-// 1,224 components): 15.0 -> 9.45 ms, 3.7 TB/s; at 4,096 atoms 1.15 -> 0.61 ms,
-// at 216 atoms of one species, a workgroup a CU, 110 -> 50 us. Stores staged through
-// LDS to be contiguous (10.5 -> 11.6 ms) and non-temporal stores (10.6) lost.
+// Bound by the 42 GB it writes at 65,536 atoms of two species (1.42 million pairs of
+// 1,224 components, two blocks): 15.0 -> 9.3 ms, 4.5 TB/s where a plain fill reaches
+// 6.3; at 4,096 atoms 1.15 -> 0.61 ms, at 216 atoms of one species, a workgroup a CU,
+// 110 -> 50 us. Stores staged through LDS to be contiguous (10.5 -> 11.6 ms) and
+// non-temporal stores (10.6) lost, as did the component codes read before the
+// expansion (0.61 -> 0.64 ms at 4,096 atoms).
 template <int LL, int J>
 __global__ __launch_bounds__(WG, 2) void k_soap_der_l(SoapParams P, SiteArgs a, int n_sites,
                                                       double* __restrict__ q_out, double* __restrict__ pnorm_out,
