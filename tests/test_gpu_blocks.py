@@ -41,3 +41,46 @@ def test_many_blocks_match_two(n):
     assert np.abs(f1 - f0).max() <= 1e-12 * np.abs(f0).max()
     assert abs(E1 - E0) <= 1e-12 * np.abs(e0).sum()
     assert np.abs(W1 - W0).max() <= 1e-12 * n * np.abs(f0).max() * 3.7
+
+
+# central_species counts within the block's own species list: entry 1 of (A, B) and entry 2 of (B, A) are
+# the same atoms
+@pytest.mark.parametrize("path", ["mixed", "fp64_plain", "fp64_adjoint", "surrogate"])
+def test_blocks_on_the_same_atoms_under_another_species_order(path):
+    from turbogap_amd import Context
+    from turbogap_amd import surrogate as SG
+    rng = np.random.default_rng(3)
+    sysm = S.binary_system(1500, seed=9)
+    blocks = []
+    for k, (types, central) in enumerate([((S.SPECIES_A, S.SPECIES_B), 1), ((S.SPECIES_B, S.SPECIES_A), 2)]):
+        h = S.soap_hypers(list(types), central_species=central)
+        Qs = rng.random((30, h.dim))
+        blocks.append((k, h, Qs / np.linalg.norm(Qs, axis=1, keepdims=True), rng.normal(scale=1e-2, size=30)))
+
+    def step(chosen, streams):
+        with Context(0) as ctx:
+            ctx.set_system(sysm.positions, sysm.species, sysm.box)
+            ctx.build_neighbors_list(3.7, fetch=False)
+            ctx.set_block_streams(streams)
+            for k, h, Qs, al in chosen:
+                mid = ctx.soap_model(h, Qs, al)
+                if path == "surrogate":
+                    for i in range(2):
+                        net = SG.MLP(ctx, h.dim, 128, 128, seed=11 + 5 * k + i)
+                        net.set_normalization(-0.5, 0.03 + 0.01 * i)
+                        net.install(mid, i)
+            if path == "surrogate":
+                SG.set_gate(ctx, 2, 1e9)
+            E, W = ctx.compute(path)
+            return (E, W) + ctx.results()
+
+    (Ea, Wa, ea, fa), (Eb, Wb, eb, fb) = [step([b], 1) for b in blocks]
+    on_a = sysm.species == S.SPECIES_A
+    assert np.all(ea[on_a] != 0.0) and np.all(eb[on_a] != 0.0) and not ea[~on_a].any() and not eb[~on_a].any()
+    for streams in (0, 1, 2):
+        E, W, e, f = step(blocks, streams)
+        # the blocks' energies and pair forces are the same numbers, added in FP64
+        assert np.array_equal(e, ea + eb), streams
+        assert np.abs(f - (fa + fb)).max() <= 1e-12 * (np.abs(fa).max() + np.abs(fb).max())
+        assert abs(E - (Ea + Eb)) <= 1e-12 * (np.abs(ea).sum() + np.abs(eb).sum())
+        assert np.abs(W - (Wa + Wb)).max() <= 1e-12 * sysm.n * 3.7 * (np.abs(fa).max() + np.abs(fb).max())

@@ -933,6 +933,13 @@ extern "C" int tgx_get_soap_energy_and_forces(tgx_ctx* ctx, int n_sites, int n_s
 int tgx_surrogate_eval(tgx_ctx* ctx, tgx_model_t* m, bool selected, int* gate_host);
 int tgx_surrogate_finish(tgx_ctx* ctx, tgx_model_t* m, int n_gated);
 
+// Whether an atom can be a centre of both blocks. central_species counts within
+// the block's own species list, so it is the species codes that are compared.
+static bool share_centres(const tgx_model_t* a, const tgx_model_t* b) {
+  if (a->central_species == 0 || b->central_species == 0) return true;  // every atom
+  return a->species_types[a->central_species - 1] == b->species_types[b->central_species - 1];
+}
+
 extern "C" int tgx_compute(tgx_ctx* ctx, int path, double* energy, double* virial) {
   TGX_CTX_CHECK(ctx);
   TGX_REQUIRE(path >= TGX_PATH_FP64_PLAIN && path <= TGX_PATH_SURROGATE, "tgx_compute: unknown path %d", path);
@@ -952,12 +959,9 @@ extern "C" int tgx_compute(tgx_ctx* ctx, int path, double* energy, double* viria
   // 3.86 ms per step in turn against 4.14 ms concurrent; the surrogate and
   // FP64 adjoint paths gain 1-2% from the overlap).
   bool disjoint = true;  // no atom is a centre of two blocks
-  for (int a = 0; a < nm && nm > 1; ++a) {
-    const int ca = ctx->models[a]->central_species;
-    if (ca == 0) disjoint = false;
+  for (int a = 0; a < nm; ++a)
     for (int b = 0; b < a; ++b)
-      if (ctx->models[b]->central_species == ca) disjoint = false;
-  }
+      if (share_centres(ctx->models[a], ctx->models[b])) disjoint = false;
   const bool concurrent = nm > 1 && disjoint && ctx->block_streams > 0 && !ctx->profiling &&
                           (path != TGX_PATH_MIXED || ctx->block_streams == 2);
   hipStream_t main_stream = ctx->stream;
@@ -979,7 +983,7 @@ extern "C" int tgx_compute(tgx_ctx* ctx, int path, double* energy, double* viria
       if (!m->stream) TGX_CHECK_HIP(hipStreamCreate(&m->stream));
       if (!m->done) TGX_CHECK_HIP(hipEventCreateWithFlags(&m->done, hipEventDisableTiming));
     }
-  std::vector<tgx_model_t*> whole;  // blocks whose energies are still to be added to the atoms'
+  std::vector<tgx_model_t*> whole;  // disjoint blocks whose energies are still to be added to the atoms', all at once
   auto block_stream = [&](tgx_model_t* m) { return concurrent ? m->stream : main_stream; };
   // Every block's selection counts in one pass and one wait, after which the
   // blocks' streams start without an event of their own. A small system's step
@@ -1019,6 +1023,8 @@ extern "C" int tgx_compute(tgx_ctx* ctx, int path, double* energy, double* viria
       ctx->gate_gated += ng;
       ctx->max_spread = std::max(ctx->max_spread, (double)sp);
       TGX_TRY(tgx_surrogate_finish(ctx, m, ng));
+      if (disjoint) whole.push_back(m);
+      else TGX_TRY(tgx_energy_scatter(ctx, m));
       if (concurrent) TGX_CHECK_HIP(hipEventRecord(m->done, m->stream));
     }
     ctx->gated_fraction = ctx->gate_sites > 0 ? (double)ctx->gate_gated / (double)ctx->gate_sites : 0.0;
@@ -1033,7 +1039,8 @@ extern "C" int tgx_compute(tgx_ctx* ctx, int path, double* energy, double* viria
       } else {
         TGX_TRY(tgx_block_select_fill(ctx, m));
         TGX_TRY(run_selected_block(ctx, m, path, true));
-        whole.push_back(m);
+        if (disjoint) whole.push_back(m);
+        else TGX_TRY(tgx_energy_scatter(ctx, m));  // onto shared centres in block order
       }
       if (concurrent) TGX_CHECK_HIP(hipEventRecord(m->done, m->stream));
     }
@@ -1042,10 +1049,7 @@ extern "C" int tgx_compute(tgx_ctx* ctx, int path, double* energy, double* viria
   if (concurrent)
     for (auto* m : ctx->models) TGX_CHECK_HIP(hipStreamWaitEvent(main_stream, m->done, 0));
   restore.blocks = false;  // the context stream now orders everything after the blocks
-  if (path == TGX_PATH_SURROGATE) whole = ctx->models;
-  if (disjoint) TGX_TRY(tgx_energy_scatter_blocks(ctx, whole.data(), (int)whole.size()));
-  else
-    for (auto* m : whole) TGX_TRY(tgx_energy_scatter(ctx, m));
+  TGX_TRY(tgx_energy_scatter_blocks(ctx, whole.data(), (int)whole.size()));
   TGX_TRY(tgx_gather_forces(ctx, energy, virial));
   return TGX_OK;
 }
