@@ -244,6 +244,13 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt(0x3F70 | N);  // vmcnt(N); expcnt and lgkmcnt not waited on
 }
 
+// The same, and every LDS read of this wavefront is done.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt_lds() {
+  static_assert(N >= 0 && N < 16, "vmcnt immediate");
+  __builtin_amdgcn_s_waitcnt(0x0070 | N);
+}
+
 // FP64 NT GEMM fed by direct global-to-LDS loads: workgroup tile (32 TI) x
 // (32 TJ), four wavefronts of (16 TI) x (16 TJ), BK = 16 in a two-slot ring. A
 // stage is 32 (TI + TJ) rows of 128 bytes (the A rows, then the B rows); the
@@ -329,7 +336,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm_f64(int K, const double* __re
     f64_mfma<TI, TJ>(acc, a0, b0);
     __builtin_amdgcn_sched_barrier(0);
     // this wavefront's part of stage st + 1 has landed and its reads of stage st are done
-    __builtin_amdgcn_s_waitcnt(0x0070);
+    wait_vmcnt_lds<0>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     issue(min(st + 2, n_stages - 1), slot);  // an in-bounds repeat past the end
@@ -605,7 +612,9 @@ __device__ __forceinline__ void pf_stage(f32x4 (&acc)[TI][4], const bf16x8 (&a)[
                                          int w) {
   pf_mfma<EPI, TI, 0, TI / 2>(acc, a, b);
   __builtin_amdgcn_sched_barrier(0);
-  wait_vmcnt<(NS - 2) * P>();
+  // this wavefront's part of the next stage has landed, and its reads of this one are done: the
+  // products above need only the first half of a
+  wait_vmcnt_lds<(NS - 2) * P>();
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
   // every wavefront has read this stage's slot: it takes stage st + NS (an in-bounds repeat past the end)
