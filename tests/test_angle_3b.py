@@ -200,3 +200,21 @@ def test_gpu_angle_3b_large_centres(ctx):
     nl = O.build_neighbors_list(sysm.positions, sysm.species, sysm.box, kw["rcut"])
     assert nl["n_neigh"][sp == 3].min() - 4 > 128
     _gpu_vs_oracle(ctx, kw, sysm)
+
+
+@pytest.mark.gpu
+def test_gpu_angle_3b_refused_centre_leaves_outputs(ctx):
+    """A centre with more than 1,024 selected neighbours is an error that leaves every output as it was."""
+    from turbogap_amd import lib as L
+    n = 2500
+    pos = np.random.default_rng(8).uniform(0.0, 10.0, (n, 3))
+    sp = np.full(n, S.CARBON, np.int32)
+    sp[0] = SI
+    ctx.set_system(pos, sp, S.cubic_box(10.0))
+    nl = ctx.build_neighbors_list(4.9)
+    assert nl["n_neigh"][0] > 1025
+    mid = ctx.angle_3b_model(**synthetic_3b("pol", sc=SI, s1=S.CARBON, s2=S.CARBON, rcut=4.9, n=4))
+    e, f, w = np.full(n, 7.0), np.full((n, 3), 7.0), np.full(9, 7.0)
+    assert L.load().tgx_pair_energy_and_forces(ctx.h, mid, L.dptr(e), L.dptr(f), L.dptr(w)) != 0
+    assert b"1024" in L.load().tgx_last_error()
+    assert (e == 7.0).all() and (f == 7.0).all() and (w == 7.0).all()

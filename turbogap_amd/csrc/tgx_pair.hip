@@ -600,16 +600,20 @@ static int angle_3b_run(tgx_ctx* ctx, const tgx_pair_model* pm, double* energies
   TGX_TRY(pm->m.ktype == 0 ? angle_3b_launch<0>(ctx, pm, e, fglob, big) : angle_3b_launch<1>(ctx, pm, e, fglob, big));
   TGX_CHECK_HIP(hipMemcpyAsync(h, big, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   // the gather's wait also brings the counters; it is repeated in the rare case
-  // that large centres were left over
-  TGX_TRY(tgx_gather_pair_forces(ctx, fglob, F, virial));
+  // that large centres were left over, which may still be refused: the caller's
+  // arrays are written at the end
+  double w[9];
+  double* wp = virial ? w : nullptr;
+  TGX_TRY(tgx_gather_pair_forces(ctx, fglob, F, wp));
   if (h[0] > 0) {
     TGX_TRY(pm->m.ktype == 0 ? angle_3b_launch_large<0>(ctx, pm, h[0], e, fglob, big)
                              : angle_3b_launch_large<1>(ctx, pm, h[0], e, fglob, big));
     TGX_CHECK_HIP(hipMemcpyAsync(h, big, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     TGX_REQUIRE(!h[1], "angle_3b: a centre has more than 1024 neighbours of the selected species inside rcut");
-    TGX_TRY(tgx_gather_pair_forces(ctx, fglob, F, virial));
+    TGX_TRY(tgx_gather_pair_forces(ctx, fglob, F, wp));
   }
+  if (virial) std::memcpy(virial, w, sizeof(w));
   if (energies) TGX_CHECK_HIP(hipMemcpyAsync(energies, e, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
   if (forces) TGX_CHECK_HIP(hipMemcpyAsync(forces, F, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, ctx->stream));
   TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
