@@ -218,3 +218,17 @@ def test_gpu_angle_3b_refused_centre_leaves_outputs(ctx):
     assert L.load().tgx_pair_energy_and_forces(ctx.h, mid, L.dptr(e), L.dptr(f), L.dptr(w)) != 0
     assert b"1024" in L.load().tgx_last_error()
     assert (e == 7.0).all() and (f == 7.0).all() and (w == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernel_type", ["exp", "pol"])
+def test_gpu_angle_3b_point_out_of_reach(ctx, kernel_type):
+    """A sparse point so far away that its squared distance overflows adds nothing."""
+    sysm, kw = silicon_crystal(cells=2), synthetic_3b(kernel_type)
+    far = dict(kw, Qs=np.vstack([kw["Qs"], [1e200, 0.0, 0.0]]), alphas=np.append(kw["alphas"], 1.0),
+               cutoff=np.append(kw["cutoff"], 1.0))
+    ctx.set_system(sysm.positions, sysm.species, sysm.box)
+    ctx.build_neighbors_list(kw["rcut"], fetch=False)
+    near = ctx.pair_energy_and_forces(ctx.angle_3b_model(**kw))
+    for a, b in zip(ctx.pair_energy_and_forces(ctx.angle_3b_model(**far)), near):
+        assert np.array_equal(a, b)

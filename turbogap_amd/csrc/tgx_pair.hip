@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void k_virial_sum(int n, const double* __restr
 // sqrt(x), x >= 0: coupled Newton (Goldschmidt) steps on v_rsq_f64, whose
 // relative error is below 2^-20, and a last residual correction; within one ulp.
 // x is kept away from zero, where the reciprocal root is infinite: a squared
-// distance below 1e-200 is zero to every use of its root.
+// distance below 1e-200 is zero to every use of its root. NaN for an infinite x.
 __device__ __forceinline__ double sqrt_pos(double x) {
   x = fmax(x, 1e-200);
   const double y = __builtin_amdgcn_rsq(x);
@@ -307,10 +307,11 @@ __global__ __launch_bounds__(64) void k_angle_3b(const int* __restrict__ centres
             kd = Q.w * exp(-0.5 * r2);
             K += kd;
           } else {
-            // (1 - r)^4 (4 r + 1) and 20 (1 - r)^3, both zero from r = 1 on
-            const double r = sqrt_pos(r2), om = fmax(1.0 - r, 0.0);
+            // (1 - r)^4 (4 r + 1) and 20 (1 - r)^3, both zero from r = 1 on and where r2 overflows
+            // (its root is NaN, and fmax takes the zero; so r itself is not used again)
+            const double om = fmax(1.0 - sqrt_pos(r2), 0.0);
             kd = Q.w * (om * om) * om;
-            K += kd * om * (4.0 * r + 1.0);
+            K += kd * om * (5.0 - 4.0 * om);
           }
           H1 += kd * d1;
           H2 += kd * d2;
