@@ -1,5 +1,6 @@
 """Weight gradients of the training pass at the edges of its tiles: one 64-row tile pair, widths and
-descriptor sizes that leave remainders of the padding, batches that are no multiple of 256."""
+descriptor sizes that leave remainders of the padding, batches that are no multiple of 256, and the
+widest rows that the loss keeps in LDS (10,240 components) and the narrowest that it does not."""
 import numpy as np
 import pytest
 
@@ -16,7 +17,8 @@ def ctx():
         yield c
 
 
-@pytest.mark.parametrize("D,Hd,B", [(40, 128, 128), (130, 256, 1152), (324, 128, 384), (1224, 384, 256)])
+@pytest.mark.parametrize("D,Hd,B", [(40, 128, 128), (130, 256, 1152), (324, 128, 384), (1224, 384, 256),
+                                    (10240, 128, 128), (10241, 128, 128)])
 def test_weight_gradients(ctx, D, Hd, B):
     rng = np.random.default_rng(D + B)
     net = SG.MLP(ctx, D, Hd, B + 128, seed=3)

@@ -250,15 +250,16 @@ __global__ void k_esum(int rows, int np, const float* __restrict__ epart, const 
 
 // Per row: residuals of the normalised targets, u = P(g - g_n), loss partials,
 // dE = 2 w_E (E - E_n)/B. One wavefront per row, the row's g - g_n in LDS between
-// the two passes. Row r of q and g_ref is row idx[r] of their arrays (idx null: r).
+// the two passes (staged; formed again in rows too wide for that). Row r of q and
+// g_ref is row idx[r] of their arrays (idx null: r).
 // The energies come from E, or, E null, from the second layer's partials.
 __global__ __launch_bounds__(256) void k_loss(int rows, int Dp, const float* __restrict__ E,
                                               const float* __restrict__ epart, int np, const float* __restrict__ b3,
                                               const double* __restrict__ e_ref, const float* __restrict__ g,
                                               const float* __restrict__ g_ref, const float* __restrict__ q,
                                               const int* __restrict__ idx, double shift, double inv_scale, float w_e,
-                                              float* __restrict__ u, __bf16* __restrict__ ub, float* __restrict__ dE,
-                                              double* __restrict__ le, double* __restrict__ lg) {
+                                              bool staged, float* __restrict__ u, __bf16* __restrict__ ub,
+                                              float* __restrict__ dE, double* __restrict__ le, double* __restrict__ lg) {
   extern __shared__ float sdiff[];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int row = blockIdx.x * 4 + w;
@@ -272,8 +273,10 @@ __global__ __launch_bounds__(256) void k_loss(int rows, int Dp, const float* __r
   for (int j = lane; j < Dp / 2; j += 64) {
     const float2 a = gr[j], t = gf[j], x = qr[j];
     const float d0 = a.x - (float)(t.x * inv_scale), d1 = a.y - (float)(t.y * inv_scale);
-    diff[2 * j] = d0;
-    diff[2 * j + 1] = d1;
+    if (staged) {
+      diff[2 * j] = d0;
+      diff[2 * j + 1] = d1;
+    }
     qd += x.x * d0;
     qd += x.y * d1;
   }
@@ -282,8 +285,16 @@ __global__ __launch_bounds__(256) void k_loss(int rows, int Dp, const float* __r
   for (int j = lane; j < Dp / 2; j += 64) {
     const float2 x = qr[j];
     float2 v;
-    v.x = diff[2 * j] - x.x * qd;
-    v.y = diff[2 * j + 1] - x.y * qd;
+    if (staged) {
+      v.x = diff[2 * j];
+      v.y = diff[2 * j + 1];
+    } else {
+      const float2 a = gr[j], t = gf[j];
+      v.x = a.x - (float)(t.x * inv_scale);
+      v.y = a.y - (float)(t.y * inv_scale);
+    }
+    v.x -= x.x * qd;
+    v.y -= x.y * qd;
     reinterpret_cast<float2*>(u + (size_t)row * Dp)[j] = v;
     __bf16* o = ub + (size_t)row * Dp + 2 * j;
     o[0] = (__bf16)v.x;
@@ -774,24 +785,32 @@ static int mlp_forward(tgx_mlp* m, int B, const __bf16* xb, bool train, float* E
 
 static int mlp_backward_dirs(tgx_mlp* m, int B, float cG, const float* q, const int* idx);
 
+// k_loss for B rows of the batch: E, or null for the second layer's partials.
+static int mlp_loss(tgx_mlp* m, int B, const float* E, const float* q, const float* g, const int* idx, float w_e) {
+  tgx_ctx* ctx = m->ctx;
+  const size_t lds = sizeof(float) * 4 * (size_t)m->Dp;
+  const bool staged = lds <= 160 * 1024;  // a CU's LDS: descriptors of up to 10,240 components
+  double* le = m->lossb.as<double>();
+  TGX_LAUNCH(ctx, "mlp_loss", k_loss, dim3((B + 3) / 4), dim3(256), staged ? lds : 0, B, m->Dp, E,
+             (const float*)m->epart.as<float>(), m->H / 32, m->theta.as<float>() + m->ob3, m->be.as<double>(),
+             m->G.as<float>(), g, q, idx, m->shift, 1.0 / m->scale, w_e, staged, m->u.as<float>(), m->ub.as<__bf16>(),
+             m->dE.as<float>(), le, le + B);
+  return TGX_OK;
+}
+
 // Loss and weight gradients of the batch in bqb and be, with the FP32 descriptors
 // and target gradients in rows idx of q and g (idx null: the first B rows).
 static int mlp_backward(tgx_mlp* m, int B, const float* q, const float* g, const int* idx, float w_e, float w_g,
                         double* loss_e, double* loss_g) {
   tgx_ctx* ctx = m->ctx;
-  const int Dp = m->Dp;
   TGX_TRY(mlp_forward(m, B, m->bqb.as<__bf16>(), true, nullptr, m->G.as<float>(), 1.0));
-  double* le = m->lossb.as<double>();
-  double* lg = le + B;
-  TGX_LAUNCH(ctx, "mlp_loss", k_loss, dim3((B + 3) / 4), dim3(256), sizeof(float) * 4 * Dp, B, Dp, (const float*)nullptr,
-             (const float*)m->epart.as<float>(), m->H / 32, m->theta.as<float>() + m->ob3, m->be.as<double>(),
-             m->G.as<float>(), g, q, idx, m->shift, 1.0 / m->scale, w_e, m->u.as<float>(), m->ub.as<__bf16>(),
-             m->dE.as<float>(), le, lg);
+  TGX_TRY(mlp_loss(m, B, nullptr, q, g, idx, w_e));
   TGX_TRY(mlp_backward_dirs(m, B, 2.0f * w_g / (float)B, q, idx));
   if (loss_e || loss_g) {
     double se = 0.0, sg = 0.0;
+    const double* le = m->lossb.as<double>();
     TGX_TRY(tgx_device_sum(ctx, le, B, &se));
-    TGX_TRY(tgx_device_sum(ctx, lg, B, &sg));
+    TGX_TRY(tgx_device_sum(ctx, le + B, B, &sg));
     if (loss_e) *loss_e = se / B;
     if (loss_g) *loss_g = sg / B;
   }
@@ -993,11 +1012,8 @@ extern "C" int tgx_mlp_evaluate(tgx_mlp* m, int begin, int end, double* e_mae, d
     TGX_LAUNCH(ctx, "mlp_gather", k_gather_rows, dim3(B), dim3(256), 0, B, m->Dp, m->idx.as<int>(), m->dq.as<float>(),
                m->de.as<double>(), m->bqb.as<__bf16>(), m->be.as<double>());
     TGX_TRY(mlp_forward(m, B, m->bqb.as<__bf16>(), false, m->E.as<float>(), m->G.as<float>(), 1.0));
-    double* le = m->lossb.as<double>();
-    TGX_LAUNCH(ctx, "mlp_loss", k_loss, dim3((B + 3) / 4), dim3(256), sizeof(float) * 4 * m->Dp, B, m->Dp,
-               (const float*)m->E.as<float>(), (const float*)nullptr, 0, (const float*)nullptr, m->be.as<double>(),
-               m->G.as<float>(), m->dg.as<float>(), m->dq.as<float>(), m->idx.as<int>(), m->shift, 1.0 / m->scale, 1.0f,
-               m->u.as<float>(), m->ub.as<__bf16>(), m->dE.as<float>(), le, le + B);
+    TGX_TRY(mlp_loss(m, B, m->E.as<float>(), m->dq.as<float>(), m->dg.as<float>(), m->idx.as<int>(), 1.0f));
+    const double* le = m->lossb.as<double>();
     TGX_CHECK_HIP(hipMemcpyAsync(er.data(), le, sizeof(double) * B, hipMemcpyDeviceToHost, ctx->stream));
     TGX_CHECK_HIP(hipMemcpyAsync(lg.data(), le + B, sizeof(double) * B, hipMemcpyDeviceToHost, ctx->stream));
     TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
