@@ -84,3 +84,32 @@ def test_blocks_on_the_same_atoms_under_another_species_order(path):
         assert np.abs(f - (fa + fb)).max() <= 1e-12 * (np.abs(fa).max() + np.abs(fb).max())
         assert abs(E - (Ea + Eb)) <= 1e-12 * (np.abs(ea).sum() + np.abs(eb).sum())
         assert np.abs(W - (Wa + Wb)).max() <= 1e-12 * sysm.n * 3.7 * (np.abs(fa).max() + np.abs(fb).max())
+
+
+# results pass through pinned memory of up to 2,048 atoms that the context always holds, of a size of their
+# own above, grown where a system is larger than any before it, and by a copy above 16,384 atoms
+def test_results_of_systems_of_changing_size():
+    from turbogap_amd import Context
+    rng = np.random.default_rng(1)
+    hyp = S.soap_binary()
+    Qs = rng.random((5, hyp[0].dim))
+    Qs /= np.linalg.norm(Qs, axis=1, keepdims=True)
+    al = rng.normal(scale=1e-2, size=5)
+
+    def step(ctx, sysm):
+        ctx.set_system(sysm.positions, sysm.species, sysm.box)
+        ctx.build_neighbors_list(3.7, fetch=False)
+        E, _ = ctx.compute("fp64_adjoint")
+        return (E,) + ctx.results() + ctx.get_gap_soap("fp64_adjoint")[:2]
+
+    with Context(0) as one:
+        one.soap_backend_begin(one.soap_model(hyp[0], Qs, al))
+        for n in (300, 2048, 2049, 40, 2500, 9000, 16384, 16385, 700):
+            sysm = S.binary_system(n, seed=n)
+            got = step(one, sysm)
+            with Context(0) as fresh:
+                fresh.soap_backend_begin(fresh.soap_model(hyp[0], Qs, al))
+                want = step(fresh, sysm)
+            # the same calls on the same numbers: whether the context is new does not matter
+            assert all(np.array_equal(a, b) for a, b in zip(got, want)), n
+            assert abs(got[0] - got[1].sum()) <= 1e-12 * np.abs(got[1]).sum()

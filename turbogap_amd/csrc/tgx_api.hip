@@ -145,7 +145,6 @@ static void free_model(tgx_model_t* m) {
                   &m->cp_row, &m->cp_col, &m->cp_el, &m->cpt_col, &m->cpt_row, &m->cpt_el, &m->qf64, &m->qssf64,
                   &m->derf, &m->cnorm};
   for (dbuf* b : bufs) b->release();
-  if (m->sel_host) (void)hipHostFree(m->sel_host);
   if (m->done) (void)hipEventDestroy(m->done);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
@@ -167,11 +166,8 @@ extern "C" int tgx_finalize(tgx_ctx* ctx) {
                   &ctx->pos_prev, &ctx->gate_mask, &ctx->cell_pos, &ctx->nbr_hits, &ctx->md_disp, &ctx->md_flag,
                   &ctx->md_fix, &ctx->md_gd0, &ctx->md_cm};
   for (dbuf* b : bufs) b->release();
-  if (ctx->gate_host) (void)hipHostFree(ctx->gate_host);
-  if (ctx->md_flag_host) (void)hipHostFree(ctx->md_flag_host);
-  if (ctx->red_host) (void)hipHostFree(ctx->red_host);
-  if (ctx->pairs_host) (void)hipHostFree(ctx->pairs_host);
-  if (ctx->fold_host) (void)hipHostFree(ctx->fold_host);
+  if (ctx->fold_own) (void)hipHostFree(ctx->fold_own);
+  ctx->pinned.release();
   for (auto& r : ctx->prof) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
   for (auto e : ctx->ev_pool) (void)hipEventDestroy(e);
   (void)hipStreamDestroy(ctx->stream);
@@ -997,11 +993,9 @@ extern "C" int tgx_compute(tgx_ctx* ctx, int path, double* energy, double* viria
     // every block's network first; its last kernel leaves the gate counters in
     // pinned memory
     if (ctx->gate_host_n < 2 * nm) {
-      if (ctx->gate_host) (void)hipHostFree(ctx->gate_host);
-      ctx->gate_host = nullptr;
-      ctx->gate_host_n = 0;
-      TGX_CHECK_HIP(hipHostMalloc((void**)&ctx->gate_host, sizeof(int) * 2 * nm, hipHostMallocDefault));
-      ctx->gate_host_n = 2 * nm;
+      const int want = std::max(2 * nm, 2 * ctx->gate_host_n);
+      TGX_TRY(ctx->pinned.take(&ctx->gate_host, (size_t)want));
+      ctx->gate_host_n = want;
     }
     for (int k = 0; k < nm; ++k) {
       tgx_model_t* m = ctx->models[k];

@@ -50,6 +50,10 @@ static inline int64_t tgx_round_up(int64_t x, int64_t g) { return (x + g - 1) / 
 // the faster one there; at most 127 rows more work).
 static inline int tgx_rows_bf16(int64_t ns) { return (int)tgx_round_up(ns, ns >= 4096 ? 256 : 128); }
 
+// Atoms whose results (36 bytes each) are kept in the context's first chunk of
+// pinned memory, beside the 37 KB of the force gather.
+constexpr int TGX_FOLD_POOL = 2048;
+
 // Growable device buffer.
 struct dbuf {
   void* p = nullptr;
@@ -86,6 +90,40 @@ struct dbuf {
     bytes = 0;
   }
   template <class T> T* as() const { return reinterpret_cast<T*>(p); }
+};
+
+// Pinned host memory of a context, handed out in pieces that live as long as it
+// does: the words and small arrays that kernels leave for the host. A pinned
+// allocation costs tens of microseconds and its release some 250 us, so a small
+// system's context makes one of them (two blocks of 1,009 atoms, mixed path: a
+// new context's first list, step and results 540 -> 400 us against one
+// allocation per word or array, its release 1,150 -> 330).
+struct pinned_pool {
+  static constexpr size_t CHUNK = 128 * 1024;
+  std::vector<void*> chunks;
+  char* at = nullptr;
+  size_t left = 0;
+  template <class T> int take(T** out, size_t n) {
+    const size_t bytes = ((n ? n : 1) * sizeof(T) + 127) & ~(size_t)127;
+    if (bytes > left) {
+      void* c = nullptr;
+      const size_t want = bytes > CHUNK ? bytes : CHUNK;
+      TGX_CHECK_HIP(hipHostMalloc(&c, want, hipHostMallocDefault));
+      chunks.push_back(c);
+      at = static_cast<char*>(c);
+      left = want;
+    }
+    *out = reinterpret_cast<T*>(at);
+    at += bytes;
+    left -= bytes;
+    return TGX_OK;
+  }
+  void release() {
+    for (void* c : chunks) (void)hipHostFree(c);
+    chunks.clear();
+    at = nullptr;
+    left = 0;
+  }
 };
 
 // Per-species SOAP parameters as the kernels see them (lengths in Å unless
@@ -163,7 +201,7 @@ struct tgx_model_t {
   dbuf sel_scratch; // block selection: flags, pair counts and their scans
   dbuf scan_tmp;    // block totals of the selection scans
   dbuf pair_site;   // int[n_pairs_b]: centre of every kept pair (plain force pass)
-  int64_t* sel_host = nullptr;  // pinned: the selection's site and pair totals
+  int64_t* sel_host = nullptr;  // the context's pinned memory: the selection's site and pair totals
   int sel_lo = 0, sel_hi = -1;  // centres are taken from atoms [sel_lo, sel_hi) only (sel_hi < 0: all)
   bool der_whole = false;       // soap_der holds dq/dr of every centre of the block (last FP64 plain evaluation)
   dbuf mlp_ws;      // surrogate work space (activations, member energies)
@@ -237,20 +275,23 @@ struct tgx_ctx {
   dbuf md_cm;                  // centre-of-mass partial sums
   bool gd_started = false, gd_backtracking = false, gd_initialized = false;
   double gd_energy0 = 0.0, gd_gamma_prev = 0.0, gd_m_prev = 0.0, gd_gamma_back0 = 0.0;
-  int* md_flag_host = nullptr;  // pinned
+  int* md_flag_host = nullptr;  // in pinned
   double dt_prev = 0.0;
   // surrogate gate
   int gate_members = 1;
   double gate_threshold = 1e30;
   double gated_fraction = 0.0, max_spread = 0.0;  // over every block of the last tgx_compute
   int64_t gate_sites = 0, gate_gated = 0;
-  int* gate_host = nullptr;  // pinned: {count, max spread bits} of every block
-  double* red_host = nullptr;  // pinned: virial and energy partials of the force gather
-  int gather_parts[2] = {0, 0};   // virial and energy partials of the last gather
-  double* fold_host = nullptr;    // pinned: a block's forces, energies and atom marks (get_gap_soap)
-  int fold_n = 0;
-  int64_t* pairs_host = nullptr;  // pinned: the list build's pair count
+  // host words and arrays that kernels write, in pinned unless said otherwise
+  pinned_pool pinned;
+  int* gate_host = nullptr;  // {count, max spread bits} of every block
   int gate_host_n = 0;
+  double* red_host = nullptr;  // virial and energy partials of the force gather
+  int gather_parts[2] = {0, 0};   // virial and energy partials of the last gather
+  double* fold_host = nullptr;    // a block's forces, energies and atom marks (get_gap_soap, get_results)
+  int fold_n = 0;                 // atoms it holds
+  void* fold_own = nullptr;       // its own pinned allocation, above TGX_FOLD_POOL atoms
+  int64_t* pairs_host = nullptr;  // the list build's pair count
   dbuf gate_mask;
   int block_streams = 1;           // blocks of distinct central species on streams of their own: 0 off, 1 default, 2 every path
   // profiling
@@ -318,6 +359,8 @@ int tgx_plain_pair_forces_q(tgx_ctx* ctx, tgx_model_t* m, const double* qss);
 // compressed blocks: q64 / soap_der from qf64 / derf, and qssf64 from qss64
 int tgx_compress_descriptors(tgx_ctx* ctx, tgx_model_t* m, bool with_der);
 int tgx_compress_gradient(tgx_ctx* ctx, tgx_model_t* m);
+// The pinned array of the partials, red_host, on first use.
+int tgx_red_host(tgx_ctx* ctx);
 int tgx_gather_forces(tgx_ctx* ctx, double* energy_out, double* virial_out);
 // tgx_gather_forces without its wait: the launch, and, once the caller has
 // synchronised the stream, the check and the virial.

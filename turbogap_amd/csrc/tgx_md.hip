@@ -521,7 +521,7 @@ extern "C" int tgx_md_displacement(tgx_ctx* ctx, double neighbors_buffer, int re
   const int n = ctx->n_sites;
   TGX_TRY(ctx->md_disp.ensure(sizeof(double) * 3 * (size_t)n));
   TGX_TRY(ctx->md_flag.ensure(sizeof(int)));
-  if (!ctx->md_flag_host) TGX_CHECK_HIP(hipHostMalloc((void**)&ctx->md_flag_host, sizeof(int), hipHostMallocDefault));
+  if (!ctx->md_flag_host) TGX_TRY(ctx->pinned.take(&ctx->md_flag_host, 1));
   if (reset) {
     TGX_TRY(tgx_zero(ctx, ctx->md_disp.p, sizeof(double) * 3 * (size_t)n));
     *rebuild = 0;
@@ -577,10 +577,7 @@ extern "C" int tgx_md_advance(tgx_ctx* ctx, double dt, int first_step, int remov
     TGX_LAUNCH(ctx, "md_disp", k_disp, dim3((n + 255) / 256), dim3(256), 0, n, b[0], b[4], b[8], ctx->pos.as<double>(),
                ctx->pos_prev.as<double>(), ctx->md_disp.as<double>(), lim * lim, flag);
   }
-  if (!ctx->red_host) {
-    const size_t nred = 9 * 512 + (size_t)TGX_SUM_PARTS + 1;
-    TGX_CHECK_HIP(hipHostMalloc((void**)&ctx->red_host, sizeof(double) * nred, hipHostMallocDefault));
-  }
+  TGX_TRY(tgx_red_host(ctx));
   TGX_CHECK_HIP(hipMemcpyAsync(ctx->red_host, part, sizeof(double) * (TGX_SUM_PARTS + 1), hipMemcpyDeviceToHost,
                                ctx->stream));
   TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));

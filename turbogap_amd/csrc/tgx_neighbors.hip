@@ -624,8 +624,7 @@ int tgx_neighbors_run(tgx_ctx* ctx, double rcut_max, const int* indices, const i
     TGX_LAUNCH(ctx, "nbr_count_brute", k_brute_neigh<0>, wgrid, wblk, 0, n, n_sc, ctx->pos.as<double>(), bx, rcut_max,
                d_do, ctx->species_sc.as<int>(), ctx->n_neigh.as<int>(), nullptr, nullptr, nullptr, nullptr, nullptr);
   }
-  if (!ctx->pairs_host)
-    TGX_CHECK_HIP(hipHostMalloc((void**)&ctx->pairs_host, sizeof(int64_t), hipHostMallocDefault));
+  if (!ctx->pairs_host) TGX_TRY(ctx->pinned.take(&ctx->pairs_host, 1));
   TGX_TRY(tgx_scan_i32(ctx, ctx->n_neigh.as<int>(), ctx->nl_off.as<int64_t>(), n, ctx->pairs_host));
   TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   const int64_t P = *ctx->pairs_host;

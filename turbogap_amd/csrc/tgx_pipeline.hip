@@ -268,7 +268,7 @@ int tgx_blocks_select_count(tgx_ctx* ctx, tgx_model_t* const* models, int count)
       tgx_model_t* m = models[k0 + k];
       // the block's own scratch: blocks may be selected while another block's kernels still run
       TGX_TRY(m->sel_scratch.ensure(sizeof(int) * 2 * (size_t)n + sizeof(int64_t) * 2 * (size_t)(n + 1) + 256));
-      if (!m->sel_host) TGX_CHECK_HIP(hipHostMalloc((void**)&m->sel_host, 2 * sizeof(int64_t), hipHostMallocDefault));
+      if (!m->sel_host) TGX_TRY(ctx->pinned.take(&m->sel_host, 2));
       const SelectView v = select_view(m, n);
       const int lo = m->sel_lo > 0 ? m->sel_lo : 0, hi = (m->sel_hi >= 0 && m->sel_hi < n) ? m->sel_hi : n;
       st.t[k] = SelectTask{species_map(m), lo, hi, m->central_species, m->rcut_max, v.flag, v.npairs};
@@ -333,11 +333,15 @@ int tgx_gather_forces(tgx_ctx* ctx, double* energy_out, double* virial_out) {
                                 ctx->energies.as<double>(), energy_out);
 }
 
-// Layout of ctx->red_host (pinned): VIRIAL_PARTS x 9 virial partials,
-// TGX_SUM_PARTS energy partials, the missing-reverse flag.
+// ctx->red_host: VIRIAL_PARTS x 9 virial partials, TGX_SUM_PARTS energy partials,
+// the missing-reverse flag.
+int tgx_red_host(tgx_ctx* ctx) {
+  if (ctx->red_host) return TGX_OK;
+  return ctx->pinned.take(&ctx->red_host, 9 * (size_t)VIRIAL_PARTS + TGX_SUM_PARTS + 1);
+}
+
 static int gather_launch(tgx_ctx* ctx, const double* fglob, double* F, bool with_virial, const double* d_energies) {
-  const size_t nred = 9 * (size_t)VIRIAL_PARTS + TGX_SUM_PARTS + 1;
-  if (!ctx->red_host) TGX_CHECK_HIP(hipHostMalloc((void**)&ctx->red_host, sizeof(double) * nred, hipHostMallocDefault));
+  TGX_TRY(tgx_red_host(ctx));
   FinishArgs a;
   a.n = ctx->n_sites;
   a.P = ctx->n_pairs;
@@ -450,13 +454,24 @@ __global__ void k_fold_out(int n, const double* __restrict__ F, const double* __
 
 int tgx_fold_out(tgx_ctx* ctx, const double* F, const int* d_mark) {
   const int n = ctx->n_sites;
-  if (ctx->fold_n < n) {
-    if (ctx->fold_host) (void)hipHostFree(ctx->fold_host);
-    ctx->fold_host = nullptr;
+  constexpr size_t row = sizeof(double) * 4 + sizeof(int);
+  if (ctx->fold_n < n && n <= TGX_FOLD_POOL) {
+    TGX_TRY(ctx->pinned.take(reinterpret_cast<char**>(&ctx->fold_host), row * TGX_FOLD_POOL));
+    ctx->fold_n = TGX_FOLD_POOL;
+  } else if (ctx->fold_n < n) {
+    // a size that rises again gets 25% headroom, as the device buffers: releasing it costs 250 us
+    int want = ctx->fold_own ? n + n / 4 : n;
+    if (ctx->fold_own) (void)hipHostFree(ctx->fold_own);
+    ctx->fold_own = ctx->fold_host = nullptr;
     ctx->fold_n = 0;
-    TGX_CHECK_HIP(hipHostMalloc((void**)&ctx->fold_host, (sizeof(double) * 4 + sizeof(int)) * (size_t)n,
-                                hipHostMallocDefault));
-    ctx->fold_n = n;
+    if (want > n && hipHostMalloc(&ctx->fold_own, row * (size_t)want, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->fold_own = nullptr;
+      want = n;
+    }
+    if (!ctx->fold_own) TGX_CHECK_HIP(hipHostMalloc(&ctx->fold_own, row * (size_t)n, hipHostMallocDefault));
+    ctx->fold_host = static_cast<double*>(ctx->fold_own);
+    ctx->fold_n = want;
   }
   TGX_LAUNCH(ctx, "fold_out", k_fold_out, dim3((n + 255) / 256), dim3(256), 0, n, F, ctx->energies.as<double>(), d_mark,
              ctx->fold_host);
