@@ -83,3 +83,27 @@ def test_noalloc_matches_allocating_entry(ctx, orc):
         None) == 1
     assert b"16384" in L.load().tgx_last_error() or b"16,384" in L.load().tgx_last_error()
     ctx.soap_backend_end()
+
+
+# one launch a scan of the offsets up to 8,192 sites, two up to the entry's limit
+@pytest.mark.parametrize("n", [8192, 8193, 16384])
+def test_noalloc_scans_of_many_sites(ctx, n):
+    from turbogap_amd import structures as S
+    rng = np.random.default_rng(n)
+    h = S.soap_hypers([S.CARBON], n_max=4, l_max=4)
+    q = rng.random((n, h.dim))
+    q /= np.linalg.norm(q, axis=1)[:, None]
+    nn = rng.integers(1, 4, n).astype(np.int32)
+    P = int(nn.sum())
+    der, xyz = rng.normal(size=(P, h.dim, 3)), rng.normal(size=(P, 3))
+    nlist = rng.integers(1, n + 1, P)
+    ctx.set_system(np.zeros((1, 3)), np.full(1, S.CARBON, np.int32), S.cubic_box(20.0))
+    ctx.soap_backend_begin(ctx.soap_model(h, q[:100], rng.normal(size=100)))
+    e_ref, f_ref, w_ref = ctx.get_soap_energy_and_forces(q, der, nn, nlist, xyz, n)
+    dev = _Device()
+    e, f, w = _noalloc(ctx, dev, h, q, der, nn, nlist, xyz, n)
+    dev.free()
+    ctx.soap_backend_end()
+    assert np.array_equal(e, e_ref) and np.array_equal(f, f_ref) and np.abs(f).max() > 0.0
+    # a sum of P terms of either sign in another order
+    assert np.abs(w - w_ref).max() <= 2.0 ** -53 * P * np.abs(f_ref).max() * np.abs(xyz).max()

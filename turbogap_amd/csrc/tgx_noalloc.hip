@@ -28,7 +28,7 @@
 
 #define TGX_NOALLOC_SCRATCH_BYTES (64u << 20)
 #define TGX_NOALLOC_MAX_DEVICES 64
-#define TGX_NOALLOC_MAX_SITES 16384  // one-workgroup scans of the offsets
+#define TGX_NOALLOC_MAX_SITES 16384
 
 static __device__ __align__(256) unsigned char scratch[TGX_NOALLOC_SCRATCH_BYTES];
 
@@ -38,6 +38,9 @@ std::mutex g_scratch_mu;
 void* g_scratch[TGX_NOALLOC_MAX_DEVICES] = {};
 
 constexpr int VIR_PARTS = 256;
+// words of the offsets' scans: enough for every site count that is taken, so that the
+// scan, given a view of them, finds its buffer large enough and never allocates
+constexpr int64_t SCAN_WORDS = tgx_scan_tmp_words(TGX_NOALLOC_MAX_SITES);
 
 // q_pad[i][d] = soap[i][d] for i < ns, d < D, zero in the padding (rows up to Mp,
 // columns up to Dp).
@@ -219,9 +222,9 @@ extern "C" int tgx_get_soap_energy_and_forces_noalloc(tgx_ctx* ctx, int n_sites,
   int* cnt = cv.take<int>((size_t)n0);
   double* fpair = cv.take<double>(3 * (size_t)P);
   double* vpart = cv.take<double>(9 * (size_t)VIR_PARTS);
-  dbuf scan_sums;  // a view (never ensured past its size: one-workgroup scans)
-  scan_sums.p = cv.take<int64_t>(64);
-  scan_sums.bytes = 64 * sizeof(int64_t);
+  dbuf scan_sums;  // a view, not owned
+  scan_sums.p = cv.take<int64_t>(SCAN_WORDS);
+  scan_sums.bytes = SCAN_WORDS * sizeof(int64_t);
   TGX_REQUIRE(cv.used <= TGX_NOALLOC_SCRATCH_BYTES,
               "tgx_get_soap_energy_and_forces_noalloc: %d sites, %lld pairs need %zu bytes of work space, more than "
               "the %u bytes this entry point has (split the sites into smaller calls)",

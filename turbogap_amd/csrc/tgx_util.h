@@ -15,6 +15,9 @@ int tgx_scan_i32(tgx_ctx* ctx, const int* in, int64_t* out, int64_t n, int64_t* 
 // The same for several arrays of n values at once (one launch for all of them up
 // to 8,192 values, two up to 65,536, three each above).
 constexpr int TGX_SCAN_TASKS = 16;
+constexpr int TGX_SCAN_BLOCK = 1024;  // values whose total is one word of tmp
+// Words of tmp that the scan of one array of n values uses, whatever its launches.
+constexpr int64_t tgx_scan_tmp_words(int64_t n) { return (n + TGX_SCAN_BLOCK - 1) / TGX_SCAN_BLOCK + 2; }
 struct tgx_scan_task {
   const int* in;
   int64_t* out;

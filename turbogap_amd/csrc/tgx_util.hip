@@ -5,7 +5,7 @@
 
 namespace {
 
-constexpr int SCAN_BLOCK = 1024;
+constexpr int SCAN_BLOCK = TGX_SCAN_BLOCK;
 constexpr int64_t SCAN_SINGLE_MAX = 8 * 1024;  // one workgroup scans up to this many values (8,192: 6 us; 16,001: 18, in two launches 10)
 
 __global__ void k_fill_zero(uint32_t* __restrict__ p, size_t n_words) {
@@ -244,7 +244,7 @@ int tgx_scan_many(tgx_ctx* ctx, const tgx_scan_tasks& ts, int count, int64_t n, 
                (const int64_t*)sb.as<int64_t>());
   } else {
     // one after the other, all through the same block totals
-    if (n > 0) TGX_TRY(sb.ensure(sizeof(int64_t) * (size_t)(nb + 2)));
+    if (n > 0) TGX_TRY(sb.ensure(sizeof(int64_t) * (size_t)tgx_scan_tmp_words(n)));
     for (int k = 0; k < count; ++k) {
       const tgx_scan_task& t = ts.t[k];
       if (n > 0) {
