@@ -8,10 +8,11 @@ from turbogap_amd import structures as S
 pytestmark = pytest.mark.gpu
 
 
-# atoms (half of them a block's centres), sparse points: 128 x 128 tiles per block of the kernel and
-# Qss products are (4, 20), (63, 70), (128, 160), (384 with 24 columns, 170), (1,184, 360), (2,304, 720)
-@pytest.mark.parametrize("n,n_sparse", [(300, 200), (1700, 1100), (4000, 1000), (4300, 3000), (9100, 4000),
-                                        (18300, 4000)])
+# atoms (half of them a block's centres), sparse points: 128 x 128 tiles per block of the kernel and Qss
+# products are (4, 20), (63, 70), (128, 160), (408, 170), (1,056, 330) with an odd number of 128-row tiles,
+# (1,152, 360) and (2,304, 720) with an even one
+@pytest.mark.parametrize("n,n_sparse", [(300, 200), (1700, 1100), (4000, 1000), (4300, 3000), (8300, 4000),
+                                        (9100, 4000), (18300, 4000)])
 def test_mixed_matches_fp64(n, n_sparse):
     from turbogap_amd import Context
     rng = np.random.default_rng(n)

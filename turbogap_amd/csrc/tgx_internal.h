@@ -46,9 +46,11 @@ void tgx_set_error(const char* fmt, ...);
 static inline int64_t tgx_round_up(int64_t x, int64_t g) { return (x + g - 1) / g * g; }
 
 // Rows of a block's arrays that the BF16 products read or write, for ns centres:
-// whole 128-row tiles, and from 4,096 on whole 256-row ones (the wider tile is
-// the faster one there; at most 127 rows more work).
-static inline int tgx_rows_bf16(int64_t ns) { return (int)tgx_round_up(ns, ns >= 4096 ? 256 : 128); }
+// whole 128-row tiles, and from 6,144 on whole 256-row ones, at most 127 rows more
+// work for the wider tile (two blocks of 4,000 sparse points, a mixed step with
+// 128-row and with 256-row padding: 0.558 and 0.572 ms at 4,100 centres, 0.728 and
+// 0.726 at 6,200, 0.930 and 0.920 at 8,200, 1.67 and 1.58 at 16,500).
+static inline int tgx_rows_bf16(int64_t ns) { return (int)tgx_round_up(ns, ns >= 6144 ? 256 : 128); }
 
 // Atoms whose results (36 bytes each) are kept in the context's first chunk of
 // pinned memory, beside the 37 KB of the force gather.
