@@ -886,9 +886,11 @@ static int launch_f64_few(tgx_ctx* ctx, const char* name, int M, int N, int K, c
 // rule. shared: another block's kernels run beside this one and take the CUs a
 // last round leaves idle, so that the wide tile pays earlier (two blocks of
 // 8,000 centres, FP64 adjoint step: 11.33 ms with 64 x 64 tiles, 11.08 with 128 x
-// 128, although alone the latter's 630 tiles take 2.06 ms against 1.39). Every
-// tile adds an element's products in the same order, so the results do not
-// depend on it.
+// 128, although alone the latter's 630 tiles take 2.06 ms against 1.39). The tiles
+// of 64 and 128 rows add an element's products in the same order, so that results
+// do not depend on which of them, or on shared; the kernel that splits K adds its
+// wavefronts' partial sums, another order, so they change in the last bits with the
+// row count at its line.
 template <int EPI, bool ZINT>
 static int launch_f64(tgx_ctx* ctx, bool shared, int M, int N, int K, const double* A, int lda, const double* B,
                       int ldb, EpiArgs e, const char* name) {

@@ -680,8 +680,10 @@ __global__ __launch_bounds__(WG, 2) void k_soap_der(SoapParams P, SiteArgs a, in
     if (code[j] >= 0) out[tid + WG * j] = self[j];
 }
 
-// ---- The same dq/dr for a compile-time l_max and at most two species of at
-// most eight radial functions each (16 stacked rows).
+// ---- The same dq/dr, and FP64 descriptors and adjoint forces, for l_max = 8 and at
+// most two species of at most eight radial functions each (16 stacked rows). LL
+// names the 8 in sizes and indexes; the degree sets of der_lm, the calls of
+// der_channel and the (l, m) tiles of l_channel are laid out for it alone.
 
 template <int LL> struct DerL {
   static constexpr int L1 = LL + 1, NLM = L1 * L1, NL = 16 * L1, D = 16 * 17 / 2 * L1;
@@ -1008,6 +1010,7 @@ __device__ __forceinline__ double l_spectrum(const SoapParams& P, const LSite<LL
 // (l, m) 64..79 and 80 of l = 8.
 template <int LL>
 __device__ __forceinline__ void l_channel(const SoapParams& P, const LSite<LL>& S, const double* X) {
+  static_assert(LL == 8, "degree 8 takes two tiles, the others one");
   using G = DerL<LL>;
   constexpr int L1 = G::L1, CP = G::CP;
   const int w = S.w, li = S.li, lg = S.lg, N = P.N;
@@ -1050,7 +1053,7 @@ __device__ __forceinline__ void l_harmonics(const LSite<LL>& S, int g, int cnt, 
   }
 }
 
-// Plain-path dq/dr for l_max = LL (the output and element layout of
+// Plain-path dq/dr for l_max = 8 (the output and element layout of
 // k_soap_der), one workgroup per site.
 //   * Pairs are prepared 32 at a time, eight lanes each (der_prepare), and their
 //     harmonics 16 at a time, a row of lanes each: with a wavefront per pair, five or
@@ -1219,7 +1222,7 @@ __global__ __launch_bounds__(WG, 2) void k_soap_der_l(SoapParams P, SiteArgs a, 
   }
 }
 
-// FP64 descriptors for l_max = LL by the first half of k_soap_der_l, one workgroup
+// FP64 descriptors for l_max = 8 by the first half of k_soap_der_l, one workgroup
 // per site (listed or in order): a wavefront per site prepared its pairs 16 at a
 // time with four lanes each and formed the rest in loops over LDS. Bound by the
 // preparation's chains at three workgroups a CU (its floor, the pairs read and the
@@ -1237,7 +1240,7 @@ __global__ __launch_bounds__(WG, 3) void k_desc_l(SoapParams P, SiteArgs a, int 
   l_spectrum<LL, J>(P, S, S.U + G::NLM * G::CP + 1, qd, q_out + (size_t)row * P.Dpad, pnorm_out + row);
 }
 
-// FP64 adjoint pair forces for l_max = LL, one workgroup per site: c as above, H from
+// FP64 adjoint pair forces for l_max = 8, one workgroup per site: c as above, H from
 // g = (Qss - (Qss . q) q) / |p|, then sixteen pairs at a time: x = sum_n R_n H(n, lm) and
 // y = sum_n R_n' H(n, lm) of all of them on the FP64 matrix cores, one (l, m) tile after
 // the other, and
