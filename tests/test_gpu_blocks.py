@@ -113,3 +113,40 @@ def test_results_of_systems_of_changing_size():
             # the same calls on the same numbers: whether the context is new does not matter
             assert all(np.array_equal(a, b) for a, b in zip(got, want)), n
             assert abs(got[0] - got[1].sum()) <= 1e-12 * np.abs(got[1]).sum()
+
+
+# a block assigns the energies of its centres and the forces of the atoms its pairs reach, and nothing else,
+# in one batch and in several
+@pytest.mark.parametrize("n,budget", [(400, 0.0), (3000, 0.0), (3000, 0.05)])
+def test_get_gap_soap_assigns_what_the_block_touches(n, budget):
+    from turbogap_amd import Context
+    rng = np.random.default_rng(n)
+    sysm = S.binary_system(n, seed=n)
+    pos, box = np.vstack([sysm.positions, sysm.box.diagonal() + 20.0]), sysm.box + np.diag([40.0, 40.0, 40.0])
+    species = np.append(sysm.species, S.SPECIES_B).astype(np.int32)  # the last atom is alone and no centre
+    h = S.soap_binary()[0]
+    Qs = rng.random((5, h.dim))
+    Qs /= np.linalg.norm(Qs, axis=1, keepdims=True)
+    al = rng.normal(scale=1e-2, size=5)
+    with Context(0) as ctx:
+        ctx.set_system(pos, species, box)
+        nl = ctx.build_neighbors_list(3.7)
+        ctx.soap_backend_begin(ctx.soap_model(h, Qs, al))
+        ctx.set_memory_budget(budget)
+        e, f = np.full(n + 1, 7.0), np.full((n + 1, 3), 7.0)
+        _, _, w, ns, _ = ctx.get_gap_soap("fp64_plain", energies=e, forces=f)
+        e2, f2 = np.full(n + 1, 7.0), np.full((n + 1, 3), 7.0)
+        _, _, w2, ns2, _ = ctx.get_gap_soap("fp64_plain", do_forces=False, energies=e2, forces=f2)
+        E, W = ctx.compute("fp64_adjoint")
+        e3, f3 = ctx.results()
+    centre = species == S.SPECIES_A
+    reached = np.zeros(n + 1, bool)
+    first = np.concatenate([[0], np.cumsum(nl["n_neigh"])])
+    for i in np.flatnonzero(centre):
+        near = nl["rjs"][first[i]:first[i + 1]] < h.rcut_max
+        reached[(nl["neighbors_list"][first[i]:first[i + 1]][near] - 1) % (n + 1)] = True
+    assert ns == ns2 == centre.sum() and not reached[n]
+    for en in (e, e2):
+        assert (en[~centre] == 7.0).all() and np.abs(en - e3)[centre].max() <= 1e-13
+    assert (f[~reached] == 7.0).all() and np.abs(f - f3)[reached].max() <= 1e-10 and (f2 == 7.0).all()
+    assert np.abs(w - W).max() <= 1e-10 * n and not w2.any()

@@ -10,8 +10,9 @@
 
 int tgx_energy_scatter(tgx_ctx* ctx, tgx_model_t* m);
 int tgx_energy_scatter_blocks(tgx_ctx* ctx, tgx_model_t* const* models, int count);
-int tgx_block_seen(tgx_ctx* ctx, tgx_model_t* m, int* d_mark);
-int tgx_fold_out(tgx_ctx* ctx, const double* F, const int* d_mark);
+int tgx_fold_ensure(tgx_ctx* ctx);
+int tgx_fold_sites(tgx_ctx* ctx, tgx_model_t* m, int first, int* d_mark);
+int tgx_fold_out(tgx_ctx* ctx, const double* energies, const int* d_mark);
 int tgx_radial_table_build(tgx_ctx* ctx, tgx_model_t* m);
 
 
@@ -639,10 +640,11 @@ static int plain_batches(tgx_ctx* ctx, tgx_model_t* m, int lo, int hi, std::vect
 
 // A block's energies and pair forces over the centres of atoms [lo, hi),
 // batched by the memory budget on the FP64 plain path. Energies are added into
-// the context's per-atom energies and pair forces into fglob. d_mark (device,
-// may be null) marks the atoms the block touches. Runs on ctx->stream.
-static int run_block_range(tgx_ctx* ctx, tgx_model_t* m, int path, bool do_forces, int lo, int hi, int* d_mark,
-                           int* n_sites_tot, int64_t* n_pairs_tot) {
+// the context's per-atom energies and pair forces into fglob. With fold, the
+// centres' atoms and energies are left in fold_host and d_mark (device, may be
+// null) marks the atoms the pairs reach. Runs on ctx->stream.
+static int run_block_range(tgx_ctx* ctx, tgx_model_t* m, int path, bool do_forces, int lo, int hi, bool fold,
+                           int* d_mark, int* n_sites_tot, int64_t* n_pairs_tot) {
   const int save_lo = m->sel_lo, save_hi = m->sel_hi;
   struct Restore {
     tgx_model_t* m;
@@ -668,9 +670,9 @@ static int run_block_range(tgx_ctx* ctx, tgx_model_t* m, int path, bool do_force
     TGX_TRY(tgx_block_select_fill(ctx, m));
     TGX_TRY(run_selected_block(ctx, m, path, do_forces));
     TGX_TRY(tgx_energy_scatter(ctx, m));
+    if (fold) TGX_TRY(tgx_fold_sites(ctx, m, ns_tot, d_mark));
     ns_tot += m->n_sites_b;
     np_tot += m->n_pairs_b;
-    if (d_mark) TGX_TRY(tgx_block_seen(ctx, m, d_mark));
   }
   if (n_sites_tot) *n_sites_tot = ns_tot;
   if (n_pairs_tot) *n_pairs_tot = np_tot;
@@ -694,25 +696,32 @@ static int get_gap_soap_impl(tgx_ctx* ctx, int path, int do_forces, int lo, int 
   TGX_TRY(begin_step(ctx));
   const int n = ctx->n_sites;
   TGX_REQUIRE(lo >= 0 && lo <= hi && hi <= n, "tgx_get_gap_soap: sites [%d, %d) outside [0, %d)", lo, hi, n);
-  TGX_TRY(ctx->gate_mask.ensure(sizeof(int) * 2 * (size_t)n));
-  int* mark = ctx->gate_mask.as<int>();
-  TGX_TRY(tgx_zero(ctx, mark, sizeof(int) * 2 * (size_t)n));
+  TGX_TRY(tgx_fold_ensure(ctx));
+  int* mark = nullptr;
+  if (do_forces) {
+    TGX_TRY(ctx->gate_mask.ensure(sizeof(int) * (size_t)n));
+    mark = ctx->gate_mask.as<int>();
+    TGX_TRY(tgx_zero(ctx, mark, sizeof(int) * (size_t)n));
+  }
   int ns_b = 0;
   int64_t np_b = 0;
-  TGX_TRY(run_block_range(ctx, m, path, do_forces != 0, lo, hi, mark, &ns_b, &np_b));
+  TGX_TRY(run_block_range(ctx, m, path, do_forces != 0, lo, hi, true, mark, &ns_b, &np_b));
   double vir[9] = {0};
-  if (do_forces) TGX_TRY(tgx_gather_forces_launch(ctx));
-  TGX_TRY(tgx_fold_out(ctx, do_forces ? ctx->forces.as<double>() : nullptr, mark));
+  if (do_forces) {
+    TGX_TRY(tgx_gather_forces_launch(ctx));
+    TGX_TRY(tgx_fold_out(ctx, nullptr, mark));
+  }
   TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   if (do_forces) TGX_TRY(tgx_gather_collect(ctx, vir, nullptr));
   // fold back like src/gap_interface.f90:422-431: assign, for touched atoms only
   const double *F = ctx->fold_host, *E = F + 3 * (size_t)n;
-  const int* touched = reinterpret_cast<const int*>(E + n);
-  for (int i = 0; i < n; ++i) {
-    if (energies && (touched[i] & 2)) energies[i] = E[i];
-    if (do_forces && forces && (touched[i] & 1))
-      for (int k = 0; k < 3; ++k) forces[3 * (size_t)i + k] = F[3 * (size_t)i + k];
-  }
+  const int *atom = reinterpret_cast<const int*>(E + n), *touched = atom + n;
+  if (energies)
+    for (int s = 0; s < ns_b; ++s) energies[atom[s]] = E[s];
+  if (do_forces && forces)
+    for (int i = 0; i < n; ++i)
+      if (touched[i])
+        for (int k = 0; k < 3; ++k) forces[3 * (size_t)i + k] = F[3 * (size_t)i + k];
   if (virial)
     for (int k = 0; k < 9; ++k) virial[k] = vir[k];
   if (n_sites_block) *n_sites_block = ns_b;
@@ -1029,7 +1038,7 @@ extern "C" int tgx_compute(tgx_ctx* ctx, int path, double* energy, double* viria
       ctx->stream = block_stream(m);
       if (path == TGX_PATH_FP64_PLAIN && plain_block_bytes(m, m->sel_host[0], m->sel_host[1]) > budget) {
         // dq/dr of the whole block does not fit: its centres in memory-bounded batches
-        TGX_TRY(run_block_range(ctx, m, path, true, 0, ctx->n_sites, nullptr, nullptr, nullptr));
+        TGX_TRY(run_block_range(ctx, m, path, true, 0, ctx->n_sites, false, nullptr, nullptr, nullptr));
       } else {
         TGX_TRY(tgx_block_select_fill(ctx, m));
         TGX_TRY(run_selected_block(ctx, m, path, true));
@@ -1055,8 +1064,9 @@ extern "C" int tgx_get_results(tgx_ctx* ctx, double* energies, double* forces) {
   if (n <= 16384) {
     // through pinned memory, one launch and one wait, against two copies: 17 us for 47 at 1,009 atoms, 21 for 73
     // at 4,096, 26 for 31 at 8,192, 39 for 41 at 16,384; above, up to 65,536 atoms (120 for 126), too little
-    // between them to hold 36 bytes of pinned memory an atom
-    TGX_TRY(tgx_fold_out(ctx, ctx->forces.as<double>(), nullptr));
+    // between them to hold 40 bytes of pinned memory an atom
+    TGX_TRY(tgx_fold_ensure(ctx));
+    TGX_TRY(tgx_fold_out(ctx, ctx->energies.as<double>(), nullptr));
     TGX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     if (forces) std::memcpy(forces, ctx->fold_host, sizeof(double) * 3 * n);
     if (energies) std::memcpy(energies, ctx->fold_host + 3 * n, sizeof(double) * n);

@@ -52,7 +52,7 @@ static inline int64_t tgx_round_up(int64_t x, int64_t g) { return (x + g - 1) / 
 // 0.726 at 6,200, 0.930 and 0.920 at 8,200, 1.67 and 1.58 at 16,500).
 static inline int tgx_rows_bf16(int64_t ns) { return (int)tgx_round_up(ns, ns >= 6144 ? 256 : 128); }
 
-// Atoms whose results (36 bytes each) are kept in the context's first chunk of
+// Atoms whose results (40 bytes each) are kept in the context's first chunk of
 // pinned memory, beside the 37 KB of the force gather.
 constexpr int TGX_FOLD_POOL = 2048;
 
@@ -290,7 +290,7 @@ struct tgx_ctx {
   int gate_host_n = 0;
   double* red_host = nullptr;  // virial and energy partials of the force gather
   int gather_parts[2] = {0, 0};   // virial and energy partials of the last gather
-  double* fold_host = nullptr;    // a block's forces, energies and atom marks (get_gap_soap, get_results)
+  double* fold_host = nullptr;    // results on their way to the caller (get_gap_soap, get_results)
   int fold_n = 0;                 // atoms it holds
   void* fold_own = nullptr;       // its own pinned allocation, above TGX_FOLD_POOL atoms
   int64_t* pairs_host = nullptr;  // the list build's pair count
