@@ -40,7 +40,8 @@ void* g_scratch[TGX_NOALLOC_MAX_DEVICES] = {};
 constexpr int VIR_PARTS = 256;
 // words of the offsets' scans: enough for every site count that is taken, so that the
 // scan, given a view of them, finds its buffer large enough and never allocates
-constexpr int64_t SCAN_WORDS = tgx_scan_tmp_words(TGX_NOALLOC_MAX_SITES);
+constexpr int64_t SCAN_WORDS = 64;
+static_assert(tgx_scan_tmp_words(TGX_NOALLOC_MAX_SITES) <= SCAN_WORDS, "the scans would grow a view");
 
 // q_pad[i][d] = soap[i][d] for i < ns, d < D, zero in the padding (rows up to Mp,
 // columns up to Dp).
