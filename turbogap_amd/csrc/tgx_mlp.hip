@@ -981,7 +981,9 @@ extern "C" int tgx_mlp_train(tgx_mlp* m, int n_train, int epochs, int batch, flo
       TGX_LAUNCH(ctx, "mlp_gather", k_gather_rows, dim3(batch), dim3(256), 0, batch, m->Dp, m->idx.as<int>(),
                  m->dq.as<float>(), m->de.as<double>(), m->bqb.as<__bf16>(), m->be.as<double>());
       double le = 0.0, lg = 0.0;
-      TGX_TRY(mlp_backward(m, batch, m->dq.as<float>(), m->dg.as<float>(), m->idx.as<int>(), w_e, w_g, (ep == epochs - 1) ? &le : nullptr, (ep == epochs - 1) ? &lg : nullptr));
+      const bool last = ep == epochs - 1;
+      TGX_TRY(mlp_backward(m, batch, m->dq.as<float>(), m->dg.as<float>(), m->idx.as<int>(), w_e, w_g,
+                           last ? &le : nullptr, last ? &lg : nullptr));
       TGX_TRY(adam_step(m, lr));
       le_sum += le;
       lg_sum += lg;
